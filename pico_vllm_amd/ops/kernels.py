@@ -225,7 +225,7 @@ def clipped_glu(gate_up: torch.Tensor, limit: float, alpha: float) -> torch.Tens
 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
              out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """float32 out = a @ w.T + bias with plain FMA.  a: [M, K] float32 or bfloat16 (rows may be
+    """float32 out = a @ w.T + bias in float32 products and sums.  a: [M, K] float32 or bfloat16 (rows may be
     strided), w: [N, K] float32."""
     _gpu(a, w, bias)
     M, K = a.shape
@@ -241,7 +241,9 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = No
     elif out.shape != (M, N) or out.dtype != torch.float32 or out.stride(1) != 1:
         raise KernelError("gemm_f32: out has the wrong shape or dtype")
     lib = library.core()
-    _check(lib, lib.pico_gemm_f32(_ptr(a), _dt(a), _ptr(w), _ptr(bias), _ptr(out), M, N, K,
+    n = lib.pico_gemm_f32_slabs(M, N, K)
+    slabs = torch.empty(n, M, N, dtype=torch.float32, device=a.device) if n else None
+    _check(lib, lib.pico_gemm_f32(_ptr(a), _dt(a), _ptr(w), _ptr(bias), _ptr(out), _ptr(slabs), M, N, K,
                                   a.stride(0) if M > 1 else K, w.stride(0), out.stride(0) if M > 1 else N, _stream()))
     return out
 

@@ -107,6 +107,24 @@ def test_gemm_f32(K, M, N, K_):
     assert torch.allclose(out3.cpu().double(), ab.double() @ w.double().T, rtol=1e-5, atol=1e-4)
 
 
+@pytest.mark.parametrize("M", [1, 31, 33, 64, 65])
+@pytest.mark.parametrize("N,K_", [(63, 3), (65, 33), (129, 255), (64, 256), (200, 260), (70, 1028), (33000, 516)])
+def test_gemm_f32_at_the_edges_of_tiles_and_ranges(K, M, N, K_):
+    # a row has the same bits in any call: alone or in tiles of 32 or 64 rows, its ranges of K in one workgroup (33,000
+    # columns) or in one each (fewer)
+    g = torch.Generator().manual_seed(M * K_)
+    a, w, b = (torch.randn(*s, generator=g).to(DEV) for s in ((M, K_), (N, K_), (N,)))
+    out = K.gemm_f32(a, w, b)
+    rows = slice(0, None) if N < 1000 else slice(N - 300, None)
+    want = a.cpu().double() @ w[rows].cpu().double().T
+    err = out[:, rows].cpu().double() - b[rows].cpu().double() - want
+    # the tree's bound (below) at four levels, and the bias's own rounding; five sigma for the largest
+    bound = (1.69 * 2 + 1) * 2.0 ** -24 * float((K_ + 1) ** 0.5)
+    assert float(err.abs().max()) <= 5 * bound
+    assert torch.equal(K.gemm_f32(a[M // 2:M // 2 + 1].contiguous(), w, b)[0], out[M // 2])
+    assert torch.equal(K.gemm_f32(a, w[rows].contiguous(), b[rows].contiguous()), out[:, rows])
+
+
 @pytest.mark.parametrize("K_", [64, 1000, 1536, 3584, 5120, 8960, 18944, 27648])
 def test_gemm_f32_rounding_does_not_grow_with_the_inner_size(K, K_):
     # The sums are trees of radix 16 with L = ceil(log16 K) levels (at most 4).  An addition rounds its partial sum
