@@ -1,0 +1,271 @@
+// Tiled bfloat16 product (prompt portions): C = X W^T (+ bias) and an epilogue, tiles as tile_stream.h has them, the tiles of
+// a call dealt out to workgroups that stay.  What an activation behind the library's product costs is a pass over [T, 2 I]
+// and back; here it is made of the sums in registers.  2,048 rows, 8,960 pairs, K 1,536: 115 us (0.98 PFLOP/s) against 117 and
+// 20 for product and pass; 832 rows, 18,944 pairs, K 3,584: 223 against 266 and 20; 65 rows of a 152,064 x 3,584 output matrix in
+// float32: 225 against 965 with the kernel for few rows (which reads the matrix once a 64 rows and unstaged).
+#include "tile_stream.h"
+
+// what becomes of the sums (the numbers are those of the weight-streaming product)
+#define GT_BF16 0     // + bias
+#define GT_F32 1      // + bias, float32
+#define GT_SWIGLU 2   // W = [gate rows; up rows]: silu(gate) up, N / 2 columns
+#define GT_RELU2 3    // max(x W^T + bias, 0)^2
+#define GT_CLIPPED 5  // W = [gate rows; up rows]: g sigmoid(alpha g) (u + 1), g = min(gate, limit), u = up within -limit .. limit
+#define GT_GELU 7     // gelu(x W^T + bias) with the error function
+
+struct GemmArgs {
+  const bf16_t* X;
+  const bf16_t* W;
+  const float* bias;
+  void* out;
+  int M, cols, K, ldx, ldw, ldo;     // cols: output columns of this launch
+  int up;                            // paired epilogues: from a gate row of W to the up row of the same column
+  int m_tiles, n_tiles;
+  float limit, alpha;
+};
+
+#define GT_COLS(NB, EPI) (gt_paired(EPI) ? 32 * (NB) : 64 * (NB))     // output columns of a tile
+constexpr bool gt_paired(int epi) { return epi == GT_SWIGLU || epi == GT_CLIPPED; }
+
+template <int EPI>
+__device__ __forceinline__ float gt_pair(float g, float u, const GemmArgs& a) {
+  if (EPI == GT_SWIGLU) return silu_f(g) * u;
+  g = fminf(g, a.limit);
+  u = fminf(fmaxf(u, -a.limit), a.limit);
+  return g / (1.0f + expf(-a.alpha * g)) * (u + 1.0f);
+}
+template <int EPI>
+__device__ __forceinline__ float gt_one(float v) {
+  if (EPI == GT_RELU2) { v = fmaxf(v, 0.f); return v * v; }
+  return EPI == GT_GELU ? gelu_erf_f(v) : v;
+}
+
+// Tile `t` of the order in which tiles are dealt out: strips of up to 8 tiles of rows, inside a strip column by column, so
+// that the 32 tiles a die works on at a time are about 8 x 4 and share their operands in its L2.
+__device__ __forceinline__ void gt_place(const GemmArgs& a, int t, int& m, int& n) {
+  const int per = 8 * a.n_tiles, strip = t / per, rest = t - strip * per, rows = min(8, a.m_tiles - strip * 8);
+  n = rest / rows;
+  m = strip * 8 + rest - n * rows;
+}
+
+template <int MB, int NB, int EPI>
+__global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const GemmArgs a) {
+#ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  typedef TileStream<MB, NB> TS;
+  TS ts(smem);
+  constexpr int TM = 64 * MB, TN = 64 * NB, COLS = gt_paired(EPI) ? TN / 2 : TN;      // output columns of a tile
+  const int tiles = a.m_tiles * a.n_tiles, step = gridDim.x;
+  // workgroups go to the dies in turn; a die's share of a round is a run of neighbouring tiles
+  const int first = gridDim.x % 8 == 0 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  if (first >= tiles) return;
+  const int stages = (a.K + TS_BK - 1) / TS_BK;
+
+  // the stage that is asked for next
+  int at_tile = first, at_stage = 0;
+  TileRowsSource<MB> xs;
+  TileRowsSource<NB> ws;
+  auto aim = [&](int t) {
+    int m, n;
+    gt_place(a, t, m, n);
+    const int m0 = m * TM;
+    xs.rsrc = ts_buffer(a.X + (size_t)m0 * a.ldx, ((long long)(a.M - m0 - 1) * a.ldx + a.K) * 2);
+#pragma unroll
+    for (int j = 0; j < 2 * MB; j++) xs.off[j] = (uint32_t)(ts.row(j) * a.ldx) * 2;
+    if (gt_paired(EPI)) {
+      // blocks of 32 tile rows are 16 gate rows and the 16 up rows of the same columns
+      const int c0 = n * COLS;
+      ws.rsrc = ts_buffer(a.W, ((long long)(a.up + a.cols - 1) * a.ldw + a.K) * 2);
+#pragma unroll
+      for (int j = 0; j < 2 * NB; j++) {
+        const int r = ts.row(j), c = c0 + (r >> 5) * 16 + (r & 15);
+        ws.off[j] = c < a.cols ? (uint32_t)((c + ((r & 16) ? a.up : 0)) * a.ldw) * 2 : TS_OUT;
+      }
+    } else {
+      const int n0 = n * TN;
+      ws.rsrc = ts_buffer(a.W + (size_t)n0 * a.ldw, ((long long)(a.cols - n0 - 1) * a.ldw + a.K) * 2);
+#pragma unroll
+      for (int j = 0; j < 2 * NB; j++) ws.off[j] = (uint32_t)(ts.row(j) * a.ldw) * 2;
+    }
+  };
+  // copies of the next stage into buffer b, and on to the one behind it
+  int fill = 0;
+  auto copies = [&](auto r) { ts.template ask<decltype(r)::from, decltype(r)::to>(fill, xs, ws, at_tile < tiles ? at_stage * TS_BK : a.K, a.K); };
+  auto on = [&] {
+    fill = fill + 1 == TS::NBUF ? 0 : fill + 1;
+    if (++at_stage == stages && at_tile < tiles) {
+      at_stage = 0;
+      at_tile += step;
+      if (at_tile < tiles) aim(at_tile);
+    }
+  };
+  aim(first);
+#pragma unroll
+  for (int b = 0; b < TS::NBUF - 1; b++) {
+    copies(Range<0, TS::LOADS>());
+    on();
+  }
+  __builtin_amdgcn_s_waitcnt(ts_wait((TS::NBUF - 2) * TS::LOADS, true));
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  copies(Range<0, TS::part(1)>());
+  ts.read(0, 0, 0);
+  int buf = 0;
+  for (int t = first; t < tiles; t += step) {
+    ts.clear();
+    for (int s = 0; s < stages; s++) {
+      const int next = buf + 1 == TS::NBUF ? 0 : buf + 1;
+      ts.stage(buf, next, copies, on);
+      buf = next;
+    }
+    // lane (l, h): row l of a block of X, tile rows 8 (r / 4) + 4 h + r % 4 of a block of W in register r
+    int mt, nt;
+    gt_place(a, t, mt, nt);
+    const int l = ts.lane & 31, h = ts.lane >> 5;
+#pragma unroll
+    for (int i = 0; i < MB; i++) {
+      const int m = mt * TM + (ts.wave >> 1) * (32 * MB) + 32 * i + l;
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        const ts_f32x16& v = ts.acc[j][i];
+        const int blk = (ts.wave & 1) * NB + j;
+        if (EPI == GT_F32) {
+          float* o = (float*)a.out + (size_t)m * a.ldo;
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const int n = nt * TN + blk * 32 + 8 * q + 4 * h;
+            if (m < a.M && n < a.cols) {
+              float4 f = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+              if (a.bias) { f.x += a.bias[n]; f.y += a.bias[n + 1]; f.z += a.bias[n + 2]; f.w += a.bias[n + 3]; }
+              *reinterpret_cast<float4*>(o + n) = f;
+            }
+          }
+        } else {
+          constexpr int G = gt_paired(EPI) ? 1 : 2;            // groups of 16 output columns in a block
+#pragma unroll
+          for (int g = 0; g < G; g++) {
+            const int n = nt * COLS + blk * (16 * G) + 16 * g;
+            uint32_t p[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              float u0, u1;
+              if (gt_paired(EPI)) {
+                u0 = gt_pair<EPI>(v[2 * q], v[8 + 2 * q], a);
+                u1 = gt_pair<EPI>(v[2 * q + 1], v[8 + 2 * q + 1], a);
+              } else {
+                const int c = n + 8 * (q >> 1) + 4 * h + 2 * (q & 1);
+                u0 = gt_one<EPI>(v[8 * g + 2 * q] + (a.bias && c < a.cols ? a.bias[c] : 0.f));
+                u1 = gt_one<EPI>(v[8 * g + 2 * q + 1] + (a.bias && c < a.cols ? a.bias[c + 1] : 0.f));
+              }
+              p[q] = pack2_bf16(u0, u1);
+            }
+            // the halves of the wave hold columns 0..3 and 8..11, 4..7 and 12..15: swapped, eight neighbours each
+            const auto s0 = __builtin_amdgcn_permlane32_swap(p[0], p[2], false, false);
+            const auto s1 = __builtin_amdgcn_permlane32_swap(p[1], p[3], false, false);
+            const int c = n + 8 * h;
+            if (m < a.M && c < a.cols)
+              *reinterpret_cast<uint4*>((bf16_t*)a.out + (size_t)m * a.ldo + c) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+          }
+        }
+      }
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(ts_wait(0, true));          // the last copies (zeros) are in before LDS is given back
+#endif
+}
+
+template <int MB, int NB, int EPI>
+static int gt_launch(GemmArgs a, hipStream_t stream) {
+  static const hipError_t room = hipFuncSetAttribute((const void*)&gemm_tiles_kernel<MB, NB, EPI>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, ts_lds_bytes(MB, NB));
+  PICO_REQUIRE(room == hipSuccess, "pico_gemm_tiles: %s", hipGetErrorString(room));
+  a.m_tiles = (a.M + 64 * MB - 1) / (64 * MB);
+  a.n_tiles = (a.cols + GT_COLS(NB, EPI) - 1) / GT_COLS(NB, EPI);
+  const long long tiles = (long long)a.m_tiles * a.n_tiles;
+  PICO_REQUIRE(tiles < (1LL << 30), "pico_gemm_tiles: %d x %d outputs are too many for one launch", a.M, a.cols);
+  const int most = 256 * ts_share(MB, NB);
+  gemm_tiles_kernel<MB, NB, EPI><<<tiles < most ? (int)tiles : most, 256, ts_lds_bytes(MB, NB), stream>>>(a);
+  PICO_LAUNCH_CHECK();
+  return 0;
+}
+
+// Which tile.  All make the same sums, so it is a question of how many rounds of workgroups a call takes and what one costs:
+// microseconds `each` a stage + `more`, fitted to calls of 24 and 56 stages with operands from memory.  A tile of which
+// two share a compute unit costs `lone` a stage while every unit has one.  Outputs a microsecond of a full round are alike
+// (0.34 to 0.36 million a microsecond and 24 stages), so what is left idle in the last round decides.
+struct GtTile { int mb, nb, share; float each, lone, more; };
+static const GtTile gt_tiles[] = {{2, 3, 2, 1.45f, 1.20f, 3.f}, {4, 2, 1, 0.84f, 0.84f, 3.8f}, {3, 3, 1, 1.00f, 1.00f, 2.f}, {2, 1, 2, 0.80f, 0.35f, 3.f}};
+
+// The tile for M rows and `cols` columns and its cost.  `first`: how many columns to make in whole rounds with it, the
+// others being better left to a launch of their own with the tile that suits them (2,052 rows of 8,960 pairs: three rounds
+// and 62 tiles; the 62 as a fourth round cost 32 us, as 170 tiles of a third their size 12); else all.
+static int gt_choose(int M, int cols, int stages, bool paired, bool split, int& first, float& cost) {
+  int best = 0;
+  cost = 3e38f;
+  for (int i = 0; i < 4; i++) {
+    const GtTile& t = gt_tiles[i];
+    const int tile_cols = GT_COLS(t.nb, paired ? GT_SWIGLU : GT_BF16), m_tiles = (M + 64 * t.mb - 1) / (64 * t.mb);
+    const long long tiles = (long long)m_tiles * ((cols + tile_cols - 1) / tile_cols), round = 256 * t.share, full = tiles / round, rest = tiles % round;
+    const float whole = (float)full * (t.each * stages + t.more);
+    const float c = whole + (rest ? (rest <= 256 ? t.lone : t.each) * stages + t.more : 0.f);
+    if (c < cost) { cost = c; best = i; first = cols; }
+    const int n1 = (int)(full * round / m_tiles) * tile_cols;
+    if (split && rest && n1 > 0 && n1 < cols) {
+      int all;
+      float other;
+      gt_choose(M, cols - n1, stages, paired, false, all, other);
+      if (whole + other + 3.f < cost) { cost = whole + other + 3.f; best = i; first = n1; }      // 3 us: a launch
+    }
+  }
+  return best;
+}
+
+template <int EPI>
+static int gt_run(GemmArgs a, hipStream_t stream) {
+  const int stages = (a.K + TS_BK - 1) / TS_BK, cols = a.cols;
+  int first, all, rc = 0;
+  float cost;
+  const int tile = gt_choose(a.M, cols, stages, gt_paired(EPI), true, first, cost);
+  auto run = [&](int i) {
+    switch (i) {
+      case 0: return gt_launch<2, 3, EPI>(a, stream);
+      case 1: return gt_launch<4, 2, EPI>(a, stream);
+      case 2: return gt_launch<3, 3, EPI>(a, stream);
+      default: return gt_launch<2, 1, EPI>(a, stream);
+    }
+  };
+  a.cols = first;
+  rc = run(tile);
+  if (rc || first == cols) return rc;
+  a.W += (size_t)first * a.ldw;
+  if (a.bias) a.bias += first;
+  a.out = (char*)a.out + (size_t)first * (EPI == GT_F32 ? 4 : 2);
+  a.cols = cols - first;
+  return run(gt_choose(a.M, a.cols, stages, gt_paired(EPI), false, all, cost));
+}
+
+// X [M, K] row stride ldx, W [N, K] row stride ldw, bfloat16; out [M, N] (N / 2 columns for the paired epilogues) row stride
+// ldo, bfloat16 or (GT_F32) float32.  All strides, K and the columns multiples of 8, the pointers on 16 bytes, each
+// operand's span below 2^31 bytes.
+extern "C" int pico_gemm_tiles(const void* X, const void* W, const float* bias, void* out, int epi, int M, int N,
+                               int K, int ldx, int ldw, int ldo, float limit, float alpha, hipStream_t stream) {
+  PICO_REQUIRE(M >= 0 && N > 0 && K > 0, "pico_gemm_tiles: bad sizes M=%d N=%d K=%d", M, N, K);
+  const int cols = gt_paired(epi) ? N / 2 : N;
+  PICO_REQUIRE(ldx >= K && ldw >= K && ldo >= cols, "pico_gemm_tiles: a row stride is smaller than its row");
+  PICO_REQUIRE(K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldo % 8 == 0 && cols % 8 == 0 && (!gt_paired(epi) || N % 2 == 0),
+               "pico_gemm_tiles: sizes and strides must be multiples of 8");
+  PICO_REQUIRE(((uintptr_t)X | (uintptr_t)W | (uintptr_t)out) % 16 == 0, "pico_gemm_tiles: operands must start on 16 bytes");
+  PICO_REQUIRE((long long)M * ldx < (1LL << 30) && (long long)N * ldw < (1LL << 30), "pico_gemm_tiles: an operand spans 2^31 bytes or more");
+  PICO_REQUIRE(!bias || !gt_paired(epi), "pico_gemm_tiles: the paired epilogues take no bias");
+  if (M == 0) return 0;
+  GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, bias, out, M, cols, K, ldx, ldw, ldo, N - cols, 0, 0, limit, alpha};
+  switch (epi) {
+    case GT_BF16: return gt_run<GT_BF16>(a, stream);
+    case GT_F32: return gt_run<GT_F32>(a, stream);
+    case GT_SWIGLU: return gt_run<GT_SWIGLU>(a, stream);
+    case GT_RELU2: return gt_run<GT_RELU2>(a, stream);
+    case GT_CLIPPED: return gt_run<GT_CLIPPED>(a, stream);
+    case GT_GELU: return gt_run<GT_GELU>(a, stream);
+  }
+  PICO_REQUIRE(false, "pico_gemm_tiles: unknown epilogue %d", epi);
+}

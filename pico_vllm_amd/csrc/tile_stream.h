@@ -1,0 +1,170 @@
+// The inner part of a tiled bfloat16 product on the matrix cores: tiles of 64 MB rows of X by 64 NB rows of W, both
+// contiguous along k, four waves (2 x 2), each with MB x NB blocks of v_mfma_f32_32x32x16_bf16; one workgroup a compute
+// unit, or two that hide each other's waits (ts_share).  Every sum runs over k in the same order whatever the tile.
+//
+// A stage is 64 k of all rows of the tile.  Its 128-byte rows go from memory straight to LDS (buffer_load .. lds, sixteen
+// bytes a lane, whole lines), the sixteen-byte chunks of a row xor-swizzled by the row so that the operand reads (32 rows,
+// one chunk each) meet every bank once.  What lies outside a matrix (rows behind the last, k behind K) is an offset behind
+// the buffer's end and arrives as zeros: no clamps, no selects.
+//
+// With one or two waves a SIMD little else hides a wait, so the products of a quarter stage (16 k) run while the operands of the
+// next are read, and the only barrier of a stage stands where its last operands are in registers: behind it the next
+// stage has landed and this one's buffer is asked to fill for the stage after.  The stages of all of a workgroup's tiles
+// are one sequence, so the next tile's first stages travel under the last products and the epilogue of this one.
+//
+// What bounds it, measured: operands that the L2 holds, a 256 x 128 stage takes 1,290 cycles (1,024 of products, 1,175 for
+// its 48 KB at the 41 bytes a cycle at which a compute unit takes in lines), a 256 x 256 one 2,230 (2,048); from memory the
+// latency of a copy shows, because LDS holds two or three stages: 0.8 to 0.9 us a 256 x 128 stage.  Lines asked for
+// further ahead (four bytes each into the L2, 2 to 6 stages before their copies) made it slower (113 to 117 us and 122 to
+// 145): the copies' counter retires in order, behind the far lines.
+#pragma once
+#include "common.h"
+
+typedef __bf16 ts_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float ts_f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t ts_u32x4 __attribute__((ext_vector_type(4)));
+
+#define TS_BK 64
+#define TS_OUT 0x80000000u          // added to an offset: behind the end of any buffer (at most 2^31 - 1 bytes)
+
+constexpr int ts_stage_bytes(int MB, int NB) { return (MB + NB) * 64 * TS_BK * 2; }
+// workgroups that share a compute unit, and buffers of a workgroup
+constexpr int ts_share(int MB, int NB) { return MB * NB <= 6 ? 2 : 1; }
+constexpr int ts_buffers(int MB, int NB) { return ts_stage_bytes(MB, NB) * 3 * ts_share(MB, NB) <= 160 * 1024 ? 3 : 2; }
+constexpr int ts_lds_bytes(int MB, int NB) { return ts_stage_bytes(MB, NB) * ts_buffers(MB, NB); }
+// s_waitcnt: at most n vector memory operations outstanding; with `lds` also no LDS read
+constexpr int ts_wait(int n, bool lds) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | ((lds ? 0 : 15) << 8); }
+
+#ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
+// The rows of one operand of a tile, as what a lane asks for: `rsrc` over the matrix from the tile's first row on, and the
+// byte offset of this lane's chunk in its row of each of the wave's copies (eight rows each), at k = 0.
+template <int B>
+struct TileRowsSource {
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off[2 * B];
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ts_buffer(const void* base, long long bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)min(bytes, (long long)0x7fffffff), 0x00020000);
+}
+
+template <int FROM, int TO> struct Range { static constexpr int from = FROM, to = TO; };
+
+template <int MB, int NB>
+struct TileStream {
+  static constexpr int NBUF = ts_buffers(MB, NB), STAGE = ts_stage_bytes(MB, NB), LOADS = 2 * (MB + NB);
+  char* lds;
+  int wave, lane;
+  uint32_t kbyte;                       // the byte of this lane's chunk within a row's 128 bytes
+  const char *xrd, *wrd;                // this wave's operand rows in buffer 0
+  int sw[4];                            // where lane (row l, half h) finds the chunk of quarter ks
+  ts_f32x16 acc[NB][MB];
+  ts_u32x4 w[2][NB], x[2][MB];
+
+  __device__ __forceinline__ TileStream(char* smem) : lds(smem) {
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    lane = threadIdx.x & 63;
+    const int rho = lane >> 3, pos = lane & 7, l = lane & 31, h = lane >> 5;
+    kbyte = (uint32_t)((pos ^ rho) << 4);
+#pragma unroll
+    for (int s = 0; s < 4; s++) sw[s] = l * 128 + (((4 * h + s) ^ (l & 7)) << 4);
+    xrd = smem + (wave >> 1) * (MB * 32 * 128);
+    wrd = smem + MB * 64 * 128 + (wave & 1) * (NB * 32 * 128);
+  }
+  // the tile row behind this lane in the wave's copy j
+  __device__ __forceinline__ int row(int j) const { return (4 * j + wave) * 8 + (lane >> 3); }
+
+  // Copies FROM .. TO - 1 of the 2 (MB + NB) that bring 64 k from k0 on of the rows of `xs` and `ws` into buffer b
+  // (k0 >= K: zeros).
+  template <int FROM, int TO>
+  __device__ __forceinline__ void ask(int b, const TileRowsSource<MB>& xs, const TileRowsSource<NB>& ws, int k0, int K) {
+    const uint32_t k = (uint32_t)k0 * 2 + kbyte;
+    const uint32_t at = k < (uint32_t)K * 2 ? k : TS_OUT;
+    char* dst = lds + b * STAGE + wave * 1024;
+#pragma unroll
+    for (int j = FROM; j < TO; j++) {
+      if (j < 2 * MB)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xs.rsrc, (__attribute__((address_space(3))) void*)(dst + j * 4096), 16, xs.off[j < 2 * MB ? j : 0] + at, 0, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ws.rsrc, (__attribute__((address_space(3))) void*)(dst + j * 4096), 16, ws.off[j < 2 * MB ? 0 : j - 2 * MB] + at, 0, 0, 0);
+    }
+  }
+  // in the order in which the products want them
+  __device__ __forceinline__ void read(int set, int b, int ks) {
+    w[set][0] = *reinterpret_cast<const ts_u32x4*>(wrd + b * STAGE + sw[ks]);
+#pragma unroll
+    for (int i = 0; i < MB; i++) x[set][i] = *reinterpret_cast<const ts_u32x4*>(xrd + b * STAGE + sw[ks] + i * 4096);
+#pragma unroll
+    for (int j = 1; j < NB; j++) w[set][j] = *reinterpret_cast<const ts_u32x4*>(wrd + b * STAGE + sw[ks] + j * 4096);
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+      for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[j][i][r] = 0.f;
+  }
+  __device__ __forceinline__ void multiply(int set) {
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+      for (int i = 0; i < MB; i++)
+        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ts_bf16x8, w[set][j]),
+                                                            __builtin_bit_cast(ts_bf16x8, x[set][i]), acc[j][i], 0, 0, 0);
+  }
+  // The MB NB products of a quarter with its operand reads between the first and its copies between the last of them: the
+  // reads are back long before their products (and before the barrier), and a copy is never asked for faster than a compute
+  // unit takes them in (about 41 bytes a cycle of whole lines; a wave that asks faster stands still, its products with it).
+  // Copies write LDS, so the compiler keeps them behind the reads in any case.
+  template <int READS, int COPIES, int I = 0>
+  __device__ __forceinline__ void weave() {
+    constexpr int P = MB * NB, H = READS < P ? (READS > 0 ? READS : 0) : P - 1, L = P - H;
+    if constexpr (I < P) {
+      constexpr int R = I < H ? (I + 1) * READS / (H > 0 ? H : 1) - I * READS / (H > 0 ? H : 1) : 0;
+      constexpr int C = I < H ? 0 : (I - H + 1) * COPIES / L - (I - H) * COPIES / L;
+      if constexpr (R > 0) __builtin_amdgcn_sched_group_barrier(0x100, R, 0);
+      if constexpr (C > 0) __builtin_amdgcn_sched_group_barrier(0x020, C, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      weave<READS, COPIES, I + 1>();
+    }
+  }
+  // The copies that take the place of a finished stage go out in PARTS quarters from its last one on: all four where there
+  // is a third buffer, else three, so that the last has a quarter to land.
+  static constexpr int PARTS = NBUF == 3 ? 4 : 3;
+  static constexpr int part(int i) { return LOADS * i / PARTS; }
+  // The products of the stage in buffer b, whose first operands are in set 0; leaves the first operands of the stage in
+  // buffer `next` there.  `copies` is called with the numbers of the copies to ask for: first what is left of those that
+  // have begun, then `on` (they are all on their way), then the first of those that fill b again.
+  template <typename Copies, typename On>
+  __device__ __forceinline__ void stage(int b, int next, Copies copies, On on) {
+    __builtin_amdgcn_sched_barrier(0);
+    read(1, b, 1);
+    copies(Range<part(1), part(2)>());
+    multiply(0);
+    weave<MB + NB, part(2) - part(1)>();
+    __builtin_amdgcn_sched_barrier(0);
+    read(0, b, 2);
+    copies(Range<part(2), part(3)>());
+    multiply(1);
+    weave<MB + NB, part(3) - part(2)>();
+    __builtin_amdgcn_sched_barrier(0);
+    if (PARTS == 3) on();
+    read(1, b, 3);
+    if (PARTS == 4) copies(Range<part(3), LOADS>());
+    multiply(0);
+    weave<MB + NB, PARTS == 4 ? LOADS - part(3) : 0>();
+    __builtin_amdgcn_sched_barrier(0);
+    if (PARTS == 4) on();
+    // this wave's copies of the next stage have landed and its reads of this one are done; then so are all waves'
+    __builtin_amdgcn_s_waitcnt(ts_wait((NBUF - 2) * LOADS, true));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    read(0, next, 0);
+    copies(Range<0, part(1)>());
+    multiply(1);
+    weave<MB + NB, part(1)>();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+};
+#endif

@@ -299,6 +299,53 @@ def skinny_ok(a: torch.Tensor, w: torch.Tensor) -> bool:
             and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def tiles_ok(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the tiled product takes these operands (whole aligned eights, spans below 2^31 bytes)."""
+    return (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and a.shape[0] > 0
+            and a.shape[1] == w.shape[1] and a.shape[1] % 8 == 0 and w.shape[0] % 16 == 0 and a.stride(1) == 1 and w.stride(1) == 1
+            and (a.stride(0) % 8 == 0 or a.shape[0] == 1) and w.stride(0) % 8 == 0 and a.stride(0) >= a.shape[1]
+            and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and a.shape[0] * a.stride(0) < 1 << 30 and w.shape[0] * w.stride(0) < 1 << 30)
+
+
+# Activations ride on the tiled product where that beats the library's product and a pass of its own.  Inner sizes up to
+# TILES_SHORT_K: always (8,960 pairs, K 1,536, microseconds of both: 31 / 21 at 65 rows, 35 / 29 at 300, 50 / 50 at 600, 82 / 67
+# at 1,024, 137 / 115 at 2,048; 13,440 squared outputs 30 / 15, 31 / 26, 46 / 43, 59 / 54, 106 / 101).  Beyond, the library's longer
+# pipeline is ahead until its tiles of 256 rows leave many of them empty: pairs only, above TILES_ROWS rows (18,944 pairs,
+# K 3,584: 120 / 133 at 300 rows, 183 / 197 at 700, 294 / 226 at 900, 318 / 255 at 1,024, 556 / 493 at 2,048).
+TILES_SHORT_K, TILES_ROWS = 2048, 768
+
+
+def tiles_act_ok(a: torch.Tensor, w: torch.Tensor, paired: bool) -> bool:
+    return tiles_ok(a, w) and (a.shape[1] <= TILES_SHORT_K or (paired and a.shape[0] > TILES_ROWS))
+
+
+def gemm_tiles(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, epilogue: int = EPI_BF16,
+               clip: Optional[tuple] = None) -> torch.Tensor:
+    """a [M, K] x w [N, K]^T, both bfloat16, any number of rows; epilogues and results as ``gemm_skinny``'s (EPI_BF16,
+    EPI_F32, EPI_SWIGLU, EPI_RELU2, EPI_CLIPPED, EPI_GELU)."""
+    _gpu(a, w, bias)
+    M, K = a.shape
+    N, K2 = w.shape
+    if K != K2:
+        raise KernelError(f"gemm: inner sizes differ ({K} and {K2})")
+    if not tiles_ok(a, w):
+        raise KernelError("gemm_tiles: operands must be bfloat16 rows of whole 16-byte aligned eights (tiles_ok)")
+    if bias is not None and (bias.dtype != torch.float32 or bias.shape != (N,) or not bias.is_contiguous()):
+        raise KernelError("gemm_tiles: bias must be contiguous float32 [N]")
+    if epilogue not in (EPI_BF16, EPI_F32, EPI_SWIGLU, EPI_RELU2, EPI_CLIPPED, EPI_GELU):
+        raise KernelError(f"gemm_tiles: no epilogue {epilogue}")
+    if epilogue == EPI_CLIPPED and (clip is None or not clip[0] > 0):
+        raise KernelError("gemm_tiles: the clipped activation needs a positive limit and a factor")
+    cols = N // 2 if epilogue in (EPI_SWIGLU, EPI_CLIPPED) else N
+    out = torch.empty(M, cols, dtype=torch.float32 if epilogue == EPI_F32 else torch.bfloat16, device=a.device)
+    limit, alpha = clip or (0.0, 0.0)
+    lib = library.core()
+    _check(lib, lib.pico_gemm_tiles(_ptr(a), _ptr(w), _ptr(bias), _ptr(out), epilogue, M, N, K, a.stride(0) if M > 1 else K,
+                                    w.stride(0), cols, c_float(limit), c_float(alpha), _stream()))
+    return out
+
+
 def gemm_skinny(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, epilogue: int = EPI_BF16,
                 k_splits: int = 1, out: Optional[torch.Tensor] = None, clip: Optional[tuple] = None,
                 token_rows: Optional[tuple] = None) -> torch.Tensor:

@@ -2,8 +2,9 @@
 
 bfloat16 weights: with up to 64 rows of activations (decode, small mixed
 steps; up to 256 for small matrices) the weight-streaming matrix-core kernel of this package, with bias,
-SwiGLU or float32 output as its epilogue (for shapes it refuses, this package's plain matrix-core product); with more rows the library GEMM
-(hipBLASLt through torch), as the reference uses the library for every
+SwiGLU or float32 output as its epilogue (for shapes it refuses, this package's plain matrix-core product); with more rows this
+package's tiled product where an activation or a float32 result follows (``kernels.tiles_act_ok`` says where), else the library
+GEMM (hipBLASLt through torch), as the reference uses the library for every
 projection (pico_vllm/model.py:200,225,316,318).  float32 weights: this package's plain-FMA kernel, never a library
 call, so the 32-bit engine has no reduced-precision matrix mode anywhere; if
 the activations are bfloat16 (a tensor stored in 32 bit inside a bfloat16
@@ -106,6 +107,8 @@ class Linear:
             epi = kernels.EPI_F32 if out_dtype == torch.float32 else kernels.EPI_BF16
             return kernels.gemm_skinny(x, self.weight, self.bias_f32, epi)
         if out_dtype == torch.float32:
+            if kernels.tiles_ok(x, self.weight):
+                return kernels.gemm_tiles(x, self.weight, self.bias_f32, kernels.EPI_F32)
             return kernels.gemm_bf16(x, self.weight, self.bias_f32, torch.float32)
         if kernels.skinny_rows(x, self.weight):
             # few rows of a shape that the weight-streaming kernel refuses (an inner size that is no multiple of 8):
@@ -130,6 +133,8 @@ class Linear:
             x = x.run()
         if self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight):
             return kernels.gemm_skinny(x, self.weight, None, kernels.EPI_SWIGLU)
+        if self.bias is None and kernels.tiles_act_ok(x, self.weight, True):
+            return kernels.gemm_tiles(x, self.weight, None, kernels.EPI_SWIGLU)
         return kernels.swiglu(self(x))
 
     def clipped_glu(self, x: torch.Tensor, limit: float, alpha: float) -> torch.Tensor:
@@ -137,6 +142,8 @@ class Linear:
         rows the epilogue of the weight-streaming kernel."""
         if self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight):
             return kernels.gemm_skinny(x, self.weight, None, kernels.EPI_CLIPPED, clip=(limit, alpha))
+        if self.bias is None and kernels.tiles_act_ok(x, self.weight, True):
+            return kernels.gemm_tiles(x, self.weight, None, kernels.EPI_CLIPPED, clip=(limit, alpha))
         return kernels.clipped_glu(self(x), limit, alpha)
 
     def gelu_token(self, x: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, col: int) -> torch.Tensor:
@@ -150,6 +157,8 @@ class Linear:
         """max(x W^T, 0)^2; with few rows the activation is the epilogue of the weight-streaming kernel."""
         if self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight):
             return kernels.gemm_skinny(x, self.weight, None, kernels.EPI_RELU2)
+        if self.bias is None and kernels.tiles_act_ok(x, self.weight, False):
+            return kernels.gemm_tiles(x, self.weight, None, kernels.EPI_RELU2)
         y = self(x)
         return kernels.relu2(y, out=y)
 
@@ -157,6 +166,8 @@ class Linear:
         """gelu(x W^T + b) with the error function; with few rows the epilogue of the weight-streaming kernel."""
         if self.weight.dtype == torch.bfloat16 and kernels.skinny_ok(x, self.weight):
             return kernels.gemm_skinny(x, self.weight, self.bias_f32, kernels.EPI_GELU)
+        if kernels.tiles_act_ok(x, self.weight, False):
+            return kernels.gemm_tiles(x, self.weight, self.bias_f32, kernels.EPI_GELU)
         y = self(x)
         return kernels.gelu(y, out=y)
 

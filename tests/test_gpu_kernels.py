@@ -143,6 +143,44 @@ def test_gemm_f32_rounding_does_not_grow_with_the_inner_size(K, K_):
     assert float(err.abs().max() / want.pow(2).mean().sqrt()) <= 5 * 1.69 * math.sqrt(levels) * eps     # 768 outputs: five sigma
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 16, 8), (65, 48, 64), (128, 400, 72), (129, 208, 1000), (200, 4112, 192), (257, 640, 136),
+                                   (450, 2576, 64), (600, 6160, 328)])
+@pytest.mark.parametrize("name", ["bf16", "f32", "swiglu", "clipped", "relu2", "gelu"])
+def test_gemm_tiles(K, M, N, K_, name):
+    # the edges of tiles of 64 to 256 rows and columns, of the stages of 64 k, of one and several rounds of workgroups
+    g = torch.Generator().manual_seed(M + N)
+    wide = torch.randn(M, K_ + 8, generator=g).bfloat16().to(DEV)
+    a, w = wide[:, 8:], (torch.randn(N, K_, generator=g) * K_ ** -0.5).bfloat16().to(DEV)      # rows with a stride
+    b = torch.randn(N, generator=g).to(DEV) if name in ("bf16", "f32", "gelu") else None
+    epi = {"bf16": K.EPI_BF16, "f32": K.EPI_F32, "swiglu": K.EPI_SWIGLU, "clipped": K.EPI_CLIPPED, "relu2": K.EPI_RELU2, "gelu": K.EPI_GELU}[name]
+    clip = (0.7, 1.702) if name == "clipped" else None
+    out = K.gemm_tiles(a, w, b, epi, clip)
+    z = a.double() @ w.double().T + (b.double() if b is not None else 0.0)
+    half = N // 2
+    want = {"bf16": lambda: z, "f32": lambda: z, "swiglu": lambda: F.silu(z[:, :half]) * z[:, half:],
+            "clipped": lambda: z[:, :half].clamp(max=0.7) * torch.sigmoid(1.702 * z[:, :half].clamp(max=0.7)) * (z[:, half:].clamp(-0.7, 0.7) + 1),
+            "relu2": lambda: torch.relu(z) ** 2, "gelu": lambda: F.gelu(z)}[name]()
+    # float32 sums of at most 1,000 terms (relative error below 1e-5 of a row's size, which is about 1) through activations
+    # with slopes of at most about 2 |z|; then one rounding to bfloat16 (2^-9)
+    slack = 1e-5 * (1 + 2 * float(z.abs().max()))
+    if name == "f32":
+        assert out.dtype == torch.float32 and float((out.double() - want).abs().max()) <= slack
+    else:
+        assert out.dtype == torch.bfloat16 and bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + slack).all())
+    # a row's bits do not depend on the rows beside it, nor on the tile that a call of its size takes
+    assert torch.equal(K.gemm_tiles(a[M // 2:M // 2 + 1], w, b, epi, clip)[0], out[M // 2])
+    assert torch.equal(K.gemm_tiles(a[:(M + 1) // 2], w, b, epi, clip), out[:(M + 1) // 2])
+
+
+def test_gemm_tiles_refuses(K):
+    a, w = torch.zeros(70, 72, device=DEV).bfloat16(), torch.zeros(48, 72, device=DEV).bfloat16()
+    for bad in (lambda: K.gemm_tiles(a[:, :68], w[:, :68]), lambda: K.gemm_tiles(a, w[:40]), lambda: K.gemm_tiles(a.float(), w),
+                lambda: K.gemm_tiles(a, w, None, K.EPI_CLIPPED), lambda: K.gemm_tiles(a[:, 1:65], w[:, :64]),
+                lambda: K.gemm_tiles(a, w, torch.zeros(47, device=DEV)), lambda: K.gemm_tiles(a, w[:, :64])):
+        with pytest.raises(RuntimeError):
+            bad()
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 301, 136), (3, 256, 64), (8, 384, 192), (33, 130, 172), (64, 1000, 1536),
                                    (100, 77, 40)])
 @pytest.mark.parametrize("out_dtype", DTYPES)
