@@ -17,6 +17,15 @@ from ..parts.spec import CacheSpec
 from .manager import CacheManager
 
 
+def device_index(values, device: torch.device) -> torch.Tensor:
+    """int64 indices on ``device`` without waiting for it: from pinned memory, in the stream's order.  (A tensor made from a
+    list on the device waits until everything launched before it has run: 1.8 ms in front of a prompt step, in which
+    nothing of the next step could be launched.)"""
+    if device.type != "cuda":
+        return torch.tensor(values, dtype=torch.long, device=device)
+    return torch.tensor(values, dtype=torch.long, pin_memory=True).to(device, non_blocking=True)
+
+
 @dataclass
 class PagedKVLayer:
     """The page tensors of one layer by name (also as attributes: ``layer.k``)."""
@@ -102,7 +111,7 @@ class CacheStorage:
         for l in self._layers.values():
             if isinstance(l, StateLayer):
                 if idx is None:
-                    idx = torch.tensor(sorted(set(slots)), dtype=torch.long, device=l.state.device)
+                    idx = device_index(sorted(set(slots)), l.state.device)
                 l.state.index_fill_(0, idx, 0)
 
     def num_bytes(self) -> int:

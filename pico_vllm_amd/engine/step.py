@@ -24,7 +24,7 @@ from typing import Dict, List, Optional
 import torch
 
 from ..cache.manager import CacheManager
-from ..cache.storage import CacheStorage
+from ..cache.storage import CacheStorage, device_index
 from ..parts.model import DecoderModel
 from .batch import BatchBuffers, BatchError, SeqStep, build_context
 
@@ -124,7 +124,7 @@ class ModelRunner:
         elif size:
             logits = self._step_prompt_graph(seqs, size)
             if back is not None:
-                logits = logits.index_select(0, torch.tensor(back, dtype=torch.long, device=logits.device))
+                logits = logits.index_select(0, device_index(back, logits.device))
         else:
             ctx = build_context(seqs, self.manager, self.buffers, self.model.dtype, self.model.spec.vocab_size)
             # the kernel choices of a recorded step for its single tokens (how their contexts are split over
@@ -138,7 +138,7 @@ class ModelRunner:
                 ctx.token_ids[:len(seqs)].copy_(device_tokens[:len(seqs)])
             logits = self.model.forward(ctx, self.storage)
             if back is not None and logits.shape[0]:
-                logits = logits.index_select(0, torch.tensor(back, dtype=torch.long, device=logits.device))
+                logits = logits.index_select(0, device_index(back, logits.device))
         self.steps += 1
         self.tokens += sum(len(s.tokens) for s in seqs)
         return logits
