@@ -10,9 +10,8 @@
 // column, and feeds P^T from registers as the B operand of O^T += V^T P^T, whose A operand is 16 contiguous bytes of
 // V^T as the pages hold it.  Scores, softmax statistics and sums are float32; P is rounded to bfloat16 for the product.
 //
-// Two shapes of workgroup (four waves): SPLIT, one block whose key range the waves share in steps of 32 and merge
-// through LDS (few blocks: decoding, short portions); or four neighbouring blocks, one a wave, whose key ranges
-// overlap so that their loads meet in the first-level cache (long portions).
+// Small steps (attn_bias_kernel): a workgroup of four waves has one block, whose key range the waves share in steps of 32 and
+// merge through LDS.  Long portions (attn_bias_staged_kernel): eight blocks, one a wave, their keys staged in LDS.
 #include "common.h"
 
 #ifndef PICO_DK
@@ -42,7 +41,7 @@ struct BiasArgs {
   bf16_t* out;                 // [T, nq * DV]
   int num_seqs, nq, nkv, P, num_pages, window, temp_every;
   float scale, temp_coef, slope_span;
-  // chunks > 1 (SPLIT only): workgroup z of a block takes the z-th piece of the block's keys and leaves its sums
+  // chunks > 1 (small steps only): workgroup z of a block takes the z-th piece of the block's keys and leaves its sums
   // unnormalised in parts_o [chunks][columns][DV] and its (maximum, sum) in parts_ml [chunks][columns][2]
   int chunks, ncols;
   float* parts_o;
@@ -65,17 +64,47 @@ struct BiasArgs {
 
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
-template <bool SPLIT>
+// A finished column's output: lane (column, kq) holds value dimensions 16 tt + 4 kq + r; M and L its maximum and sum.
+__device__ __forceinline__ void write_column(const BiasArgs& a, const f32x4 (&o)[DT], int t, int head, int kq, float M_all, float L) {
+  // the column's own key is always seen: M_all is finite.  (A sink so far above every key that its exponential overflows
+  // leaves the keys no weight: the output is 0.)
+  if (a.sink) L += __expf((a.sinks ? a.sinks[head] : 0.f) - M_all);
+  float inv = a.out_scale / L;
+  if (a.gate && a.gate_heads) inv *= sigmoid_f32(bf16_to_f32(a.gate[(size_t)t * a.gate_stride + head]));
+  bf16_t* orow = a.out + (size_t)t * a.out_stride + (size_t)head * DV + 4 * kq;
+  const bf16_t* grow = a.gate && !a.gate_heads ? a.gate + (size_t)t * a.gate_stride + (size_t)head * DV + 4 * kq : nullptr;
+#pragma unroll
+  for (int tt = 0; tt < DT; tt++) {
+    float g0 = inv, g1 = inv, g2 = inv, g3 = inv;
+    if (a.out_f32) {
+      float* o32 = reinterpret_cast<float*>(a.out) + (size_t)t * a.out_stride + (size_t)head * DV + 4 * kq + 16 * tt;
+      *reinterpret_cast<f32x4*>(o32) = f32x4{o[tt][0] * g0, o[tt][1] * g1, o[tt][2] * g2, o[tt][3] * g3};
+      continue;
+    }
+    if (grow) {
+      const uint2 gv = *reinterpret_cast<const uint2*>(grow + 16 * tt);
+      g0 *= sigmoid_f32(__uint_as_float(gv.x << 16));
+      g1 *= sigmoid_f32(__uint_as_float(gv.x & 0xffff0000u));
+      g2 *= sigmoid_f32(__uint_as_float(gv.y << 16));
+      g3 *= sigmoid_f32(__uint_as_float(gv.y & 0xffff0000u));
+    }
+    uint2 w;
+    w.x = pack2_bf16(o[tt][0] * g0, o[tt][1] * g1);
+    w.y = pack2_bf16(o[tt][2] * g2, o[tt][3] * g3);
+    *reinterpret_cast<uint2*>(orow + 16 * tt) = w;
+  }
+}
+
 __global__ __launch_bounds__(256, 2) void attn_bias_kernel(const BiasArgs a) {
-  __shared__ float xo[SPLIT ? 3 : 1][SPLIT ? DV : 1][16];
-  __shared__ float xml[SPLIT ? 3 : 1][2][16];
+  __shared__ float xo[3][DV][16];
+  __shared__ float xml[3][2][16];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, kq = lane >> 4;
   const int g = blockIdx.y;
   const int R = a.nq / a.nkv;
   const int tpb = R >= 16 ? 1 : 16 / R;                 // tokens a block
   const int hb = R > 16 ? (R + 15) / 16 : 1;            // blocks a token (R > 16)
   // which block of which sequence: blocks are counted sequence by sequence
-  int tile = SPLIT ? (int)blockIdx.x : 4 * (int)blockIdx.x + wave;
+  int tile = blockIdx.x;
   int b = 0, t_begin = 0, t_end = 0;
   bool found = false;
   for (; b < a.num_seqs; b++) {
@@ -85,18 +114,15 @@ __global__ __launch_bounds__(256, 2) void attn_bias_kernel(const BiasArgs a) {
     if (tile < tiles) { found = true; break; }
     tile -= tiles;
   }
-  if (!found) {
-    if (SPLIT) return;          // the whole workgroup
-    t_begin = t_end = 0;        // this wave has nothing; it still meets no barrier below
-  }
+  if (!found) return;
   const int t0 = t_begin + (tile / hb) * tpb;           // first token of the block
-  const int ntok = found ? min(tpb, t_end - t0) : 0;
+  const int ntok = min(tpb, t_end - t0);
   const int hc = tile % hb;                             // which 16 heads of the token (R > 16)
   const int my_tok = R >= 16 ? 0 : col / R, my_h = R >= 16 ? 16 * hc + col : col % R;
   const bool col_ok = my_tok < ntok && my_h < R;
   const int t = t0 + (col_ok ? my_tok : 0);
   const int head = g * R + (col_ok ? my_h : 0);
-  const int p0 = found ? a.positions[t0] : 0;           // the block's first position; its tokens follow one another
+  const int p0 = a.positions[t0];           // the block's first position; its tokens follow one another
   const int my_pos = p0 + (col_ok ? my_tok : 0);
   const int hi = p0 + ntok;                             // keys below hi are read
   const int lo = a.chunk > 0 ? p0 / a.chunk * a.chunk : a.window > 0 ? max(0, p0 - a.window + 1) : 0;
@@ -125,9 +151,8 @@ __global__ __launch_bounds__(256, 2) void attn_bias_kernel(const BiasArgs a) {
   for (int tt = 0; tt < DT; tt++) o[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int pshift = 31 - __clz(a.P);                   // page sizes are powers of two
-  const int stride = SPLIT ? 128 : 32;
   int begin = lo & ~31, end = hi;
-  if (SPLIT && a.chunks > 1) {
+  if (a.chunks > 1) {
     // pieces of whole turns of the four waves (128 keys), so the tiles are those of the uncut loop
     const int piece = ((hi - begin + a.chunks - 1) / a.chunks + 127) & ~127;
     begin += (int)blockIdx.z * piece;
@@ -136,12 +161,12 @@ __global__ __launch_bounds__(256, 2) void attn_bias_kernel(const BiasArgs a) {
   // kept first keys in front of the window's first tile: tiles of their own, taken by the first piece (those inside
   // the window's tiles are let through by the mask below)
   const int sink_end = min(keep, lo & ~31);
-  const bool sinks = sink_end > 0 && (!SPLIT || blockIdx.z == 0);
-  const int first = begin + (SPLIT ? 32 * wave : 0);
+  const bool sinks = sink_end > 0 && blockIdx.z == 0;
+  const int first = begin + 32 * wave;
   if (ntok > 0 && (first < end || sinks)) {
     const int last_key = hi - 1, last_group = last_key / 8 * 8;
     const int row_key = 8 * (col >> 2) + (col & 3);     // key of this lane's row in tile 0; tile 1: 4 more
-    int key0 = sinks ? (SPLIT ? 32 * wave : 0) : first;
+    int key0 = sinks ? 32 * wave : first;
     bool in_sinks = sinks;
     if (in_sinks && key0 >= sink_end) { in_sinks = false; key0 = first; }
     while (in_sinks || key0 < end) {
@@ -222,47 +247,44 @@ __global__ __launch_bounds__(256, 2) void attn_bias_kernel(const BiasArgs a) {
         o[tt] *= alpha;
         o[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vr[tt]), pb, o[tt], 0, 0, 0);
       }
-      key0 += stride;
+      key0 += 128;
       if (in_sinks && key0 >= sink_end) { in_sinks = false; key0 = first; }
     }
   }
-  float a0 = 1.f, L = l, M_all = m;
-  if (SPLIT) {
-    // merge the four waves; lane (col, kq) of wave 0 holds value dimensions 16 tt + 4 kq + r of column `col`
-    if (wave > 0) {
-#pragma unroll
-      for (int tt = 0; tt < DT; tt++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) xo[wave - 1][16 * tt + 4 * kq + r][col] = o[tt][r];
-      if (kq == 0) { xml[wave - 1][0][col] = m; xml[wave - 1][1][col] = l; }
-    }
-    __syncthreads();
-    if (wave != 0) return;
-    float M = m;
-#pragma unroll
-    for (int w = 0; w < 3; w++) M = fmaxf(M, xml[w][0][col]);
-    const float m_use = (M == -INFINITY) ? 0.f : M;
-    M_all = M;
-    a0 = __expf(m - m_use);
-    float aw[3];
-    L = l * a0;
-#pragma unroll
-    for (int w = 0; w < 3; w++) {
-      aw[w] = __expf(xml[w][0][col] - m_use);
-      L += xml[w][1][col] * aw[w];
-    }
+  // merge the four waves; lane (col, kq) of wave 0 holds value dimensions 16 tt + 4 kq + r of column `col`
+  if (wave > 0) {
 #pragma unroll
     for (int tt = 0; tt < DT; tt++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        float acc = o[tt][r] * a0;
-#pragma unroll
-        for (int w = 0; w < 3; w++) acc += xo[w][16 * tt + 4 * kq + r][col] * aw[w];
-        o[tt][r] = acc;
-      }
+      for (int r = 0; r < 4; r++) xo[wave - 1][16 * tt + 4 * kq + r][col] = o[tt][r];
+    if (kq == 0) { xml[wave - 1][0][col] = m; xml[wave - 1][1][col] = l; }
   }
+  __syncthreads();
+  if (wave != 0) return;
+  float M = m;
+#pragma unroll
+  for (int w = 0; w < 3; w++) M = fmaxf(M, xml[w][0][col]);
+  const float m_use = (M == -INFINITY) ? 0.f : M;
+  const float M_all = M;
+  const float a0 = __expf(m - m_use);
+  float aw[3];
+  float L = l * a0;
+#pragma unroll
+  for (int w = 0; w < 3; w++) {
+    aw[w] = __expf(xml[w][0][col] - m_use);
+    L += xml[w][1][col] * aw[w];
+  }
+#pragma unroll
+  for (int tt = 0; tt < DT; tt++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      float acc = o[tt][r] * a0;
+#pragma unroll
+      for (int w = 0; w < 3; w++) acc += xo[w][16 * tt + 4 * kq + r][col] * aw[w];
+      o[tt][r] = acc;
+    }
   if (!col_ok) return;
-  if (SPLIT && a.chunks > 1) {
+  if (a.chunks > 1) {
     const size_t c = (size_t)blockIdx.z * a.ncols + (size_t)t * a.nq + head;
     float* po = a.parts_o + c * DV + 4 * kq;
 #pragma unroll
@@ -270,33 +292,203 @@ __global__ __launch_bounds__(256, 2) void attn_bias_kernel(const BiasArgs a) {
     if (kq == 0) { a.parts_ml[2 * c] = M_all; a.parts_ml[2 * c + 1] = L; }
     return;
   }
-  // the column's own key is always seen: M_all is finite.  (A sink so far above every key that its exponential overflows
-  // leaves the keys no weight: the output is 0.)
-  if (a.sink) L += __expf((a.sinks ? a.sinks[head] : 0.f) - M_all);
-  float inv = a.out_scale / L;
-  if (a.gate && a.gate_heads) inv *= sigmoid_f32(bf16_to_f32(a.gate[(size_t)t * a.gate_stride + head]));
-  bf16_t* orow = a.out + (size_t)t * a.out_stride + (size_t)head * DV + 4 * kq;
-  const bf16_t* grow = a.gate && !a.gate_heads ? a.gate + (size_t)t * a.gate_stride + (size_t)head * DV + 4 * kq : nullptr;
-#pragma unroll
-  for (int tt = 0; tt < DT; tt++) {
-    float g0 = inv, g1 = inv, g2 = inv, g3 = inv;
-    if (a.out_f32) {
-      float* o32 = reinterpret_cast<float*>(a.out) + (size_t)t * a.out_stride + (size_t)head * DV + 4 * kq + 16 * tt;
-      *reinterpret_cast<f32x4*>(o32) = f32x4{o[tt][0] * g0, o[tt][1] * g1, o[tt][2] * g2, o[tt][3] * g3};
-      continue;
-    }
-    if (grow) {
-      const uint2 gv = *reinterpret_cast<const uint2*>(grow + 16 * tt);
-      g0 *= sigmoid_f32(__uint_as_float(gv.x << 16));
-      g1 *= sigmoid_f32(__uint_as_float(gv.x & 0xffff0000u));
-      g2 *= sigmoid_f32(__uint_as_float(gv.y << 16));
-      g3 *= sigmoid_f32(__uint_as_float(gv.y & 0xffff0000u));
-    }
-    uint2 w;
-    w.x = pack2_bf16(o[tt][0] * g0, o[tt][1] * g1);
-    w.y = pack2_bf16(o[tt][2] * g2, o[tt][3] * g3);
-    *reinterpret_cast<uint2*>(orow + 16 * tt) = w;
+  write_column(a, o, t, head, kq, M_all, L);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Long portions.  A workgroup owns 128 columns of one sequence and kv group, token by token with all heads of the group
+// (columns run on over tokens: no column stays empty because 16 is no multiple of the heads), and brings every key and
+// value to LDS once for all of them.  The next SK keys travel in registers under this tile's products, from there into the
+// other half of LDS: one barrier a tile.  Rows of K lie in the order in which the score tiles want them (see above), with
+// strides that put 16 neighbouring rows on 16 different banks.  The sums are those of one wave over a block's keys in steps
+// of 32, bit for bit; they are scaled only where a maximum rose, and masks looked at only where a tile meets an edge.
+//
+// With a block a wave reading its keys itself, every 16 columns brought all keys through the L2 (12 TB/s of it), which
+// bounded it.  Now LDS and the softmax's chain do: eight waves, two a SIMD, read 36 KB each for 32 keys of 320 and values of
+// 256.  Four waves of two blocks halve that and were slower, one wave a SIMD hides nothing (377 against 203 us below).
+// Microseconds before / now, 2,048 tokens: 12 heads of 320 and 256 over one 271 / 203, behind 4,096 others 947 / 573; 28
+// heads 444 / 206; two maps of 12 heads of 64 and 128 168 / 94; 12 heads of 128 over 2 in chunks of 1,024 78 / 47, capped with
+// a window of 1,024 91 / 68.
+// ---------------------------------------------------------------------------------------------------------------------
+constexpr int SK = DK + DV <= 256 ? 64 : 32;            // keys of a stage
+constexpr int ST_WAVES = 8, ST_COLS = 16 * ST_WAVES, ST_NT = 64 * ST_WAVES;
+constexpr int ST_KROW = DK + 8, ST_VROW = SK + 8;
+constexpr int ST_BYTES = (SK * ST_KROW + DV * ST_VROW) * 2;
+constexpr int ST_KC = SK * DK / 8, ST_VC = DV * SK / 8;  // pieces of 16 bytes of a stage
+constexpr int ST_NK = (ST_KC + ST_NT - 1) / ST_NT, ST_NV = (ST_VC + ST_NT - 1) / ST_NT;
+
+__global__ __launch_bounds__(ST_NT, DK <= 128 && DV <= 128 ? 4 : 2) void attn_bias_staged_kernel(const BiasArgs a) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t st_smem[];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, kq = lane >> 4;
+  const int g = blockIdx.y, R = a.nq / a.nkv;
+  // which columns of which sequence: tiles are counted sequence by sequence, the ones with the most keys first
+  int tile = blockIdx.x, b = 0, t_begin = 0, ntok = 0, tiles = 0;
+  for (; b < a.num_seqs; b++) {
+    t_begin = a.cu_seqlens[b];
+    ntok = a.cu_seqlens[b + 1] - t_begin;
+    tiles = (ntok * R + ST_COLS - 1) / ST_COLS;
+    if (tile < tiles) break;
+    tile -= tiles;
   }
+  if (b == a.num_seqs) return;
+  tile = tiles - 1 - tile;
+  const int ncol = ntok * R, c_first = tile * ST_COLS, c_last = min(c_first + ST_COLS, ncol) - 1;
+  const int p_seq = a.positions[t_begin];
+  const int p_lo = p_seq + c_first / R, p_hi = p_seq + c_last / R;       // first and last position of the workgroup
+  const int hi = p_hi + 1;
+  const int lo = a.chunk > 0 ? p_lo / a.chunk * a.chunk : a.window > 0 ? max(0, p_lo - a.window + 1) : 0;
+  const int keep = a.window > 0 ? a.keep_first : 0;
+  const int gv = g / a.v_div, nv = a.nkv / a.v_div;
+  const float inv_cap = a.softcap > 0.f ? 1.0f / a.softcap : 0.f;
+  const int* bt = a.block_table + (size_t)b * a.max_pages;
+  const int pshift = 31 - __clz(a.P);
+  const int last_key = hi - 1, last_group = last_key / 8 * 8;
+
+  const int c = c_first + wave * 16 + col, cc = min(c, c_last), tok = cc / R;
+  const int t = t_begin + tok, head = g * R + cc - tok * R, my_pos = p_seq + tok;
+  const int my_lo = a.chunk > 0 ? my_pos / a.chunk * a.chunk : a.window > 0 ? max(0, my_pos - a.window + 1) : 0;
+  float qscale = a.scale, slope = 0.f, m = -INFINITY, l = 0.f;
+  if (a.temp_every > 0) qscale *= 1.0f + a.temp_coef * logf((float)((my_pos + 1) / a.temp_every + 1));
+  if (a.slope_span > 0.f) slope = exp2f(-a.slope_span * (float)(head + 1) / (float)a.nq);
+  bf16x8 qf[KS];
+  const bf16_t* qrow = a.q + (size_t)t * a.q_stride + (size_t)head * DK + 8 * kq;
+#pragma unroll
+  for (int st = 0; st < KS; st++) qf[st] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qrow + 32 * st));
+  f32x4 o[DT];
+#pragma unroll
+  for (int tt = 0; tt < DT; tt++) o[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // of the wave's columns (the same for all lanes): the lowest and highest position, the highest first key
+  const int c_wave = c_first + wave * 16, c_wend = min(c_wave + 15, c_last);
+  const bool any = c_wave <= c_last;
+  const int w_lo = p_seq + min(c_wave, c_last) / R, w_hi = p_seq + c_wend / R;
+  const int w_first = a.chunk > 0 ? w_hi / a.chunk * a.chunk : a.window > 0 ? max(0, w_hi - a.window + 1) : 0;
+
+  // a stage's pages are looked up a stage before it is fetched: a fetch is one latency, not two
+  uint4 kr[ST_NK], vr[ST_NV];
+  int kpage[ST_NK], vpage[ST_NV];
+  auto lookup = [&](int key0) {
+#pragma unroll
+    for (int i = 0; i < ST_NK; i++) kpage[i] = bt[min(key0 + min(tid + ST_NT * i, ST_KC - 1) / (DK / 8), last_key) >> pshift];
+#pragma unroll
+    for (int i = 0; i < ST_NV; i++) vpage[i] = bt[min(key0 + min(tid + ST_NT * i, ST_VC - 1) % (SK / 8) * 8, last_group) >> pshift];
+  };
+  auto fetch = [&](int key0) {
+#pragma unroll
+    for (int i = 0; i < ST_NK; i++) {
+      const int c = min(tid + ST_NT * i, ST_KC - 1), pos = min(key0 + c / (DK / 8), last_key), page = min(max(kpage[i], 0), a.num_pages - 1);
+      kr[i] = *reinterpret_cast<const uint4*>(a.k_cache + ((((size_t)page * a.nkv + g) << pshift) + (pos & (a.P - 1))) * DK + c % (DK / 8) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < ST_NV; i++) {
+      const int c = min(tid + ST_NT * i, ST_VC - 1), pos = min(key0 + c % (SK / 8) * 8, last_group), page = min(max(vpage[i], 0), a.num_pages - 1);
+      vr[i] = *reinterpret_cast<const uint4*>(a.v_cache + ((((size_t)page * nv + gv) * DV + c / (SK / 8)) << pshift) + (pos & (a.P - 1)));
+    }
+  };
+  auto commit = [&](int buf, int key0) {
+    bf16_t* ks = st_smem + buf * (ST_BYTES / 2);
+    bf16_t* vs = ks + SK * ST_KROW;
+#pragma unroll
+    for (int i = 0; i < ST_NK; i++) {
+      const int c = tid + ST_NT * i, key = c / (DK / 8);
+      const int row = (key & ~31) + ((key >> 2) & 1) * 16 + ((key & 31) >> 3) * 4 + (key & 3);
+      if (ST_KC % ST_NT == 0 || c < ST_KC) *reinterpret_cast<uint4*>(ks + row * ST_KROW + c % (DK / 8) * 8) = kr[i];
+    }
+    const bool edge = key0 + SK > hi || key0 < lo;
+#pragma unroll
+    for (int i = 0; i < ST_NV; i++) {
+      const int c = tid + ST_NT * i;
+      uint4 v = vr[i];
+      if (edge) {
+        // values of keys outside the range hold whatever the page held before: zero (0 * NaN is NaN)
+        const int k = key0 + c % (SK / 8) * 8;
+        uint32_t live[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int k0 = k + 2 * j, k1 = k0 + 1;
+          const bool v0 = k0 < hi && (k0 >= lo || k0 < keep), v1 = k1 < hi && (k1 >= lo || k1 < keep);
+          live[j] = (v0 ? 0x0000ffffu : 0u) | (v1 ? 0xffff0000u : 0u);
+        }
+        v = make_uint4(v.x & live[0], v.y & live[1], v.z & live[2], v.w & live[3]);
+      }
+      if (ST_VC % ST_NT == 0 || c < ST_VC) *reinterpret_cast<uint4*>(vs + c / (SK / 8) * ST_VROW + c % (SK / 8) * 8) = v;
+    }
+  };
+
+  // kept first keys in front of the window's first tile are tiles of their own
+  const int begin = lo & ~(SK - 1), sink_end = min(keep, begin);
+  auto after = [&](int k) { return k < begin && k + SK >= sink_end ? begin : k + SK; };
+  int key0 = sink_end > 0 ? 0 : begin, next = after(key0);
+  lookup(key0);
+  fetch(key0);
+  lookup(next);
+  commit(0, key0);
+  int buf = 0;
+  while (true) {
+    const bool more = next < hi;
+    __syncthreads();
+    if (more) {
+      fetch(next);
+      lookup(after(next));
+    }
+    const bf16_t* ks = st_smem + buf * (ST_BYTES / 2) + col * ST_KROW + 8 * kq;
+    const bf16_t* vs = st_smem + buf * (ST_BYTES / 2) + SK * ST_KROW + col * ST_VROW + 8 * kq;
+#pragma unroll
+    for (int u = 0; u < SK; u += 32) {
+      const int k0 = key0 + u;
+      if (!any || k0 > w_hi) continue;                    // (nothing that a column of this wave sees)
+      f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+      for (int st = 0; st < KS; st++) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(ks + u * ST_KROW + 32 * st), qf[st], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(ks + (u + 16) * ST_KROW + 32 * st), qf[st], s1, 0, 0, 0);
+      }
+      float sv[8], mx = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        float v = (r < 4 ? s0[r & 3] : s1[r & 3]) * qscale - slope * (float)(my_pos - (k0 + 8 * kq + r));
+        if (a.softcap > 0.f) v = a.softcap * tanhf(v * inv_cap);
+        sv[r] = v;
+      }
+      if (k0 + 31 > w_lo || k0 < w_first) {
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+          const int key = k0 + 8 * kq + r;
+          if (key > my_pos || (key < my_lo && key >= keep)) sv[r] = -INFINITY;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 8; r++) mx = fmaxf(mx, sv[r]);
+      mx = max_across_16(mx);
+      mx = max_across_32(mx);
+      const float m_new = fmaxf(m, mx), m_use = m_new == -INFINITY ? 0.f : m_new;      // a column that has seen no key yet
+      const float alpha = __expf(m - m_use);
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        sv[r] = __expf(sv[r] - m_use);
+        sum += sv[r];
+      }
+      sum = sum_across_16(sum);
+      sum = sum_across_32(sum);
+      l = l * alpha + sum;
+      if (__any(m_new > m)) {
+#pragma unroll
+        for (int tt = 0; tt < DT; tt++) o[tt] *= alpha;
+      }
+      m = m_new;
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, make_uint4(pack2_bf16(sv[0], sv[1]), pack2_bf16(sv[2], sv[3]),
+                                                               pack2_bf16(sv[4], sv[5]), pack2_bf16(sv[6], sv[7])));
+#pragma unroll
+      for (int tt = 0; tt < DT; tt++)
+        o[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(vs + tt * 16 * ST_VROW + u), pb, o[tt], 0, 0, 0);
+    }
+    if (!more) break;
+    commit(buf ^ 1, next);
+    buf ^= 1;
+    key0 = next;
+    next = after(next);
+  }
+  if (c <= c_last) write_column(a, o, t, head, kq, m, l);
 }
 
 #define MAX_PIECES 64
@@ -332,7 +524,8 @@ __global__ __launch_bounds__(DV <= 64 ? 64 : DV <= 128 ? 128 : 256) void attn_bi
   else out[at] = f32_to_bf16(v);
 }
 
-// split != 0: one block of 16 columns a workgroup, its keys shared by the four waves; else four blocks a workgroup.
+// split != 0: one block of 16 columns a workgroup, its keys shared by the four waves; else 128 columns a workgroup, keys and
+// values through LDS.
 extern "C" int pico_attnb(const void* q, int q_stride, const void* k_cache, const void* v_cache, const int* block_table,
                           int max_pages, const int* cu_seqlens, const int* positions, int num_seqs, int T, void* out,
                           int nq, int nkv, int dk, int dv, int P, int num_pages, float scale, int window, float temp_coef,
@@ -367,14 +560,18 @@ extern "C" int pico_attnb(const void* q, int q_stride, const void* k_cache, cons
              slope_span, chunks, T * nq, parts_o, parts_ml, softcap, keep_first, (const bf16_t*)gate, gate_stride,
              chunk, sink, gate_heads, v_div, out_f32, sinks, out_scale, out_stride};
   if (split) {
-    attn_bias_kernel<true><<<dim3((unsigned)tiles, nkv, chunks), 256, 0, stream>>>(a);
+    attn_bias_kernel<<<dim3((unsigned)tiles, nkv, chunks), 256, 0, stream>>>(a);
     if (chunks > 1 && out)                               // (no output: the caller puts the pieces together)
       attn_bias_merge_kernel<<<T * nq, DV <= 64 ? 64 : DV <= 128 ? 128 : 256, 0, stream>>>(parts_o, parts_ml, chunks, T * nq,
                                                                                            (bf16_t*)out, (const bf16_t*)gate,
                                                                                            gate_stride, nq, sink, gate_heads, out_f32, sinks,
                                                                                            out_scale, out_stride);
-  } else
-    attn_bias_kernel<false><<<dim3((unsigned)((tiles + 3) / 4), nkv), 256, 0, stream>>>(a);
+  } else {
+    static const hipError_t room = hipFuncSetAttribute((const void*)&attn_bias_staged_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * ST_BYTES);
+    PICO_REQUIRE(room == hipSuccess, "pico_attnb: %s", hipGetErrorString(room));
+    const long long wgs = ((long long)T * R + ST_COLS - 1) / ST_COLS + num_seqs;      // every sequence's last may be partly empty
+    attn_bias_staged_kernel<<<dim3((unsigned)wgs, nkv), ST_NT, 2 * ST_BYTES, stream>>>(a);
+  }
   PICO_LAUNCH_CHECK();
   return 0;
 }

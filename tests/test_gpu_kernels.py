@@ -1258,3 +1258,24 @@ def test_the_library_product_with_its_tuner_on_gives_the_same_and_hands_the_mode
     for got, ref in ((before, want), (tuned, want), (other, want[:300]), (no_bias, want[:512] - b.bfloat16().double())):
         assert got.dtype == torch.bfloat16
         assert torch.allclose(got.cpu().double(), ref, rtol=1e-2, atol=1e-2 * math.sqrt(320))
+
+
+@pytest.mark.parametrize("nq,nkv,dk,dv,more", [(12, 1, 320, 256, {}), (6, 2, 64, 128, {"window": 50, "keep_first": 5, "softcap": 20.0}),
+                                               (5, 5, 128, 16, {"chunk": 64, "sink": True}), (40, 2, 32, 96, {"slope_span": 8.0})])
+@pytest.mark.parametrize("lens,prefix", [([1], 0), ([11, 10], 0), ([65, 1, 130], 37), ([3, 300], 500)])
+@pytest.mark.parametrize("Pg", [8, 64])
+def test_bias_attention_shared_keys(nq, nkv, dk, dv, more, lens, prefix, Pg):
+    # 128 columns that share staged keys (columns run over tokens whatever the heads a group), against blocks whose keys four
+    # waves share: edges of workgroups, of stages of 32 and 64 keys, of windows, kept keys and chunks, several sequences
+    from pico_vllm_amd.ops.attention_bias_fast import FastBiasAttention
+    fast = FastBiasAttention(nq, nkv, dk, dv, dk ** -0.5, **more)
+    g = torch.Generator(device=DEV).manual_seed(dk + len(lens))
+    B, T, per = len(lens), sum(lens), -(-(max(lens) + prefix) // Pg)
+    kc, vc = (torch.randn(B * per + 3, nkv, *s, device=DEV, generator=g).bfloat16() for s in ((Pg, dk), (dv, Pg)))
+    bt = torch.randperm(B * per + 3, device=DEV, generator=g)[:B * per].int().reshape(B, per).contiguous()
+    q = torch.randn(T, nq * dk, device=DEV, generator=g).bfloat16()
+    cu = torch.tensor([0] + [sum(lens[:i + 1]) for i in range(B)], dtype=torch.int32, device=DEV)
+    pos = torch.cat([torch.arange(prefix, prefix + n) for n in lens]).int().to(DEV)
+    got, want = (fast.run(q, kc, vc, bt, cu, pos, B, split=s, chunks=1).double() for s in (False, True))
+    # both round probabilities (2^-9 each, against maxima that may differ) and the output to bfloat16
+    assert float((got - want).abs().max()) <= 2.0 ** -7 * float(vc.float().abs().max())
