@@ -76,7 +76,8 @@ extern "C" int pico_delta_prep(const void* x, int ldx, int q_col, int k_col, con
   return 0;
 }
 
-// grid (T); bc: the convolved B | C (columns b_col .., c_col .., n each); dt_raw: H columns of y from dt_col.
+// grid (T); bc: the convolved B | C (columns b_col .., c_col .., n each; not widened where bf is null); dt_raw: H columns of y
+// from dt_col.
 template <typename T>
 __global__ __launch_bounds__(256) void ssd_prep_kernel(const T* __restrict__ bc, int ldb, int b_col, int c_col, int n,
                                                        const T* __restrict__ y, int ldy, int dt_col,
@@ -85,7 +86,7 @@ __global__ __launch_bounds__(256) void ssd_prep_kernel(const T* __restrict__ bc,
                                                        float* __restrict__ dt, int H) {
   const int t = blockIdx.x;
   const T* br = bc + (size_t)t * ldb;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+  for (int i = threadIdx.x; bf && i < n; i += blockDim.x) {
     bf[(size_t)t * n + i] = load_f32(br + b_col + i);
     cf[(size_t)t * n + i] = load_f32(br + c_col + i);
   }

@@ -916,11 +916,38 @@ def _decay_chunks(x, q_col, k_col, v_col, cu_seqlens, state_slots, state, num_se
     """``gla_scan`` with a constant decay a head, its sequences in chunks on the matrix cores (operands checked there)."""
     lib = library.core()
     T = x.shape[0]
-    max_chunks = -(-T // DECAY_CHUNK)
-    ws = torch.empty(num_seqs * max_chunks, heads, dk, dv, dtype=torch.float32, device=x.device)
+    chunks = T // DECAY_CHUNK + num_seqs
+    ws = torch.empty(chunks, heads, dk, dv, dtype=torch.float32, device=x.device)
     _check(lib, lib.pico_decay_chunks(_ptr(x), x.stride(0) if T > 1 else x.shape[1], q_col, k_col, v_col, _ptr(cu_seqlens),
                                       _ptr(state_slots), _ptr(head_decay), _ptr(state), _ptr(out), _ptr(ws), num_seqs, T, heads, dk, dv,
-                                      c_float(qscale), state.shape[0], max_chunks, 1 if silu else 0, _stream()))
+                                      c_float(qscale), state.shape[0], chunks, 1 if silu else 0, _stream()))
+    return out
+
+
+def ssd_chunks(x: torch.Tensor, q_col: int, k_col: int, v_col: int, g: torch.Tensor, beta: torch.Tensor, cu_seqlens: torch.Tensor,
+               state_slots: torch.Tensor, state: torch.Tensor, num_seqs: int, heads: int, kv_heads: int, dk: int, dv: int) -> torch.Tensor:
+    """``delta_scan`` without the delta rule and with one decay a head, its sequences in chunks on the matrix cores (float32
+    products): q, k and v are columns of bfloat16 rows x (``decay_chunks_ok``), g and beta float32 [T, heads]."""
+    _gpu(x, g, beta, cu_seqlens, state_slots, state)
+    T = x.shape[0]
+    if x.dim() != 2 or x.stride(1) != 1 or not decay_chunks_ok(x, q_col, k_col, v_col, dk, dv) or heads % kv_heads \
+            or x.shape[1] < max(q_col + kv_heads * dk, k_col + kv_heads * dk, v_col + heads * dv):
+        raise KernelError("ssd_chunks: bfloat16 rows that hold q, k and v in whole aligned eights, keys of up to 128")
+    for t in (g, beta):
+        if t.dtype != torch.float32 or tuple(t.shape) != (T, heads) or not t.is_contiguous():
+            raise KernelError(f"ssd_chunks: decays and factors are contiguous float32 [T, {heads}]")
+    if state.dtype != torch.float32 or state.dim() != 4 or tuple(state.shape[1:]) != (heads, dk, dv) or not state.is_contiguous():
+        raise KernelError(f"ssd_chunks: the state must be contiguous float32 [slots, {heads}, {dk}, {dv}]")
+    _i32(cu_seqlens, "cu_seqlens", num_seqs + 1)
+    _i32(state_slots, "state_slots", num_seqs)
+    chunks = T // DECAY_CHUNK + num_seqs
+    out = torch.empty(T, heads * dv, dtype=torch.float32, device=x.device)
+    ws = torch.empty(chunks, heads, dk, dv, dtype=torch.float32, device=x.device)
+    ws_decay = torch.empty(chunks, heads, dtype=torch.float32, device=x.device)
+    lib = library.core()
+    _check(lib, lib.pico_ssd_chunks(_ptr(x), x.stride(0) if T > 1 else x.shape[1], q_col, k_col, v_col, _ptr(cu_seqlens), _ptr(state_slots),
+                                    _ptr(g), _ptr(beta), _ptr(state), _ptr(out), _ptr(ws), _ptr(ws_decay), num_seqs, T, heads, heads // kv_heads,
+                                    dk, dv, state.shape[0], chunks, _stream()))
     return out
 
 
@@ -1668,8 +1695,9 @@ def delta_prep(x: torch.Tensor, q_col: int, k_col: int, y: torch.Tensor, b_col: 
 
 
 def ssd_prep(bc: torch.Tensor, b_col: int, c_col: int, n: int, y: torch.Tensor, dt_col: int, dt_bias: torch.Tensor,
-             a_log: torch.Tensor, heads: int):
-    """What enters a state-space walk, in float32: B and C (n columns each of bc from b_col, c_col) widened;
+             a_log: torch.Tensor, heads: int, widen: bool = True):
+    """What enters a state-space walk, in float32: B and C (n columns each of bc from b_col, c_col) widened (None without
+    ``widen``);
     dt = softplus(y[:, dt_col : dt_col + heads] + dt_bias) and the decay exp(-exp(a_log) dt), both [T, heads]."""
     _gpu(bc, y, dt_bias, a_log)
     T = bc.shape[0]
@@ -1679,8 +1707,8 @@ def ssd_prep(bc: torch.Tensor, b_col: int, c_col: int, n: int, y: torch.Tensor, 
         raise KernelError("ssd_prep: the rows do not hold what is read")
     _vec(dt_bias, heads, "dt bias"); _vec(a_log, heads, "A_log")
     dev = bc.device
-    bf = torch.empty(T, n, dtype=torch.float32, device=dev)
-    cf = torch.empty(T, n, dtype=torch.float32, device=dev)
+    bf = torch.empty(T, n, dtype=torch.float32, device=dev) if widen else None
+    cf = torch.empty(T, n, dtype=torch.float32, device=dev) if widen else None
     g = torch.empty(T, heads, dtype=torch.float32, device=dev)
     dt = torch.empty(T, heads, dtype=torch.float32, device=dev)
     lib = library.core()

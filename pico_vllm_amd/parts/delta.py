@@ -193,7 +193,15 @@ class StateSpaceDuality(Mixer):
         gn = self.groups * self.n
         y = self.in_proj(x)                                 # [T, z | x | B | C | dt]
         xbc = kernels.causal_conv(y[:, self.inner:], self.channels, self.conv_w, self.conv_b, ctx, hist.state, 0, single=ctx.all_decode)
-        bf, cf, g, dt = kernels.ssd_prep(xbc, self.inner, self.inner + gn, gn, y, self.dt_col, self.dt_bias, self.a_log, self.heads)
-        o = kernels.delta_scan(cf, bf, xbc, g, dt, ctx.cu_seqlens, ctx.state_slots, state.state, ctx.num_seqs, self.heads,
-                               self.groups, self.n, self.dv, delta=False, chunk=_chunk(self.act_dtype, ctx))
+        chunk = _chunk(self.act_dtype, ctx)
+        # prompt portions in chunks on the matrix cores where their sizes allow it, straight from the convolved rows
+        products = chunk == kernels.DECAY_CHUNK and kernels.decay_chunks_ok(xbc, self.inner + gn, self.inner, 0, self.n, self.dv)
+        bf, cf, g, dt = kernels.ssd_prep(xbc, self.inner, self.inner + gn, gn, y, self.dt_col, self.dt_bias, self.a_log, self.heads,
+                                         widen=not products)
+        if products:
+            o = kernels.ssd_chunks(xbc, self.inner + gn, self.inner, 0, g, dt, ctx.cu_seqlens, ctx.state_slots, state.state, ctx.num_seqs,
+                                   self.heads, self.groups, self.n, self.dv)
+        else:
+            o = kernels.delta_scan(cf, bf, xbc, g, dt, ctx.cu_seqlens, ctx.state_slots, state.state, ctx.num_seqs, self.heads,
+                                   self.groups, self.n, self.dv, delta=False, chunk=chunk)
         return kernels.gated_group_norm(o, xbc, y, self.d, self.norm_weight, self.norm_eps, self.heads, self.dv, self.norm_groups)

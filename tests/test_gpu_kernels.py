@@ -1279,3 +1279,38 @@ def test_bias_attention_shared_keys(nq, nkv, dk, dv, more, lens, prefix, Pg):
     got, want = (fast.run(q, kc, vc, bt, cu, pos, B, split=s, chunks=1).double() for s in (False, True))
     # both round probabilities (2^-9 each, against maxima that may differ) and the output to bfloat16
     assert float((got - want).abs().max()) <= 2.0 ** -7 * float(vc.float().abs().max())
+
+
+@pytest.mark.parametrize("H,G,dk,dv", [(4, 2, 128, 64), (6, 1, 40, 72), (3, 3, 96, 128)])
+@pytest.mark.parametrize("lens", [[1], [64, 63], [65, 1, 200], [130]])
+@pytest.mark.parametrize("steps", [(0.01, 0.2), (0.5, 60.0)])
+def test_ssd_chunks(K, H, G, dk, dv, lens, steps):
+    # a decay a token and head, from slow ones to ones that a float cannot hold, over the edges of chunks of 64 and several
+    # sequences, against the walk token by token in 64 bits
+    g = torch.Generator().manual_seed(dk + sum(lens))
+    T, B = sum(lens), len(lens)
+    x = torch.randn(T, H * dv + 2 * G * dk, generator=g).bfloat16()
+    dt = torch.empty(T, H).uniform_(*steps, generator=g)
+    a = torch.empty(H).uniform_(0.5, 4.5, generator=g)
+    decay = torch.exp(-a * dt)
+    state = torch.randn(B + 1, H, dk, dv, generator=g)
+    cu = torch.tensor([0] + [sum(lens[:i + 1]) for i in range(B)], dtype=torch.int32)
+    slots = torch.arange(B, 0, -1, dtype=torch.int32)
+    st = state.to(DEV)
+    out = K.ssd_chunks(x.to(DEV), H * dv + G * dk, H * dv, 0, decay.to(DEV), dt.to(DEV), cu.to(DEV), slots.to(DEV), st, B, H, G, dk, dv).cpu().double()
+    v, k, q = x[:, :H * dv].double().view(T, H, dv), x[:, H * dv:H * dv + G * dk].double().view(T, G, dk), x[:, H * dv + G * dk:].double().view(T, G, dk)
+    k, q = k.repeat_interleave(H // G, 1), q.repeat_interleave(H // G, 1)
+    for b in range(B):
+        S = state[slots[b]].double()
+        size = S.abs()                              # the same sums of absolute values: what rounding is relative to
+        for t in range(cu[b], cu[b + 1]):
+            w = decay[t].double().view(H, 1, 1)
+            add = k[t].unsqueeze(-1) * (dt[t].double().view(H, 1) * v[t]).unsqueeze(1)
+            S, size = w * S + add, w * size + add.abs()
+            bound = (size * q[t].abs().unsqueeze(-1)).sum(1)
+            # sums of up to dk + 64 float32 products of float32 products: 2^-24 of the absolute sums a rounding, at most
+            # some twenty in a row (chains of 64 at random, decays and factors)
+            err = (out[t].view(H, dv) - (S * q[t].unsqueeze(-1)).sum(1)).abs()
+            assert bool((err <= 20 * 2.0 ** -24 * bound + 1e-30).all())
+        assert bool(((st[slots[b]].cpu().double() - S).abs() <= 20 * 2.0 ** -24 * size + 1e-30).all())
+    assert torch.equal(st[0].cpu(), state[0])       # a slot that no sequence holds
