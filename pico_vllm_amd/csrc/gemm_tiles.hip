@@ -40,14 +40,6 @@ __device__ __forceinline__ float gt_one(float v) {
   return EPI == GT_GELU ? gelu_erf_f(v) : v;
 }
 
-// Tile `t` of the order in which tiles are dealt out: strips of up to 8 tiles of rows, inside a strip column by column, so
-// that the 32 tiles a die works on at a time are about 8 x 4 and share their operands in its L2.
-__device__ __forceinline__ void gt_place(const GemmArgs& a, int t, int& m, int& n) {
-  const int per = 8 * a.n_tiles, strip = t / per, rest = t - strip * per, rows = min(8, a.m_tiles - strip * 8);
-  n = rest / rows;
-  m = strip * 8 + rest - n * rows;
-}
-
 template <int MB, int NB, int EPI>
 __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const GemmArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
@@ -55,19 +47,13 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
   typedef TileStream<MB, NB> TS;
   TS ts(smem);
   constexpr int TM = 64 * MB, TN = 64 * NB, COLS = gt_paired(EPI) ? TN / 2 : TN;      // output columns of a tile
-  const int tiles = a.m_tiles * a.n_tiles, step = gridDim.x;
-  // workgroups go to the dies in turn; a die's share of a round is a run of neighbouring tiles
-  const int first = gridDim.x % 8 == 0 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int tiles = a.m_tiles * a.n_tiles, first = ts_first();
   if (first >= tiles) return;
-  const int stages = (a.K + TS_BK - 1) / TS_BK;
-
-  // the stage that is asked for next
-  int at_tile = first, at_stage = 0;
   TileRowsSource<MB> xs;
   TileRowsSource<NB> ws;
   auto aim = [&](int t) {
     int m, n;
-    gt_place(a, t, m, n);
+    ts_place(a.m_tiles, a.n_tiles, t, m, n);
     const int m0 = m * TM;
     xs.rsrc = ts_buffer(a.X + (size_t)m0 * a.ldx, ((long long)(a.M - m0 - 1) * a.ldx + a.K) * 2);
 #pragma unroll
@@ -88,39 +74,10 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
       for (int j = 0; j < 2 * NB; j++) ws.off[j] = (uint32_t)(ts.row(j) * a.ldw) * 2;
     }
   };
-  // copies of the next stage into buffer b, and on to the one behind it
-  int fill = 0;
-  auto copies = [&](auto r) { ts.template ask<decltype(r)::from, decltype(r)::to>(fill, xs, ws, at_tile < tiles ? at_stage * TS_BK : a.K, a.K); };
-  auto on = [&] {
-    fill = fill + 1 == TS::NBUF ? 0 : fill + 1;
-    if (++at_stage == stages && at_tile < tiles) {
-      at_stage = 0;
-      at_tile += step;
-      if (at_tile < tiles) aim(at_tile);
-    }
-  };
-  aim(first);
-#pragma unroll
-  for (int b = 0; b < TS::NBUF - 1; b++) {
-    copies(Range<0, TS::LOADS>());
-    on();
-  }
-  __builtin_amdgcn_s_waitcnt(ts_wait((TS::NBUF - 2) * TS::LOADS, true));
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  copies(Range<0, TS::part(1)>());
-  ts.read(0, 0, 0);
-  int buf = 0;
-  for (int t = first; t < tiles; t += step) {
-    ts.clear();
-    for (int s = 0; s < stages; s++) {
-      const int next = buf + 1 == TS::NBUF ? 0 : buf + 1;
-      ts.stage(buf, next, copies, on);
-      buf = next;
-    }
+  ts.run(first, gridDim.x, tiles, a.K, xs, ws, aim, [&](int t) {
     // lane (l, h): row l of a block of X, tile rows 8 (r / 4) + 4 h + r % 4 of a block of W in register r
     int mt, nt;
-    gt_place(a, t, mt, nt);
+    ts_place(a.m_tiles, a.n_tiles, t, mt, nt);
     const int l = ts.lane & 31, h = ts.lane >> 5;
 #pragma unroll
     for (int i = 0; i < MB; i++) {
@@ -169,8 +126,7 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
         }
       }
     }
-  }
-  __builtin_amdgcn_s_waitcnt(ts_wait(0, true));          // the last copies (zeros) are in before LDS is given back
+  });
 #endif
 }
 

@@ -3,27 +3,24 @@
 // Few rows (a row is one (token, chosen expert) pair; single tokens and small steps): every row streams its expert's
 // matrices once, 16 bytes a lane, sixteen lanes to an output element.
 //
-// Many rows (prompt portions): the rows are sorted by expert on the device (nothing comes back to the host), every
-// expert's rows padded to whole tiles of MOE_BM rows, and two grouped products run on the matrix cores, their operands
-// staged through LDS:
-//   first:  y[p, f] = act(gate_e[f] . x_p, up_e[f] . x_p),  x_p = bf16(w_p * h[token of p])   (gathered while staging)
-//   second: out[slot of p][token of p][n] = down_e[n] . y[p]                                   (float32, scattered)
+// More rows: they are sorted by expert on the device (nothing comes back to the host), every expert's rows padded to whole
+// tiles, and two grouped products run on the matrix cores, tiles as tile_stream.h has them:
+//   first:  y[p, f] = act(gate_e[f] . h[token of p], up_e[f] . h[token of p], w_p)      (rows gathered by the copies to LDS)
+//   second: out[slot of p][token of p][n] = down_e[n] . y[p]                             (float32, scattered)
+// While experts have few rows the matrices' stream bounds it: 128 rows over 32 experts of 4,736 x 3,584, 368 and 188 us the two
+// products (5.8 TB/s) against 478 and 250 with operands that pass through registers; from about 100 rows an expert the
+// latency of the copies: 4,096 rows over 16 experts of 2,240 x 1,536 92 and 47 us against 145 and 75, 2,754 rows 93 and 48
+// against 101 and 54 (tiles of 128 rows are 69 and 65 percent full then).
+//
 // A row's result does not depend on which other rows share its tile: a matrix instruction keeps rows apart and the sums
 // over k run in the same order for every row.
-#include "common.h"
+#include "tile_stream.h"
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-#define MOE_BM 128         // rows of a tile
-#define MOE_BN 128         // matrix rows (output columns) of a tile
-#define MOE_BK 64          // k of one stage
-#define MOE_LD 72          // LDS row stride in bfloat16: 144 bytes, a multiple of 16 that spreads rows over the banks
-
-// mode 0: the clipped activation, the row's weight w already in the input; mode 1: w silu(g) u (the weight on the
-// expert's output, taken in front of the linear second product); mode 2: w times the clipped activation
+// mode 0: the clipped activation, the row's weight w on its input; mode 1: w silu(g) u (the weight on the expert's
+// output, taken in front of the linear second product); mode 2: w times the clipped activation
 __device__ __forceinline__ float moe_act(float g, float u, float limit, float alpha, int mode, float w) {
   if (mode == 1) return w * (g / (1.0f + expf(-g))) * u;
+  if (mode == 0) { g *= w; u *= w; }
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
   return (mode == 2 ? w : 1.0f) * (g / (1.0f + expf(-alpha * g)) * (u + 1.0f));
@@ -34,24 +31,6 @@ __device__ __forceinline__ void unpack8(const uint4& v, float* f) {
   f[2] = __uint_as_float(v.y << 16); f[3] = __uint_as_float(v.y & 0xffff0000u);
   f[4] = __uint_as_float(v.z << 16); f[5] = __uint_as_float(v.z & 0xffff0000u);
   f[6] = __uint_as_float(v.w << 16); f[7] = __uint_as_float(v.w & 0xffff0000u);
-}
-
-// 8 bfloat16 times w, each rounded to bfloat16 again
-__device__ __forceinline__ uint4 scale8(const uint4& v, float w) {
-  float f[8];
-  unpack8(v, f);
-  uint4 o;
-  o.x = pack2_bf16(f[0] * w, f[1] * w);
-  o.y = pack2_bf16(f[2] * w, f[3] * w);
-  o.z = pack2_bf16(f[4] * w, f[5] * w);
-  o.w = pack2_bf16(f[6] * w, f[7] * w);
-  return o;
-}
-
-// v where keep, else zeros (component by component: the values stay in registers)
-__device__ __forceinline__ uint4 keep8(const uint4& v, bool keep) {
-  const uint32_t m = keep ? 0xffffffffu : 0u;
-  return make_uint4(v.x & m, v.y & m, v.z & m, v.w & m);
 }
 
 __device__ __forceinline__ float dot8(const uint4& a, const float* x, float acc) {
@@ -83,16 +62,14 @@ __global__ __launch_bounds__(256) void moe_up_rows_kernel(const bf16_t* __restri
   const int f = blockIdx.y * 16 + (threadIdx.x >> 4);
   const int e = experts[r];
   if (e < 0 || e >= E || f >= F) return;
-  const float wr = weights[r];
-  const float w = mode != 0 ? 1.f : wr;
+  const float w = weights[r];
   const bf16_t* x = h + (size_t)(r / top) * ldh;
   const bf16_t* wg = gate_up + ((size_t)e * 2 * F + f) * D;
   const bf16_t* wu = wg + (size_t)F * D;
   float g = 0.f, u = 0.f;
 #pragma unroll 2
   for (int k = sub * 8; k < D; k += 128) {
-    const uint4 x8 = *reinterpret_cast<const uint4*>(x + k);
-    const uint4 xv = mode != 0 ? x8 : scale8(x8, w);
+    const uint4 xv = *reinterpret_cast<const uint4*>(x + k);
     const uint4 gv = *reinterpret_cast<const uint4*>(wg + k);
     const uint4 uv = *reinterpret_cast<const uint4*>(wu + k);
     float xf[8];
@@ -102,7 +79,7 @@ __global__ __launch_bounds__(256) void moe_up_rows_kernel(const bf16_t* __restri
   }
   g = row16_sum(g);
   u = row16_sum(u);
-  if (sub == 0) y[(size_t)r * F + f] = f32_to_bf16(moe_act(g, u, limit, alpha, mode, wr));
+  if (sub == 0) y[(size_t)r * F + f] = f32_to_bf16(moe_act(g, u, limit, alpha, mode, w));
 }
 
 // ---------------------------------------------------------------------------
@@ -165,14 +142,20 @@ extern "C" int pico_moe_experts_rows(const void* h, int ldh, const void* gate_up
 // ---------------------------------------------------------------------------
 // Sorting the rows by expert.  One workgroup an expert: it counts every expert's rows (to know where its own begin),
 // then writes its own rows' numbers in ascending order; its last tile is filled up with -1.
-//   sorted[tiles_cap * MOE_BM]: row numbers (token * top + slot) or -1;  tile_expert[tiles_cap]: the expert of a tile, -1: unused
+//   sorted[tiles_cap * bm]: row numbers (token * top + slot) or -1;  sorted_w: their weights;
+//   tiles[2 t]: MOE_TILE(expert, rows) of tile t;  tiles[2 t + 1]: MOE_STRIP(first tile, tiles) of the strip it is in, up to
+//   MOE_STRIP_TILES neighbouring tiles of one expert;  tiles[2 tiles_cap]: how many tiles there are
 // ---------------------------------------------------------------------------
 #define MOE_SORT_THREADS 1024
 #define MOE_SORT_MAX_E 1024
+#define MOE_TILE(e, rows) ((e) << 10 | (rows))
+#define MOE_STRIP(first, n) ((first) << 4 | (n))
+#define MOE_STRIP_TILES 8
 
-__global__ __launch_bounds__(MOE_SORT_THREADS) void moe_sort_kernel(const int* __restrict__ experts, int R, int E,
+__global__ __launch_bounds__(MOE_SORT_THREADS) void moe_sort_kernel(const int* __restrict__ experts,
+                                                                    const float* __restrict__ weights, int R, int E, int bm,
                                                                     int tiles_cap, int* __restrict__ sorted,
-                                                                    int* __restrict__ tile_expert) {
+                                                                    float* __restrict__ sorted_w, int* __restrict__ tiles_out) {
   __shared__ int hist[MOE_SORT_MAX_E];
   __shared__ int wave_count[MOE_SORT_THREADS / 64];
   __shared__ int base_tiles;
@@ -186,13 +169,16 @@ __global__ __launch_bounds__(MOE_SORT_THREADS) void moe_sort_kernel(const int* _
   }
   __syncthreads();
   int before = 0;
-  for (int i = tid; i < e; i += MOE_SORT_THREADS) before += (hist[i] + MOE_BM - 1) / MOE_BM;
+  for (int i = tid; i < e; i += MOE_SORT_THREADS) before += (hist[i] + bm - 1) / bm;
   if (before) atomicAdd(&base_tiles, before);
   __syncthreads();
-  const int count = hist[e], tiles = (count + MOE_BM - 1) / MOE_BM, base = base_tiles;
-  for (int i = tid; i < tiles; i += MOE_SORT_THREADS) tile_expert[base + i] = e;
-  if (e == E - 1)
-    for (int i = base + tiles + tid; i < tiles_cap; i += MOE_SORT_THREADS) tile_expert[i] = -1;
+  const int count = hist[e], tiles = (count + bm - 1) / bm, base = base_tiles;
+  for (int i = tid; i < tiles; i += MOE_SORT_THREADS) {
+    const int first = i / MOE_STRIP_TILES * MOE_STRIP_TILES;
+    tiles_out[2 * (base + i)] = MOE_TILE(e, min(bm, count - i * bm));
+    tiles_out[2 * (base + i) + 1] = MOE_STRIP(base + first, min(MOE_STRIP_TILES, tiles - first));
+  }
+  if (e == E - 1 && tid == 0) tiles_out[2 * tiles_cap] = base + tiles;
   // every wave takes a stretch of the rows: counts its own, then writes them behind those of the waves before it
   const int seg = ((R + nw - 1) / nw + 63) / 64 * 64, lo = wave * seg, hi = min(R, lo + seg);
   int mine = 0;
@@ -205,187 +191,227 @@ __global__ __launch_bounds__(MOE_SORT_THREADS) void moe_sort_kernel(const int* _
   __syncthreads();
   int at = 0;
   for (int i = 0; i < wave; i++) at += wave_count[i];
-  int* dst = sorted + (size_t)base * MOE_BM;
+  int* dst = sorted + (size_t)base * bm;
+  float* dst_w = sorted_w + (size_t)base * bm;
   for (int r0 = lo; r0 < hi; r0 += 64) {
     const int r = r0 + lane;
     const bool is = r < hi && experts[r] == e;
     const unsigned long long m = __ballot(is);
-    if (is) dst[at + __popcll(m & ((1ull << lane) - 1ull))] = r;
+    if (is) {
+      const int to = at + __popcll(m & ((1ull << lane) - 1ull));
+      dst[to] = r;
+      dst_w[to] = weights[r];
+    }
     at += __popcll(m);
   }
-  for (int i = count + tid; i < tiles * MOE_BM; i += MOE_SORT_THREADS) dst[i] = -1;
+  for (int i = count + tid; i < tiles * bm; i += MOE_SORT_THREADS) { dst[i] = -1; dst_w[i] = 0.f; }
 }
 
 // ---------------------------------------------------------------------------
-// The grouped product.  grid (tiles_cap, ceil(N / columns of a tile)); a tile is MOE_BM rows x MOE_BN matrix rows, staged
-// MOE_BK k at a time (the next stage travels in registers while this one is multiplied); 4 waves as 2 x 2, a wave makes
-// 64 rows x 2 blocks of 32 columns with four v_mfma_f32_32x32x16_bf16 a k step.
-// UP:   A = gathered, scaled rows of h (K = D); B rows = 64 gate rows f0.. and 64 up rows F + f0..; a wave holds gate and
-//       up of the same 32 columns and writes act(gate, up) to y[p, f] (bfloat16).
-// DOWN: A = y rows of the tile (K = F); B rows = 128 rows n0.. of down_e; float32 to out[slot][token][n].
+// The grouped product: tiles as tile_stream.h has them, of 64 MB sorted rows of one expert by 64 NB rows of its matrix.
+// UP:   X = gathered rows of h (K = D); the matrix's rows in blocks of 16 gate rows and the 16 up rows of the same columns;
+//       act(gate, up) to y[p, f] (bfloat16).
+// DOWN: X = y rows of the tile (K = F); float32 to out[slot][token][n].
 // ---------------------------------------------------------------------------
+struct MoeArgs {
+  const bf16_t* X;
+  const bf16_t* W;
+  const int* sorted;
+  const float* sorted_w;
+  const int* tiles;
+  bf16_t* y;
+  float* out;
+  int tiles_cap, ldx, T, top, F, D, n_tiles, mode;
+  float limit, alpha;
+};
+
+#ifdef __HIP_DEVICE_COMPILE__
+// a read of what an earlier kernel wrote, at an address that is the same in all lanes: it goes through the scalar cache and
+// so does not wait behind the copies, which the vector loads' counter retires in order
+__device__ __forceinline__ int moe_scalar(const int* p) {
+  return *(const __attribute__((address_space(4))) int*)(uintptr_t)p;
+}
+
+// Tile t of the order in which tiles are dealt out: strip by strip, inside a strip column by column.  The tiles that share rows
+// of a matrix are neighbours, so they run on one die at one time, and a matrix is read from memory once; a die at work on
+// one strip also holds all of its rows in its L2.  (Strips of 8 tiles across experts read the rows on all dies and a matrix
+// twice where a strip ends in it.)
+__device__ __forceinline__ void moe_place(const MoeArgs& a, int t, int& m, int& n) {
+  const int strip = moe_scalar(a.tiles + 2 * (t / a.n_tiles) + 1), first = strip >> 4, rows = strip & 15, rest = t - first * a.n_tiles;
+  n = rest / rows;
+  m = first + rest - n * rows;
+}
+#endif
+
+template <int MB, int NB, bool UP>
+__global__ __launch_bounds__(256, ts_share(MB, NB)) void moe_grouped_kernel(const MoeArgs a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  typedef TileStream<MB, NB> TS;
+  TS ts(smem);
+  constexpr int TM = 64 * MB, TN = 64 * NB, COLS = UP ? TN / 2 : TN;
+  const int K = UP ? a.D : a.F, tiles = moe_scalar(a.tiles + 2 * a.tiles_cap) * a.n_tiles, first = ts_first();
+  if (first >= tiles) return;
+  TileRowsSource<MB> xs;
+  TileRowsSource<NB> ws;
+  auto aim = [&](int t) {
+    int m, n;
+    moe_place(a, t, m, n);
+    const int tile = moe_scalar(a.tiles + 2 * m), e = tile >> 10, rows = tile & 1023;
+    const int c0 = n * COLS;
+    if (UP) {
+      xs.rsrc = ts_buffer(a.X, ((long long)(a.T - 1) * a.ldx + K) * 2);
+      ws.rsrc = ts_buffer(a.W + (size_t)e * 2 * a.F * K, (long long)a.F * K * 4);
+#pragma unroll
+      for (int j = 0; j < 2 * MB; j++) {
+        const int* list = a.sorted + (size_t)m * TM + (4 * j + ts.wave) * 8;
+        int r = moe_scalar(list);
+#pragma unroll
+        for (int i = 1; i < 8; i++) {
+          const int v = moe_scalar(list + i);
+          r = (ts.lane >> 3) == i ? v : r;
+        }
+        xs.off[j] = r < 0 ? TS_OUT : (uint32_t)(r / a.top * a.ldx) * 2;
+      }
+#pragma unroll
+      for (int j = 0; j < 2 * NB; j++) {
+        const int r = ts.row(j), c = c0 + (r >> 5) * 16 + (r & 15);
+        ws.off[j] = c < a.F ? (uint32_t)((c + ((r & 16) ? a.F : 0)) * K) * 2 : TS_OUT;
+      }
+    } else {
+      xs.rsrc = ts_buffer(a.X + (size_t)m * TM * K, (long long)rows * K * 2);
+      ws.rsrc = ts_buffer(a.W + ((size_t)e * a.D + c0) * K, (long long)(a.D - c0) * K * 2);
+#pragma unroll
+      for (int j = 0; j < 2 * MB; j++) xs.off[j] = (uint32_t)(ts.row(j) * K) * 2;
+#pragma unroll
+      for (int j = 0; j < 2 * NB; j++) ws.off[j] = (uint32_t)(ts.row(j) * K) * 2;
+    }
+  };
+  ts.run(first, gridDim.x, tiles, K, xs, ws, aim, [&](int t) {
+    // lane (l, h): row l of a block of X, tile rows 8 (r / 4) + 4 h + r % 4 of a block of W in register r
+    int mt, nt;
+    moe_place(a, t, mt, nt);
+    const int l = ts.lane & 31, h = ts.lane >> 5, rows = moe_scalar(a.tiles + 2 * mt) & 1023;
+#pragma unroll
+    for (int i = 0; i < MB; i++) {
+      const int in = (ts.wave >> 1) * (32 * MB) + 32 * i;      // the block's first row in its tile
+      if (in >= rows) continue;
+      const size_t p0 = (size_t)mt * TM + in;
+      int mine = 0;                                            // the row's weight (UP) or number
+#pragma unroll
+      for (int j = 0; j < 32; j++) {
+        const int v = moe_scalar((UP ? (const int*)a.sorted_w : a.sorted) + p0 + j);
+        mine = l == j ? v : mine;
+      }
+      const bool there = in + l < rows;
+      const float w = __int_as_float(mine);
+      float* o = UP ? nullptr : a.out + ((size_t)(there ? mine % a.top : 0) * a.T + (there ? mine / a.top : 0)) * a.D;
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        const ts_f32x16& v = ts.acc[j][i];
+        const int blk = (ts.wave & 1) * NB + j;
+        if (UP) {
+          uint32_t p[4];
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            p[q] = pack2_bf16(moe_act(v[2 * q], v[8 + 2 * q], a.limit, a.alpha, a.mode, w),
+                              moe_act(v[2 * q + 1], v[8 + 2 * q + 1], a.limit, a.alpha, a.mode, w));
+          // the halves of the wave hold columns 0..3 and 8..11, 4..7 and 12..15: swapped, eight neighbours each
+          const auto s0 = __builtin_amdgcn_permlane32_swap(p[0], p[2], false, false);
+          const auto s1 = __builtin_amdgcn_permlane32_swap(p[1], p[3], false, false);
+          const int c = nt * COLS + blk * 16 + 8 * h;
+          if (there && c < a.F)
+            *reinterpret_cast<uint4*>(a.y + (p0 + l) * a.F + c) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const int n = nt * TN + blk * 32 + 8 * q + 4 * h;
+            if (there && n < a.D) *reinterpret_cast<float4*>(o + n) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+          }
+        }
+      }
+    }
+  });
+#endif
+}
+
+template <int MB, int NB, bool UP>
+static int moe_launch(MoeArgs a, hipStream_t stream) {
+  static const hipError_t room = hipFuncSetAttribute((const void*)&moe_grouped_kernel<MB, NB, UP>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, ts_lds_bytes(MB, NB));
+  PICO_REQUIRE(room == hipSuccess, "pico_moe_experts_grouped: %s", hipGetErrorString(room));
+  const int cols = UP ? 32 * NB : 64 * NB, n = UP ? a.F : a.D, most = 256 * ts_share(MB, NB);
+  a.n_tiles = (n + cols - 1) / cols;
+  const long long tiles = (long long)a.tiles_cap * a.n_tiles;
+  PICO_REQUIRE(tiles < (1LL << 30), "pico_moe_experts_grouped: sizes beyond one launch");
+  moe_grouped_kernel<MB, NB, UP><<<tiles < most ? (int)tiles : most, 256, ts_lds_bytes(MB, NB), stream>>>(a);
+  return 0;
+}
+
+// Rows of a tile: 64 up to 48 rows an expert (most experts then have one tile), else 128.  37 rows an expert of 2,240 x 1,536:
+// 56 and 26 us the two products with tiles of 64, 54 and 35 with 128; 87 of 4,736 x 3,584: 495 and 263 with 64, 426 and 217
+// with 128; 256 of 2,240 x 1,536: 119 and 67, 92 and 47.  Taller tiles pad more than they save.
+extern "C" int pico_moe_tile_rows(long long rows, int E) { return rows <= 48LL * E ? 64 : 128; }
+
+// Columns of a tile: as many rounds of workgroups as a call is expected to take (its rows spread over the experts at
+// random), at the cost of a stage in a full round and in a last one that leaves a compute unit at most one workgroup, in
+// microseconds; the operands come from memory, so a stage costs its latency more than its products.
+struct MoeTile { int nb, share; float each, lone; };
+static const MoeTile moe_tiles[2][2] = {{{1, 2, 0.72f, 0.6f}, {2, 2, 1.3f, 1.1f}}, {{3, 2, 1.9f, 1.65f}, {4, 1, 1.4f, 1.4f}}};
+
+static double moe_live(double rows, int E, int bm) {           // tiles that are expected to have rows
+  const double mean = rows / E;
+  double tiles = E * -expm1(-mean);
+  for (int j = 1; j * (double)bm < rows; j++) {
+    const double p = 0.5 * erfc((j * bm - mean) / sqrt(2 * mean));
+    if (p < 1e-3) break;
+    tiles += E * p;
+  }
+  return tiles;
+}
+
 template <bool UP>
-__global__ __launch_bounds__(256) void moe_grouped_kernel(const bf16_t* __restrict__ A, int lda,
-                                                          const bf16_t* __restrict__ W, const int* __restrict__ sorted,
-                                                          const int* __restrict__ tile_expert,
-                                                          const float* __restrict__ weights, bf16_t* __restrict__ y,
-                                                          float* __restrict__ out, int T, int top, int F, int D,
-                                                          float limit, float alpha, int ntile, int ncol, int mode) {
-  __shared__ __attribute__((aligned(16))) bf16_t As[MOE_BM * MOE_LD];
-  __shared__ __attribute__((aligned(16))) bf16_t Bs[MOE_BN * MOE_LD];
-  __shared__ int rows[MOE_BM];
-  // Which tile and which columns.  Workgroups go to the chip's eight dies in turn, and every die has a second-level
-  // cache of its own.  Tiles are taken in pairs (neighbours in the sorted order: mostly one expert's); pair p belongs to
-  // die p % 8, and a die's consecutive workgroups are the two tiles of a pair at the same columns, then at the next
-  // columns: what runs together on a die shares its operands.  grid: 8 * ceil(pairs / 8) * 2 * ncol, one-dimensional.
-  const int die = blockIdx.x & 7, idx = blockIdx.x >> 3;
-  const int pair = (idx / (2 * ncol)) * 8 + die, rest = idx % (2 * ncol);
-  const int tile = 2 * pair + (rest & 1), col = rest >> 1;
-  if (tile >= ntile) return;
-  const int e = tile_expert[tile];
-  if (e < 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-  const int K = UP ? D : F;
-  const int c0 = col * (UP ? MOE_BN / 2 : MOE_BN);            // first output column of this tile
-  if (tid < MOE_BM) rows[tid] = sorted[(size_t)tile * MOE_BM + tid];
-
-  // what this thread stages: 8 k of four A rows and of four B rows (rows srow, srow + 32, ...); rows that do not exist
-  // point at a row that does and are cleared after the load, so that every load is unconditional
-  const int srow = tid >> 3, sk = (tid & 7) * 8;
-  const size_t erows = UP ? (size_t)2 * F : (size_t)D;
-#define MOE_STAGE_ROW(i, A_SRC, A_W, A_OK, B_SRC, B_OK)                                   \
-  const bf16_t* A_SRC;                                                                    \
-  const bf16_t* B_SRC;                                                                    \
-  float A_W = 1.f;                                                                        \
-  bool A_OK = true, B_OK;                                                                 \
-  {                                                                                       \
-    const int m = srow + 32 * (i);                                                        \
-    if (UP) {                                                                             \
-      const int r = sorted[(size_t)tile * MOE_BM + m];                                    \
-      A_OK = r >= 0;                                                                      \
-      A_SRC = A + (size_t)(A_OK ? r / top : 0) * lda + sk;                                \
-      A_W = A_OK ? (mode != 0 ? 1.f : weights[r]) : 0.f;                                  \
-      const int f = c0 + (m & 63);                                                        \
-      B_OK = f < F;                                                                       \
-      B_SRC = W + ((size_t)e * erows + (B_OK ? (m >> 6) * F + f : 0)) * K + sk;           \
-    } else {                                                                              \
-      A_SRC = A + ((size_t)tile * MOE_BM + m) * lda + sk;                                 \
-      B_OK = c0 + m < D;                                                                  \
-      B_SRC = W + ((size_t)e * erows + (B_OK ? c0 + m : 0)) * K + sk;                     \
-    }                                                                                     \
+static int moe_product(int bm, int E, const MoeArgs& a, hipStream_t stream) {
+  const double live = moe_live((double)a.T * a.top, E, bm);
+  double cost[2];
+  for (int i = 0; i < 2; i++) {
+    const MoeTile& t = moe_tiles[bm == 128][i];
+    const int cols = (UP ? 32 : 64) * t.nb, n = UP ? a.F : a.D;
+    const double rounds = ceil(live) * ((n + cols - 1) / cols) / (256.0 * t.share), full = floor(rounds), rest = rounds - full;
+    cost[i] = full * t.each + (rest == 0 ? 0 : rest * t.share <= 1 ? t.lone : t.each);
   }
-  MOE_STAGE_ROW(0, a_src0, a_w0, a_ok0, b_src0, b_ok0)
-  MOE_STAGE_ROW(1, a_src1, a_w1, a_ok1, b_src1, b_ok1)
-  MOE_STAGE_ROW(2, a_src2, a_w2, a_ok2, b_src2, b_ok2)
-  MOE_STAGE_ROW(3, a_src3, a_w3, a_ok3, b_src3, b_ok3)
-#undef MOE_STAGE_ROW
-
-  f32x16 acc00, acc01, acc10, acc11;
-#pragma unroll
-  for (int r = 0; r < 16; r++) { acc00[r] = 0.f; acc01[r] = 0.f; acc10[r] = 0.f; acc11[r] = 0.f; }
-
-  uint4 ra0, ra1, ra2, ra3, rb0, rb1, rb2, rb3;
-  // K is a multiple of 8: the 8 k of a load are in or out together; a load beyond K reads k = 0 .. instead.  What must
-  // read as zero (rows that do not exist, k beyond K) is cleared where the stage is written to LDS, not here: a select
-  // on a register that a load has just been asked for would wait for that load in front of the products
-#define MOE_FETCH(k0)                                                      \
-  {                                                                        \
-    const bool k_ok = (k0) + sk < K;                                       \
-    const int ko = k_ok ? (k0) : -sk;   /* the row's first 8, not 8 behind its end (the last row ends the tensor) */ \
-    ra0 = *reinterpret_cast<const uint4*>(a_src0 + ko);                    \
-    ra1 = *reinterpret_cast<const uint4*>(a_src1 + ko);                    \
-    ra2 = *reinterpret_cast<const uint4*>(a_src2 + ko);                    \
-    ra3 = *reinterpret_cast<const uint4*>(a_src3 + ko);                    \
-    rb0 = *reinterpret_cast<const uint4*>(b_src0 + ko);                    \
-    rb1 = *reinterpret_cast<const uint4*>(b_src1 + ko);                    \
-    rb2 = *reinterpret_cast<const uint4*>(b_src2 + ko);                    \
-    rb3 = *reinterpret_cast<const uint4*>(b_src3 + ko);                    \
-  }
-  MOE_FETCH(0)
-  const int frag = (lane & 31) * MOE_LD + (lane >> 5) * 8;    // a lane's place in a block of 32 rows
-  const int a_off = wm * 64 * MOE_LD + frag;
-  const int b_off0 = (UP ? wn * 32 : wn * 64) * MOE_LD + frag;
-  const int b_off1 = (UP ? 64 + wn * 32 : wn * 64 + 32) * MOE_LD + frag;
-  for (int k0 = 0; k0 < K; k0 += MOE_BK) {
-    __syncthreads();                                          // the last stage has been read
-    {
-      bf16_t* as = As + srow * MOE_LD + sk;
-      bf16_t* bs = Bs + srow * MOE_LD + sk;
-      const bool k_in = k0 + sk < K;
-      const bool scaled = UP && mode == 0;        // the other modes put the weight on the activation instead
-      *reinterpret_cast<uint4*>(as) = keep8(scaled ? scale8(ra0, a_w0) : ra0, a_ok0 && k_in);
-      *reinterpret_cast<uint4*>(as + 32 * MOE_LD) = keep8(scaled ? scale8(ra1, a_w1) : ra1, a_ok1 && k_in);
-      *reinterpret_cast<uint4*>(as + 64 * MOE_LD) = keep8(scaled ? scale8(ra2, a_w2) : ra2, a_ok2 && k_in);
-      *reinterpret_cast<uint4*>(as + 96 * MOE_LD) = keep8(scaled ? scale8(ra3, a_w3) : ra3, a_ok3 && k_in);
-      *reinterpret_cast<uint4*>(bs) = keep8(rb0, b_ok0 && k_in);
-      *reinterpret_cast<uint4*>(bs + 32 * MOE_LD) = keep8(rb1, b_ok1 && k_in);
-      *reinterpret_cast<uint4*>(bs + 64 * MOE_LD) = keep8(rb2, b_ok2 && k_in);
-      *reinterpret_cast<uint4*>(bs + 96 * MOE_LD) = keep8(rb3, b_ok3 && k_in);
-    }
-    if (k0 + MOE_BK < K) MOE_FETCH(k0 + MOE_BK)               // the next stage travels while this one is multiplied
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < MOE_BK; ks += 16) {
-      const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(As + a_off + ks);
-      const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(As + a_off + 32 * MOE_LD + ks);
-      const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(Bs + b_off0 + ks);
-      const bf16x8 b1 = *reinterpret_cast<const bf16x8*>(Bs + b_off1 + ks);
-      acc00 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, acc00, 0, 0, 0);
-      acc01 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b1, acc01, 0, 0, 0);
-      acc10 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b0, acc10, 0, 0, 0);
-      acc11 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, acc11, 0, 0, 0);
-    }
-  }
-#undef MOE_FETCH
-  // a lane holds column lane % 32 of its blocks and rows 8 (r / 4) + 4 (lane / 32) + r % 4
-#define MOE_WRITE(i, ACC0, ACC1)                                                                                     \
-  _Pragma("unroll") for (int r = 0; r < 16; r++) {                                                                   \
-    const int m = wm * 64 + 32 * (i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);                                     \
-    if (UP) {                                                                                                        \
-      const int f = c0 + wn * 32 + (lane & 31);                                                                      \
-      const float wrow = (mode != 0 && rows[m] >= 0) ? weights[rows[m]] : 0.f;                                       \
-      if (f < F) y[((size_t)tile * MOE_BM + m) * F + f] = f32_to_bf16(moe_act(ACC0[r], ACC1[r], limit, alpha, mode, wrow)); \
-    } else {                                                                                                         \
-      const int row = rows[m];                                                                                       \
-      if (row < 0) continue;                                                                                         \
-      float* o = out + ((size_t)(row % top) * T + row / top) * D;                                                    \
-      const int n = c0 + wn * 64 + (lane & 31);                                                                      \
-      if (n < D) o[n] = ACC0[r];                                                                                     \
-      if (n + 32 < D) o[n + 32] = ACC1[r];                                                                           \
-    }                                                                                                                \
-  }
-  MOE_WRITE(0, acc00, acc01)
-  MOE_WRITE(1, acc10, acc11)
-#undef MOE_WRITE
+  const bool second = cost[1] < cost[0];
+  if (bm == 64) return second ? moe_launch<1, 2, UP>(a, stream) : moe_launch<1, 1, UP>(a, stream);
+  return second ? moe_launch<2, 4, UP>(a, stream) : moe_launch<2, 3, UP>(a, stream);
 }
 
-extern "C" int pico_moe_tile_rows() { return MOE_BM; }
-
+// sorted: int32 [2 tiles_cap bm] (row numbers, then weights), tiles: int32 [2 tiles_cap + 1]
 extern "C" int pico_moe_experts_grouped(const void* h, int ldh, const void* gate_up, const void* down, const int* experts,
-                                        const float* weights, int* sorted, int* tile_expert, int tiles_cap, void* y,
+                                        const float* weights, int* sorted, int* tiles, int tiles_cap, int bm, void* y,
                                         float* out, int T, int top, int E, int F, int D, float limit, float alpha,
                                         int mode, hipStream_t stream) {
   PICO_REQUIRE(mode >= 0 && mode <= 2, "pico_moe_experts_grouped: unknown mode %d", mode);
   PICO_REQUIRE(T >= 0 && top > 0 && E > 0 && F > 0 && D > 0 && ldh >= D, "pico_moe_experts_grouped: bad sizes");
   PICO_REQUIRE(E <= MOE_SORT_MAX_E, "pico_moe_experts_grouped: at most %d experts", MOE_SORT_MAX_E);
   PICO_REQUIRE(F % 8 == 0 && D % 8 == 0 && ldh % 8 == 0, "pico_moe_experts_grouped: sizes must be multiples of 8");
-  PICO_REQUIRE(((uintptr_t)h | (uintptr_t)gate_up | (uintptr_t)down | (uintptr_t)y) % 16 == 0,
+  PICO_REQUIRE(((uintptr_t)h | (uintptr_t)gate_up | (uintptr_t)down | (uintptr_t)y | (uintptr_t)out) % 16 == 0,
                "pico_moe_experts_grouped: operands must start on 16 bytes");
   if (T == 0) return 0;
   const long long R = (long long)T * top;
   PICO_REQUIRE(R < (1ll << 30), "pico_moe_experts_grouped: too many rows");
-  const long long need = (R + (long long)E * (MOE_BM - 1)) / MOE_BM;
+  PICO_REQUIRE((long long)T * ldh < (1ll << 30) && (long long)F * D < (1ll << 29),
+               "pico_moe_experts_grouped: the activations or an expert's matrix span 2^31 bytes or more");
+  PICO_REQUIRE(bm == pico_moe_tile_rows(R, E), "pico_moe_experts_grouped: tiles of %d rows", bm);
+  const long long need = (R + (long long)E * (bm - 1)) / bm;
   PICO_REQUIRE(tiles_cap >= need, "pico_moe_experts_grouped: room for %d tiles, %lld may be needed", tiles_cap, need);
-  const long long ncol1 = (F + MOE_BN / 2 - 1) / (MOE_BN / 2), ncol2 = (D + MOE_BN - 1) / MOE_BN;
-  const long long slots = ((tiles_cap + 1) / 2 + 7) / 8 * 8 * 2;       // tiles in pairs, pairs in eights
-  PICO_REQUIRE(slots * ncol1 < (1ll << 31) && slots * ncol2 < (1ll << 31), "pico_moe_experts_grouped: sizes beyond the grid");
-  moe_sort_kernel<<<E, MOE_SORT_THREADS, 0, stream>>>(experts, (int)R, E, tiles_cap, sorted, tile_expert);
-  moe_grouped_kernel<true><<<(unsigned)(slots * ncol1), 256, 0, stream>>>(
-      (const bf16_t*)h, ldh, (const bf16_t*)gate_up, sorted, tile_expert, weights, (bf16_t*)y, nullptr, T, top, F, D, limit,
-      alpha, tiles_cap, (int)ncol1, mode);
-  moe_grouped_kernel<false><<<(unsigned)(slots * ncol2), 256, 0, stream>>>(
-      (const bf16_t*)y, F, (const bf16_t*)down, sorted, tile_expert, nullptr, nullptr, out, T, top, F, D, limit, alpha,
-      tiles_cap, (int)ncol2, mode);
+  float* sorted_w = (float*)sorted + (size_t)tiles_cap * bm;
+  moe_sort_kernel<<<E, MOE_SORT_THREADS, 0, stream>>>(experts, weights, (int)R, E, bm, tiles_cap, sorted, sorted_w, tiles);
+  const MoeArgs up{(const bf16_t*)h, (const bf16_t*)gate_up, sorted, sorted_w, tiles, (bf16_t*)y, nullptr, tiles_cap, ldh, T, top, F, D, 0, mode, limit, alpha};
+  MoeArgs dn = up;
+  dn.X = (const bf16_t*)y; dn.W = (const bf16_t*)down; dn.out = out;
+  int rc = moe_product<true>(bm, E, up, stream);
+  if (!rc) rc = moe_product<false>(bm, E, dn, stream);
+  if (rc) return rc;
   PICO_LAUNCH_CHECK();
   return 0;
 }

@@ -166,5 +166,55 @@ struct TileStream {
     weave<MB + NB, part(1)>();
     __builtin_amdgcn_sched_barrier(0);
   }
+  // Tiles first, first + step, .. below `tiles`, each over K: `aim(t)` points xs and ws at tile t, `done(t)` takes its sums.
+  template <typename Aim, typename Done>
+  __device__ __forceinline__ void run(int first, int step, int tiles, int K, const TileRowsSource<MB>& xs,
+                                      const TileRowsSource<NB>& ws, Aim aim, Done done) {
+    const int stages = (K + TS_BK - 1) / TS_BK;
+    int at_tile = first, at_stage = 0, fill = 0;             // the stage that is asked for next, into buffer `fill`
+    auto copies = [&](auto r) { ask<decltype(r)::from, decltype(r)::to>(fill, xs, ws, at_tile < tiles ? at_stage * TS_BK : K, K); };
+    auto on = [&] {
+      fill = fill + 1 == NBUF ? 0 : fill + 1;
+      if (++at_stage == stages && at_tile < tiles) {
+        at_stage = 0;
+        at_tile += step;
+        if (at_tile < tiles) aim(at_tile);
+      }
+    };
+    aim(first);
+#pragma unroll
+    for (int b = 0; b < NBUF - 1; b++) {
+      copies(Range<0, LOADS>());
+      on();
+    }
+    __builtin_amdgcn_s_waitcnt(ts_wait((NBUF - 2) * LOADS, true));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    copies(Range<0, part(1)>());
+    read(0, 0, 0);
+    int buf = 0;
+    for (int t = first; t < tiles; t += step) {
+      clear();
+      for (int s = 0; s < stages; s++) {
+        const int next = buf + 1 == NBUF ? 0 : buf + 1;
+        stage(buf, next, copies, on);
+        buf = next;
+      }
+      done(t);
+    }
+    __builtin_amdgcn_s_waitcnt(ts_wait(0, true));          // the last copies (zeros) are in before LDS is given back
+  }
 };
+
+// Tile t of the order in which tiles are dealt out: strips of up to 8 tiles of rows, inside a strip column by column, so
+// that the 32 tiles a die works on at a time are about 8 x 4 and share their operands in its L2.
+__device__ __forceinline__ void ts_place(int m_tiles, int n_tiles, int t, int& m, int& n) {
+  const int per = 8 * n_tiles, strip = t / per, rest = t - strip * per, rows = min(8, m_tiles - strip * 8);
+  n = rest / rows;
+  m = strip * 8 + rest - n * rows;
+}
+// Workgroups go to the dies in turn; a die's share of a round is a run of neighbouring tiles.
+__device__ __forceinline__ int ts_first() {
+  return gridDim.x % 8 == 0 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+}
 #endif

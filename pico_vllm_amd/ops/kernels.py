@@ -1195,7 +1195,10 @@ def moe_experts_plain(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
     return out
 
 
-MOE_STREAM_ROWS = 32        # up to this many (token, expert) rows every row streams its expert's matrices
+# up to this many (token, expert) rows every row streams its expert's matrices.  Behind it rows share experts often enough
+# that sorting pays: 16, 20, 24, 32 rows over 32 experts of 4,736 x 3,584 238, 287, 337, 447 us each for itself, 238, 275, 295,
+# 375 sorted; 16 and 24 rows over 16 experts of 2,240 x 1,536 55 and 72 against 59 and 61
+MOE_STREAM_ROWS = 16
 
 
 def moe_fast_ok(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor) -> bool:
@@ -1203,7 +1206,9 @@ def moe_fast_ok(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor) -> b
     return (h.dtype == torch.bfloat16 and gate_up.dtype == torch.bfloat16 and down.dtype == torch.bfloat16
             and h.dim() == 2 and h.stride(1) == 1 and h.shape[1] % 8 == 0 and down.shape[2] % 8 == 0
             and (h.stride(0) % 8 == 0 or h.shape[0] == 1) and h.data_ptr() % 16 == 0
-            and gate_up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0 and gate_up.shape[0] <= 1024)
+            and gate_up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0 and gate_up.shape[0] <= 1024
+            # (offsets within the activations and within an expert's matrix are 31 bits of bytes)
+            and h.shape[0] * h.stride(0) < 2**30 and down.shape[1] * down.shape[2] < 2**29)
 
 
 def moe_grouped_rows(tokens: int, top: int) -> bool:
@@ -1232,17 +1237,16 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, expe
         _check(lib, lib.pico_moe_experts_rows(_ptr(h), ldh, _ptr(gate_up), _ptr(down), _ptr(experts), _ptr(weights),
                                               _ptr(y), _ptr(out), T, top, E, F, D, c_float(limit), c_float(alpha), mode, _stream()))
         return out[0] if top == 1 else out
-    bm = lib.pico_moe_tile_rows()
+    bm = lib.pico_moe_tile_rows(c_ll(T * top), E)
     tiles = (T * top + E * (bm - 1)) // bm
-    sorted_rows = torch.empty(tiles * bm, dtype=torch.int32, device=h.device)
-    tile_expert = torch.empty(tiles, dtype=torch.int32, device=h.device)
+    lists = torch.empty(2 * tiles * bm + 2 * tiles + 1, dtype=torch.int32, device=h.device)
     y = torch.empty(tiles * bm, F, dtype=h.dtype, device=h.device)
     # a slot whose expert has no matrices (a number from E on) is written by no product: with one slot a token the
     # caller adds into the rows, which then start from zero; with several, ``moe_identity`` fills the slabs' rows
     out = (torch.zeros if top == 1 else torch.empty)(top, T, D, dtype=torch.float32, device=h.device)
     _check(lib, lib.pico_moe_experts_grouped(_ptr(h), ldh, _ptr(gate_up), _ptr(down), _ptr(experts), _ptr(weights),
-                                             _ptr(sorted_rows), _ptr(tile_expert), tiles, _ptr(y), _ptr(out), T, top, E, F,
-                                             D, c_float(limit), c_float(alpha), mode, _stream()))
+                                             _ptr(lists), _ptr(lists[2 * tiles * bm:]), tiles, bm, _ptr(y), _ptr(out), T, top,
+                                             E, F, D, c_float(limit), c_float(alpha), mode, _stream()))
     return out[0] if top == 1 else out
 
 

@@ -89,6 +89,38 @@ def test_swiglu(K, dtype):
         close(K.swiglu(gu.to(DEV)), P.swiglu(gu), dtype)
 
 
+@pytest.mark.parametrize("counts,D,F_", [([0, 1, 63, 64, 65], 72, 40), ([129, 0, 48, 2], 64, 264), ([1, 127, 128, 129, 700], 136, 1000),
+                                         ([0, 1100], 328, 200), ([0, 0, 5], 1536, 8)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_moe_grouped(K, counts, D, F_, mode):
+    # experts with rows up to, at and behind the edges of tiles of 64 and 128 rows and of strips of tiles, columns and k that
+    # end inside a tile and a stage; a row with a stride; a number that has no matrices
+    g = torch.Generator().manual_seed(D + F_)
+    E, which = len(counts), [e for e, n in enumerate(counts) for _ in range(n)] + [len(counts)]
+    R = len(which)
+    which = torch.tensor(which)[torch.randperm(R, generator=g)]
+    h = torch.randn(R, D + 8, generator=g).bfloat16().to(DEV)[:, 8:]
+    gate_up = (torch.randn(E, 2 * F_, D, generator=g) * D ** -0.5).bfloat16().to(DEV)
+    down = (torch.randn(E, D, F_, generator=g) * F_ ** -0.5).bfloat16().to(DEV)
+    wt = torch.rand(R, 1, generator=g).to(DEV)
+    got = K.moe_experts(h, gate_up, down, which.int().view(R, 1).to(DEV), wt, 0.7, 1.702, grouped=True, mode=mode).double()
+    for e in range(E + 1):
+        at = (which == e).nonzero().view(-1).to(DEV)
+        if e == E:
+            assert not got[at].any()                 # one slot a token: rows of no expert are left zero
+            continue
+        w = wt[at].double()
+        z = (h[at].double() * (w if mode == 0 else 1.0)) @ gate_up[e].double().T
+        gate, up = z[:, :F_], z[:, F_:]
+        if mode != 1:
+            gate, up = gate.clamp(max=0.7), up.clamp(-0.7, 0.7) + 1
+        y = gate * torch.sigmoid((1.0 if mode == 1 else 1.702) * gate) * up * (w if mode else 1.0)
+        want = y @ down[e].double().T
+        # y is rounded once to bfloat16 (eight bits: at most 2^-8 of its size), the sums are float32 (1e-5 of a row's size each)
+        slack = (y.abs() * 2.0 ** -8 + 1e-5 * (1 + 2 * z.abs().max() if at.numel() else 1.0)) @ down[e].double().abs().T + 1e-5
+        assert bool(((got[at] - want).abs() <= slack).all())
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 301, 136), (5, 64, 172), (70, 130, 64), (130, 17, 33)])
 def test_gemm_f32(K, M, N, K_):
     a, w, b = torch.randn(M, K_), torch.randn(N, K_), torch.randn(N)
