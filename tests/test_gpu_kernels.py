@@ -315,6 +315,37 @@ def test_plain_attention_kernel_other_sizes(K, dtype, nq, nkv, d, Pg):
     close(out, want, dtype)
 
 
+@pytest.mark.parametrize("nq,nkv,d,Pg,window", [(12, 2, 128, 16, 0), (7, 1, 60, 4, 0), (5, 5, 132, 12, 100), (8, 2, 256, 64, 33), (40, 2, 8, 16, 0)])
+def test_f32_attention_keeps_columns_apart(K, nq, nkv, d, Pg, window):
+    # tiles of 16 columns with tokens of several sequences, whose keys end in the middle of a quarter; what a token does not see
+    # (its own sequence's later tokens, tokens outside its window, other sequences, the rest of a page) is not finite
+    new_lens, prefix_lens = [1, 1, 70, 5, 1], [130, 0, 15, 63, 64]
+    clean, want = _attn_case(K, torch.float32, new_lens, prefix_lens, nq, nkv, d, Pg, window, seed=5)
+    close(clean, want, torch.float32)
+    ends = [sum(new_lens[:b + 1]) for b in range(5)]
+    bad_k, bad_v = 15 + 50, 15 + 40                              # of the third sequence, among its new tokens
+
+    def spoil(qs, ks, vs):
+        ks[2][bad_k:bad_k + 3], vs[2][bad_v], vs[2][bad_v + 1], vs[4][64] = float("nan"), float("inf"), float("nan"), float("inf")
+        ks[0][:20], vs[0][:20] = (float("nan"), float("inf")) if window else (ks[0][:20], vs[0][:20])
+    got, _ = _attn_case(K, torch.float32, new_lens, prefix_lens, nq, nkv, d, Pg, window, seed=5, boost=spoil)
+    spoiled = set(range(2 + 40, 2 + 70)) | {ends[4] - 1}         # rows that see one of them
+    rows = [r for r in range(ends[4]) if r not in spoiled]
+    close(got[rows], want[rows], torch.float32)
+    assert not torch.isfinite(got[2 + 40]).all()
+    # a position's bits do not depend on how its sequence was cut into steps, nor on who shares its tile
+    g = torch.Generator().manual_seed(5)
+    totals = [n + p for n, p in zip(new_lens, prefix_lens)]
+    kv = [[torch.randn(N, nkv, d, generator=g) for N in totals] for _ in range(2)]
+    q = [torch.randn(n, nq, d, generator=g) for n in new_lens]
+
+    def last(qs, ks, vs):
+        for b in range(5):
+            qs[b][:], ks[b][:], vs[b][:] = q[b][-1:], kv[0][b], kv[1][b]
+    lone, _ = _attn_case(K, torch.float32, [1] * 5, [n - 1 for n in totals], nq, nkv, d, Pg, window, seed=6, boost=last)
+    assert torch.equal(lone, clean[[e - 1 for e in ends]])
+
+
 # Head sizes that are no multiple of 16 (the configuration allows any even one): the matrix-core kernels do not take
 # them, so both engine precisions go through this kernel there.
 @pytest.mark.parametrize("dtype", DTYPES)
