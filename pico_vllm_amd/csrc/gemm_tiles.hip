@@ -176,11 +176,20 @@ static int gt_choose(int M, int cols, int stages, bool paired, bool split, int& 
   return best;
 }
 
+// Up to 64 rows the stream of W bounds a call, and tiles of 64 rows carry it: 32 rows of a 152,064 x 3,584 output matrix in
+// float32 203 us (5.4 TB/s; the weight-streaming kernel 244), of 28,416 pairs, K 3,584, 74 (89).  128 columns of W while that
+// leaves no second round, then 64, which round up less (those two calls with the other width: 223 and 76).
+template <int EPI>
+static int gt_few(const GemmArgs& a, hipStream_t stream) {
+  return a.cols <= 512 * GT_COLS(2, EPI) ? gt_launch<1, 2, EPI>(a, stream) : gt_launch<1, 1, EPI>(a, stream);
+}
+
 template <int EPI>
 static int gt_run(GemmArgs a, hipStream_t stream) {
   const int stages = (a.K + TS_BK - 1) / TS_BK, cols = a.cols;
   int first, all, rc = 0;
   float cost;
+  if (a.M <= 64) return gt_few<EPI>(a, stream);
   const int tile = gt_choose(a.M, cols, stages, gt_paired(EPI), true, first, cost);
   auto run = [&](int i) {
     switch (i) {

@@ -320,6 +320,16 @@ def tiles_act_ok(a: torch.Tensor, w: torch.Tensor, paired: bool) -> bool:
     return tiles_ok(a, w) and (a.shape[1] <= TILES_SHORT_K or (paired and a.shape[0] > TILES_ROWS))
 
 
+def tiles_few_ok(a: torch.Tensor, w: torch.Tensor, paired: bool) -> bool:
+    """Whether the tiled product takes these few rows from the weight-streaming one: large matrices, whose tiles fill the chip
+    (256 and more of 128 rows of W), from where the activations in every wave's slices slow the stream down.  Microseconds
+    streamed / tiled, 16, 24, 32, 48, 64 rows: 152,064 x 3,584 to float32 203 / 195, 227 / 197, 244 / 203, 228 / 217, 242 / 232;
+    28,416 pairs, K 3,584, 73 / 71, 84 / 73, 89 / 74, 81 / 76, 88 / 78; 18,944 pairs 51 / 59, 59 / 60, 61 / 62, 69 / 64, 76 / 66."""
+    rows, N = a.shape[0], w.shape[0]
+    return rows <= 64 and (rows > 16 and N > 49152 if paired and rows <= 32 else N > 32768 if paired else rows >= 16 and N > 65536) \
+        and tiles_ok(a, w)
+
+
 def gemm_tiles(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, epilogue: int = EPI_BF16,
                clip: Optional[tuple] = None) -> torch.Tensor:
     """a [M, K] x w [N, K]^T, both bfloat16, any number of rows; epilogues and results as ``gemm_skinny``'s (EPI_BF16,

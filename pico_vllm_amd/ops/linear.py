@@ -105,6 +105,8 @@ class Linear:
             raise ValueError("linear: bfloat16 weights need bfloat16 activations")
         if kernels.skinny_ok(x, self.weight):
             epi = kernels.EPI_F32 if out_dtype == torch.float32 else kernels.EPI_BF16
+            if epi == kernels.EPI_F32 and kernels.tiles_few_ok(x, self.weight, False):
+                return kernels.gemm_tiles(x, self.weight, self.bias_f32, epi)
             return kernels.gemm_skinny(x, self.weight, self.bias_f32, epi)
         if out_dtype == torch.float32:
             if kernels.tiles_ok(x, self.weight):
@@ -131,18 +133,20 @@ class Linear:
                 out, x.resid = kernels.gemm_skinny_norm(x.resid_in, x.delta, x.weight, x.eps, self.weight, kernels.EPI_SWIGLU)
                 return out
             x = x.run()
-        if self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight):
+        few = self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight)
+        if few and not kernels.tiles_few_ok(x, self.weight, True):
             return kernels.gemm_skinny(x, self.weight, None, kernels.EPI_SWIGLU)
-        if self.bias is None and kernels.tiles_act_ok(x, self.weight, True):
+        if self.bias is None and (few or kernels.tiles_act_ok(x, self.weight, True)):
             return kernels.gemm_tiles(x, self.weight, None, kernels.EPI_SWIGLU)
         return kernels.swiglu(self(x))
 
     def clipped_glu(self, x: torch.Tensor, limit: float, alpha: float) -> torch.Tensor:
         """g sigmoid(alpha g) (u + 1) of [gate; up] = x W^T, g = min(gate, limit), u = up clamped to -limit .. limit; with few
         rows the epilogue of the weight-streaming kernel."""
-        if self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight):
+        few = self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight)
+        if few and not kernels.tiles_few_ok(x, self.weight, True):
             return kernels.gemm_skinny(x, self.weight, None, kernels.EPI_CLIPPED, clip=(limit, alpha))
-        if self.bias is None and kernels.tiles_act_ok(x, self.weight, True):
+        if self.bias is None and (few or kernels.tiles_act_ok(x, self.weight, True)):
             return kernels.gemm_tiles(x, self.weight, None, kernels.EPI_CLIPPED, clip=(limit, alpha))
         return kernels.clipped_glu(self(x), limit, alpha)
 

@@ -204,6 +204,27 @@ def test_gemm_tiles(K, M, N, K_, name):
     assert torch.equal(K.gemm_tiles(a[:(M + 1) // 2], w, b, epi, clip), out[:(M + 1) // 2])
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,name", [(66000, "f32"), (65536, "f32"), (65600, "swiglu"), (33024, "clipped"), (65536, "swiglu")])
+def test_few_rows_of_a_large_matrix(K, M, N, name):
+    # both widths of the tiles for few rows, at and behind the sizes where the rule changes over, through ``Linear``
+    from pico_vllm_amd.ops.linear import Linear
+    g = torch.Generator().manual_seed(M + N)
+    a, w = torch.randn(M, 72, generator=g).bfloat16().to(DEV), (torch.randn(N, 72, generator=g) * 72 ** -0.5).bfloat16().to(DEV)
+    z = a.double() @ w.double().T
+    gate, up = z[:, :N // 2], z[:, N // 2:]
+    slack = 1e-5 * (1 + 2 * float(z.abs().max()))                       # as above
+    for out in ([Linear(w)(a, torch.float32), K.gemm_tiles(a, w, None, K.EPI_F32)] if name == "f32" else
+                [Linear(w).swiglu(a), K.gemm_tiles(a, w, None, K.EPI_SWIGLU)] if name == "swiglu" else
+                [Linear(w).clipped_glu(a, 0.7, 1.702), K.gemm_tiles(a, w, None, K.EPI_CLIPPED, (0.7, 1.702))]):
+        if name == "f32":
+            assert float((out.double() - z).abs().max()) <= slack
+            continue
+        want = F.silu(gate) * up if name == "swiglu" else \
+            gate.clamp(max=0.7) * torch.sigmoid(1.702 * gate.clamp(max=0.7)) * (up.clamp(-0.7, 0.7) + 1)
+        assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + slack).all())
+
+
 def test_gemm_tiles_refuses(K):
     a, w = torch.zeros(70, 72, device=DEV).bfloat16(), torch.zeros(48, 72, device=DEV).bfloat16()
     for bad in (lambda: K.gemm_tiles(a[:, :68], w[:, :68]), lambda: K.gemm_tiles(a, w[:40]), lambda: K.gemm_tiles(a.float(), w),
