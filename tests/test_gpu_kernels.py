@@ -1398,3 +1398,38 @@ def test_ssd_chunks(K, H, G, dk, dv, lens, steps):
             assert bool((err <= 20 * 2.0 ** -24 * bound + 1e-30).all())
         assert bool(((st[slots[b]].cpu().double() - S).abs() <= 20 * 2.0 ** -24 * size + 1e-30).all())
     assert torch.equal(st[0].cpu(), state[0])       # a slot that no sequence holds
+
+
+@pytest.mark.parametrize("dk", [64, 96, 128, 192, 256])
+@pytest.mark.parametrize("lens,dv", [([1], 16), ([64, 65], 40), ([3, 700, 128], 72)])
+def test_delta_chunks(K, dk, lens, dv):
+    # the walk over the chunks' states on the matrix cores (key sizes of whole 64s) and without (96), value sizes that end inside
+    # a tile of 16 columns, one and many chunks, a slot that no sequence holds, against the rule token by token in 64 bits
+    g = torch.Generator().manual_seed(dk + sum(lens))
+    T, B, H, G = sum(lens), len(lens), 4, 2
+    q, k = (F.normalize(torch.randn(T, G, dk, generator=g), dim=-1) for _ in range(2))
+    v, decay, beta = torch.randn(T, H * dv, generator=g).bfloat16(), torch.rand(T, H, generator=g) * 0.2 + 0.8, torch.rand(T, H, generator=g)
+    state = torch.randn(B + 1, H, dk, dv, generator=g)
+    cu = torch.tensor([0] + [sum(lens[:i + 1]) for i in range(B)], dtype=torch.int32)
+    slots = torch.arange(B, 0, -1, dtype=torch.int32)
+    st = state.to(DEV)
+    out = K.delta_scan(q.reshape(T, -1).to(DEV), k.reshape(T, -1).to(DEV), v.to(DEV), decay.to(DEV), beta.to(DEV), cu.to(DEV), slots.to(DEV),
+                       st, B, H, G, dk, dv, delta=True, chunk=64).cpu().double().view(T, H, dv)
+    q, k, v = q.double().repeat_interleave(H // G, 1), k.double().repeat_interleave(H // G, 1), v.double().view(T, H, dv)
+    # a chunk's sums are chains of at most 128 and its walk of 64 steps of three roundings, each chain at random about 0.2 of
+    # the root of its length in units of 2^-24: 3.6; what a decay of 0.8 to 1 and the rule leave of earlier chunks' adds a
+    # fifth; three times that for the spread
+    tol = 13 * 2.0 ** -24
+
+    def rms(x):
+        return float(x.pow(2).mean().sqrt())
+    for b in range(B):
+        S, want = state[slots[b]].double(), []
+        for t in range(cu[b], cu[b + 1]):
+            S = S * decay[t].double().view(H, 1, 1)
+            S = S + k[t].unsqueeze(-1) * (beta[t].double().view(H, 1) * (v[t] - (S * k[t].unsqueeze(-1)).sum(1))).unsqueeze(1)
+            want.append((S * q[t].unsqueeze(-1)).sum(1))
+        want = torch.stack(want)
+        assert rms(out[cu[b]:cu[b + 1]] - want) <= tol * rms(want)
+        assert rms(st[slots[b]].cpu().double() - S) <= tol * rms(S)
+    assert torch.equal(st[0].cpu(), state[0])
