@@ -23,33 +23,45 @@
 // ---------------------------------------------------------------------------
 #define MOE_MAX_TOP 16
 
-// the `top` largest of a row's E logits z (the lowest index among equal ones) and their sigmoids
-__device__ __forceinline__ void route_row(const float* z, int E, int top, int* __restrict__ experts,
-                                          float* __restrict__ weights);
-
-__global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__ logits, int T, int E, int top,
-                                                       int* __restrict__ experts, float* __restrict__ weights) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+// The `top` largest of a row's E logits z (the lowest index among equal ones; a NaN is passed over, unless it is the first
+// that is left) and their sigmoids.  A wave a token, lane l looks after logits l, l + 64, ..: 32 tokens of 32 experts, top 4,
+// 8 us; a thread a token, whose reads and comparisons wait for one another, 28.
+__global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ logits, int T, int E, int top,
+                                                        int* __restrict__ experts, float* __restrict__ weights) {
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (t >= T) return;
-  route_row(logits + (size_t)t * E, E, top, experts + (size_t)t * top, weights + (size_t)t * top);
-}
-
-__device__ __forceinline__ void route_row(const float* z, int E, int top, int* __restrict__ experts,
-                                          float* __restrict__ weights) {
+  const float* z = logits + (size_t)t * E;
   int chosen[MOE_MAX_TOP];
-  for (int k = 0; k < top; k++) {
-    int best = -1;
-    float bz = 0.f;
-    for (int e = 0; e < E; e++) {
+#pragma unroll
+  for (int k = 0; k < MOE_MAX_TOP; k++) chosen[k] = -1;
+#pragma unroll
+  for (int k = 0; k < MOE_MAX_TOP; k++) {
+    if (k >= top) break;
+    float bz = -INFINITY;
+    int best = 0x7fffffff, first = 0x7fffffff;
+    for (int e = lane; e < E; e += 64) {
       bool taken = false;
+#pragma unroll
       for (int j = 0; j < k; j++) taken |= chosen[j] == e;
       if (taken) continue;
+      first = min(first, e);
       const float v = z[e];
-      if (best < 0 || v > bz) { best = e; bz = v; }     // NaN never wins over a number; the first of equals stays
+      if (v > bz || (v == bz && e < best)) { bz = v; best = e; }
     }
+#pragma unroll
+    for (int x = 1; x < 64; x *= 2) {
+      const float oz = __shfl_xor(bz, x);
+      const int oe = __shfl_xor(best, x);
+      if (oe != 0x7fffffff && (best == 0x7fffffff || oz > bz || (oz == bz && oe < best))) { bz = oz; best = oe; }
+      first = min(first, __shfl_xor(first, x));
+    }
+    const float zf = z[first];                       // (top <= E: there is one)
+    if (zf != zf || best == 0x7fffffff) { best = first; bz = zf; }
     chosen[k] = best;
-    experts[k] = best;
-    weights[k] = 1.0f / (1.0f + expf(-bz));
+    if (lane == k) {
+      experts[(size_t)t * top + k] = best;
+      weights[(size_t)t * top + k] = 1.0f / (1.0f + expf(-bz));
+    }
   }
 }
 
@@ -150,7 +162,7 @@ static int moe_router_impl(const void* x, int ldx, int dtype, const float* Wr, i
   if (softmax)
     moe_route_softmax_kernel<<<(T + 3) / 4, 256, 0, stream>>>(z, correction, T, E, top, scale, experts, weights);
   else
-    moe_route_kernel<<<(T + 63) / 64, 64, 0, stream>>>(z, T, E, top, experts, weights);
+    moe_route_kernel<<<(T + 3) / 4, 256, 0, stream>>>(z, T, E, top, experts, weights);
   PICO_LAUNCH_CHECK();
   return 0;
 }
@@ -160,7 +172,7 @@ extern "C" int pico_moe_route(const float* logits, int T, int E, int top, int* e
   PICO_REQUIRE(T >= 0 && E > 0 && top > 0 && top <= E && top <= MOE_MAX_TOP,
                "pico_moe_route: %d of %d experts per token is outside what the kernel takes (at most %d)", top, E, MOE_MAX_TOP);
   if (T == 0) return 0;
-  moe_route_kernel<<<(T + 63) / 64, 64, 0, stream>>>(logits, T, E, top, experts, weights);
+  moe_route_kernel<<<(T + 3) / 4, 256, 0, stream>>>(logits, T, E, top, experts, weights);
   PICO_LAUNCH_CHECK();
   return 0;
 }

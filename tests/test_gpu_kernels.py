@@ -1433,3 +1433,23 @@ def test_delta_chunks(K, dk, lens, dv):
         assert rms(out[cu[b]:cu[b + 1]] - want) <= tol * rms(want)
         assert rms(st[slots[b]].cpu().double() - S) <= tol * rms(S)
     assert torch.equal(st[0].cpu(), state[0])
+
+
+@pytest.mark.parametrize("E,top", [(1, 1), (5, 5), (63, 4), (64, 2), (65, 16), (130, 3)])
+def test_moe_route_among_equal_and_odd_logits(K, E, top):
+    # the lowest of equal logits first; a NaN only where it is the first that is left; all of a row minus infinity
+    g = torch.Generator().manual_seed(E)
+    z = torch.randint(-3, 4, (41, E), generator=g).float()
+    z[3], z[4, E // 2], z[5, 0], z[6, E - 1] = float("-inf"), float("nan"), float("nan"), float("inf")
+    z[7, ::2] = float("nan")
+    experts, weights = K.moe_route(z.to(DEV), top)
+    for t in range(41):
+        row, left = z[t].tolist(), list(range(E))
+        for k in range(top):
+            best = left[0]
+            for e in left:
+                best = e if row[e] > row[best] else best
+            left.remove(best)
+            assert int(experts[t, k]) == best, (t, k)
+    want = torch.sigmoid(torch.gather(z, 1, experts.cpu().long()))
+    assert torch.allclose(weights.cpu(), want, rtol=1e-6, atol=0, equal_nan=True)      # one exponential and a quotient
