@@ -129,25 +129,53 @@ extern "C" int pico_add_layernorm(float* resid, const void* delta, int delta_dty
 // resid[t][i] += scale[i] * (a_0[t][i] + a_1[t][i] + .. + sigmoid(gate[t * gate_stride]) * b[t][i])
 // a: `slabs` addends of type TA (or none); b of type TB with a gate logit per row (or none; no gate: b as it is);
 // scale [H] or none.
-template <typename TA, typename TB>
+// V entries a thread: four where rows and addresses allow it (1,377 rows of 1,536 with two float32 addends and a gated
+// bfloat16 one: 9.6 us against 15.6 with one).
+template <typename T, int V> __device__ __forceinline__ void scaled_load(const T* p, float* v) {
+  if constexpr (V == 1) {
+    v[0] = load_f32(p);
+  } else if constexpr (sizeof(T) == 4) {
+    const float4 r = *reinterpret_cast<const float4*>(p);
+    v[0] = r.x; v[1] = r.y; v[2] = r.z; v[3] = r.w;
+  } else {
+    const uint2 r = *reinterpret_cast<const uint2*>(p);
+    v[0] = __uint_as_float(r.x << 16); v[1] = __uint_as_float(r.x & 0xffff0000u);
+    v[2] = __uint_as_float(r.y << 16); v[3] = __uint_as_float(r.y & 0xffff0000u);
+  }
+}
+
+template <typename TA, typename TB, int V>
 __global__ __launch_bounds__(256) void scaled_add_kernel(float* __restrict__ resid, const TA* __restrict__ a, int slabs,
                                                          size_t slab_stride, const TB* __restrict__ b,
                                                          const float* __restrict__ gate, int gate_stride,
                                                          const float* __restrict__ scale, int H, size_t n) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (i >= n) return;
   const int col = (int)(i % H);
-  float d = 0.f;
+  float d[V], x[V], s[V], bv[V];
+  scaled_load<float, V>(resid + i, x);
+  if (scale) scaled_load<float, V>(scale + col, s);
+  if (b) scaled_load<TB, V>(b + i, bv);
+#pragma unroll
+  for (int v = 0; v < V; v++) d[v] = 0.f;
   if (a) {
-    d = load_f32(a + i);
-    for (int k = 1; k < slabs; k++) d += load_f32(a + k * slab_stride + i);
+    scaled_load<TA, V>(a + i, d);
+    for (int k = 1; k < slabs; k++) {
+      float more[V];
+      scaled_load<TA, V>(a + k * slab_stride + i, more);
+#pragma unroll
+      for (int v = 0; v < V; v++) d[v] += more[v];
+    }
   }
   if (b) {
-    float bv = load_f32(b + i);
-    if (gate) bv *= 1.0f / (1.0f + expf(-gate[(i / H) * (size_t)gate_stride]));
-    d += bv;
+    const float g = gate ? 1.0f / (1.0f + expf(-gate[(i / H) * (size_t)gate_stride])) : 1.f;
+#pragma unroll
+    for (int v = 0; v < V; v++) d[v] += gate ? bv[v] * g : bv[v];
   }
-  resid[i] += scale ? scale[col] * d : d;
+#pragma unroll
+  for (int v = 0; v < V; v++) x[v] += scale ? s[v] * d[v] : d[v];
+  if constexpr (V == 1) resid[i] = x[0];
+  else *reinterpret_cast<float4*>(resid + i) = make_float4(x[0], x[1], x[2], x[3]);
 }
 
 extern "C" int pico_scaled_add(float* resid, const void* a, int a_dtype, int slabs, long long slab_stride, const void* b,
@@ -157,10 +185,17 @@ extern "C" int pico_scaled_add(float* resid, const void* a, int a_dtype, int sla
   PICO_REQUIRE(a != nullptr || b != nullptr, "pico_scaled_add: nothing to add");
   if (T == 0) return 0;
   const size_t n = (size_t)T * H;
-  const unsigned grid = (unsigned)((n + 255) / 256);
+  const bool four = H % 4 == 0 && ((uintptr_t)resid | (uintptr_t)a | (uintptr_t)b | (uintptr_t)scale) % 16 == 0 && slab_stride % 4 == 0;
+  const unsigned grid = (unsigned)(((four ? n / 4 : n) + 255) / 256);
 #define LAUNCH(TA, TB)                                                                                               \
-  scaled_add_kernel<TA, TB><<<grid, 256, 0, stream>>>(resid, (const TA*)a, slabs, (size_t)slab_stride, (const TB*)b, \
-                                                      gate, gate_stride, scale, H, n)
+  do {                                                                                                               \
+    if (four)                                                                                                        \
+      scaled_add_kernel<TA, TB, 4><<<grid, 256, 0, stream>>>(resid, (const TA*)a, slabs, (size_t)slab_stride, (const TB*)b, \
+                                                             gate, gate_stride, scale, H, n);                        \
+    else                                                                                                             \
+      scaled_add_kernel<TA, TB, 1><<<grid, 256, 0, stream>>>(resid, (const TA*)a, slabs, (size_t)slab_stride, (const TB*)b, \
+                                                             gate, gate_stride, scale, H, n);                        \
+  } while (0)
   const int ad = a ? a_dtype : PICO_DTYPE_F32, bd = b ? b_dtype : PICO_DTYPE_F32;
   if (ad == PICO_DTYPE_F32 && bd == PICO_DTYPE_F32) LAUNCH(float, float);
   else if (ad == PICO_DTYPE_F32 && bd == PICO_DTYPE_BF16) LAUNCH(float, bf16_t);

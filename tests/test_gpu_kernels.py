@@ -1453,3 +1453,25 @@ def test_moe_route_among_equal_and_odd_logits(K, E, top):
             assert int(experts[t, k]) == best, (t, k)
     want = torch.sigmoid(torch.gather(z, 1, experts.cpu().long()))
     assert torch.allclose(weights.cpu(), want, rtol=1e-6, atol=0, equal_nan=True)      # one exponential and a quotient
+
+
+@pytest.mark.parametrize("T,H", [(1, 4), (7, 44), (3, 45), (130, 1536)])
+@pytest.mark.parametrize("slabs,gated,scaled,b_dtype", [(1, False, False, None), (3, True, True, torch.bfloat16), (2, False, True, torch.float32),
+                                                        (0, True, False, torch.float32)])
+def test_scaled_add(K, T, H, slabs, gated, scaled, b_dtype):
+    # four entries a thread (rows of whole fours on aligned addresses) and one
+    g = torch.Generator().manual_seed(T + H)
+    x, a = torch.randn(T, H, generator=g), torch.randn(slabs, T, H, generator=g) if slabs else None
+    b = torch.randn(T, H, generator=g).to(b_dtype) if b_dtype else None
+    gate, scale = (torch.randn(T, 1, generator=g) if gated and b_dtype else None), (torch.randn(H, generator=g) if scaled else None)
+    want = (a.double().sum(0) if slabs else 0) + (0 if b is None else b.double() * (torch.sigmoid(gate.double()) if gate is not None else 1))
+    want = x.double() + (want * scale.double() if scaled else want)
+    size = x.abs().double() + ((a.abs().double().sum(0) if slabs else 0) + (0 if b is None else b.abs().double())) * (scale.abs().double() if scaled else 1)
+    for off in (0, 1):                                                   # the stream on 16 bytes, and 4 behind
+        buf = torch.zeros(T * H + 1)
+        buf[off:off + T * H] = x.view(-1)
+        resid = buf.to(DEV)[off:off + T * H].view(T, H)
+        K.scaled_add(resid, None if a is None else a.to(DEV) if slabs > 1 else a[0].to(DEV), None if b is None else b.to(DEV),
+                     None if gate is None else gate.to(DEV), None if scale is None else scale.to(DEV))
+        # eight float32 roundings at most, of parts of `size`
+        assert bool(((resid.cpu().double() - want).abs() <= 8 * 2.0 ** -24 * size).all())
