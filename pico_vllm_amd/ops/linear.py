@@ -64,10 +64,15 @@ def _library_tuning(rows: int) -> None:
     if st["ready"] == "off":
         return
     # never while a graph is being recorded: timing candidates does not belong into a graph
-    want = rows % TUNE_ROWS == 0 and not torch.cuda.is_current_stream_capturing()
+    want = _tuned(rows) and not torch.cuda.is_current_stream_capturing()
     if st["tuning"] != want:
         tunable.tuning_enable(want)
         st["tuning"] = want
+
+
+def _tuned(rows: int) -> bool:
+    """Whether the library's tuner looks after products of this many rows."""
+    return _tuner_state["wanted"] and rows % TUNE_ROWS == 0
 
 
 class no_library_tuning:
@@ -136,7 +141,7 @@ class Linear:
         few = self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight)
         if few and not kernels.tiles_few_ok(x, self.weight, True):
             return kernels.gemm_skinny(x, self.weight, None, kernels.EPI_SWIGLU)
-        if self.bias is None and (few or kernels.tiles_act_ok(x, self.weight, True)):
+        if self.bias is None and (few or kernels.tiles_act_ok(x, self.weight, True, _tuned(x.shape[0]))):
             return kernels.gemm_tiles(x, self.weight, None, kernels.EPI_SWIGLU)
         return kernels.swiglu(self(x))
 
@@ -146,7 +151,7 @@ class Linear:
         few = self.weight.dtype == torch.bfloat16 and self.bias is None and kernels.skinny_ok(x, self.weight)
         if few and not kernels.tiles_few_ok(x, self.weight, True):
             return kernels.gemm_skinny(x, self.weight, None, kernels.EPI_CLIPPED, clip=(limit, alpha))
-        if self.bias is None and (few or kernels.tiles_act_ok(x, self.weight, True)):
+        if self.bias is None and (few or kernels.tiles_act_ok(x, self.weight, True, _tuned(x.shape[0]))):
             return kernels.gemm_tiles(x, self.weight, None, kernels.EPI_CLIPPED, clip=(limit, alpha))
         return kernels.clipped_glu(self(x), limit, alpha)
 
