@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
   typedef TileStream<MB, NB, SETS> TS;
   TS ts(smem);
   constexpr int TM = 64 * MB, TN = 64 * NB, COLS = gt_paired(EPI) ? TN / 2 : TN;      // output columns of a tile
-  const int tiles = a.m_tiles * a.n_tiles, first = ts_first();
-  if (first >= tiles) return;
+  const int tiles = a.m_tiles * a.n_tiles;
+  if (ts_tile(0, tiles) < 0) return;
   TileRowsSource<MB> xs;
   TileRowsSource<NB> ws;
   auto aim = [&](int t) {
@@ -96,7 +96,7 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
       for (int j = 0; j < 2 * NB; j++) ws.off[j] = (uint32_t)(ts.row(j) * a.ldw) * 2;
     }
   };
-  ts.run(first, gridDim.x, tiles, a.K, xs, ws, aim, [&](int t) {
+  ts.run(tiles, a.K, xs, ws, aim, [&](int t) {
     // lane (l, h): row l of a block of X, tile rows 8 (r / 4) + 4 h + r % 4 of a block of W in register r
     int mt, nt;
     ts_place(a.m_tiles, a.n_tiles, t, mt, nt);
@@ -184,16 +184,14 @@ static int gt_launch(GemmArgs a, hipStream_t stream) {
   a.n_tiles = (a.cols + GT_COLS(NB, EPI) - 1) / GT_COLS(NB, EPI);
   const long long tiles = (long long)a.m_tiles * a.n_tiles;
   PICO_REQUIRE(tiles < (1LL << 30), "pico_gemm_tiles: %d x %d outputs are too many for one launch", a.M, a.cols);
-  const int most = 256 * ts_share(MB, NB);
-  gemm_tiles_kernel<MB, NB, EPI, SETS><<<tiles < most ? (int)tiles : most, 256, ts_lds_bytes(MB, NB), stream>>>(a);
+  gemm_tiles_kernel<MB, NB, EPI, SETS><<<ts_grid(tiles, 256 * ts_share(MB, NB)), 256, ts_lds_bytes(MB, NB), stream>>>(a);
   PICO_LAUNCH_CHECK();
   return 0;
 }
 
 // Which tile.  All make the same sums, so it is a question of how many rounds of workgroups a call takes and what one costs:
 // microseconds `each` a stage + `more`, fitted to calls of 24 and 56 stages with operands from memory.  A tile of which
-// two share a compute unit costs `lone` a stage where a unit has one, as in a call of one round of them (a last round behind full
-// ones is dealt two a unit to the first dies and costs more than that).  Outputs a microsecond of a full round are alike
+// two share a compute unit costs `lone` a stage where a unit has one.  Outputs a microsecond of a full round are alike
 // (0.34 to 0.36 million a microsecond and 24 stages), so what is left idle in the last round decides.
 struct GtTile { int mb, nb, share; float each, lone, more; };
 static const GtTile gt_tiles[] = {{2, 3, 2, 1.45f, 1.20f, 3.f}, {4, 2, 1, 0.84f, 0.84f, 3.8f}, {3, 3, 1, 1.00f, 1.00f, 2.f}, {2, 1, 2, 0.80f, 0.35f, 3.f}};

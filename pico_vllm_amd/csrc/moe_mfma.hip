@@ -250,8 +250,8 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void moe_grouped_kernel(cons
   typedef TileStream<MB, NB> TS;
   TS ts(smem);
   constexpr int TM = 64 * MB, TN = 64 * NB, COLS = UP ? TN / 2 : TN;
-  const int K = UP ? a.D : a.F, tiles = moe_scalar(a.tiles + 2 * a.tiles_cap) * a.n_tiles, first = ts_first();
-  if (first >= tiles) return;
+  const int K = UP ? a.D : a.F, tiles = moe_scalar(a.tiles + 2 * a.tiles_cap) * a.n_tiles;
+  if (ts_tile(0, tiles) < 0) return;
   TileRowsSource<MB> xs;
   TileRowsSource<NB> ws;
   auto aim = [&](int t) {
@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void moe_grouped_kernel(cons
       for (int j = 0; j < 2 * NB; j++) ws.off[j] = (uint32_t)(ts.row(j) * K) * 2;
     }
   };
-  ts.run(first, gridDim.x, tiles, K, xs, ws, aim, [&](int t) {
+  ts.run(tiles, K, xs, ws, aim, [&](int t) {
     // lane (l, h): row l of a block of X, tile rows 8 (r / 4) + 4 h + r % 4 of a block of W in register r
     int mt, nt;
     moe_place(a, t, mt, nt);
@@ -340,11 +340,11 @@ static int moe_launch(MoeArgs a, hipStream_t stream) {
   static const hipError_t room = hipFuncSetAttribute((const void*)&moe_grouped_kernel<MB, NB, UP>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, ts_lds_bytes(MB, NB));
   PICO_REQUIRE(room == hipSuccess, "pico_moe_experts_grouped: %s", hipGetErrorString(room));
-  const int cols = UP ? 32 * NB : 64 * NB, n = UP ? a.F : a.D, most = 256 * ts_share(MB, NB);
+  const int cols = UP ? 32 * NB : 64 * NB, n = UP ? a.F : a.D;
   a.n_tiles = (n + cols - 1) / cols;
   const long long tiles = (long long)a.tiles_cap * a.n_tiles;
   PICO_REQUIRE(tiles < (1LL << 30), "pico_moe_experts_grouped: sizes beyond one launch");
-  moe_grouped_kernel<MB, NB, UP><<<tiles < most ? (int)tiles : most, 256, ts_lds_bytes(MB, NB), stream>>>(a);
+  moe_grouped_kernel<MB, NB, UP><<<ts_grid(tiles, 256 * ts_share(MB, NB)), 256, ts_lds_bytes(MB, NB), stream>>>(a);
   return 0;
 }
 
@@ -354,8 +354,7 @@ static int moe_launch(MoeArgs a, hipStream_t stream) {
 extern "C" int pico_moe_tile_rows(long long rows, int E) { return rows <= 48LL * E ? 64 : 128; }
 
 // Columns of a tile: as many rounds of workgroups as a call is expected to take (its rows spread over the experts at
-// random), at the cost of a stage in a full round and in a last one that leaves a compute unit at most one workgroup (measured
-// as a call's only one; behind full rounds the first dies have two a unit and the others none), in
+// random), at the cost of a stage in a full round and in a last one that leaves a compute unit at most one workgroup, in
 // microseconds; the operands come from memory, so a stage costs its latency more than its products.
 struct MoeTile { int nb, share; float each, lone; };
 static const MoeTile moe_tiles[2][2] = {{{1, 2, 0.72f, 0.6f}, {2, 2, 1.3f, 1.1f}}, {{3, 2, 1.9f, 1.65f}, {4, 1, 1.4f, 1.4f}}};

@@ -36,6 +36,9 @@ constexpr int ts_lds_bytes(int MB, int NB) { return ts_stage_bytes(MB, NB) * ts_
 // s_waitcnt: at most n vector memory operations outstanding; with `lds` also no LDS read
 constexpr int ts_wait(int n, bool lds) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | ((lds ? 0 : 15) << 8); }
 
+// workgroups for so many tiles where `most` run at once
+constexpr int ts_grid(long long tiles, int most) { return tiles < most ? (int)((tiles + 7) / 8 * 8) : most; }
+
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
 // The rows of one operand of a tile, as what a lane asks for: `rsrc` over the matrix from the tile's first row on, and the
 // byte offset of this lane's chunk in its row of each of the wave's copies (eight rows each), at k = 0.
@@ -47,6 +50,18 @@ struct TileRowsSource {
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t ts_buffer(const void* base, long long bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)min(bytes, (long long)0x7fffffff), 0x00020000);
+}
+
+// The tile a workgroup takes in round r of `tiles`, or -1.  Workgroups go to the dies in turn (the grid is a multiple of eight,
+// ts_grid), and a die's share of a round is a run of neighbouring tiles; so is its share of a last round that is not full: an
+// eighth of what is left, for the workgroups that came to the die first, one a compute unit while there are units.  (Dealt from the
+// first die on, and grids that are no multiple of eight left as they came: gelu of 13,440 columns, K 1,536, 832 rows 55 us, 45
+// so; 11,008 pairs, K 2,048, 832 rows 101, 86; 18,944 pairs, K 3,584, 300 rows 135, 117; the two products of 2,754 rows over 16
+// experts of 2,240 x 1,536 149, 134; calls of whole rounds the same.)
+__device__ __forceinline__ int ts_tile(int r, int tiles) {
+  const int die = blockIdx.x & 7, place = blockIdx.x >> 3, from = r * (int)gridDim.x, left = tiles - from;
+  const int share = left >= (int)gridDim.x ? (int)gridDim.x >> 3 : (left + 7) >> 3, at = die * share + place;
+  return place < share && at < left ? from + at : -1;
 }
 
 template <int FROM, int TO> struct Range { static constexpr int from = FROM, to = TO; };
@@ -182,22 +197,21 @@ struct TileStream {
       round(Sets<V + 1>(), s, stages, buf, copies, on);
     }
   }
-  // Tiles first, first + step, .. below `tiles`, each over K: `aim(t)` points xs and ws at tile t, `done(t)` takes its sums.
+  // This workgroup's tiles of so many (ts_tile), each over K: `aim(t)` points xs and ws at tile t, `done(t)` takes its sums.
   template <typename Aim, typename Done>
-  __device__ __forceinline__ void run(int first, int step, int tiles, int K, const TileRowsSource<MB>& xs,
-                                      const TileRowsSource<NB>& ws, Aim aim, Done done) {
+  __device__ __forceinline__ void run(int tiles, int K, const TileRowsSource<MB>& xs, const TileRowsSource<NB>& ws, Aim aim, Done done) {
     const int stages = (K + TS_BK - 1) / TS_BK;
-    int at_tile = first, at_stage = 0, fill = 0;             // the stage that is asked for next, into buffer `fill`
-    auto copies = [&](auto r) { ask<decltype(r)::from, decltype(r)::to>(fill, xs, ws, at_tile < tiles ? at_stage * TS_BK : K, K); };
+    int at_round = 0, at_tile = ts_tile(0, tiles), at_stage = 0, fill = 0;      // the stage that is asked for next, into buffer `fill`
+    auto copies = [&](auto r) { ask<decltype(r)::from, decltype(r)::to>(fill, xs, ws, at_tile >= 0 ? at_stage * TS_BK : K, K); };
     auto on = [&] {
       fill = fill + 1 == NBUF ? 0 : fill + 1;
-      if (++at_stage == stages && at_tile < tiles) {
+      if (++at_stage == stages && at_tile >= 0) {
         at_stage = 0;
-        at_tile += step;
-        if (at_tile < tiles) aim(at_tile);
+        at_tile = ts_tile(++at_round, tiles);
+        if (at_tile >= 0) aim(at_tile);
       }
     };
-    aim(first);
+    aim(at_tile);
 #pragma unroll
     for (int b = 0; b < NBUF - 1; b++) {
       copies(Range<0, LOADS>());
@@ -209,7 +223,7 @@ struct TileStream {
     copies(Range<0, part(1)>());
     read(0, 0, 0);
     int buf = 0;
-    for (int t = first; t < tiles; t += step) {
+    for (int turn = 0, t; (t = ts_tile(turn, tiles)) >= 0; turn++) {
       clear();
       for (int s = 0; s < stages; s += SETS) round(Sets<0>(), s, stages, buf, copies, on);
       done(t);
@@ -224,10 +238,5 @@ __device__ __forceinline__ void ts_place(int m_tiles, int n_tiles, int t, int& m
   const int per = 8 * n_tiles, strip = t / per, rest = t - strip * per, rows = min(8, m_tiles - strip * 8);
   n = rest / rows;
   m = strip * 8 + rest - n * rows;
-}
-// Workgroups go to the dies in turn; a die's share of a round is a run of neighbouring tiles.  (So is its share of a last round
-// that is not full: 256 tiles behind rounds of 512 run two a compute unit on four dies, and the others have none.)
-__device__ __forceinline__ int ts_first() {
-  return gridDim.x % 8 == 0 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
 }
 #endif

@@ -223,6 +223,17 @@ def test_gemm_tiles(K, M, N, K_, name):
     assert torch.equal(K.gemm_tiles(a[:(M + 1) // 2], w, b, epi, clip), out[:(M + 1) // 2])
 
 
+@pytest.mark.parametrize("tiles", [1, 7, 8, 9, 63, 255, 257, 511, 513, 520, 767, 1025, 1031])
+def test_gemm_tiles_deals_every_tile_once(K, tiles):
+    # grids of every remainder by eight, last rounds of one tile, of an eighth less one, of one tile a compute unit and more;
+    # a tile is made of exact sums (whole numbers), so a tile that is left out or written by another shows
+    g = torch.Generator(device=DEV).manual_seed(tiles)
+    a = torch.randint(-4, 5, (100, 64), device=DEV, generator=g).bfloat16()
+    w = torch.randint(-4, 5, (64 * tiles, 64), device=DEV, generator=g).bfloat16()
+    for _ in range(2):
+        assert torch.equal(K.gemm_tiles(a, w, None, K.EPI_F32), a.float() @ w.float().T)
+
+
 @pytest.mark.parametrize("M", [65, 700])
 def test_gemm_tiles_gelu_over_its_range(K, M):
     # the epilogue's own error function from end to end, a bias that starts on no 16 bytes beside it
