@@ -35,6 +35,8 @@ ATTN_SOURCES = ("errors.hip", "attention_mfma.hip")
 
 ATTN_BIAS_SOURCES = ("errors.hip", "attention_bias_mfma.hip")
 
+LATENT_SOURCES = ("errors.hip", "latent_prompt.hip")
+
 PEAK_SOURCES = ("errors.hip", "peaks.hip")
 
 _loaded: Dict[str, ctypes.CDLL] = {}
@@ -151,6 +153,16 @@ def attention_bias_library(key_dim: int, value_dim: int) -> ctypes.CDLL:
                         (f"-DPICO_DK={key_dim}", f"-DPICO_DV={value_dim}"))
 
 
+def latent_prompt_library(dim: int, rot_dim: int, value_dim: int, rank: int) -> ctypes.CDLL:
+    """Prompt attention through a latent with the heads' own keys and values, specialised for one set of sizes."""
+    return load_library(*_latent_prompt(dim, rot_dim, value_dim, rank))
+
+
+def _latent_prompt(dim: int, rot_dim: int, value_dim: int, rank: int) -> tuple:
+    return (f"pico_latent_d{dim}_r{rot_dim}_v{value_dim}_c{rank}", LATENT_SOURCES,
+            (f"-DPICO_LAT_D={dim}", f"-DPICO_LAT_R={rot_dim}", f"-DPICO_LAT_V={value_dim}", f"-DPICO_LAT_RANK={rank}"))
+
+
 def peaks() -> ctypes.CDLL:
     """The two measuring kernels of the benchmark (a read stream, a matrix-core loop)."""
     return load_library("pico_peaks", PEAK_SOURCES)
@@ -158,7 +170,8 @@ def peaks() -> ctypes.CDLL:
 
 def build_all(head_dims: Iterable[int] = tuple(range(16, 257, 16)), force: bool = True,
               bias_dims: Iterable[tuple] = ((64, 32), (64, 64), (128, 64), (128, 128), (32, 16), (32, 64), (64, 48), (64, 16), (32, 32), (32, 96), (64, 96),
-                                          (128, 96), (96, 64), (320, 256), (256, 224), (288, 224), (64, 128), (96, 96), (32, 48))) -> List[str]:
+                                          (128, 96), (96, 64), (320, 256), (256, 224), (288, 224), (64, 128), (96, 96), (32, 48)),
+              latent_dims: Iterable[tuple] = ((128, 64, 128, 256), (64, 32, 64, 128), (32, 64, 32, 96), (64, 128, 128, 32))) -> List[str]:
     """Compile everything (used by the build check); returns the paths."""
     out = [build_library("pico_core", CORE_SOURCES, force=force), build_library("pico_peaks", PEAK_SOURCES, force=force)]
     if os.path.isfile(os.path.join(CSRC, "attention_mfma.hip")):
@@ -166,4 +179,7 @@ def build_all(head_dims: Iterable[int] = tuple(range(16, 257, 16)), force: bool 
             out.append(build_library(f"pico_attn_d{d}", ATTN_SOURCES, (f"-DPICO_HEAD_DIM={d}",), force=force))
     for dk, dv in bias_dims:
         out.append(build_library(f"pico_attnb_k{dk}_v{dv}", ATTN_BIAS_SOURCES, (f"-DPICO_DK={dk}", f"-DPICO_DV={dv}"), force=force))
+    for sizes in latent_dims:
+        name, sources, defines = _latent_prompt(*sizes)
+        out.append(build_library(name, sources, defines, force=force))
     return out

@@ -67,6 +67,7 @@ class LatentAttention(Mixer):
         self.uv_t: Optional[torch.Tensor] = None  # [H, kv_rank, dv]
         self.wq = self.wkv = None
         self.fast = None
+        self.prompt = None                        # portions of many tokens with the heads' own keys and values
 
     def cache_spec(self) -> CacheSpec:
         return CacheSpec("paged_kv", page_tensors=(PageTensor("k", (1, "page", self.kv_rank + self.r)),
@@ -111,9 +112,17 @@ class LatentAttention(Mixer):
             if attention_bias_fast.supported(self.dk, self.kv_rank) and (self.heads * self.dk) % 8 == 0:
                 self.fast = attention_bias_fast.FastBiasAttention(self.nq, 1, self.dk, self.kv_rank, self.scale,
                                                                   gated=self.gate_heads, gate_heads=self.gate_heads)
+                from ..ops import latent_prompt
+                # (its query rows start on 8 bytes)
+                q_cols = self.uq.out_features if self.q_rank else self.down.out_features
+                if latent_prompt.supported(self.d, self.r, self.dv, self.kv_rank) and q_cols % 4 == 0:
+                    self.prompt = latent_prompt.LatentPrompt(H, self.d, self.r, self.dv, self.kv_rank, self.scale,
+                                                             self.uk_t.view(H * self.d, self.kv_rank), tensors[n["uv"]].to(device).contiguous())
 
     def graph_variant(self, ctx: StepContext) -> tuple:
-        return (("latent_attention",) + self.fast.plan(ctx),) if self.fast is not None else ()
+        if self.fast is None:
+            return ()
+        return (("latent_attention",) + self.fast.plan(ctx) + ((self.prompt.plan(ctx),) if self.prompt is not None else ()),)
 
     def _per_head(self, x: torch.Tensor, x_head: int, w: torch.Tensor, copy: int = 0, turn=None) -> torch.Tensor:
         """out[t, h] = [x[t, h, :in] @ w[h] | x[t, h, in : in + copy]]; x [T, >= H * x_head].  ``turn``: the table of the
@@ -150,12 +159,28 @@ class LatentAttention(Mixer):
                                     self.norm_eps, table, ctx.slot_mapping[cache.group], cache.k, cache.v)
         q = self.uq(cq) if self.q_rank else y                    # [T, >= H (d + r)]
         gate = y[:, self.g_col:] if self.gate_heads else None
+        bt = ctx.block_tables[cache.group]
+        plan = self.prompt.plan(ctx) if self.prompt is not None and cache.k.dtype == torch.bfloat16 else None
+        if plan is not None:
+            lead = int(ctx.host["cu_seqlens"][plan[0]])
+            out = torch.empty(x.shape[0], H * self.dv, dtype=x.dtype, device=x.device)
+            if lead:
+                out[:lead] = self._in_latent(q[:lead], table[:lead], cache, bt[:plan[0]], ctx, plan[0], None if gate is None else gate[:lead])
+            return self.prompt(q, table, cache, bt, ctx, plan, out, gate)
+        return self._in_latent(q, table, cache, bt, ctx, ctx.num_seqs, gate)
+
+    def _in_latent(self, q: torch.Tensor, table: Optional[torch.Tensor], cache, bt: torch.Tensor, ctx: StepContext, num_seqs: int,
+                   gate: Optional[torch.Tensor]) -> torch.Tensor:
+        """Attention in the latent's space for the rows of q, those of the step's first ``num_seqs`` sequences."""
+        H, d, r = self.heads, self.d, self.r
         # the queries in the latent's space, their rotated part turned on the way: [T, H (kv_rank + r)]
         ql = self._per_head(q, d + r, self.uk_t, copy=r, turn=table if r else None)
-        bt = ctx.block_tables[cache.group]
-        if self.fast is not None and cache.k.dtype == torch.bfloat16:
-            ol = self.fast(ql, cache, bt, ctx, gate=gate)
-        else:
-            ol = kernels.attn_bias_plain(ql, cache.k, cache.v, bt, ctx.positions, ctx.token_seq, H, 1, self.dk, self.kv_rank,
+        if self.fast is None or cache.k.dtype != torch.bfloat16:
+            T = q.shape[0]
+            ol = kernels.attn_bias_plain(ql, cache.k, cache.v, bt, ctx.positions[:T], ctx.token_seq[:T], H, 1, self.dk, self.kv_rank,
                                          self.scale, 0, gate=gate, gate_heads=self.gate_heads)
+        elif num_seqs < ctx.num_seqs:
+            ol = self.fast.run(ql, cache.k, cache.v, bt, ctx.cu_seqlens, ctx.positions, num_seqs, gate=gate)
+        else:
+            ol = self.fast(ql, cache, bt, ctx, gate=gate)
         return self._per_head(ol, self.kv_rank, self.uv_t)       # [T, H dv]
