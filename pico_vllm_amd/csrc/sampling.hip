@@ -17,27 +17,35 @@
 // faster than one compute unit takes data in: 19 us for 151,936 logits), in a chain of launches whose
 // workgroups never wait for one another: what a launch needs of the launch before it lies in memory.
 //   1. the first maximum of every chunk (argmax_part_kernel);
-//   2. for rows with top_p < 1, five rounds that narrow t* in the order of the float's bit pattern (e lies in
-//      (0, 1], where that order is the order of the values): a round lays 63 thresholds evenly between the
-//      bounds lo < t* <= hi, every workgroup sorts the e of its chunk into the 64 classes between them and
-//      sums each class; the next launch adds the classes of all chunks, finds between which two thresholds
-//      f drops below the target and takes those as its bounds: 2^30 patterns shrink by 64 a round;
-//   3. per chunk, the sum of e > t* in double and the number of e == t*;
-//   4. one workgroup a row picks the chunk, then the thread, then the token at which the running sum of the
-//      kept e passes u times their total, ties counted in vocabulary order.
-// All sums run in a fixed order, so a row's result depends on its inputs only.  e is the hardware's exponential
-// (__expf: 2^(x log2 e)) in every launch alike: what a token weighs must be the same bits wherever it is asked.
+//   2. for rows with top_p < 1, the mass of e by its bit pattern (e lies in (0, 1], where the patterns' order is the order of
+//      the values): 2,033 classes of 2^19 patterns, a sixteenth of a factor of two each (sample_classes_kernel);
+//   3. every workgroup finds from them the class in which f drops below the target, sums what its chunk has above that class, in
+//      double, and lists what it has in it (sample_collect_kernel);
+//   4. one workgroup a row finds t* among what is listed (classes of 2^9 patterns, then of one), then the chunk, the
+//      thread, and the token at which the running sum of the kept e passes u times their total, ties counted in
+//      vocabulary order (sample_pick_kernel).
+// The search sums e as whole numbers of 2^-40 (fewer bits from 2^23 tokens on): such sums are the same in any order, so they are
+// made with atomics, and off by 7e-8 of a row's mass at most.  All other sums run in a fixed order: a row's result depends
+// on its inputs only.  e is the hardware's exponential (__expf: 2^(x log2 e)) in every launch alike: what a token weighs
+// must be the same bits wherever it is asked.
+// (Five rounds of 63 thresholds and float sums, each a launch that read the row, in place of 2 and the search of 4: the chain 62 us for 8 rows
+// of 151,936 logits with top_p < 1, 32 so; 64 rows 159, 65; one row 63, 30; 5,000 logits 34, 25.  Where a class holds most of a row
+// the last launch's one workgroup has it all: logits within a twentieth of each other 61, 47, all logits equal 63, 93.)
 #include "common.h"
 
 #define SAMPLE_CHUNKS 32            // as ARGMAX_CHUNKS below: the two share the first launch
 #define ARGMAX_CHUNKS 32
 #define SAMPLE_THREADS 256
-#define SAMPLE_ROUND_THREADS 128    // of a round's workgroups: 64 classes a thread in LDS, 32 KB
-#define SAMPLE_K 63                 // thresholds a round
-#define SAMPLE_CLASSES (SAMPLE_K + 1)
-#define SAMPLE_ROUNDS 5             // ceil(2^30 / 64^5) = 1
-#define SAMPLE_PIECE 32             // the elements of the chosen chunk that a thread of the last launch holds in registers
-#define SAMPLE_ONE 0x3f800000u      // the bit pattern of 1.0f: no e is above it
+#define SAMPLE_PICK_THREADS 1024    // of the last launch where it searches (else SAMPLE_THREADS)
+#define SAMPLE_PIECE 8192           // the elements of the chosen chunk that the last launch holds in registers
+#define SAMPLE_HELD 32              // the elements of a chunk that a thread of the third launch holds in registers
+#define SAMPLE_CLASSES 2048         // of patterns: b >> SAMPLE_LOW; no e is above 1.0f, the first of class 2032
+#define SAMPLE_LOW 19
+#define SAMPLE_MID 9                // the last launch's classes: 2^(19 - 9) of 2^9 patterns, 2^9 of one
+#define SAMPLE_ONE 0x3f800000u      // the bit pattern of 1.0f
+#define SAMPLE_LISTED 4864          // elements of a class that a chunk lists (all of a chunk up to 155,648 tokens); more are read again
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct SampleChunk {
   int begin, end;
@@ -54,139 +62,116 @@ __device__ __forceinline__ float sample_row_max(const float* __restrict__ part_v
   return wave_max(lane < SAMPLE_CHUNKS ? part_val[row * SAMPLE_CHUNKS + lane] : -INFINITY);
 }
 
-// threshold j of a round with bounds lo < t* <= hi (patterns), w = hi - lo: lo + (j + 1) step with step = ceil(w / 64).
-// (The last ones may lie beyond hi, where f is below the target as it is at hi: the bounds still close in by 64 a round.)
-__device__ __forceinline__ uint32_t sample_step(uint32_t w) { return (w + SAMPLE_CLASSES - 1) / SAMPLE_CLASSES; }
-__device__ __forceinline__ uint32_t sample_threshold(uint32_t lo, uint32_t w, int j) {
-  return lo + (uint32_t)(j + 1) * sample_step(w);
+// e as a whole number of 2^-bits, rounded down
+__device__ __forceinline__ unsigned long long sample_fixed(uint32_t b, int bits) {
+  const uint32_t off = 127u - min(b >> 23, 127u);          // e in [2^-off, 2^(1 - off))
+  const unsigned long long m = (unsigned long long)((b & 0x7fffffu) | 0x800000u) << (bits - 23);
+  return off < 64u ? m >> off : 0ull;
 }
+__device__ __forceinline__ uint32_t sample_class(uint32_t b) { return min(b >> SAMPLE_LOW, (uint32_t)SAMPLE_CLASSES - 1); }
 
-// What a workgroup keeps of the search from launch to launch, every workgroup its own copy: lo, hi, f(hi), the target.
+// What the launches before the last leave of a row's search: the class, the mass above it, and the target.
+struct SampleRow {
+  unsigned long long above;
+  float target;
+  uint32_t cls;
+};
 
-// lane m of the first wave: class m of the row, the chunks' sums added in the order of the chunks
-__device__ __forceinline__ float sample_class_total(const float* __restrict__ classes) {
-  float t = 0.f;
-  if (threadIdx.x < 64) {
-    float v[SAMPLE_CHUNKS];                  // all loads in flight at once
+// Sum over the threads behind this one, and of all, of a workgroup of `waves` waves; whole numbers.
+__device__ __forceinline__ unsigned long long block_behind(unsigned long long v, unsigned long long* scratch, int waves, unsigned long long& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned long long incl = v;
 #pragma unroll
-    for (int c = 0; c < SAMPLE_CHUNKS; c++) v[c] = classes[c * SAMPLE_CLASSES + threadIdx.x];
-#pragma unroll
-    for (int c = 0; c < SAMPLE_CHUNKS; c++) t += v[c];
-  }
-  return t;
-}
-
-// The bounds after the round whose class totals the first wave holds in `t`; all threads get them.
-__device__ void sample_decide(float t, uint4 st, float tp, uint32_t& lo, uint32_t& hi, float& f_hi, float& target,
-                              uint32_t* result) {
-  static_assert(SAMPLE_CLASSES == 64, "lane m of the first wave holds class m");
-  lo = st.x; hi = st.y;
-  f_hi = __uint_as_float(st.z); target = __uint_as_float(st.w);
-  const uint32_t w = hi - lo;
-  if (w <= 1u) return;                       // found already
-  const int tid = threadIdx.x;
-  if (tid < 64) {
-    if (!(target > 0.f)) target = tp * wave_sum(t);          // the first round: the classes hold every e of the row
-    // classes m .. 63 together, in every lane m (a fixed tree of additions)
-    float above = t;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const float o = __shfl_down(above, off, 64);
-      if (tid + off < 64) above += o;
-    }
-    // f(t_j) = classes j + 1 .. 63 together; the first j at which it is below the target
-    const float f_j = __shfl_down(above, 1, 64);
-    const unsigned long long below = __ballot(tid < SAMPLE_K && f_j < target);
-    const int first = below ? __ffsll((long long)below) - 1 : SAMPLE_K;
-    const float f_new = first < SAMPLE_K ? __shfl(f_j, first, 64) : f_hi;
-    if (tid == 0) {
-      result[0] = first > 0 ? sample_threshold(lo, w, first - 1) : lo;
-      result[1] = first < SAMPLE_K ? sample_threshold(lo, w, first) : hi;
-      result[2] = __float_as_uint(f_new); result[3] = __float_as_uint(target);
-    }
+  for (int off = 1; off < 64; off <<= 1) {
+    const unsigned long long o = __shfl_down(incl, off, 64);
+    if (lane + off < 64) incl += o;
   }
   __syncthreads();
-  lo = result[0]; hi = result[1];
-  f_hi = __uint_as_float(result[2]); target = __uint_as_float(result[3]);
-  __syncthreads();                           // result may be written again
+  if (lane == 0) scratch[wave] = incl;
+  __syncthreads();
+  unsigned long long behind = 0;
+  total = 0;
+  for (int k = 0; k < waves; k++) {
+    if (k > wave) behind += scratch[k];
+    total += scratch[k];
+  }
+  return behind + incl - v;
+}
+// Of N classes a thread, in ascending order, with `above` behind them: the one at which the sum from above reaches the target.
+template <int N>
+__device__ __forceinline__ void sample_cross(const unsigned long long (&h)[N], unsigned long long above, double target, int first, int* cls,
+                                             unsigned long long* mass) {
+#pragma unroll
+  for (int j = N - 1; j >= 0; j--) {
+    if ((double)above < target && (double)(above + h[j]) >= target) {
+      *cls = first + j;
+      *mass = above;
+    }
+    above += h[j];
+  }
 }
 
-__global__ __launch_bounds__(SAMPLE_ROUND_THREADS) void sample_round_kernel(
-    const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature,
-    const float* __restrict__ top_p, const float* __restrict__ part_val, const float* __restrict__ prev,
-    float* __restrict__ next, uint32_t* __restrict__ state, int first) {
-  __shared__ float hist[SAMPLE_CLASSES][SAMPLE_ROUND_THREADS];   // a column per thread: no two threads share an entry
-  __shared__ float halves[2][SAMPLE_CLASSES];
-  __shared__ uint32_t result[4];
+// Additions to classes in LDS, a run of one class at a time: rows of equal or nearly equal logits send all lanes to one place.
+struct SampleRun {
+  unsigned long long* hist;
+  uint32_t at = 0;
+  unsigned long long sum = 0;
+  __device__ __forceinline__ void add(uint32_t cls, unsigned long long f) {
+    if (cls != at) {
+      if (sum) atomicAdd(&hist[at], sum);
+      at = cls;
+      sum = 0;
+    }
+    sum += f;
+  }
+  __device__ __forceinline__ void end() {
+    if (sum) atomicAdd(&hist[at], sum);
+  }
+};
+
+// Sums of a chunk's e by class, added to the row's (which the first launch has cleared).
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_classes_kernel(
+    const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature, const float* __restrict__ top_p,
+    const float* __restrict__ part_val, unsigned long long* __restrict__ classes, int bits) {
+  __shared__ unsigned long long hist[SAMPLE_CLASSES];
   const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
   // everything the workgroup needs from memory is asked for at once, whatever it turns out to need: what the launch
   // before wrote comes from memory, a microsecond or two away, and asking one after the other would add them up
-  const float temp = temperature[row], tp = top_p[row];
-  uint32_t* st = state + ((size_t)row * SAMPLE_CHUNKS + c) * 4;
-  const uint4 kept = first ? make_uint4(0u, SAMPLE_ONE, 0u, 0u) : *reinterpret_cast<const uint4*>(st);
-  const float t = first ? 0.f : sample_class_total(prev + (size_t)row * SAMPLE_CHUNKS * SAMPLE_CLASSES);
-  const float mx = sample_row_max(part_val, row);
+  const float temp = temperature[row], tp = top_p[row], mx = sample_row_max(part_val, row);
   const float* x = logits + (size_t)row * ld;
   const SampleChunk ch = sample_chunk(V, c);
-  // eight loads in flight per thread, those of the next eight tokens issued before these are classed
-  auto fetch = [&](int i0, float* v) {
+  auto fetch = [&](int i0, float (&v)[8]) {
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-      const int i = i0 + k * SAMPLE_ROUND_THREADS;
-      v[k] = i < ch.end ? x[i] : -INFINITY;                // exp(-inf) = 0 adds nothing to its class
+      const int i = i0 + k * SAMPLE_THREADS;
+      v[k] = i < ch.end ? x[i] : -INFINITY;                // exp(-inf) = 0 adds nothing
     }
   };
   float v[8], ahead[8];
   fetch(ch.begin + tid, v);
   if (!(temp > 0.f) || !(tp < 1.0f)) return;
-  uint32_t lo = 0u, hi = SAMPLE_ONE;
-  float f_hi = 0.f, target = 0.f;
-  if (!first) sample_decide(t, kept, tp, lo, hi, f_hi, target, result);
-  if (tid == 0) {
-    st[0] = lo; st[1] = hi;
-    st[2] = __float_as_uint(f_hi); st[3] = __float_as_uint(target);
-  }
-  const uint32_t w = hi - lo;
-  if (w <= 1u) return;
   const float inv_t = 1.0f / temp;
-#pragma unroll 8
-  for (int m = 0; m < SAMPLE_CLASSES; m++) hist[m][tid] = 0.f;
-  const uint32_t step = sample_step(w);
-  const float per_step = 1.0f / (float)step;
-  for (int i0 = ch.begin + tid; i0 < ch.end; i0 += 8 * SAMPLE_ROUND_THREADS) {
-    fetch(i0 + 8 * SAMPLE_ROUND_THREADS, ahead);
+#pragma unroll
+  for (int j = 0; j < SAMPLE_CLASSES / SAMPLE_THREADS; j++) hist[j * SAMPLE_THREADS + tid] = 0ull;
+  __syncthreads();
+  SampleRun run{hist};
+  for (int i0 = ch.begin + tid; i0 < ch.end; i0 += 8 * SAMPLE_THREADS) {
+    fetch(i0 + 8 * SAMPLE_THREADS, ahead);
 #pragma unroll
     for (int k = 0; k < 8; k++) {
       const float e = __expf((v[k] - mx) * inv_t);
-      const uint32_t b = __float_as_uint(e);
-      // the class of e: how many thresholds lie strictly below it
-      // (threshold j is below e if (j + 1) step < b - lo: floor((b - lo - 1) / step) of them, 63 at most)
-      uint32_t m = 0;
-      if (b > lo) {
-        const uint32_t d = b - lo - 1u;
-        m = min((uint32_t)((float)d * per_step), (uint32_t)SAMPLE_CLASSES);      // a guess that is off by one at most
-        if ((m + 1u) * step <= d) m++;
-        if (m * step > d) m--;
-        m = min(m, (uint32_t)SAMPLE_K);
-      }
-      hist[m][tid] += e;
+      if (e > 0.f) run.add(sample_class(__float_as_uint(e)), sample_fixed(__float_as_uint(e), bits));
     }
 #pragma unroll
     for (int k = 0; k < 8; k++) v[k] = ahead[k];
   }
+  run.end();
   __syncthreads();
-  // Thread (m, half) adds the entries of class m of one half of the threads, one after the other (no exchange between
-  // lanes: 32 reductions over a wave would be 32 chains of six exchanges); it starts at column m so that the lanes of a
-  // wave read different banks.
-  static_assert(SAMPLE_ROUND_THREADS == 128 && SAMPLE_CLASSES == 64, "two halves of 64 threads, a class a lane");
-  const int m = tid & 63, half = tid >> 6;
-  float sum = 0.f;
-#pragma unroll 16
-  for (int j = 0; j < 64; j++) sum += hist[m][half * 64 + ((j + m) & 63)];
-  halves[half][m] = sum;
-  __syncthreads();
-  if (tid < SAMPLE_CLASSES)
-    next[((size_t)row * SAMPLE_CHUNKS + c) * SAMPLE_CLASSES + tid] = halves[0][tid] + halves[1][tid];
+#pragma unroll
+  for (int j = 0; j < SAMPLE_CLASSES / SAMPLE_THREADS; j++) {
+    const unsigned long long f = hist[j * SAMPLE_THREADS + tid];
+    if (f) atomicAdd(&classes[(size_t)row * SAMPLE_CLASSES + j * SAMPLE_THREADS + tid], f);
+  }
 }
 
 __device__ __forceinline__ double wave_sum_f64(double v) {
@@ -200,73 +185,8 @@ __device__ __forceinline__ int wave_sum_i32(int v) {
   return v;
 }
 
-// The terms e = exp((x - max) / t) of the elements begin + thread, begin + thread + SAMPLE_THREADS, ... of a chunk, in
-// that order, eight loads in flight a thread: one load at a time, each used at once, is a chain of memory latencies
-// (6 us for the 19 elements a thread has of a chunk of 151,936 logits).
-template <class Use>
-__device__ __forceinline__ void sample_each_term(const float* __restrict__ x, int begin, int end, float mx, float inv_t, Use use) {
-  for (int i0 = begin + (int)threadIdx.x; i0 < end; i0 += 8 * SAMPLE_THREADS) {
-    float v[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int i = i0 + k * SAMPLE_THREADS;
-      v[k] = i < end ? x[i] : 0.f;
-    }
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int i = i0 + k * SAMPLE_THREADS;
-      if (i < end) use(i, __expf((v[k] - mx) * inv_t));
-    }
-  }
-}
-
-// per chunk: the sum of e > t* (double) and the number of e == t*; the row's t* and how many ties it keeps
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_chunk_sums_kernel(
-    const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature,
-    const float* __restrict__ top_p, const float* __restrict__ part_val, const float* __restrict__ prev,
-    const uint32_t* __restrict__ state, double* __restrict__ fin_s, int* __restrict__ fin_n, uint32_t* __restrict__ fin_par) {
-  __shared__ uint32_t result[4];
-  __shared__ double ws[SAMPLE_THREADS / 64];
-  __shared__ int wn[SAMPLE_THREADS / 64];
-  const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
-  const float temp = temperature[row], tp = top_p != nullptr ? top_p[row] : 1.0f;
-  if (!(temp > 0.f)) return;
-  float thr = 0.f;                            // keep e > thr, and the first `ties_kept` tokens with e == thr
-  int ties_kept = 0x7fffffff;
-  if (tp < 1.0f) {
-    uint32_t lo, hi;
-    float f_hi, target;
-    sample_decide(sample_class_total(prev + (size_t)row * SAMPLE_CHUNKS * SAMPLE_CLASSES),
-                  *reinterpret_cast<const uint4*>(state + ((size_t)row * SAMPLE_CHUNKS + c) * 4), tp, lo, hi, f_hi, target, result);
-    thr = __uint_as_float(hi);
-    // the mass above the threshold is below the target; tied tokens are taken, in vocabulary order, while
-    // the mass before them still is
-    ties_kept = max(1, (int)ceilf((target - f_hi) / thr));
-  }
-  const float mx = sample_row_max(part_val, row), inv_t = 1.0f / temp;
-  const float* x = logits + (size_t)row * ld;
-  const SampleChunk ch = sample_chunk(V, c);
-  double s = 0.0;
-  int n = 0;
-  sample_each_term(x, ch.begin, ch.end, mx, inv_t, [&](int, float e) {
-    if (e > thr) s += (double)e;
-    n += e == thr;
-  });
-  s = wave_sum_f64(s);
-  n = wave_sum_i32(n);
-  if ((tid & 63) == 0) { ws[tid >> 6] = s; wn[tid >> 6] = n; }
-  __syncthreads();
-  if (tid == 0) {
-    for (int k = 1; k < SAMPLE_THREADS / 64; k++) { s += ws[k]; n += wn[k]; }
-    const size_t at = (size_t)row * SAMPLE_CHUNKS + c;
-    fin_s[at] = s;
-    fin_n[at] = n;
-    fin_par[2 * at] = __float_as_uint(thr);
-    fin_par[2 * at + 1] = (uint32_t)ties_kept;
-  }
-}
-
 // exclusive prefix sums over the workgroup's threads, in a fixed order; `total` gets the sum of all
+template <int THREADS>
 __device__ __forceinline__ double block_prefix_f64(double v, double* wave_tot, double& total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double incl = v;
@@ -280,12 +200,13 @@ __device__ __forceinline__ double block_prefix_f64(double v, double* wave_tot, d
   __syncthreads();
   double before = 0.0;
   total = 0.0;
-  for (int k = 0; k < SAMPLE_THREADS / 64; k++) {
+  for (int k = 0; k < THREADS / 64; k++) {
     if (k < wave) before += wave_tot[k];
     total += wave_tot[k];
   }
   return before + incl - v;
 }
+template <int THREADS>
 __device__ __forceinline__ int block_prefix_i32(int v, int* wave_tot) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int incl = v;
@@ -302,15 +223,131 @@ __device__ __forceinline__ int block_prefix_i32(int v, int* wave_tot) {
   return before + incl - v;
 }
 
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(
-    const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature,
+// Per chunk: the sum (double) of the e above the row's class, and a list of those in it, a thread's behind the last thread's; the
+// number that there are.  Rows with top_p >= 1: the sum of all.
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
+    const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature, const float* __restrict__ top_p,
+    const float* __restrict__ part_val, const unsigned long long* __restrict__ classes, int bits, double* __restrict__ fin_s,
+    int* __restrict__ fin_n, uint32_t* __restrict__ list, SampleRow* __restrict__ rows) {
+  __shared__ unsigned long long scratch[SAMPLE_THREADS / 64], mass;
+  __shared__ int cls;
+  __shared__ double ws[SAMPLE_THREADS / 64];
+  __shared__ int wn[SAMPLE_THREADS / 64];
+  const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
+  const float temp = temperature[row], tp = top_p != nullptr ? top_p[row] : 1.0f, mx = sample_row_max(part_val, row);
+  if (!(temp > 0.f)) return;
+  const float* x = logits + (size_t)row * ld;
+  const SampleChunk ch = sample_chunk(V, c);
+  // the terms of the elements begin + thread, begin + thread + SAMPLE_THREADS, .., all asked for at once: one load at a
+  // time, each used at once, is a chain of memory latencies (6 us for the 19 elements a thread has of a chunk of 151,936 logits)
+  const float inv_t = 1.0f / temp;
+  const bool held = ch.end - ch.begin <= SAMPLE_HELD * SAMPLE_THREADS;     // the same for all threads
+  const int rounds = held ? (ch.end - ch.begin + 8 * SAMPLE_THREADS - 1) / (8 * SAMPLE_THREADS) : 0;      // of eight elements a thread
+  float mine[SAMPLE_HELD];
+#pragma unroll
+  for (int g = 0; g < SAMPLE_HELD / 8; g++) {
+    if (g < rounds) {
+#pragma unroll
+      for (int k = 8 * g; k < 8 * g + 8; k++) {
+        const int i = ch.begin + tid + k * SAMPLE_THREADS;
+        mine[k] = i < ch.end ? x[i] : 0.f;
+      }
+    }
+  }
+  int above = -1;                                          // keep what is above this class, list what is in it
+  if (tp < 1.0f) {
+    constexpr int N = SAMPLE_CLASSES / SAMPLE_THREADS;
+    unsigned long long h[N], own = 0, total;
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+      h[j] = classes[(size_t)row * SAMPLE_CLASSES + tid * N + j];
+      own += h[j];
+    }
+    if (tid == 0) cls = SAMPLE_ONE >> SAMPLE_LOW, mass = 0;                // (a target that is not above zero: the largest alone)
+    const unsigned long long behind = block_behind(own, scratch, SAMPLE_THREADS / 64, total);
+    const double one = (double)(1ull << bits);
+    const float target = tp * (float)((double)total / one);
+    sample_cross(h, behind, (double)target * one, tid * N, &cls, &mass);
+    __syncthreads();
+    above = cls;
+    if (c == 0 && tid == 0) rows[row] = {mass, target, (uint32_t)above};
+  }
+  double s = 0.0;
+  int n = 0;
+  auto each = [&](auto use) {
+    if (held) {
+#pragma unroll
+      for (int g = 0; g < SAMPLE_HELD / 8; g++) {
+        if (g < rounds) {
+#pragma unroll
+          for (int k = 8 * g; k < 8 * g + 8; k++)
+            if (ch.begin + tid + k * SAMPLE_THREADS < ch.end) use(mine[k]);
+        }
+      }
+    } else {
+      for (int i0 = ch.begin + tid; i0 < ch.end; i0 += 8 * SAMPLE_THREADS) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          const int i = i0 + k * SAMPLE_THREADS;
+          v[k] = i < ch.end ? x[i] : 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+          if (i0 + k * SAMPLE_THREADS < ch.end) use(__expf((v[k] - mx) * inv_t));
+      }
+    }
+  };
+#pragma unroll
+  for (int g = 0; g < SAMPLE_HELD / 8; g++) {
+    if (g < rounds) {
+#pragma unroll
+      for (int k = 8 * g; k < 8 * g + 8; k++) mine[k] = __expf((mine[k] - mx) * inv_t);
+    }
+  }
+  if (above < 0) {
+    each([&](float e) {
+      if (e > 0.f) s += (double)e;
+    });
+  } else {
+    each([&](float e) {
+      const int k = (int)sample_class(__float_as_uint(e));
+      if (k > above && e > 0.f) s += (double)e;
+      n += k == above;
+    });
+    const int before = block_prefix_i32<SAMPLE_THREADS>(n, wn);
+    uint32_t* mylist = list + ((size_t)row * SAMPLE_CHUNKS + c) * SAMPLE_LISTED;
+    int at = before;
+    each([&](float e) {
+      if ((int)sample_class(__float_as_uint(e)) == above) {
+        if (at < SAMPLE_LISTED) mylist[at] = __float_as_uint(e);
+        at++;
+      }
+    });
+    if (tid == SAMPLE_THREADS - 1) fin_n[(size_t)row * SAMPLE_CHUNKS + c] = before + n;
+  }
+  s = wave_sum_f64(s);
+  if ((tid & 63) == 0) ws[tid >> 6] = s;
+  __syncthreads();
+  if (tid == 0) {
+    for (int k = 1; k < SAMPLE_THREADS / 64; k++) s += ws[k];
+    fin_s[(size_t)row * SAMPLE_CHUNKS + c] = s;
+  }
+}
+
+template <int THREADS, bool SEARCH>
+__global__ __launch_bounds__(THREADS) void sample_pick_kernel(
+    const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature, const float* __restrict__ top_p,
     const float* __restrict__ u, const float* __restrict__ part_val, const int* __restrict__ part_idx,
-    const double* __restrict__ fin_s, const int* __restrict__ fin_n, const uint32_t* __restrict__ fin_par,
-    int* __restrict__ out) {
-  __shared__ double wave_tot[SAMPLE_THREADS / 64];
-  __shared__ int wave_cnt[SAMPLE_THREADS / 64];
+    const double* __restrict__ fin_s, const int* __restrict__ fin_n, const uint32_t* __restrict__ list,
+    const SampleRow* __restrict__ rows, int bits, int* __restrict__ out) {
+  constexpr int WAVES = THREADS / 64, PER = THREADS / SAMPLE_CHUNKS, PIECE = SAMPLE_PIECE / THREADS;     // PER: threads a chunk
+  __shared__ unsigned long long hist[SEARCH ? 1 << (SAMPLE_LOW - SAMPLE_MID) : 1], scratch[WAVES], mass;
+  __shared__ int cls;
+  __shared__ double wave_tot[WAVES];
+  __shared__ int wave_cnt[WAVES];
   __shared__ int chosen_chunk, chosen_ties_before;
-  __shared__ int wave_first[SAMPLE_THREADS / 64], wave_last[SAMPLE_THREADS / 64];
+  __shared__ int wave_first[WAVES], wave_last[WAVES];
   __shared__ int chunk_n[SAMPLE_CHUNKS];
   __shared__ double chunk_s[SAMPLE_CHUNKS];
   __shared__ double chosen_before, chosen_target;
@@ -320,68 +357,156 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(
   int mi = lane < SAMPLE_CHUNKS ? part_idx[row * SAMPLE_CHUNKS + lane] : 0x7fffffff;
   wave_first_max(mx, mi);
   const float temp = temperature[row], u_row = u[row];    // (asked for here: where it is used, one thread would wait for it)
+  const float tp = SEARCH ? top_p[row] : 1.0f;
   if (!(temp > 0.f)) {
     if (tid == 0) out[row] = mi;
     return;
   }
+  const float inv_t = 1.0f / temp;
+  const float* x = logits + (size_t)row * ld;
   const size_t base = (size_t)row * SAMPLE_CHUNKS;
-  const float thr = __uint_as_float(fin_par[2 * base]);
-  const int ties_kept = (int)fin_par[2 * base + 1];
-  if (tid < SAMPLE_CHUNKS) {
-    chunk_n[tid] = fin_n[base + tid];
-    chunk_s[tid] = fin_s[base + tid];
+  float thr = 0.f;                            // keep e > thr, and the first `ties_kept` tokens with e == thr
+  int ties_kept = 0x7fffffff;
+  const int my_chunk = tid / PER, part = tid % PER;
+  double kept_s = fin_s[base + my_chunk];
+  int kept_n = 0;
+  if constexpr (SEARCH) if (tp < 1.0f) {
+    const SampleRow r = rows[row];
+    const int listed = fin_n[base + my_chunk];
+    // the patterns of this chunk's elements of the class, PER threads side by side, four neighbours each: from the list, of which
+    // each thread holds the first ones, or, where it did not have room for all, from the logits
+    const u32x4* mylist = reinterpret_cast<const u32x4*>(list + (base + my_chunk) * SAMPLE_LISTED);
+    const u32x4 held = 4 * part < listed ? mylist[part] : u32x4{0, 0, 0, 0};
+    auto entries = [&](auto use) {
+      if (listed <= SAMPLE_LISTED) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (4 * part + j < listed) use(held[j]);
+        for (int k0 = part + PER; 4 * k0 < listed; k0 += 4 * PER) {
+          u32x4 v[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) v[k] = 4 * (k0 + k * PER) < listed ? mylist[k0 + k * PER] : u32x4{0, 0, 0, 0};
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+              if (4 * (k0 + k * PER) + j < listed) use(v[k][j]);
+        }
+      } else {
+        const SampleChunk ch = sample_chunk(V, my_chunk);
+        for (int i0 = ch.begin + part; i0 < ch.end; i0 += 16 * PER) {
+          float v[16];
+#pragma unroll
+          for (int k = 0; k < 16; k++) v[k] = i0 + k * PER < ch.end ? x[i0 + k * PER] : 0.f;
+#pragma unroll
+          for (int k = 0; k < 16; k++) {
+            const uint32_t b = __float_as_uint(__expf((v[k] - mx) * inv_t));
+            if (i0 + k * PER < ch.end && sample_class(b) == r.cls) use(b);
+          }
+        }
+      }
+    };
+    // among 2^(LOW - MID) classes of 2^MID patterns, then among the patterns of one
+    static_assert(PER == 32 && (1 << (SAMPLE_LOW - SAMPLE_MID)) == THREADS && (1 << SAMPLE_MID) <= THREADS, "half a wave a chunk, a class a thread");
+    const double one = (double)(1ull << bits), target = (double)r.target * one;
+    uint32_t found = r.cls;                   // the leading bits of t*
+    unsigned long long above = r.above, all;
+    bool any = true;
+#pragma unroll
+    for (int level = 0; level < 2; level++) {
+      const int shift = level ? 0 : SAMPLE_MID, width = level ? SAMPLE_MID : SAMPLE_LOW - SAMPLE_MID;
+      hist[tid] = 0ull;
+      if (tid == 0) cls = -1;
+      __syncthreads();
+      SampleRun run{hist};
+      entries([&](uint32_t b) {
+        if (b >> (shift + width) == found) run.add((b >> shift) & ((1u << width) - 1), sample_fixed(b, bits));
+      });
+      run.end();
+      __syncthreads();
+      const unsigned long long h[1] = {hist[tid]};
+      sample_cross(h, above + block_behind(h[0], scratch, WAVES, all), target, tid, &cls, &mass);
+      __syncthreads();
+      any = any && cls >= 0;
+      found = found << width | (uint32_t)max(cls, 0);
+      if (cls >= 0) above = mass;
+      __syncthreads();                        // (cls and hist are written again)
+    }
+    if (!any) found = SAMPLE_ONE, above = 0;  // a target that is not above zero: the first of the largest
+    thr = __uint_as_float(found);
+    // the mass above the threshold is below the target; tied tokens are taken, in vocabulary order, while
+    // the mass before them still is
+    ties_kept = max(1, (int)ceilf((r.target - (float)((double)above / one)) / thr));
+    double s = 0.0;
+    entries([&](uint32_t b) {
+      const float e = __uint_as_float(b);
+      if (e > thr) s += (double)e;
+      kept_n += e == thr;
+    });
+#pragma unroll
+    for (int off = PER / 2; off > 0; off >>= 1) {
+      s += __shfl_xor(s, off, 64);
+      kept_n += __shfl_xor(kept_n, off, 64);
+    }
+    kept_s += s;
+  }
+  if (part == 0) {
+    chunk_n[my_chunk] = kept_n;
+    chunk_s[my_chunk] = kept_s;
   }
   __syncthreads();
-  if (tid == 0) {
-    // what every chunk keeps: its e > thr, and of its ties those that still are among the first `ties_kept`
-    double kept[SAMPLE_CHUNKS], total = 0.0;
-    int before[SAMPLE_CHUNKS], ties = 0;
-    for (int c = 0; c < SAMPLE_CHUNKS; c++) {
-      const int n = chunk_n[c];
-      before[c] = ties;
-      const int taken = min(n, max(0, ties_kept - min(ties, ties_kept)));
-      kept[c] = chunk_s[c] + (double)thr * (double)taken;
-      total += kept[c];
-      ties += n;
+  if (tid < 64) {
+    // what every chunk keeps, a chunk a lane: its e > thr, and of its ties those that still are among the first `ties_kept`
+    const bool real = lane < SAMPLE_CHUNKS;
+    const int n = real ? chunk_n[lane] : 0;
+    int ties = n;
+#pragma unroll
+    for (int off = 1; off < SAMPLE_CHUNKS; off <<= 1) {
+      const int o = __shfl_up(ties, off, 64);
+      if (lane >= off) ties += o;
     }
-    const double target = (double)u_row * total;
-    double run = 0.0, before_last = 0.0;
-    int c = -1, last_nonzero = 0;
-    for (int i = 0; i < SAMPLE_CHUNKS; i++) {
-      if (kept[i] > 0.0) { last_nonzero = i; before_last = run; }
-      if (run + kept[i] > target) { c = i; break; }
-      run += kept[i];
+    const int before = ties - n, taken = min(n, max(0, ties_kept - min(before, ties_kept)));
+    const double kept = real ? chunk_s[lane] + (double)thr * (double)taken : 0.0;
+    double run = kept;
+#pragma unroll
+    for (int off = 1; off < SAMPLE_CHUNKS; off <<= 1) {
+      const double o = __shfl_up(run, off, 64);
+      if (lane >= off) run += o;
     }
-    if (c < 0) { c = last_nonzero; run = before_last; }
-    chosen_chunk = c;
-    chosen_before = run;
-    chosen_target = target;
-    chosen_ties_before = before[c];
+    const double target = (double)u_row * __shfl(run, SAMPLE_CHUNKS - 1, 64);
+    double in_front = __shfl_up(run, 1, 64);
+    if (lane == 0) in_front = 0.0;
+    const unsigned long long some = __ballot(kept > 0.0), reaches = __ballot(kept > 0.0 && run > target);
+    const int c = reaches ? __ffsll((long long)reaches) - 1 : some ? 63 - __clzll((long long)some) : 0;
+    if (lane == c) {
+      chosen_chunk = c;
+      chosen_before = in_front;
+      chosen_target = target;
+      chosen_ties_before = before;
+    }
   }
   __syncthreads();
   const SampleChunk ch = sample_chunk(V, chosen_chunk);
-  const float inv_t = 1.0f / temp;
-  const float* x = logits + (size_t)row * ld;
   // A thread owns a contiguous piece of the chunk and goes through it three times.  One element after the other from
   // memory, each pass is a chain of latencies (2 to 2.6 us each for the 19 elements a thread has of a chunk of
-  // 151,936 logits): a piece of up to SAMPLE_PIECE elements (vocabularies up to 262,144) is asked for at once and
+  // 151,936 logits): a piece of a chunk of up to SAMPLE_PIECE elements (vocabularies up to 262,144) is asked for at once and
   // its terms wait in registers.
   auto term = [&](int i) { return __expf((x[i] - mx) * inv_t); };
-  const int piece = (ch.end - ch.begin + SAMPLE_THREADS - 1) / SAMPLE_THREADS;
+  const int piece = (ch.end - ch.begin + THREADS - 1) / THREADS;
   const int b = min(ch.end, ch.begin + tid * piece), e_ = min(ch.end, b + piece);
-  const bool held = piece <= SAMPLE_PIECE;                                 // the same for all threads
-  float mine[SAMPLE_PIECE];
+  const bool held = piece <= PIECE;                                 // the same for all threads
+  float mine[PIECE];
   if (held) {
 #pragma unroll
-    for (int k = 0; k < SAMPLE_PIECE; k++) mine[k] = b + k < e_ ? x[b + k] : 0.f;
+    for (int k = 0; k < PIECE; k++) mine[k] = b + k < e_ ? x[b + k] : 0.f;
 #pragma unroll
-    for (int k = 0; k < SAMPLE_PIECE; k++) mine[k] = __expf((mine[k] - mx) * inv_t);
+    for (int k = 0; k < PIECE; k++) mine[k] = __expf((mine[k] - mx) * inv_t);
   }
   // use(i, e) for the elements of the piece in their order, until it returns false
   auto each = [&](auto use) {
     if (held) {
 #pragma unroll
-      for (int k = 0; k < SAMPLE_PIECE; k++) {
+      for (int k = 0; k < PIECE; k++) {
         if (b + k >= e_ || !use(b + k, mine[k])) break;
       }
     } else {
@@ -391,7 +516,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(
   };
   int my_ties = 0;
   each([&](int, float e) { my_ties += e == thr; return true; });
-  const int ties_before = chosen_ties_before + block_prefix_i32(my_ties, wave_cnt);
+  const int ties_before = chosen_ties_before + block_prefix_i32<THREADS>(my_ties, wave_cnt);
   double s = 0.0;
   {
     int tie = ties_before;
@@ -401,7 +526,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(
     });
   }
   double chunk_total;
-  const double before = chosen_before + block_prefix_f64(s, wave_tot, chunk_total);
+  const double before = chosen_before + block_prefix_f64<THREADS>(s, wave_tot, chunk_total);
   const double target = chosen_target;
   // the first thread whose piece reaches the target, and the last that keeps anything (a vote in each wave, then
   // the waves side by side: every thread asking for one word of LDS at once takes 4 us)
@@ -415,7 +540,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(
   __syncthreads();
   int first = 0x7fffffff, last = -1;
 #pragma unroll
-  for (int w = 0; w < SAMPLE_THREADS / 64; w++) {
+  for (int w = 0; w < WAVES; w++) {
     first = min(first, wave_first[w]);
     last = max(last, wave_last[w]);
   }
@@ -445,10 +570,13 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(
 // first maximum of a chunk each, a second launch picks among them (the lowest index on a tie, as above).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void argmax_part_kernel(const float* __restrict__ logits, int ld, int V,
-                                                          float* __restrict__ part_val, int* __restrict__ part_idx) {
+                                                          float* __restrict__ part_val, int* __restrict__ part_idx,
+                                                          unsigned long long* __restrict__ clear = nullptr) {
   __shared__ float vals[4];
   __shared__ int idxs[4];
   const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
+  constexpr int SHARE = SAMPLE_CLASSES / ARGMAX_CHUNKS;    // what the second launch of sampling adds to
+  if (clear != nullptr && tid < SHARE) clear[(size_t)row * SAMPLE_CLASSES + c * SHARE + tid] = 0ull;
   const float* x = logits + (size_t)row * ld;
   const int len = (V + ARGMAX_CHUNKS - 1) / ARGMAX_CHUNKS;
   const int begin = min(V, c * len), end = min(V, begin + len);
@@ -500,9 +628,10 @@ extern "C" int pico_argmax(const float* logits, int ld, int R, int V, float* par
 }
 
 // work: pico_sample_workspace_words(R) 4-byte words, 16-byte aligned.  top_p_rows == 0: no row has top_p < 1 (every
-// row is treated so), and the rounds that look for the threshold are not launched.
+// row is treated so), and the launch that looks for the threshold is left out.
 extern "C" long long pico_sample_workspace_words(int R) {
-  return (long long)R * SAMPLE_CHUNKS * (2 + 1 + 1 + 2 * SAMPLE_CLASSES + 4 + 1 + 2);
+  static_assert(sizeof(SampleRow) == 16, "four words a row");
+  return (long long)R * (2 * SAMPLE_CLASSES + 4 + SAMPLE_CHUNKS * (2 + 1 + 1 + 1 + SAMPLE_LISTED));
 }
 
 extern "C" int pico_sample(const float* logits, int ld, int R, int V, const float* temperature, const float* top_p,
@@ -511,27 +640,29 @@ extern "C" int pico_sample(const float* logits, int ld, int R, int V, const floa
   PICO_REQUIRE(R >= 0 && V > 0 && ld >= V, "pico_sample: bad sizes R=%d V=%d ld=%d", R, V, ld);
   PICO_REQUIRE(R <= 65535, "pico_sample: too many rows");
   if (R == 0) return 0;
-  // (the rounds read their state with 16-byte loads; every part of the workspace is a multiple of 16 bytes long)
+  // (every part of the workspace is a multiple of 16 bytes long)
   PICO_REQUIRE(work != nullptr && (uintptr_t)work % 16 == 0, "pico_sample: the workspace is missing or not 16-byte aligned");
   const size_t n = (size_t)R * SAMPLE_CHUNKS;
-  double* fin_s = (double*)work;
+  unsigned long long* classes = (unsigned long long*)work;
+  SampleRow* rows = (SampleRow*)(classes + (size_t)R * SAMPLE_CLASSES);
+  double* fin_s = (double*)(rows + R);
   float* part_val = (float*)(fin_s + n);
   int* part_idx = (int*)(part_val + n);
-  float* classes[2] = {(float*)(part_idx + n), (float*)(part_idx + n) + n * SAMPLE_CLASSES};
-  uint32_t* state = (uint32_t*)(classes[1] + n * SAMPLE_CLASSES);
-  int* fin_n = (int*)(state + 4 * n);
-  uint32_t* fin_par = (uint32_t*)(fin_n + n);
+  int* fin_n = part_idx + n;
+  uint32_t* list = (uint32_t*)(fin_n + n);
+  int bits = 40;                              // a row's sum of whole numbers of 2^-bits stays below 2^63
+  while (bits > 31 && V > (1LL << (63 - bits))) bits--;
   const dim3 grid(R, SAMPLE_CHUNKS);
-  argmax_part_kernel<<<grid, 256, 0, stream>>>(logits, ld, V, part_val, part_idx);
+  argmax_part_kernel<<<grid, 256, 0, stream>>>(logits, ld, V, part_val, part_idx, top_p_rows ? classes : nullptr);
   const float* asked = top_p_rows ? top_p : nullptr;
+  if (top_p_rows) sample_classes_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, top_p, part_val, classes, bits);
+  sample_collect_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, part_val, classes, bits, fin_s, fin_n, list, rows);
   if (top_p_rows)
-    for (int r = 0; r < SAMPLE_ROUNDS; r++)
-      sample_round_kernel<<<grid, SAMPLE_ROUND_THREADS, 0, stream>>>(logits, ld, V, temperature, top_p, part_val,
-                                                                    classes[(r + 1) & 1], classes[r & 1], state, r == 0);
-  sample_chunk_sums_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, part_val,
-                                                               classes[(SAMPLE_ROUNDS - 1) & 1], state, fin_s, fin_n, fin_par);
-  sample_pick_kernel<<<R, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, u, part_val, part_idx, fin_s, fin_n,
-                                                      fin_par, out);
+    sample_pick_kernel<SAMPLE_PICK_THREADS, true><<<R, SAMPLE_PICK_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, u, part_val, part_idx,
+                                                                                        fin_s, fin_n, list, rows, bits, out);
+  else
+    sample_pick_kernel<SAMPLE_THREADS, false><<<R, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, u, part_val, part_idx,
+                                                                               fin_s, fin_n, list, rows, bits, out);
   PICO_LAUNCH_CHECK();
   return 0;
 }

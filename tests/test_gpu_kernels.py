@@ -626,6 +626,25 @@ def test_sampling_at_the_real_vocabulary_row_by_row(K):
         K.sample(dev, temps.to(DEV), top_ps.to(DEV), us.to(DEV), work=K.sample_workspace(R - 1, DEV))
 
 
+@pytest.mark.parametrize("V", [40, 3000, 151936, 300001])
+def test_sampling_searches_classes_of_any_size(K, V):
+    # classes that hold a few elements, more than a chunk lists (nearly flat rows), the whole row (equal logits), and chunks of more
+    # elements than a thread holds: every draw against the plain rule, as far from a boundary of the CDF as sums of 32-bit
+    # exponentials are off (the exponentials by 3e-7 each, at 17,000 kept tokens a row and more)
+    g = torch.Generator().manual_seed(V)
+    R = 12
+    logits = torch.randn(R, V, generator=g) * torch.tensor([3, 3, 1, 1, 0.2, 0.2, 0.01, 0.01, 0, 0, 6, 6.0])[:, None]
+    top_ps = torch.tensor([0.9, 0.3, 0.9, 0.999, 0.5, 0.95, 0.9, 0.02, 0.25, 0.9, 0.99, 1e-5])
+    temps, us = torch.full((R,), 0.8), torch.rand(R, generator=g)
+    out = K.sample(logits.to(DEV), temps.to(DEV), top_ps.to(DEV), us.to(DEV)).tolist()
+    assert out == K.sample(logits.to(DEV), temps.to(DEV), top_ps.to(DEV), us.to(DEV)).tolist()
+    for r in range(R):
+        p = P.top_p_probs(logits[r].double(), 0.8, float(top_ps[r]))
+        want, cum = P.inverse_cdf(p, float(us[r])), torch.cumsum(p, 0)
+        assert 0 <= out[r] < V and (out[r] == want or abs(float(cum[min(out[r], want)]) - float(us[r])) < 2e-6), (r, out[r], want)
+        assert float(p[out[r]]) > 0 or abs(float(us[r]) - 1) < 2e-6, (r, "a token outside the kept set")
+
+
 def test_sampling_at_the_edges_of_its_options(K):
     # a nucleus so small that only the likeliest token fits, a temperature so low that it holds all the mass, one so high
     # that the distribution is flat, and a vocabulary smaller than the number of chunks a row is read in
