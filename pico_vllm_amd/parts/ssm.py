@@ -28,7 +28,9 @@ class SelectiveStateSpace(Mixer):
     graph_safe_prompts = True
 
     # In the bfloat16 engine a step with a prompt portion cuts its sequences into chunks of this many tokens that run
-    # side by side (``kernels.selective_scan``); decided from the step's shape alone.  The 32-bit engine walks every
+    # side by side (``kernels.selective_scan``); decided from the step's shape alone.  (16 state elements: as many as
+    # ``kernels.scan_chunk`` says, from a dozen tokens on that are not a sequence's only one: 16 tokens of 3,072 channels 18 us, 28
+    # walked whole; 64: 21 and 91; 30 single tokens and 16: 34 and 36.)  The 32-bit engine walks every
     # sequence whole, so that its sums do not depend on how a prompt was cut.
     CHUNK, CHUNKED_FROM = 64, 128
 
@@ -81,6 +83,11 @@ class SelectiveStateSpace(Mixer):
         u = kernels.causal_conv(uz, I, self.conv_w, self.conv_b, ctx, cache.state, N, single=ctx.all_decode)
         dbc = self.x_proj(u)                                                         # [T, d | B | C]
         dt_pre = self.dt_proj(dbc[:, :R], out_dtype=torch.float32)                   # step sizes stay float32 from here on
-        chunked = self.act_dtype == torch.bfloat16 and not ctx.all_decode and ctx.num_tokens >= self.CHUNKED_FROM
+        chunk = 0
+        if kernels.scan_rows_held(N, self.act_dtype):
+            if not ctx.all_decode and ctx.num_tokens - ctx.num_seqs >= 12:
+                chunk = kernels.scan_chunk(ctx.num_tokens, I, ctx.num_seqs)
+        elif self.act_dtype == torch.bfloat16 and not ctx.all_decode and ctx.num_tokens >= self.CHUNKED_FROM:
+            chunk = self.CHUNK
         return kernels.selective_scan(u, dt_pre, self.dt_bias, dbc, R, R + N, self.a_log, self.d, uz[:, I:], ctx, cache.state,
-                                      self.taps - 1, chunk=self.CHUNK if chunked else 0)
+                                      self.taps - 1, chunk=chunk)

@@ -275,6 +275,36 @@ def test_convolution_and_recurrence_in_portions_and_token_by_token(dtype, C, N, 
         assert float(state[1].min()) == 9.0 and float(state[3].max()) == 9.0           # other requests' slots untouched
 
 
+@pytest.mark.parametrize("C,lens,chunk", [(300, [1] * 66 + [37, 0, 9], 8), (256, [33], 33), (8, [70, 1, 0, 200], 16), (520, [150, 40, 1], 1),
+                                          (40, [400, 300], 128), (64, [5, 4, 3, 2, 1], 4)])
+def test_recurrence_in_chunks_numbered_through(C, lens, chunk):
+    """16 state elements: chunks of all sequences side by side, sequences of single tokens, of none and of more than a chunk,
+    more sequences than lanes, channels that fill no workgroup; from states that are not zero."""
+    from pico_vllm_amd.ops import kernels
+    g = torch.Generator().manual_seed(C)
+    T, N, R = sum(lens), 16, 6
+    mk = lambda *s: torch.randn(*s, generator=g)
+    u, z, dbc, dtp = mk(T, C).bfloat16(), mk(T, C).bfloat16(), mk(T, R + 2 * N).bfloat16(), 0.5 * mk(T, C) - 1
+    a_log, D, dtb, start = torch.log(0.5 + 4 * torch.rand(C, N, generator=g)), 1 + 0.3 * mk(C), 0.1 * mk(C), mk(len(lens) + 1, C, N + 3)
+    ctx = step_ctx(lens, [0] * len(lens), list(range(len(lens))))
+    state = start.to(DEV)
+    got = kernels.selective_scan(u.to(DEV), dtp.to(DEV), dtb.to(DEV), dbc.to(DEV), R, R + N, a_log.to(DEV), D.to(DEV), z.to(DEV), ctx, state, 3, chunk=chunk)
+    dt, A, at = P.softplus(dtp.double() + dtb.double()), -torch.exp(a_log.double()), 0
+    for b, n in enumerate(lens):
+        S = start[b, :, :N].double()
+        want = []
+        for t in range(at, at + n):
+            S = torch.exp(dt[t][:, None] * A) * S + (dt[t] * u[t].double())[:, None] * dbc[t, R:R + N].double()
+            want.append((S @ dbc[t, R + N:].double() + D.double() * u[t].double()) * P.silu(z[t].double()))
+        if n:
+            close(got[at:at + n], torch.stack(want), "bfloat16")
+        # the state: float32 sums over the sequence, decays off by a few 1e-7 each
+        assert (state[b, :, :N].cpu().double() - S).abs().max() <= 4e-6 * max(1.0, float(S.abs().max()))
+        assert torch.equal(state[b, :, N:].cpu(), start[b, :, N:])
+        at += n
+    assert torch.equal(state[-1].cpu(), start[-1])
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,dk,dv,decay", [(2, 24, 40, (0.9, 0.996)), (4, 64, 64, (0.97, 0.99, 0.999, 1.0)), (3, 16, 8, (0.5, 0.9375, 0.99)), (1, 80, 100, (0.999,))])
 def test_retention_recurrence_with_fixed_decays(dtype, H, dk, dv, decay):
