@@ -19,6 +19,8 @@
 //   pico_gated_group_norm: (y + D_h x) silu(z), RMS-normed in equal parts of the row, times a weight
 #include "common.h"
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
 
@@ -138,17 +140,23 @@ extern "C" int pico_ssd_prep(const void* bc, int ldb, int b_col, int c_col, int 
 #define DS_LOCAL 1
 #define DS_FROM 2
 
-template <typename TV, int KPL, int VPL, bool DELTA, int MODE>
+// FOUR: four lanes a column and four waves (key sizes of 33 to 128, 64 and more columns).  What a thread stages of the next block
+// is asked for before this block's tokens are walked, a token's k, g and q are read from LDS under the token before, and the
+// sums over key channels meet by lane swaps instead of through the LDS crossbar: a token is a chain, and with one or two waves
+// a SIMD nothing else hides its waits.  The two passes over 2,052 tokens, 12 heads of 64 keys and 128 values: 60 and 51 us, 71
+// and 93 without all that; the same bits.
+template <typename TV, int KPL, int VPL, bool DELTA, int MODE, bool FOUR = false>
 __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                          const TV* __restrict__ v, int ldv, const float* __restrict__ g,
                                                          int g_channels, const float* __restrict__ beta,
                                                          const int* __restrict__ cu_seqlens, const int* __restrict__ state_slots,
                                                          float* __restrict__ state, float* __restrict__ out, int H, int KVH,
-                                                         int dk, int dv, int KS, int TB, int num_slots, int chunk,
+                                                         int dk, int dv, int ks_lanes, int tb, int num_slots, int chunk,
                                                          int max_chunks, float* __restrict__ ws_S, float* __restrict__ ws_P) {
-  extern __shared__ float lds[];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
   const int b = MODE == DS_WHOLE ? blockIdx.x : blockIdx.x / max_chunks, h = blockIdx.y;
-  const int nw = blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int KS = FOUR ? 4 : ks_lanes, TB = FOUR ? 16 : tb;
+  const int nw = FOUR ? 4 : blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int VC = 64 / KS, vc = lane % VC, ks = lane / VC;
   const int DKP = KS * KPL;                            // key channels with padding
   const int tile = nw * VC * VPL;                      // columns of the workgroup
@@ -193,9 +201,55 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
   float gprod[KPL];                                    // DS_LOCAL without the delta rule: the chunk's decays multiplied up
 #pragma unroll
   for (int i = 0; i < KPL; i++) gprod[i] = 1.f;
+  // a thread's share of a block's staged values, of which FOUR keeps the next block's in registers
+  constexpr int NK = KPL / 4, NV = 4 * VPL;
+  float nk[NK], nq[NK], ng[NK], nv[NV], nbeta = 0.f;
+  auto fetch = [&](int t0) {
+    const int nb = min(TB, t_end - t0);
+#pragma unroll
+    for (int x = 0; x < NK; x++) {
+      const int idx = threadIdx.x + 256 * x, t = t0 + min(idx / (4 * KPL), nb - 1), cc = min(idx % (4 * KPL), dk - 1);
+      nk[x] = k[((size_t)t * KVH + kvh) * dk + cc];
+      nq[x] = MODE == DS_LOCAL ? 0.f : q[((size_t)t * KVH + kvh) * dk + cc];
+      ng[x] = g_channels ? g[((size_t)t * H + h) * dk + cc] : g[(size_t)t * H + h];
+    }
+#pragma unroll
+    for (int x = 0; x < NV; x++) {
+      const int idx = threadIdx.x + 256 * x;
+      nv[x] = load_f32(v + (size_t)(t0 + min(idx / (64 * VPL), nb - 1)) * ldv + (size_t)h * dv + min(col0 + idx % (64 * VPL), dv - 1));
+    }
+    if (threadIdx.x < 16) nbeta = beta[(size_t)(t0 + min((int)threadIdx.x, nb - 1)) * H + h];
+  };
+  auto put = [&] {
+#pragma unroll
+    for (int x = 0; x < NK; x++) {
+      const int idx = threadIdx.x + 256 * x;
+      const bool in = idx % (4 * KPL) < dk;
+      ks_[idx] = in ? nk[x] : 0.f;
+      if (MODE != DS_LOCAL) qs_[idx] = in ? nq[x] : 0.f;
+      gs_[idx] = in ? ng[x] : 1.f;
+    }
+#pragma unroll
+    for (int x = 0; x < NV; x++) {
+      const int idx = threadIdx.x + 256 * x;
+      vs_[idx] = col0 + idx % (64 * VPL) < dv ? nv[x] : 0.f;       // the unit vectors' columns have values of zero
+    }
+    if (threadIdx.x < 16) bs_[threadIdx.x] = nbeta;
+  };
+  // the sum over the lanes that share a column, in a fixed tree
+  auto across = [&](float x) {
+    if (FOUR) return sum_across_32(sum_across_16(x));
+    for (int o = VC; o < 64; o <<= 1) x += __shfl_xor(x, o);
+    return x;
+  };
+  const bool idle = col0 + wave * VC * VPL >= ncols;               // the same for all lanes: a wave behind the last column
+  if (FOUR) fetch(t_begin);
   for (int t0 = t_begin; t0 < t_end; t0 += TB) {
     const int nb = min(TB, t_end - t0);
     __syncthreads();                                   // the last block's staged values have been read
+    if (FOUR) {
+      put();
+    } else {
     for (int idx = threadIdx.x; idx < nb * DKP; idx += blockDim.x) {      // only the block's tokens: a single token is one turn
       const int tt = idx / DKP, c = idx % DKP;
       const int t = t0 + min(tt, nb - 1), cc = min(c, dk - 1);
@@ -213,18 +267,30 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
       vs_[idx] = (tt < nb && col < dv) ? x : 0.f;       // the unit vectors' columns have values of zero
     }
     if ((int)threadIdx.x < TB) bs_[threadIdx.x] = beta[(size_t)(t0 + min((int)threadIdx.x, nb - 1)) * H + h];
+    }
     __syncthreads();
-    for (int tt = 0; tt < nb; tt++) {
-      const float4* k4 = reinterpret_cast<const float4*>(ks_ + tt * DKP + c0);
-      const float4* g4 = reinterpret_cast<const float4*>(gs_ + tt * DKP + c0);
-      const float4* q4 = reinterpret_cast<const float4*>(qs_ + tt * DKP + c0);
+    if (FOUR && t0 + TB < t_end) fetch(t0 + TB);
+    if (FOUR && idle) continue;
+    f32x4 kt[2][KPL / 4], gt[2][KPL / 4], qt[2][KPL / 4];
+    auto read = [&](int set, int tt) {
+      const f32x4* k4 = reinterpret_cast<const f32x4*>(ks_ + tt * DKP + c0);
+      const f32x4* g4 = reinterpret_cast<const f32x4*>(gs_ + tt * DKP + c0);
+      const f32x4* q4 = reinterpret_cast<const f32x4*>(qs_ + tt * DKP + c0);
+#pragma unroll
+      for (int i = 0; i < KPL / 4; i++) {
+        kt[set][i] = k4[i];
+        gt[set][i] = g4[i];
+        if (MODE != DS_LOCAL) qt[set][i] = q4[i];
+      }
+    };
+    auto token = [&](int set, int tt) {
       const float bt = bs_[tt];
       float kc[KPL], u[VPL];
 #pragma unroll
       for (int j = 0; j < VPL; j++) u[j] = 0.f;
 #pragma unroll
       for (int i = 0; i < KPL / 4; i++) {
-        const float4 kv = k4[i], gv = g4[i];
+        const f32x4 kv = kt[set][i], gv = gt[set][i];
         kc[4 * i] = kv.x; kc[4 * i + 1] = kv.y; kc[4 * i + 2] = kv.z; kc[4 * i + 3] = kv.w;
         if (MODE == DS_LOCAL && !DELTA) { gprod[4 * i] *= gv.x; gprod[4 * i + 1] *= gv.y; gprod[4 * i + 2] *= gv.z; gprod[4 * i + 3] *= gv.w; }
 #pragma unroll
@@ -240,9 +306,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
       for (int j = 0; j < VPL; j++) {
         const float vt = vs_[tt * tile + lcol0 + j * VC];
         if (DELTA) {
-          float sk = u[j];
-          for (int o = VC; o < 64; o <<= 1) sk += __shfl_xor(sk, o);
-          u[j] = bt * (vt - sk);
+          u[j] = bt * (vt - across(u[j]));
         } else {
           u[j] = bt * vt;
         }
@@ -252,14 +316,14 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
         for (int j = 0; j < VPL; j++)
 #pragma unroll
           for (int i = 0; i < KPL; i++) S[j][i] = fmaf(kc[i], u[j], S[j][i]);
-        continue;
+        return;
       }
       float so[VPL];
 #pragma unroll
       for (int j = 0; j < VPL; j++) so[j] = 0.f;
 #pragma unroll
       for (int i = 0; i < KPL / 4; i++) {
-        const float4 qv = q4[i];
+        const f32x4 qv = qt[set][i];
 #pragma unroll
         for (int j = 0; j < VPL; j++) {
           S[j][4 * i] = fmaf(kc[4 * i], u[j], S[j][4 * i]); so[j] = fmaf(S[j][4 * i], qv.x, so[j]);
@@ -270,11 +334,18 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
       }
 #pragma unroll
       for (int j = 0; j < VPL; j++) {
-        float x = so[j];
-        for (int o = VC; o < 64; o <<= 1) x += __shfl_xor(x, o);
+        const float x = across(so[j]);
         const int col = col0 + lcol0 + j * VC;
         if (ks == 0 && col < dv) out[((size_t)(t0 + tt) * H + h) * dv + col] = x;
       }
+    };
+    read(0, 0);
+    for (int tt = 0; tt < nb; tt += 2) {
+      if (tt + 1 < nb) read(1, tt + 1);
+      token(0, tt);
+      if (tt + 1 >= nb) break;
+      if (tt + 2 < nb) read(0, tt + 2);
+      token(1, tt + 1);
     }
   }
   if (MODE == DS_FROM) return;
@@ -549,12 +620,16 @@ extern "C" int pico_delta_scan(const float* q, const float* k, const void* v, in
 #define COMBINE(RB)                                                                                                          \
   delta_combine_mfma_kernel<RB><<<dim3(num_seqs, H, (dv + 15) / 16), 256, 0, stream>>>(cu_seqlens, state_slots, state, ws_S, ws_P, \
                                                                                        H, dv, num_slots, chunk, max_chunks)
+  // (fewer key channels a lane leave nothing to read ahead)
+  const bool four = chunk > 0 && KS == 4 && kpl >= 8 && vpl == 2 && nw_v == 4 && nw_l == 4 && TB == 16;
+#define FOUR_OK(KPL, VPL) (KPL >= 8 && VPL == 2)
 #define GO(TV, KPL, VPL, D)                                                                                                  \
   do {                                                                                                                       \
     if (chunk == 0) {                                                                                                        \
       delta_scan_kernel<TV, KPL, VPL, D, DS_WHOLE><<<dim3(nblk, H, tiles(dv, nw_v)), 64 * nw_v, lds_bytes(nw_v), stream>>>(ARGS(TV)); \
     } else {                                                                                                                 \
-      delta_scan_kernel<TV, KPL, VPL, D, DS_LOCAL><<<dim3(nblk, H, tiles(cols_local, nw_l)), 64 * nw_l, lds_bytes(nw_l), stream>>>(ARGS(TV)); \
+      if (FOUR_OK(KPL, VPL) && four) delta_scan_kernel<TV, KPL, VPL, D, DS_LOCAL, FOUR_OK(KPL, VPL)><<<dim3(nblk, H, tiles(cols_local, nw_l)), 256, lds_bytes(nw_l), stream>>>(ARGS(TV)); \
+      else delta_scan_kernel<TV, KPL, VPL, D, DS_LOCAL><<<dim3(nblk, H, tiles(cols_local, nw_l)), 64 * nw_l, lds_bytes(nw_l), stream>>>(ARGS(TV)); \
       if (D && dk == 64) COMBINE(1);                                                                                         \
       else if (D && dk == 128) COMBINE(2);                                                                                   \
       else if (D && dk == 192) COMBINE(3);                                                                                   \
@@ -565,7 +640,8 @@ extern "C" int pico_delta_scan(const float* q, const float* k, const void* v, in
       else                                                                                                                   \
         decay_combine_kernel<<<dim3(num_seqs, H, (dk * dv + 255) / 256), 256, 0, stream>>>(                                  \
             cu_seqlens, state_slots, state, ws_S, ws_P, H, dk, dv, num_slots, chunk, max_chunks);                            \
-      delta_scan_kernel<TV, KPL, VPL, D, DS_FROM><<<dim3(nblk, H, tiles(dv, nw_v)), 64 * nw_v, lds_bytes(nw_v), stream>>>(ARGS(TV)); \
+      if (FOUR_OK(KPL, VPL) && four) delta_scan_kernel<TV, KPL, VPL, D, DS_FROM, FOUR_OK(KPL, VPL)><<<dim3(nblk, H, tiles(dv, nw_v)), 256, lds_bytes(nw_v), stream>>>(ARGS(TV)); \
+      else delta_scan_kernel<TV, KPL, VPL, D, DS_FROM><<<dim3(nblk, H, tiles(dv, nw_v)), 64 * nw_v, lds_bytes(nw_v), stream>>>(ARGS(TV)); \
     }                                                                                                                        \
   } while (0)
 #define PICK2(TV, KPL, D)                  \
@@ -586,6 +662,7 @@ extern "C" int pico_delta_scan(const float* q, const float* k, const void* v, in
 #undef PICK
 #undef PICK2
 #undef GO
+#undef FOUR_OK
 #undef COMBINE
 #undef ARGS
   PICO_LAUNCH_CHECK();
