@@ -691,6 +691,49 @@ __global__ __launch_bounds__(1024) void gated_group_norm_kernel(const float* __r
   for (int i = threadIdx.x; i < n; i += blockDim.x) store_f32(out + (size_t)t * H * dv + base + i, part[i] * r * w[base + i]);
 }
 
+// The same in bfloat16 with four neighbouring entries a thread and turn, the part in registers and its loads all asked for at once.
+// 2,052 tokens, two parts of 1,536: 16.6 us, entry by entry through LDS 20.7.
+template <int VPT>
+__global__ __launch_bounds__(1024) void gated_group_norm4_kernel(const float* __restrict__ y, const bf16_t* __restrict__ x, int ldx,
+                                                                const bf16_t* __restrict__ z, int ldz, const float* __restrict__ D,
+                                                                const float* __restrict__ w, float eps, bf16_t* __restrict__ out,
+                                                                int H, int dv, int groups) {
+  __shared__ float scratch[16];
+  const int t = blockIdx.x, n = H * dv / groups, base = blockIdx.y * n;
+  f32x4 yv[VPT], wv[VPT];
+  uint2 xv[VPT], zv[VPT];
+  float dh[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; j++) {
+    const int c = base + min(4 * (int)(j * blockDim.x + threadIdx.x), n - 4);
+    yv[j] = *reinterpret_cast<const f32x4*>(y + (size_t)t * H * dv + c);
+    xv[j] = *reinterpret_cast<const uint2*>(x + (size_t)t * ldx + c);
+    zv[j] = *reinterpret_cast<const uint2*>(z + (size_t)t * ldz + c);
+    wv[j] = *reinterpret_cast<const f32x4*>(w + c);
+    dh[j] = D[c / dv];
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPT; j++) {
+    const bool in = 4 * (int)(j * blockDim.x + threadIdx.x) < n;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t xw = k < 2 ? xv[j].x : xv[j].y, zw = k < 2 ? zv[j].x : zv[j].y;
+      const float xx = __uint_as_float(k & 1 ? xw & 0xffff0000u : xw << 16), zz = __uint_as_float(k & 1 ? zw & 0xffff0000u : zw << 16);
+      yv[j][k] = fmaf(dh[j], xx, yv[j][k]) * (zz / (1.0f + expf(-zz)));
+      ss = in ? fmaf(yv[j][k], yv[j][k], ss) : ss;
+    }
+  }
+  const float r = 1.0f / sqrtf(block_sum(ss, scratch) / (float)n + eps);
+#pragma unroll
+  for (int j = 0; j < VPT; j++) {
+    const int i = 4 * (int)(j * blockDim.x + threadIdx.x);
+    if (i < n)
+      *reinterpret_cast<uint2*>(out + (size_t)t * H * dv + base + i) = make_uint2(pack2_bf16(yv[j][0] * r * wv[j][0], yv[j][1] * r * wv[j][1]),
+                                                                                 pack2_bf16(yv[j][2] * r * wv[j][2], yv[j][3] * r * wv[j][3]));
+  }
+}
+
 extern "C" int pico_gated_group_norm(const float* y, const void* x, int ldx, const void* z, int ldz, int dtype, const float* D,
                                      const float* w, float eps, void* out, int T, int H, int dv, int groups,
                                      hipStream_t stream) {
@@ -699,6 +742,18 @@ extern "C" int pico_gated_group_norm(const float* y, const void* x, int ldx, con
   if (T == 0) return 0;
   const size_t lds = (size_t)(H * dv / groups) * sizeof(float);
   const dim3 grid(T, groups);
+  // whole aligned fours of a head and of a part, parts that fit a workgroup's registers
+  const int n = H * dv / groups;
+  if (dtype == PICO_DTYPE_BF16 && dv % 4 == 0 && n % 4 == 0 && n <= 8192 && ldx % 4 == 0 && ldz % 4 == 0 && ((uintptr_t)y | (uintptr_t)w) % 16 == 0 &&
+      ((uintptr_t)x | (uintptr_t)z | (uintptr_t)out) % 8 == 0) {
+    const int vpt = n <= 4096 ? 1 : 2, threads = ((n / 4 + vpt - 1) / vpt + 63) / 64 * 64;
+#define GATED(VPT) gated_group_norm4_kernel<VPT><<<grid, threads, 0, stream>>>(y, (const bf16_t*)x, ldx, (const bf16_t*)z, ldz, D, w, eps, (bf16_t*)out, H, dv, groups)
+    if (vpt == 1) GATED(1);
+    else GATED(2);
+#undef GATED
+    PICO_LAUNCH_CHECK();
+    return 0;
+  }
   const int threads = T >= 64 ? 256 : 1024;       // few tokens: a thread's loads are one turn and travel together
   if (dtype == PICO_DTYPE_F32)
     gated_group_norm_kernel<float><<<grid, threads, lds, stream>>>(y, (const float*)x, ldx, (const float*)z, ldz, D, w, eps, (float*)out, H, dv, groups);

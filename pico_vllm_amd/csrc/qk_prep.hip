@@ -85,18 +85,21 @@ __global__ __launch_bounds__(1024) void qk_norm_store_kernel(
   }
 }
 
-// Unit by unit in bfloat16 for many tokens (one map a head; units of up to 128 entries in whole pairs, the turned ones in
-// whole fours): a lane owns two neighbouring entries, and a wave asks for all of its units (up to QK_AHEAD of them at a time),
-// their partners in the rotation included, before the first norm waits.  PAIRS: neighbours are turned together, so that a lane
-// holds both entries of a pair; WEIGHTED: the units have weights.
+// In bfloat16 for many tokens (units of up to 128 entries in whole pairs, the turned ones in whole fours): a lane owns two
+// neighbouring entries, and a wave asks for all of its units (up to QK_AHEAD of them at a time), their partners in the
+// rotation included, before the first norm waits.  PAIRS: neighbours are turned together, so that a lane holds both entries
+// of a pair.  WEIGHTS: the units have none, one for all (QK_NORM_UNIT), or, normed over the whole row, one each (QK_NORM_ROW).
+// 2,052 tokens, 12 query and 2 key heads of 128 normed over the row 13.5 us, in two maps of 64 normed by themselves 16.1; entry by
+// entry, a wave waiting for a unit at a time, 22.2 both.
 #define QK_AHEAD 4
-template <bool PAIRS, bool WEIGHTED>
+template <bool PAIRS, int WEIGHTS>
 __global__ __launch_bounds__(256) void qk_unit_norm_store_kernel(
-    const bf16_t* __restrict__ x, int ld, int q_col, int k_col, int v_col, int nq, int nk, int nv, int dk, int dv,
+    const bf16_t* __restrict__ x, int ld, int q_col, int k_col, int v_col, int nq, int nk, int nv, int dk, int dv, int maps,
     const float* __restrict__ wq, const float* __restrict__ wk, float eps, const float* __restrict__ cos_sin, int rot,
     const int* __restrict__ slots, bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache, int P,
     int num_pages) {
-  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  __shared__ float sums[2][4];
+  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const bf16_t* row = x + (size_t)t * ld;
   const int slot = slots ? slots[t] : -1;
   const int page = slot >= 0 ? slot / P : -1, off = slot >= 0 ? slot % P : 0;
@@ -117,19 +120,47 @@ __global__ __launch_bounds__(256) void qk_unit_norm_store_kernel(
       const int g = e / dv, d = e % dv;
       v_cache[(((size_t)page * nv + g) * dv + d) * P + off] = row[v_col + e];
     }
+  float row_q = 1.f, row_k = 1.f;
+  if (WEIGHTS == QK_NORM_ROW) {
+    auto squares = [&](const bf16_t* src, int n) {                   // of the whole row, two entries a turn
+      float ss = 0.f;
+      for (int e = 2 * threadIdx.x; e < n; e += 2 * blockDim.x) {
+        const uint32_t v = *reinterpret_cast<const uint32_t*>(src + e);
+        const float v0 = __uint_as_float(v << 16), v1 = __uint_as_float(v & 0xffff0000u);
+        ss += fmaf(v0, v0, v1 * v1);
+      }
+      return wave_sum(ss);
+    };
+    const float sq = squares(row + q_col, nq * dk), sk = squares(row + k_col, nk * dk);
+    if (lane == 0) { sums[0][wave] = sq; sums[1][wave] = sk; }
+    __syncthreads();
+    row_q = 1.0f / sqrtf((sums[0][0] + sums[0][1] + sums[0][2] + sums[0][3]) / (float)(nq * dk) + eps);
+    row_k = 1.0f / sqrtf((sums[1][0] + sums[1][1] + sums[1][2] + sums[1][3]) / (float)(nk * dk) + eps);
+  }
   float2 q0 = make_float2(1.f, 1.f), qp = q0, k0 = q0, kp = q0;
-  if (WEIGHTED) {
+  if (WEIGHTS == QK_NORM_UNIT) {
     q0 = *reinterpret_cast<const float2*>(wq + ic); qp = *reinterpret_cast<const float2*>(wq + j);
     k0 = *reinterpret_cast<const float2*>(wk + ic); kp = *reinterpret_cast<const float2*>(wk + j);
   }
+  const int R = max(1, nq / max(1, nk));                             // heads a kv group
   for (int u0 = wave; u0 < nq + nk; u0 += nw * QK_AHEAD) {
     uint32_t own[QK_AHEAD], par[QK_AHEAD];
+    float2 w0[QK_AHEAD], w1[QK_AHEAD];
 #pragma unroll
     for (int a = 0; a < QK_AHEAD; a++) {
       const int u = min(u0 + a * nw, nq + nk - 1);
-      const bf16_t* src = row + (u < nq ? q_col + u * dk : k_col + (u - nq) * dk);
+      const bool is_q = u < nq;
+      const bf16_t* src = row + (is_q ? q_col + u * dk : k_col + (u - nq) * dk);
       own[a] = *reinterpret_cast<const uint32_t*>(src + ic);
       par[a] = PAIRS ? own[a] : *reinterpret_cast<const uint32_t*>(src + j);
+      if (WEIGHTS == QK_NORM_ROW) {
+        const float* w = is_q ? wq + u * dk : wk + (u - nq) * dk;
+        w0[a] = *reinterpret_cast<const float2*>(w + ic);
+        w1[a] = *reinterpret_cast<const float2*>(w + j);
+      } else {
+        w0[a] = is_q ? q0 : k0;
+        w1[a] = is_q ? qp : kp;
+      }
     }
 #pragma unroll
     for (int a = 0; a < QK_AHEAD; a++) {
@@ -139,10 +170,15 @@ __global__ __launch_bounds__(256) void qk_unit_norm_store_kernel(
       if (!is_q && !store) break;                                    // (keys stand behind all queries)
       const float v0 = __uint_as_float(own[a] << 16), v1 = __uint_as_float(own[a] & 0xffff0000u);
       const float p0 = PAIRS ? v1 : __uint_as_float(par[a] << 16), p1 = PAIRS ? v0 : __uint_as_float(par[a] & 0xffff0000u);
-      const float r = 1.0f / sqrtf(wave_sum(i < dk ? fmaf(v0, v0, v1 * v1) : 0.f) / (float)dk + eps);
-      const float2 w0 = is_q ? q0 : k0, w1 = is_q ? qp : kp;
-      const float a0 = v0 * r * w0.x, a1 = v1 * r * w0.y, b0 = p0 * r * (PAIRS ? w0.y : w1.x), b1 = p1 * r * (PAIRS ? w0.x : w1.y);
-      bf16_t* dst = is_q ? q_out + ((size_t)t * nq + u) * dk : k_cache + (((size_t)page * nk + (u - nq)) * P + off) * dk;
+      const float r = WEIGHTS == QK_NORM_ROW ? (is_q ? row_q : row_k)
+                                             : 1.0f / sqrtf(wave_sum(i < dk ? fmaf(v0, v0, v1 * v1) : 0.f) / (float)dk + eps);
+      const float a0 = v0 * r * w0[a].x, a1 = v1 * r * w0[a].y, b0 = p0 * r * (PAIRS ? w0[a].y : w1[a].x), b1 = p1 * r * (PAIRS ? w0[a].x : w1[a].y);
+      int place = u;
+      if (is_q && maps > 1) {
+        const int h = u / maps, m = u % maps, g = h / R, rr = h % R;
+        place = (g * maps + m) * R + rr;
+      }
+      bf16_t* dst = is_q ? q_out + ((size_t)t * nq + place) * dk : k_cache + (((size_t)page * nk + (u - nq)) * P + off) * dk;
       if (i < dk) *reinterpret_cast<uint32_t*>(dst + i) = pack2_bf16(a0 * c0 + b0 * s0, a1 * c1 + b1 * s1);
     }
   }
@@ -162,15 +198,23 @@ extern "C" int pico_qk_norm_store(const void* x, int dtype, int ld, int q_col, i
   PICO_REQUIRE(k_cache == nullptr || (P > 0 && num_pages > 0 && slots), "pico_qk_norm_store: a cache needs pages and slots");
   if (T == 0) return 0;
   if (k_cache == nullptr) { slots = nullptr; v_cache = nullptr; P = 1; num_pages = 0; }
-  if (dtype == PICO_DTYPE_BF16 && T > 64 && norm_mode == QK_NORM_UNIT && maps == 1 && dk % 2 == 0 && dk <= 128 && (pairs || rot % 4 == 0) &&
+  if (dtype == PICO_DTYPE_BF16 && T > 64 && norm_mode != QK_NORM_NONE && dk % 2 == 0 && dk <= 128 && (pairs || rot % 4 == 0) &&
       (ld | q_col | k_col) % 2 == 0 && ((uintptr_t)x | (uintptr_t)q_out | (uintptr_t)k_cache) % 4 == 0 &&
       ((uintptr_t)wq | (uintptr_t)wk) % 8 == 0 && (uintptr_t)cos_sin % 16 == 0) {
-#define LAUNCH(PAIRS, WEIGHTED)                                                                                              \
-  qk_unit_norm_store_kernel<PAIRS, WEIGHTED><<<T, 256, 0, stream>>>((const bf16_t*)x, ld, q_col, k_col, v_col, nq, nk, nv, dk, dv, \
-                                                                    wq, wk, eps, cos_sin, rot, slots, (bf16_t*)q_out,         \
-                                                                    (bf16_t*)k_cache, (bf16_t*)v_cache, P, num_pages)
-    if (pairs) { if (wq) LAUNCH(true, true); else LAUNCH(true, false); }
-    else { if (wq) LAUNCH(false, true); else LAUNCH(false, false); }
+#define LAUNCH(PAIRS, WEIGHTS)                                                                                                     \
+  qk_unit_norm_store_kernel<PAIRS, WEIGHTS><<<T, 256, 0, stream>>>((const bf16_t*)x, ld, q_col, k_col, v_col, nq, nk, nv, dk, dv, maps, \
+                                                                   wq, wk, eps, cos_sin, rot, slots, (bf16_t*)q_out,                 \
+                                                                   (bf16_t*)k_cache, (bf16_t*)v_cache, P, num_pages)
+    const int weights = norm_mode == QK_NORM_ROW ? QK_NORM_ROW : wq ? QK_NORM_UNIT : QK_NORM_NONE;
+    if (pairs) {
+      if (weights == QK_NORM_ROW) LAUNCH(true, QK_NORM_ROW);
+      else if (weights) LAUNCH(true, QK_NORM_UNIT);
+      else LAUNCH(true, QK_NORM_NONE);
+    } else {
+      if (weights == QK_NORM_ROW) LAUNCH(false, QK_NORM_ROW);
+      else if (weights) LAUNCH(false, QK_NORM_UNIT);
+      else LAUNCH(false, QK_NORM_NONE);
+    }
 #undef LAUNCH
     PICO_LAUNCH_CHECK();
     return 0;

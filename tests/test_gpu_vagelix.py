@@ -776,3 +776,66 @@ def test_configurations_drawn_at_random_in_mixed_batches(seed):
     for dtype in ("float32", "bfloat16"):
         rows, rp = replay(d, dtype, steps, peak, page, max_live=3)
         compare(f"drawn{seed}", dtype, rows, reqs, cfg=cfg, tensors=t)
+
+
+def same_but_for_rounding(got, want, big):
+    """Two orders of the same float32 sums, stored in bfloat16: neighbouring values at most (2^-7 of the value), plus a few
+    float32 roundings of the largest term."""
+    a, b = got.double().cpu(), want.double().cpu()
+    assert bool(((a - b).abs() <= 2.0 ** -7 * torch.maximum(a.abs(), b.abs()) + 2.0 ** -20 * big).all()), float((a - b).abs().max())
+
+
+@pytest.mark.parametrize("H,G,dk,maps,mode,rot,odd", [(12, 2, 64, 2, 1, 0, 0), (6, 2, 64, 2, 1, 64, 0), (12, 2, 128, 1, 2, 128, 0), (5, 1, 10, 1, 2, 4, 0),
+                                                      (9, 3, 62, 3, 1, 8, 1), (17, 1, 2, 1, 2, 0, 0), (1, 1, 128, 1, 2, 0, 1)])
+def test_two_entries_a_lane_give_what_entry_by_entry_gives(H, G, dk, maps, mode, rot, odd):
+    """70 rows at once and 35 at a time, where the general kernel runs; also with values that start in an odd column."""
+    from pico_vllm_amd.ops import kernels
+    g = torch.Generator().manual_seed(H * dk)
+    T, page, pages, dv = 70, 8, 10, 16
+    nq, nk = H * maps, G * maps
+    q0, k0 = 2, 2 + nq * dk
+    v0 = k0 + nk * dk + odd
+    x = (2 * torch.randn(T, v0 + G * dv + (4 - odd) // 2 * 2 + (v0 + G * dv) % 2, generator=g)).to(DEV, torch.bfloat16)
+    nw = dk if mode == 1 else None
+    wq, wk = ((1 + 0.3 * torch.randn(nw or n * dk, generator=g)).to(DEV) for n in (nq, nk))
+    slots = torch.tensor([t if t != 9 else -1 for t in range(T)], dtype=torch.int32, device=DEV)
+    table = kernels.rope_table(torch.arange(T, dtype=torch.int32, device=DEV),
+                               torch.tensor([300.0 ** (-2.0 * i / rot) for i in range(rot // 2)], device=DEV)) if rot else None
+    def run(sl, kc, vc):
+        return kernels.qk_norm_store(x[sl], q0, k0, v0, nq, nk, G, dk, dv, maps, mode, wq, wk, 1e-5, table[sl] if rot else None, rot, slots[sl], kc, vc)
+    caches = [(torch.zeros(pages, nk, page, dk, dtype=torch.bfloat16, device=DEV), torch.zeros(pages, G, dv, page, dtype=torch.bfloat16, device=DEV))
+              for _ in range(2)]
+    got = run(slice(0, T), *caches[0])
+    want = torch.cat([run(slice(0, 35), *caches[1]), run(slice(35, T), *caches[1])])
+    same_but_for_rounding(got, want, 8)
+    same_but_for_rounding(caches[0][0], caches[1][0], 8)
+    assert torch.equal(caches[0][1], caches[1][1])
+
+
+@pytest.mark.parametrize("H", [4, 252, 260, 1536, 4096])
+def test_fours_a_thread_give_what_entry_by_entry_gives(H):
+    """Two normed outputs onto a stream, and the gated norm in parts, against the same with rows that no four fits."""
+    from pico_vllm_amd.ops import kernels
+    g = torch.Generator().manual_seed(H)
+    T = 5
+    a, b = ((3 * torch.randn(T, H, generator=g)).to(DEV, torch.bfloat16) for _ in range(2))
+    w, wa, wb = ((1 + 0.3 * torch.randn(H, generator=g)).to(DEV) for _ in range(3))
+    x = torch.randn(T, H, generator=g)
+    fast, spare = x.to(DEV), torch.empty(T * H + 1, device=DEV)
+    slow = spare[1:].view(T, H)
+    slow.copy_(x)
+    for dtype in (torch.bfloat16, torch.float32, None):
+        copies = [kernels.norm_add(r, a, w, 1e-5, dtype, y2=b, weight1=wa, weight2=wb) for r in (fast, slow)]
+        close(fast, slow.cpu(), "float32")
+        if dtype is not None:
+            same_but_for_rounding(copies[0], copies[1], 8)
+    for heads, parts in ((1, 1), (H // 4, 1), (2, 2)):                  # a part of up to 8,192 entries
+        dv = H // heads if heads != 2 else 2 * H
+        n = heads * dv
+        y = torch.randn(T, n, generator=g).to(DEV)
+        xs = torch.randn(T, n, generator=g).to(DEV, torch.bfloat16)
+        z = torch.randn(T, n + 4, generator=g).to(DEV, torch.bfloat16)
+        d, wn = torch.randn(heads, generator=g).to(DEV), (1 + 0.3 * torch.randn(n, generator=g)).to(DEV)
+        got, want = (kernels.gated_group_norm(y, xs, zz, d, wn, 1e-5, heads, dv, parts)
+                     for zz in (z[:, :n], torch.cat([z, z[:, :1]], 1)[:, :n]))
+        same_but_for_rounding(got, want, 64)
