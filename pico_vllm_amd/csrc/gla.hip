@@ -13,51 +13,92 @@
 // on the sizes alone, so a token's output does not depend on how its sequence was cut into steps.
 #include "common.h"
 
+// log(sigmoid(z)) = -log(1 + e^-z), without overflow on either side; one logarithm and exponential serve both, as lanes of a
+// wave that differ in sign would go through the two in turn.
+__device__ __forceinline__ float log_sigmoid(float z) {
+  const float l = log1pf(expf(-fabsf(z)));
+  return z >= 0.f ? -l : z - l;
+}
+
 // ---------------------------------------------------------------------------
 // Logarithm of the decay: out[t][c] = log(sigmoid(z)) / tau, z = sum_r a2[c][r] * x[t][r] + b[c].
-// x: the low-rank activations (columns of a wider row, stride ldx); a2 [C, R]; b float32 [C].  grid (T), any C and R.
+// x: the low-rank activations (columns of a wider row, stride ldx); a2 [C, R]; b float32 [C].  grid (ceil(T / TOK), ceil(C / 256)),
+// any C and R.  A thread makes one channel of TOK tokens, so that a2 is read once for them: 2,048 tokens, 768 channels of
+// rank 32 13.7 us, 16.5 with a token a workgroup and a logarithm for either sign; few tokens keep one, to fill the chip.
 // ---------------------------------------------------------------------------
-template <typename T>
+#define GLA_DECAY_TOKENS 8
+template <typename T, int TOK>
 __global__ __launch_bounds__(256) void gla_decay_kernel(const T* __restrict__ x, int ldx, const T* __restrict__ a2,
                                                         const float* __restrict__ b, float inv_tau, float* __restrict__ out,
-                                                        int C, int R) {
-  extern __shared__ float xs[];
-  const int t = blockIdx.x;
-  for (int r = threadIdx.x; r < R; r += blockDim.x) xs[r] = load_f32(x + (size_t)t * ldx + r);
+                                                        int tokens, int C, int R) {
+  extern __shared__ float xs[];                         // [R][TOK]
+  const int t0 = blockIdx.x * TOK, c = blockIdx.y * 256 + threadIdx.x;
+  for (int i = threadIdx.x; i < R * TOK; i += blockDim.x) xs[i] = load_f32(x + (size_t)min(t0 + i % TOK, tokens - 1) * ldx + i / TOK);
   __syncthreads();
-  for (int c = threadIdx.x; c < C; c += blockDim.x) {
-    const T* w = a2 + (size_t)c * R;
-    float z = b ? b[c] : 0.f;
-    for (int r = 0; r < R; r++) z = fmaf(load_f32(w + r), xs[r], z);
-    // log(sigmoid(z)) = -log(1 + e^-z), without overflow on either side
-    const float ls = z >= 0.f ? -log1pf(expf(-z)) : z - log1pf(expf(z));
-    out[(size_t)t * C + c] = ls * inv_tau;
+  if (c >= C) return;
+  const T* w = a2 + (size_t)c * R;
+  float z[TOK];
+#pragma unroll
+  for (int k = 0; k < TOK; k++) z[k] = b ? b[c] : 0.f;
+  constexpr int V = 16 / sizeof(T);
+  int r = 0;
+  if (R % V == 0 && (uintptr_t)a2 % 16 == 0)            // a lane's row of a2 in whole aligned sixteens: its lines are asked for once
+#pragma unroll 2
+    for (; r < R; r += V) {
+      alignas(16) T wv[V];
+      *reinterpret_cast<uint4*>(wv) = *reinterpret_cast<const uint4*>(w + r);
+#pragma unroll
+      for (int i = 0; i < V; i++)
+#pragma unroll
+        for (int k = 0; k < TOK; k++) z[k] = fmaf(load_f32(wv + i), xs[(r + i) * TOK + k], z[k]);
+    }
+  for (; r < R; r++) {
+    const float wr = load_f32(w + r);
+#pragma unroll
+    for (int k = 0; k < TOK; k++) z[k] = fmaf(wr, xs[r * TOK + k], z[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < TOK; k++) {
+    if (t0 + k >= tokens) break;
+    out[(size_t)(t0 + k) * C + c] = log_sigmoid(z[k]) * inv_tau;
   }
 }
 
 extern "C" int pico_gla_decay(const void* x, int ldx, int dtype, const void* a2, const float* b, float tau, float* out,
                               int T, int C, int R, hipStream_t stream) {
   PICO_REQUIRE(T >= 0 && C > 0 && R > 0 && ldx >= R && R <= 8192, "pico_gla_decay: bad sizes");
+  PICO_REQUIRE((C + 255) / 256 <= 65535, "pico_gla_decay: sizes beyond the grid");
   PICO_REQUIRE(tau > 0.f, "pico_gla_decay: tau must be positive");
   if (T == 0) return 0;
-  const size_t lds = (size_t)R * sizeof(float);
-  if (dtype == PICO_DTYPE_F32)
-    gla_decay_kernel<float><<<T, 256, lds, stream>>>((const float*)x, ldx, (const float*)a2, b, 1.0f / tau, out, C, R);
-  else if (dtype == PICO_DTYPE_BF16)
-    gla_decay_kernel<bf16_t><<<T, 256, lds, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)a2, b, 1.0f / tau, out, C, R);
-  else
-    PICO_REQUIRE(false, "pico_gla_decay: unknown dtype %d", dtype);
+  // blocks of tokens where they still fill the chip and their activations fit LDS
+  const bool many = T >= 64 && R <= 1024;
+  const int tok = many ? GLA_DECAY_TOKENS : 1;
+  const size_t lds = (size_t)R * tok * sizeof(float);
+  const dim3 grid((T + tok - 1) / tok, (C + 255) / 256);
+#define DECAY(TT)                                                                                                            \
+  do {                                                                                                                       \
+    if (many) gla_decay_kernel<TT, GLA_DECAY_TOKENS><<<grid, 256, lds, stream>>>((const TT*)x, ldx, (const TT*)a2, b, 1.0f / tau, out, T, C, R); \
+    else gla_decay_kernel<TT, 1><<<grid, 256, lds, stream>>>((const TT*)x, ldx, (const TT*)a2, b, 1.0f / tau, out, T, C, R);  \
+  } while (0)
+  if (dtype == PICO_DTYPE_F32) DECAY(float);
+  else if (dtype == PICO_DTYPE_BF16) DECAY(bf16_t);
+  else PICO_REQUIRE(false, "pico_gla_decay: unknown dtype %d", dtype);
+#undef DECAY
   PICO_LAUNCH_CHECK();
   return 0;
 }
 
 // ---------------------------------------------------------------------------
-// The recurrence, token by token.  grid (sequences, heads, ceil(dv / 64 VPL)); a workgroup owns 64 VPL value channels of
-// one head of one sequence; wave w of its ceil(dk / GLA_CPT) waves owns key channels GLA_CPT w .., lane l value channels
-// l, l + 64, .. (VPL of them: 2 where a head has more than 64):
-// a thread keeps GLA_CPT state elements in registers over all tokens of the step.  Tokens are taken TB (8 or 16) at a
-// time: their q, k and decays are staged in LDS (every thread reads all of its channels' from there) while the next
-// block's travel from memory in registers; the waves' partial outputs meet in LDS and are summed in wave order.
+// The recurrence, token by token.  grid (sequences, heads, ceil(dv / 64)); a workgroup owns 64 value channels of one head of
+// one sequence; wave w of its NW owns key channels 32 w ..  A thread keeps a patch of 8 key by 4 value channels of the state in
+// registers over all tokens of the step (lane l: values 4 (l mod 16) .., keys 8 (l / 16) ..), so that the 24 numbers of q, k
+// and decays and the 4 of v that it reads of a token out of LDS serve 96 operations; the wave's four partial outputs of a
+// value are added by lane swaps that leave each lane one value.  Tokens are taken TB (8 or 16) at a time: they are staged in
+// LDS while the next block's travel from memory in registers; the waves' partial outputs meet in LDS and are summed in
+// wave order.
+// What bounds it is the vector pipe, 3 operations a state element and token (2 where no outputs are made); with one value
+// and 32 key channels a lane it was LDS, which hands every lane its own copy of 96 numbers a token.  A prompt of 2,048 tokens,
+// 12 heads of 64 x 128: chunks of 64 take 43 us with outputs and 26 without, before 81 and 48.
 //
 // Long portions are cut into chunks of `chunk` tokens that run side by side (the recurrence is linear in the state):
 //   GLA_LOCAL:  every chunk from a state of zero, no outputs; leaves its state in ws[chunk] and the sum of its decays'
@@ -66,14 +107,17 @@ extern "C" int pico_gla_decay(const void* x, int ldx, int dtype, const void* a2,
 //   GLA_FROM:   every chunk again from ws[chunk], writing the outputs
 // GLA_WHOLE is the plain walk from the slot's state (a sequence is one chunk).  blockIdx.x = sequence * max_chunks + chunk.
 // ---------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 #define GLA_CPT 32
+#define GLA_KEYS 8          // of a lane
 #define GLA_WHOLE 0
 #define GLA_LOCAL 1
 #define GLA_FROM 2
 
-// FUSED: the decays are made inside the walk (log_decay is null) instead of read.
-template <typename T, int MODE, int TB, int VPL, bool FUSED>
-__global__ __launch_bounds__(TB == 16 ? 256 : 512) void gla_scan_kernel(const T* __restrict__ x, int ldx, int q_col, int k_col, int v_col,
+// FUSED: the decays are made inside the walk (log_decay is null) instead of read.  wide: the states' rows are whole aligned fours.
+template <typename T, int MODE, int NW, bool FUSED>
+__global__ __launch_bounds__(64 * NW) void gla_scan_kernel(const T* __restrict__ x, int ldx, int q_col, int k_col, int v_col,
                                                        const float* __restrict__ log_decay,
                                                        const int* __restrict__ cu_seqlens,
                                                        const int* __restrict__ state_slots, float* __restrict__ state,
@@ -81,28 +125,14 @@ __global__ __launch_bounds__(TB == 16 ? 256 : 512) void gla_scan_kernel(const T*
                                                        int num_slots, int chunk, int max_chunks, float* __restrict__ ws,
                                                        float* __restrict__ ws_decay, const T* __restrict__ a2,
                                                        const float* __restrict__ a2_bias, int a_col, int R, float inv_tau,
-                                                       const float* __restrict__ head_decay, int silu) {
-  extern __shared__ float lds[];
+                                                       const float* __restrict__ head_decay, int silu, int wide) {
+  constexpr int TB = NW <= 4 ? 16 : 8, CP = NW * GLA_CPT, NL = TB / 2, NV = TB / NW;
+  __shared__ float qs[TB * CP], ks[TB * CP], as[TB * CP], vs[TB * 64], po[TB * NW * 64];
   // head_decay given: every key channel of head h decays by the constant head_decay[h] at every token (log_decay, a2
   // are not read); the decay is multiplied in as it is, no logarithm and exponential between
   const float fixed = head_decay ? head_decay[blockIdx.y] : 0.f;
-  const int nw = blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int CP = nw * GLA_CPT;                          // key channels with padding
-  float* qs = lds;                                      // [TB][CP]
-  float* ks = qs + TB * CP;
-  float* as = ks + TB * CP;
-  float* po = as + TB * CP;                             // [TB][nw][64 VPL]
-  // a lane owns VPL value channels, 64 apart: what it reads of a token's q, k and decays out of LDS serves them all
-  // (every wave of a compute unit reads the same staged values, and LDS hands each lane its own copy)
-  constexpr int VW = 64 * VPL;
-  const int b = MODE == GLA_WHOLE ? blockIdx.x : blockIdx.x / max_chunks, h = blockIdx.y, v = blockIdx.z * VW + lane;
-  bool v_ok[VPL];
-  int v_in[VPL];                                        // a value channel that exists, else the head's last one
-#pragma unroll
-  for (int j = 0; j < VPL; j++) {
-    v_ok[j] = v + 64 * j < dv;
-    v_in[j] = min(v + 64 * j, dv - 1) - v;
-  }
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int b = MODE == GLA_WHOLE ? blockIdx.x : blockIdx.x / max_chunks, h = blockIdx.y, v0 = blockIdx.z * 64;
   int t_begin = cu_seqlens[b], t_end = cu_seqlens[b + 1];
   if (MODE != GLA_WHOLE) {
     t_begin += (blockIdx.x % max_chunks) * chunk;
@@ -110,40 +140,34 @@ __global__ __launch_bounds__(TB == 16 ? 256 : 512) void gla_scan_kernel(const T*
   }
   const int slot = state_slots[b];
   if (slot < 0 || slot >= num_slots || t_end <= t_begin) return;
-  const int c0 = wave * GLA_CPT;
-  float* sp = MODE == GLA_WHOLE ? state + (((size_t)slot * H + h) * dk + c0) * dv + v
-                                : ws + (((size_t)blockIdx.x * H + h) * dk + c0) * dv + v;
+  const int live = (dk + GLA_CPT - 1) / GLA_CPT;        // waves that own key channels at all
+  const int ck = (lane >> 4) * GLA_KEYS, c0 = wave * GLA_CPT + ck, vl = 4 * (lane & 15), v = v0 + vl;
+  float* sp = MODE == GLA_WHOLE ? state + ((size_t)slot * H + h) * dk * dv : ws + ((size_t)blockIdx.x * H + h) * dk * dv;
   // Every load below is unconditional, from an address clamped into the tensor, and what must not count is cleared
   // afterwards: a load inside a branch is waited for inside that branch, and a thread's loads of a block then queue
   // one behind the other's latency instead of travelling together.
-  float S[VPL][GLA_CPT];
+  f32x4 S[GLA_KEYS];
   if (MODE != GLA_LOCAL) {
+    if (wide) {
 #pragma unroll
-    for (int j = 0; j < VPL; j++)
+      for (int c = 0; c < GLA_KEYS; c++) S[c] = *reinterpret_cast<const f32x4*>(sp + (size_t)min(c0 + c, dk - 1) * dv + min(v, dv - 4));
+    } else {
 #pragma unroll
-      for (int c = 0; c < GLA_CPT; c++) S[j][c] = sp[(size_t)(min(c0 + c, dk - 1) - c0) * dv + v_in[j]];
-  }
+      for (int c = 0; c < GLA_KEYS; c++)
 #pragma unroll
-  for (int j = 0; j < VPL; j++)
-#pragma unroll
-    for (int c = 0; c < GLA_CPT; c++) S[j][c] = (MODE != GLA_LOCAL && v_ok[j] && c0 + c < dk) ? S[j][c] : 0.f;
-  if (MODE == GLA_LOCAL && blockIdx.z == 0) {
-    // the chunk's decays multiplied up, as the sum of their logarithms, for the walk over the chunks
-    for (int c = threadIdx.x; c < dk; c += blockDim.x) {
-      float sum = 0.f;
-      if (head_decay) sum = (float)(t_end - t_begin) * logf(fixed);
-      else
-        for (int t = t_begin; t < t_end; t++) sum += log_decay[(size_t)t * H * dk + (size_t)h * dk + c];
-      ws_decay[((size_t)blockIdx.x * H + h) * dk + c] = sum;
+        for (int j = 0; j < 4; j++) S[c][j] = sp[(size_t)min(c0 + c, dk - 1) * dv + min(v + j, dv - 1)];
     }
   }
-  // A thread stages TB / 2 elements (token tt, channel c) of a block: i = threadIdx.x + j * blockDim.x.  The next
-  // block's values travel in registers while this block is walked.
-  constexpr int NL = TB / 2;
+#pragma unroll
+  for (int c = 0; c < GLA_KEYS; c++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) S[c][j] = (MODE != GLA_LOCAL && v + j < dv && c0 + c < dk) ? S[c][j] : 0.f;
+  // A thread stages TB / 2 elements (tokens tt0, tt0 + 2, .., channel cc) of a block's q, k and decays and TB / NW of its v
+  // (tokens wave, wave + NW, .., channel lane).  The next block's values travel in registers while this block is walked.
   const int tt0 = (int)threadIdx.x >= CP ? 1 : 0, cc = (int)threadIdx.x - tt0 * CP;
-  T rq[NL], rk[NL], rv[VPL][TB];
-  float ra[NL];
-  const int c_in = min(cc, dk - 1);
+  T rq[NL], rk[NL], rv[NV];
+  float ra[NL], decayed = 0.f;                          // (decayed: the logarithms of this thread's tokens in the chunk, added up)
+  const int c_in = min(cc, dk - 1), v_in = min(v0 + lane, dv - 1);
   auto fetch = [&](int t0) {
     const int nb = min(TB, t_end - t0);
 #pragma unroll
@@ -164,14 +188,11 @@ __global__ __launch_bounds__(TB == 16 ? 256 : 512) void gla_scan_kernel(const T*
         const T* w = a2 + ((size_t)h * dk + c_in) * R;
         float z = a2_bias ? a2_bias[h * dk + c_in] : 0.f;
         for (int r = 0; r < R; r++) z = fmaf(load_f32(w + r), load_f32(xa + r), z);
-        const float ls = z >= 0.f ? -log1pf(expf(-z)) : z - log1pf(expf(z));
-        ra[j] = ls * inv_tau;
+        ra[j] = log_sigmoid(z) * inv_tau;
       }
     }
 #pragma unroll
-    for (int j = 0; j < VPL; j++)
-#pragma unroll
-      for (int tt = 0; tt < TB; tt++) rv[j][tt] = x[(size_t)(t0 + min(tt, nb - 1)) * ldx + v_col + (size_t)h * dv + v + v_in[j]];
+    for (int j = 0; j < NV; j++) rv[j] = x[(size_t)(t0 + min(wave + j * NW, nb - 1)) * ldx + v_col + (size_t)h * dv + v_in];
   };
   fetch(t_begin);
   for (int t0 = t_begin; t0 < t_end; t0 += TB) {
@@ -179,79 +200,95 @@ __global__ __launch_bounds__(TB == 16 ? 256 : 512) void gla_scan_kernel(const T*
     __syncthreads();                                    // the last block's staged values and partial outputs have been read
 #pragma unroll
     for (int j = 0; j < NL; j++) {
-      const int tt = tt0 + 2 * j, c = cc, i = tt * CP + c;      // = threadIdx.x + j * blockDim.x: a workgroup has 2 CP threads
-      const bool in = tt < nb && c < dk;
+      const int tt = tt0 + 2 * j, i = tt * CP + cc;     // a workgroup has 2 CP threads
+      const bool in = tt < nb && cc < dk;
       const float qv = load_f32(&rq[j]), kv = load_f32(&rk[j]);
-      qs[i] = (in && MODE != GLA_LOCAL) ? (silu ? silu_f(qv) : qv) * qscale : 0.f;
+      if (MODE != GLA_LOCAL) qs[i] = in ? (silu ? silu_f(qv) : qv) * qscale : 0.f;
       ks[i] = in ? (silu ? silu_f(kv) : kv) : 0.f;
       as[i] = in ? (head_decay ? fixed : expf(ra[j])) : 1.f;
+      if (MODE == GLA_LOCAL) decayed += in ? ra[j] : 0.f;
     }
-    float vv[VPL][TB];
 #pragma unroll
-    for (int j = 0; j < VPL; j++)
-#pragma unroll
-      for (int tt = 0; tt < TB; tt++) {
-        const float x0 = load_f32(&rv[j][tt]);
-        vv[j][tt] = (tt < nb && v_ok[j]) ? (silu ? silu_f(x0) : x0) : 0.f;
-      }
+    for (int j = 0; j < NV; j++) {
+      const float x0 = load_f32(&rv[j]);
+      vs[(wave + j * NW) * 64 + lane] = (wave + j * NW < nb && v0 + lane < dv) ? (silu ? silu_f(x0) : x0) : 0.f;
+    }
     __syncthreads();
     if (t0 + TB < t_end) fetch(t0 + TB);
+    auto token = [&](int tt) {
+      const f32x4* a4 = reinterpret_cast<const f32x4*>(as + tt * CP + c0);
+      const f32x4* k4 = reinterpret_cast<const f32x4*>(ks + tt * CP + c0);
+      const f32x4* q4 = reinterpret_cast<const f32x4*>(qs + tt * CP + c0);
+      const f32x4 vt = *reinterpret_cast<const f32x4*>(vs + tt * 64 + vl);
+      float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int tt = 0; tt < TB; tt++) {
-      if (tt >= nb) break;
-      const float4* a4 = reinterpret_cast<const float4*>(as + tt * CP + c0);
-      const float4* k4 = reinterpret_cast<const float4*>(ks + tt * CP + c0);
-      const float4* q4 = reinterpret_cast<const float4*>(qs + tt * CP + c0);
-      // four partial sums over the channels (c mod 4), added at the end: four short chains instead of one long one
-      float acc0[VPL], acc1[VPL], acc2[VPL], acc3[VPL];
-#pragma unroll
-      for (int j = 0; j < VPL; j++) acc0[j] = acc1[j] = acc2[j] = acc3[j] = 0.f;
-#pragma unroll
-      for (int c = 0; c < GLA_CPT / 4; c++) {
-        const float4 av = a4[c], kv = k4[c];
-        float4 qv = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int c = 0; c < GLA_KEYS / 4; c++) {
+        const f32x4 av = a4[c], kv = k4[c];
+        f32x4 qv = {0.f, 0.f, 0.f, 0.f};
         if (MODE != GLA_LOCAL) qv = q4[c];
 #pragma unroll
-        for (int j = 0; j < VPL; j++) {
-          const float vt = vv[j][tt];
-          S[j][4 * c + 0] = fmaf(av.x, S[j][4 * c + 0], kv.x * vt);
-          S[j][4 * c + 1] = fmaf(av.y, S[j][4 * c + 1], kv.y * vt);
-          S[j][4 * c + 2] = fmaf(av.z, S[j][4 * c + 2], kv.z * vt);
-          S[j][4 * c + 3] = fmaf(av.w, S[j][4 * c + 3], kv.w * vt);
-          if (MODE != GLA_LOCAL) {
-            acc0[j] = fmaf(S[j][4 * c + 0], qv.x, acc0[j]);
-            acc1[j] = fmaf(S[j][4 * c + 1], qv.y, acc1[j]);
-            acc2[j] = fmaf(S[j][4 * c + 2], qv.z, acc2[j]);
-            acc3[j] = fmaf(S[j][4 * c + 3], qv.w, acc3[j]);
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            S[4 * c + i][j] = fmaf(av[i], S[4 * c + i][j], kv[i] * vt[j]);
+            if (MODE != GLA_LOCAL) acc[j] = fmaf(S[4 * c + i][j], qv[i], acc[j]);
           }
-        }
       }
       if (MODE != GLA_LOCAL) {
+        // lane (group g, l) is left with value 4 l + g of the four groups' sums
+        const auto e = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0]), __float_as_uint(acc[2]), false, false);
+        const auto f = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[1]), __float_as_uint(acc[3]), false, false);
+        const float e2 = __uint_as_float(e[0]) + __uint_as_float(e[1]), f2 = __uint_as_float(f[0]) + __uint_as_float(f[1]);
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(e2), __float_as_uint(f2), false, false);
+        po[(tt * NW + wave) * 64 + vl + (lane >> 4)] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      }
+    };
+    if (wave < live) {
+      if (nb == TB) {                                   // whole blocks in one piece: a token's reads travel under the one before
 #pragma unroll
-        for (int j = 0; j < VPL; j++) po[(tt * nw + wave) * VW + 64 * j + lane] = (acc0[j] + acc1[j]) + (acc2[j] + acc3[j]);
+        for (int tt = 0; tt < TB; tt++) token(tt);
+      } else {
+#pragma unroll 1
+        for (int tt = 0; tt < nb; tt++) token(tt);
       }
     }
     if (MODE == GLA_LOCAL) continue;
     __syncthreads();
-    for (int i = threadIdx.x; i < nb * VW; i += blockDim.x) {
-      const int tt = i / VW, l = i % VW, vo = blockIdx.z * VW + l;
-      if (vo >= dv) continue;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+      const int tt = wave + j * NW;
       float sum = 0.f;
-      for (int w = 0; w < nw; w++) sum += po[(tt * nw + w) * VW + l];
-      out[(size_t)(t0 + tt) * H * dv + (size_t)h * dv + vo] = sum;
+      for (int w = 0; w < live; w++) sum += po[(tt * NW + w) * 64 + lane];
+      if (tt < nb && v0 + lane < dv) out[(size_t)(t0 + tt) * H * dv + (size_t)h * dv + v0 + lane] = sum;
     }
   }
   if (MODE != GLA_FROM) {
+    if (wide) {
 #pragma unroll
-    for (int j = 0; j < VPL; j++)
+      for (int c = 0; c < GLA_KEYS; c++)
+        if (v < dv && c0 + c < dk) *reinterpret_cast<f32x4*>(sp + (size_t)(c0 + c) * dv + v) = S[c];
+    } else {
 #pragma unroll
-      for (int c = 0; c < GLA_CPT; c++)
-        if (v_ok[j] && c0 + c < dk) sp[(size_t)c * dv + 64 * j] = S[j][c];
+      for (int c = 0; c < GLA_KEYS; c++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (v + j < dv && c0 + c < dk) sp[(size_t)(c0 + c) * dv + v + j] = S[c][j];
+    }
+  }
+  if (MODE == GLA_LOCAL && blockIdx.z == 0) {
+    // the chunk's decays multiplied up, as the sum of their logarithms, for the walk over the chunks
+    __syncthreads();
+    if (tt0) as[cc] = decayed;
+    __syncthreads();
+    if (!tt0 && cc < dk)
+      ws_decay[((size_t)blockIdx.x * H + h) * dk + cc] = head_decay ? (float)(t_end - t_begin) * logf(fixed) : decayed + as[cc];
   }
 }
 
 // The walk over a sequence's chunks, one thread per state element: ws[j] becomes the state in front of chunk j, the
-// slot gets the state behind the last chunk.  grid (sequences, heads, ceil(dk dv / 256)).
+// slot gets the state behind the last chunk.  grid (sequences, heads, ceil(dk dv / 256)).  32 chunks of 12 states of 64 x 128
+// 10.3 us, with every chunk's state asked for in its turn 15.6.
+#define GLA_AHEAD 8
 __global__ __launch_bounds__(256) void gla_combine_kernel(const int* __restrict__ cu_seqlens,
                                                           const int* __restrict__ state_slots, float* __restrict__ state,
                                                           float* __restrict__ ws, const float* __restrict__ ws_decay, int H,
@@ -264,12 +301,31 @@ __global__ __launch_bounds__(256) void gla_combine_kernel(const int* __restrict_
   float* sp = state + ((size_t)slot * H + h) * dk * dv + e;
   float S = *sp;
   const int chunks = (n + chunk - 1) / chunk;
-  for (int j = 0; j < chunks; j++) {
-    const size_t at = (size_t)b * max_chunks + j;
-    float* w = ws + (at * H + h) * dk * dv + e;
-    const float local = *w;
-    *w = S;
-    S = fmaf(expf(ws_decay[(at * H + h) * dk + c]), S, local);
+  const size_t step = (size_t)H * dk * dv, step_d = (size_t)H * dk;
+  float* w = ws + ((size_t)b * max_chunks * H + h) * dk * dv + e;
+  const float* wd = ws_decay + ((size_t)b * max_chunks * H + h) * dk + c;
+  // the next chunks' states and decays are asked for before the ones in hand are walked
+  float local[GLA_AHEAD], decay[GLA_AHEAD];
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int a = 0; a < GLA_AHEAD; a++) {
+      const int j = min(j0 + a, chunks - 1);
+      local[a] = w[j * step];
+      decay[a] = wd[j * step_d];
+    }
+  };
+  fetch(0);
+  for (int j0 = 0; j0 < chunks; j0 += GLA_AHEAD) {
+    float L[GLA_AHEAD], D[GLA_AHEAD];
+#pragma unroll
+    for (int a = 0; a < GLA_AHEAD; a++) { L[a] = local[a]; D[a] = expf(decay[a]); }
+    if (j0 + GLA_AHEAD < chunks) fetch(j0 + GLA_AHEAD);
+#pragma unroll
+    for (int a = 0; a < GLA_AHEAD; a++) {
+      if (j0 + a >= chunks) break;
+      w[(j0 + a) * step] = S;
+      S = fmaf(D[a], S, L[a]);
+    }
   }
   *sp = S;
 }
@@ -295,35 +351,22 @@ extern "C" int pico_gla_scan(const void* x, int ldx, int dtype, int q_col, int k
                               (long long)max_chunks * chunk >= T && (long long)num_seqs * max_chunks < (1ll << 31)),
                "pico_gla_scan: chunks need room for their states and must cover the step's tokens");
   if (num_seqs == 0 || T == 0) return 0;
-  const int nw = (dk + GLA_CPT - 1) / GLA_CPT;
-  // tokens of a block: 16 where the staged values fit (up to 128 key channels), else 8
-  const int tb = nw <= 4 ? 16 : 8;
-  // value channels a lane: one.  (Two, where a head has more than 64, halve what is read out of LDS for the same
-  // arithmetic, but a wave then takes nearly twice as long and half as many fill the chip: 136 against 100 us for the
-  // chunks of a 2,048-token prompt with 12 heads of 64 x 128.)
-  const int vpl = 1;
-  const size_t lds = (size_t)(3 * tb * nw * GLA_CPT + tb * nw * 64 * vpl) * sizeof(float);
-  PICO_REQUIRE(lds <= 64 * 1024, "pico_gla_scan: key channels beyond the staging memory");
-  const int vb = (dv + 64 * vpl - 1) / (64 * vpl);
+  const int wide = dv % 4 == 0 && ((uintptr_t)state | (uintptr_t)ws) % 16 == 0, vb = (dv + 63) / 64;
 #define GLA_ARGS(TT)                                                                                                       \
   (const TT*)x, ldx, q_col, k_col, v_col, log_decay, cu_seqlens, state_slots, state, out, H, dk, dv, qscale, num_slots,   \
-      chunk, max_chunks, ws, ws_decay, (const TT*)a2, a2_bias, a_col, R, 1.0f / (tau > 0.f ? tau : 1.f), head_decay, silu
+      chunk, max_chunks, ws, ws_decay, (const TT*)a2, a2_bias, a_col, R, 1.0f / (tau > 0.f ? tau : 1.f), head_decay, silu, wide
+#define GLA_WAVES(TT, MODE, GX, FUSED)                                                                                     \
+  do {                                                                                                                     \
+    if (dk <= 32) gla_scan_kernel<TT, MODE, 1, FUSED><<<dim3(GX, H, vb), 64, 0, stream>>>(GLA_ARGS(TT));                   \
+    else if (dk <= 64) gla_scan_kernel<TT, MODE, 2, FUSED><<<dim3(GX, H, vb), 128, 0, stream>>>(GLA_ARGS(TT));             \
+    else if (dk <= 128) gla_scan_kernel<TT, MODE, 4, FUSED><<<dim3(GX, H, vb), 256, 0, stream>>>(GLA_ARGS(TT));            \
+    else gla_scan_kernel<TT, MODE, 8, FUSED><<<dim3(GX, H, vb), 512, 0, stream>>>(GLA_ARGS(TT));                           \
+  } while (0)
 #define GLA_LAUNCH(TT, MODE, GX)                                                                                           \
   do {                                                                                                                     \
-    constexpr bool fused = MODE == GLA_WHOLE;     /* with FUSED the launch below is taken only when log_decay is null */ \
-    if (log_decay == nullptr && head_decay == nullptr && fused) {                                                                                   \
-      if (tb == 16)                                                                                                        \
-        gla_scan_kernel<TT, MODE, 16, 1, fused><<<dim3(GX, H, vb), 64 * nw, lds, stream>>>(GLA_ARGS(TT));                  \
-      else                                                                                                                 \
-        gla_scan_kernel<TT, MODE, 8, 1, fused><<<dim3(GX, H, vb), 64 * nw, lds, stream>>>(GLA_ARGS(TT));                   \
-    } else if (tb == 16 && vpl == 2)                                                                                       \
-      gla_scan_kernel<TT, MODE, 16, 2, false><<<dim3(GX, H, vb), 64 * nw, lds, stream>>>(GLA_ARGS(TT));                    \
-    else if (tb == 16)                                                                                                     \
-      gla_scan_kernel<TT, MODE, 16, 1, false><<<dim3(GX, H, vb), 64 * nw, lds, stream>>>(GLA_ARGS(TT));                    \
-    else if (vpl == 2)                                                                                                     \
-      gla_scan_kernel<TT, MODE, 8, 2, false><<<dim3(GX, H, vb), 64 * nw, lds, stream>>>(GLA_ARGS(TT));                     \
-    else                                                                                                                   \
-      gla_scan_kernel<TT, MODE, 8, 1, false><<<dim3(GX, H, vb), 64 * nw, lds, stream>>>(GLA_ARGS(TT));                     \
+    constexpr bool whole = MODE == GLA_WHOLE;                                                                              \
+    if (log_decay == nullptr && head_decay == nullptr && whole) GLA_WAVES(TT, MODE, GX, whole);                            \
+    else GLA_WAVES(TT, MODE, GX, false);                                                                                   \
   } while (0)
 #define GLA_RUN(TT)                                                                                                        \
   if (chunk == 0) {                                                                                                        \
@@ -344,6 +387,7 @@ extern "C" int pico_gla_scan(const void* x, int ldx, int dtype, int q_col, int k
   }
 #undef GLA_RUN
 #undef GLA_LAUNCH
+#undef GLA_WAVES
 #undef GLA_ARGS
   PICO_LAUNCH_CHECK();
   return 0;

@@ -325,7 +325,7 @@ def test_one_key_that_stands_out_at_every_edge(dtype, Pg):
 # ---------------------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,dk,dv,rank,tau", [(2, 24, 40, 5, 4.0), (4, 64, 64, 12, 12.0), (1, 80, 100, 3, 1.0), (3, 16, 8, 2, 30.0),
-                                              (2, 256, 72, 8, 8.0)])
+                                              (2, 256, 72, 8, 8.0), (2, 33, 67, 3, 2.0), (1, 7, 3, 2, 5.0)])
 def test_gla_kernels_in_portions_and_token_by_token(dtype, H, dk, dv, rank, tau):
     from pico_vllm_amd.ops import kernels as K
     dt = DT[dtype]
@@ -421,6 +421,24 @@ def test_gla_kernels_in_portions_and_token_by_token(dtype, H, dk, dv, rank, tau)
     ref = (P.rms_norm(torch.cat(outs).double().view(T, H, dv), w.double(), eps).reshape(T, H * dv) * P.silu(gate))
     assert torch.allclose(out.cpu().double(), ref, rtol=1e-5 if dtype == "float32" else 1e-2, atol=1e-5 if dtype == "float32" else 1e-2)
     assert torch.allclose(ref, want_out, rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,C,R", [(64, 256, 32), (71, 300, 5), (65, 1, 16), (130, 257, 1024), (64, 3, 1025)])
+def test_decays_of_many_tokens_are_those_of_one_at_a_time(dtype, T, C, R):
+    """Blocks of tokens, rows of a2 in sixteens of bytes or entry by entry: the same sums in the same order, so the same bits."""
+    from pico_vllm_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(T * C)
+    x = torch.randn(T, R + 3, generator=g).to(DEV, DT[dtype])
+    a2 = (8 * R ** -0.5 * torch.randn(C, R, generator=g)).to(DEV, DT[dtype])
+    b = torch.randn(C, generator=g).to(DEV)
+    got = K.gla_decay(x, 3, a2, b, 4.0)
+    assert torch.equal(got, torch.cat([K.gla_decay(x[t:t + 1], 3, a2, b, 4.0) for t in range(T)]))
+    z = x[:, 3:].double().cpu() @ a2.double().cpu().T + b.double().cpu()
+    want = torch.nn.functional.logsigmoid(z) / 4.0
+    # R float32 sums of terms of up to |x| |a2|, then two functions good to a few roundings
+    bound = 2.0 ** -24 * (R * (x[:, 3:].double().cpu().abs() @ a2.double().cpu().abs().T) + 8 * (want.abs() + 1))
+    assert bool(((got.double().cpu() - want).abs() <= bound).all())
 
 
 def test_a_decay_near_one_keeps_a_far_token_in_the_state():
