@@ -21,6 +21,7 @@ struct GemmArgs {
   int M, cols, K, ldx, ldw, ldo;     // cols: output columns of this launch
   int up;                            // paired epilogues: from a gate row of W to the up row of the same column
   int m_tiles, n_tiles;
+  int splits, part;                  // of K: so many parts of `part` each, a part's sums in out + s M ldo (GT_F32; else one)
   float limit, alpha;
 };
 
@@ -66,18 +67,20 @@ template <int MB, int NB, int EPI, int SETS>
 __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const GemmArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  typedef TileStream<MB, NB, SETS> TS;
+  typedef TileStream<MB, NB, SETS, EPI == GT_F32> TS;
   TS ts(smem);
   constexpr int TM = 64 * MB, TN = 64 * NB, COLS = gt_paired(EPI) ? TN / 2 : TN;      // output columns of a tile
-  const int tiles = a.m_tiles * a.n_tiles;
+  const int tiles = a.m_tiles * a.n_tiles * (EPI == GT_F32 ? a.splits : 1);
   if (ts_tile(0, tiles) < 0) return;
   TileRowsSource<MB> xs;
   TileRowsSource<NB> ws;
   auto aim = [&](int t) {
     int m, n;
-    ts_place(a.m_tiles, a.n_tiles, t, m, n);
-    const int m0 = m * TM;
-    xs.rsrc = ts_buffer(a.X + (size_t)m0 * a.ldx, ((long long)(a.M - m0 - 1) * a.ldx + a.K) * 2);
+    ts_place(a.m_tiles, a.n_tiles * (EPI == GT_F32 ? a.splits : 1), t, m, n);
+    const int m0 = m * TM, s = EPI == GT_F32 ? n / a.n_tiles : 0, k0 = s * a.part, k = EPI == GT_F32 ? min(a.part, a.K - k0) : a.K;
+    n -= s * a.n_tiles;
+    if (EPI == GT_F32) ts.k_end = k;
+    xs.rsrc = ts_buffer(a.X + (size_t)m0 * a.ldx + k0, ((long long)(a.M - m0 - 1) * a.ldx + k) * 2);
 #pragma unroll
     for (int j = 0; j < 2 * MB; j++) xs.off[j] = (uint32_t)(ts.row(j) * a.ldx) * 2;
     if (gt_paired(EPI)) {
@@ -91,15 +94,17 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
       }
     } else {
       const int n0 = n * TN;
-      ws.rsrc = ts_buffer(a.W + (size_t)n0 * a.ldw, ((long long)(a.cols - n0 - 1) * a.ldw + a.K) * 2);
+      ws.rsrc = ts_buffer(a.W + (size_t)n0 * a.ldw + k0, ((long long)(a.cols - n0 - 1) * a.ldw + k) * 2);
 #pragma unroll
       for (int j = 0; j < 2 * NB; j++) ws.off[j] = (uint32_t)(ts.row(j) * a.ldw) * 2;
     }
   };
-  ts.run(tiles, a.K, xs, ws, aim, [&](int t) {
+  ts.run(tiles, EPI == GT_F32 ? a.part : a.K, xs, ws, aim, [&](int t) {
     // lane (l, h): row l of a block of X, tile rows 8 (r / 4) + 4 h + r % 4 of a block of W in register r
     int mt, nt;
-    ts_place(a.m_tiles, a.n_tiles, t, mt, nt);
+    ts_place(a.m_tiles, a.n_tiles * (EPI == GT_F32 ? a.splits : 1), t, mt, nt);
+    const int split = EPI == GT_F32 ? nt / a.n_tiles : 0;
+    nt -= split * a.n_tiles;
     const int l = ts.lane & 31, h = ts.lane >> 5;
     // of the bias what this lane adds, all of it asked for at once (a pair at a time between the outputs it was waited for each
     // time: 32 us of a call of 2,048 rows, 13,440 columns).  Not with float32 results, which do
@@ -132,7 +137,7 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
         }
         const int blk = (ts.wave & 1) * NB + j;
         if (EPI == GT_F32) {
-          float* o = (float*)a.out + (size_t)m * a.ldo;
+          float* o = (float*)a.out + ((size_t)split * a.M + m) * a.ldo;
 #pragma unroll
           for (int q = 0; q < 4; q++) {
             const int n = nt * TN + blk * 32 + 8 * q + 4 * h;
@@ -182,7 +187,7 @@ static int gt_launch(GemmArgs a, hipStream_t stream) {
   PICO_REQUIRE(room == hipSuccess, "pico_gemm_tiles: %s", hipGetErrorString(room));
   a.m_tiles = (a.M + 64 * MB - 1) / (64 * MB);
   a.n_tiles = (a.cols + GT_COLS(NB, EPI) - 1) / GT_COLS(NB, EPI);
-  const long long tiles = (long long)a.m_tiles * a.n_tiles;
+  const long long tiles = (long long)a.m_tiles * a.n_tiles * a.splits;
   PICO_REQUIRE(tiles < (1LL << 30), "pico_gemm_tiles: %d x %d outputs are too many for one launch", a.M, a.cols);
   gemm_tiles_kernel<MB, NB, EPI, SETS><<<ts_grid(tiles, 256 * ts_share(MB, NB)), 256, ts_lds_bytes(MB, NB), stream>>>(a);
   PICO_LAUNCH_CHECK();
@@ -199,13 +204,13 @@ static const GtTile gt_tiles[] = {{2, 3, 2, 1.45f, 1.20f, 3.f}, {4, 2, 1, 0.84f,
 // The tile for M rows and `cols` columns and its cost.  `first`: how many columns to make in whole rounds with it, the
 // others being better left to a launch of their own with the tile that suits them (2,052 rows of 8,960 pairs: three rounds
 // and 62 tiles; the 62 as a fourth round cost 32 us, as 170 tiles of a third their size 12); else all.
-static int gt_choose(int M, int cols, int stages, bool paired, bool split, int& first, float& cost) {
+static int gt_choose(int M, int cols, int stages, bool paired, bool split, int& first, float& cost, int parts = 1) {
   int best = 0;
   cost = 3e38f;
   for (int i = 0; i < 4; i++) {
     const GtTile& t = gt_tiles[i];
     const int tile_cols = GT_COLS(t.nb, paired ? GT_SWIGLU : GT_BF16), m_tiles = (M + 64 * t.mb - 1) / (64 * t.mb);
-    const long long tiles = (long long)m_tiles * ((cols + tile_cols - 1) / tile_cols), round = 256 * t.share, full = tiles / round, rest = tiles % round;
+    const long long tiles = (long long)m_tiles * ((cols + tile_cols - 1) / tile_cols) * parts, round = 256 * t.share, full = tiles / round, rest = tiles % round;
     const float whole = (float)full * (t.each * stages + t.more);
     const float c = whole + (rest ? (rest <= 256 ? t.lone : t.each) * stages + t.more : 0.f);
     if (c < cost) { cost = c; best = i; first = cols; }
@@ -222,10 +227,10 @@ static int gt_choose(int M, int cols, int stages, bool paired, bool split, int& 
 
 template <int EPI>
 static int gt_run(GemmArgs a, hipStream_t stream) {
-  const int stages = (a.K + TS_BK - 1) / TS_BK, cols = a.cols;
+  const int stages = (a.part + TS_BK - 1) / TS_BK, cols = a.cols;
   int first, all, rc = 0;
   float cost;
-  const int tile = gt_choose(a.M, cols, stages, gt_paired(EPI), true, first, cost);
+  const int tile = gt_choose(a.M, cols, stages, gt_paired(EPI), a.splits == 1, first, cost, a.splits);
   auto run = [&](int i) {
     switch (i) {
       case 0: return gt_launch<2, 3, EPI>(a, stream);
@@ -269,7 +274,7 @@ extern "C" int pico_gemm_tiles(const void* X, const void* W, const float* bias, 
   PICO_REQUIRE((long long)M * ldx < (1LL << 30) && (long long)N * ldw < (1LL << 30), "pico_gemm_tiles: an operand spans 2^31 bytes or more");
   PICO_REQUIRE(!bias || !gt_paired(epi), "pico_gemm_tiles: the paired epilogues take no bias");
   if (M == 0) return 0;
-  GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, bias, out, M, cols, K, ldx, ldw, ldo, N - cols, 0, 0, limit, alpha};
+  GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, bias, out, M, cols, K, ldx, ldw, ldo, N - cols, 0, 0, 1, K, limit, alpha};
   if (few) {
     PICO_REQUIRE(M <= 64, "pico_gemm_tiles: %d rows are not few", M);
     switch (epi) {
@@ -288,4 +293,65 @@ extern "C" int pico_gemm_tiles(const void* X, const void* W, const float* bias, 
     case GT_GELU: return gt_run<GT_GELU>(a, stream);
   }
   PICO_REQUIRE(false, "pico_gemm_tiles: unknown epilogue %d", epi);
+}
+
+// A long K with few tiles: K in parts that run side by side, each into float32 rows of its own, and one pass that adds a row's
+// parts up in their order and rounds once.  832 rows of 3,584 outputs, K 18,944: two parts 125 us (0.90 PFLOP/s), whole
+// 215 with 112 to 392 tiles on 256 compute units, the library's product 175.
+// The pass, eight neighbours a thread, is bound by memory.
+__global__ __launch_bounds__(256) void gemm_join_kernel(const float* __restrict__ parts, int splits, const float* __restrict__ bias,
+                                                        bf16_t* __restrict__ out, long long eights, int N) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= eights) return;
+  const gt_f32x4* p = reinterpret_cast<const gt_f32x4*>(parts) + 2 * i;
+  gt_f32x4 lo = p[0], hi = p[1];
+  for (int s = 1; s < splits; s++) {
+    lo += p[2 * s * eights];
+    hi += p[2 * s * eights + 1];
+  }
+  if (bias) {
+    const gt_f32x4* b = reinterpret_cast<const gt_f32x4*>(bias + 8 * i % N);
+    lo += b[0];
+    hi += b[1];
+  }
+  reinterpret_cast<uint4*>(out)[i] = make_uint4(pack2_bf16(lo[0], lo[1]), pack2_bf16(lo[2], lo[3]), pack2_bf16(hi[0], hi[1]), pack2_bf16(hi[2], hi[3]));
+}
+
+#define GT_SPLITS 8
+static int gt_part(int K, int splits) { return ((K + splits - 1) / splits + TS_BK - 1) / TS_BK * TS_BK; }
+
+// Into how many parts: by the tiles' cost (gt_choose) and the pass's, which moves 4 bytes a part and output and 2 at 4.5 TB/s.
+// 1: whole, without a pass.
+extern "C" int pico_gemm_tiles_parts(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 1;
+  int best = 1, first;
+  float least = 3e38f;
+  for (int s = 1; s <= GT_SPLITS; s++) {
+    const int part = gt_part(K, s);
+    if (s > 1 && (long long)(s - 1) * part >= K) break;
+    float cost;
+    gt_choose(M, N, part / TS_BK, false, s == 1, first, cost, s);
+    if (s > 1) cost += 3.f + (float)M * N * (4 * s + 2) / 4.5e6f;
+    if (cost < least) { least = cost; best = s; }
+  }
+  return best;
+}
+
+// out [M, N] bfloat16 = X W^T + bias with K in `splits` parts; parts float32 [splits, M, N].  Operands as pico_gemm_tiles.
+extern "C" int pico_gemm_tiles_split(const void* X, const void* W, const float* bias, float* parts, void* out, int splits, int M, int N,
+                                     int K, int ldx, int ldw, hipStream_t stream) {
+  PICO_REQUIRE(M >= 0 && N > 0 && K > 0, "pico_gemm_tiles_split: bad sizes M=%d N=%d K=%d", M, N, K);
+  PICO_REQUIRE(splits > 1 && splits <= GT_SPLITS && (long long)(splits - 1) * gt_part(K, splits) < K, "pico_gemm_tiles_split: %d parts of %d", splits, K);
+  PICO_REQUIRE(ldx >= K && ldw >= K && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && N % 8 == 0,
+               "pico_gemm_tiles_split: sizes and strides must be multiples of 8");
+  PICO_REQUIRE(((uintptr_t)X | (uintptr_t)W | (uintptr_t)out | (uintptr_t)parts | (uintptr_t)bias) % 16 == 0, "pico_gemm_tiles_split: operands must start on 16 bytes");
+  PICO_REQUIRE((long long)M * ldx < (1LL << 30) && (long long)N * ldw < (1LL << 30), "pico_gemm_tiles_split: an operand spans 2^31 bytes or more");
+  if (M == 0) return 0;
+  GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, nullptr, parts, M, N, K, ldx, ldw, N, 0, 0, 0, splits, gt_part(K, splits), 0.f, 0.f};
+  const int rc = gt_run<GT_F32>(a, stream);
+  if (rc) return rc;
+  const long long eights = (long long)M * N / 8;
+  gemm_join_kernel<<<(unsigned)((eights + 255) / 256), 256, 0, stream>>>(parts, splits, bias, (bf16_t*)out, eights, N);
+  PICO_LAUNCH_CHECK();
+  return 0;
 }

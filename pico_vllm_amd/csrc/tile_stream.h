@@ -66,11 +66,13 @@ __device__ __forceinline__ int ts_tile(int r, int tiles) {
 
 template <int FROM, int TO> struct Range { static constexpr int from = FROM, to = TO; };
 
-template <int MB, int NB, int SETS = 1>
+// ENDS: tiles end at a k of their own (k_end).
+template <int MB, int NB, int SETS = 1, bool ENDS = false>
 struct TileStream {
   static constexpr int NBUF = ts_buffers(MB, NB), STAGE = ts_stage_bytes(MB, NB), LOADS = 2 * (MB + NB);
   char* lds;
   int wave, lane;
+  int k_end;                            // ENDS: k from here on is asked for as zeros, set by `aim` (at most `run`'s K)
   uint32_t kbyte;                       // the byte of this lane's chunk within a row's 128 bytes
   const char *xrd, *wrd;                // this wave's operand rows in buffer 0
   int sw[4];                            // where lane (row l, half h) finds the chunk of quarter ks
@@ -202,7 +204,7 @@ struct TileStream {
   __device__ __forceinline__ void run(int tiles, int K, const TileRowsSource<MB>& xs, const TileRowsSource<NB>& ws, Aim aim, Done done) {
     const int stages = (K + TS_BK - 1) / TS_BK;
     int at_round = 0, at_tile = ts_tile(0, tiles), at_stage = 0, fill = 0;      // the stage that is asked for next, into buffer `fill`
-    auto copies = [&](auto r) { ask<decltype(r)::from, decltype(r)::to>(fill, xs, ws, at_tile >= 0 ? at_stage * TS_BK : K, K); };
+    auto copies = [&](auto r) { ask<decltype(r)::from, decltype(r)::to>(fill, xs, ws, at_tile >= 0 ? at_stage * TS_BK : K, ENDS ? k_end : K); };
     auto on = [&] {
       fill = fill + 1 == NBUF ? 0 : fill + 1;
       if (++at_stage == stages && at_tile >= 0) {

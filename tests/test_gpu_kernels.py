@@ -1735,3 +1735,31 @@ def test_scaled_add(K, T, H, slabs, gated, scaled, b_dtype):
                      None if gate is None else gate.to(DEV), None if scale is None else scale.to(DEV))
         # eight float32 roundings at most, of parts of `size`
         assert bool(((resid.cpu().double() - want).abs() <= 8 * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("M,N,K_,parts", [(65, 16, 200, 2), (1, 16, 520, 5), (64, 80, 128, 2), (129, 208, 1000, 4), (300, 1552, 8960, 8), (257, 3584, 18944, 3)])
+def test_products_in_parts_of_the_inner_size(K, M, N, K_, parts):
+    """Parts of whole 64, the last one shorter and in remainders of 8; rows in a wider matrix; with a bias and without."""
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K_ + 8, generator=g).bfloat16().to(DEV)[:, :K_]
+    w = torch.randn(N, K_, generator=g).bfloat16().to(DEV)
+    b = torch.randn(N, generator=g).to(DEV)
+    xd, wd = x.double().cpu(), w.double().cpu()
+    size = xd.abs() @ wd.abs().T
+    for bias in (b, None):
+        got = K.gemm_tiles_split(x, w, bias, parts).double().cpu()
+        want = xd @ wd.T + (0 if bias is None else bias.double().cpu())
+        # one rounding to bfloat16, and float32 sums of K terms
+        assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + K_ * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("M,N,K_", [(65, 1536, 8960), (1000, 3584, 18944), (1536, 16, 6656)])
+def test_the_layer_takes_a_long_inner_size_in_parts(K, M, N, K_):
+    from pico_vllm_amd.ops.linear import Linear
+    g = torch.Generator().manual_seed(N)
+    x, w = torch.randn(M, K_, generator=g).bfloat16().to(DEV), torch.randn(N, K_, generator=g).bfloat16().to(DEV)
+    b = torch.randn(N, generator=g).bfloat16().to(DEV)
+    parts = K.tiles_parts(x, w)
+    assert parts > 1
+    assert torch.equal(Linear(w, b)(x), K.gemm_tiles_split(x, w, b.float(), parts))
+    assert K.tiles_parts(x[:, :K_ - 4], w[:, :K_ - 4]) == 1 and K.tiles_parts(x[:, :6144], w[:, :6144]) == 1
