@@ -375,3 +375,11 @@ def test_a_description_that_does_not_hold_together_is_refused_when_the_model_is_
         lin(torch.zeros(2, 6, dtype=torch.bfloat16))
     with pytest.raises(ValueError, match="bfloat16 weights need bfloat16 activations"):
         lin(torch.zeros(2, 8))
+
+
+def test_a_long_inner_size_on_host_tensors_goes_to_the_library():
+    import torch
+    from pico_vllm_amd.ops.linear import Linear
+    g = torch.Generator().manual_seed(1)
+    w, x = torch.randn(32, 6656, generator=g).bfloat16(), torch.randn(300, 6656, generator=g).bfloat16()
+    assert torch.equal(Linear(w)(x), torch.mm(x, w.t()))
