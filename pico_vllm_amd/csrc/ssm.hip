@@ -465,8 +465,8 @@ __global__ __launch_bounds__(256) void ssm_combine_kernel(const int* __restrict_
 
 // chunk == 0: every sequence walked whole from its slot.  chunk > 0: sequences cut into chunks of that many tokens that
 // run side by side (three launches); ws float32 [num_seqs * max_chunks, C, N], ws_dt [num_seqs * max_chunks, C],
-// max_chunks at least the chunks of the longest sequence; dt_ws [T, C] (may be null: then the general kernels serve; with it, 16
-// state elements and bfloat16, ws and ws_dt hold T / chunk + num_seqs chunks).
+// max_chunks at least the chunks of the longest sequence.  dt_ws [T, C] chooses the passes for 16 state elements and bfloat16, for
+// which ws and ws_dt hold T / chunk + num_seqs chunks, numbered through; null: the general kernels.
 extern "C" int pico_selective_scan(const void* xc, const float* dtp, const float* dt_bias, const void* bc, int ldbc, int b_col,
                                    int c_col, const float* A_log, const float* D, const void* z, int ldz, int dtype,
                                    const int* cu_seqlens, const int* state_slots, float* state, int num_slots, int B, int T,
@@ -487,7 +487,10 @@ extern "C" int pico_selective_scan(const void* xc, const float* dtp, const float
   const int per = 256 / lpc;
   const int gy = (C + per - 1) / per;
   PICO_REQUIRE(gy <= 65535 && ((long long)C * N + 255) / 256 <= 65535, "pico_selective_scan: too many channels");
-  if (dtype == PICO_DTYPE_BF16 && chunk > 0 && N == 16 && dt_ws != nullptr && chunk <= 256 && (uintptr_t)A_log % 16 == 0 && (uintptr_t)ws % 16 == 0) {
+  if (dt_ws != nullptr) {
+    // (no way back to the general kernels: they number the chunks otherwise, and need room for more of them)
+    PICO_REQUIRE(dtype == PICO_DTYPE_BF16 && N == 16 && chunk > 0 && chunk <= 256 && ((uintptr_t)A_log | (uintptr_t)ws) % 16 == 0,
+                 "pico_selective_scan: chunks numbered through want 16 state elements, bfloat16, chunks of up to 256 tokens and aligned A_log and ws");
     const dim3 grid(T / chunk + B, (C + 255) / 256);
 #define SSM_16 (const bf16_t*)xc, dtp, dt_bias, (const bf16_t*)bc, ldbc, b_col, c_col, A_log, D, (const bf16_t*)z, ldz, cu_seqlens, \
                state_slots, num_slots, C, (bf16_t*)out, chunk, B, ws, ws_dt, dt_ws

@@ -305,6 +305,29 @@ def test_recurrence_in_chunks_numbered_through(C, lens, chunk):
     assert torch.equal(state[-1].cpu(), start[-1])
 
 
+def test_recurrence_in_chunks_with_decays_that_start_anywhere():
+    """16 state elements a channel whose logarithms begin one float into a buffer, several sequences: the same numbers as from an aligned
+    start (the passes that read them in fours are not taken, and the workspace is the other passes')."""
+    from pico_vllm_amd.ops import kernels
+    lens, C, N, R, chunk = [1800, 3, 40], 40, 16, 6, 35
+    g = torch.Generator().manual_seed(1)
+    mk = lambda *s: torch.randn(*s, generator=g)
+    T = sum(lens)
+    u, z, dbc, dtp = (t.to(DEV) for t in (mk(T, C).bfloat16(), mk(T, C).bfloat16(), mk(T, R + 2 * N).bfloat16(), 0.5 * mk(T, C) - 1))
+    a_log = torch.log(0.5 + 4 * torch.rand(C, N, generator=g)).to(DEV)
+    odd = torch.empty(C * N + 1, device=DEV)[1:].view(C, N)
+    odd.copy_(a_log)
+    D, dtb, start = (1 + 0.3 * mk(C)).to(DEV), (0.1 * mk(C)).to(DEV), mk(len(lens) + 1, C, N + 3).to(DEV)
+    ctx = step_ctx(lens, [0] * len(lens), list(range(len(lens))))
+    out = []
+    for a in (a_log, odd):
+        state = start.clone()
+        out.append((kernels.selective_scan(u, dtp, dtb, dbc, R, R + N, a, D, z, ctx, state, 3, chunk=chunk), state))
+    close(out[1][0], out[0][0].cpu().double(), "bfloat16")
+    assert (out[1][1] - out[0][1]).abs().max() <= 8e-6 * max(1.0, float(start.abs().max()))
+    assert torch.equal(out[1][1][-1], start[-1])
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,dk,dv,decay", [(2, 24, 40, (0.9, 0.996)), (4, 64, 64, (0.97, 0.99, 0.999, 1.0)), (3, 16, 8, (0.5, 0.9375, 0.99)), (1, 80, 100, (0.999,))])
 def test_retention_recurrence_with_fixed_decays(dtype, H, dk, dv, decay):
