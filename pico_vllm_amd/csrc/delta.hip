@@ -140,23 +140,17 @@ extern "C" int pico_ssd_prep(const void* bc, int ldb, int b_col, int c_col, int 
 #define DS_LOCAL 1
 #define DS_FROM 2
 
-// FOUR: four lanes a column and four waves (key sizes of 33 to 128, 64 and more columns).  What a thread stages of the next block
-// is asked for before this block's tokens are walked, a token's k, g and q are read from LDS under the token before, and the
-// sums over key channels meet by lane swaps instead of through the LDS crossbar: a token is a chain, and with one or two waves
-// a SIMD nothing else hides its waits.  The two passes over 2,052 tokens, 12 heads of 64 keys and 128 values: 60 and 51 us, 71
-// and 93 without all that; the same bits.
-template <typename TV, int KPL, int VPL, bool DELTA, int MODE, bool FOUR = false>
+template <typename TV, int KPL, int VPL, bool DELTA, int MODE>
 __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                          const TV* __restrict__ v, int ldv, const float* __restrict__ g,
                                                          int g_channels, const float* __restrict__ beta,
                                                          const int* __restrict__ cu_seqlens, const int* __restrict__ state_slots,
                                                          float* __restrict__ state, float* __restrict__ out, int H, int KVH,
-                                                         int dk, int dv, int ks_lanes, int tb, int num_slots, int chunk,
+                                                         int dk, int dv, int KS, int TB, int num_slots, int chunk,
                                                          int max_chunks, float* __restrict__ ws_S, float* __restrict__ ws_P) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];
+  extern __shared__ float lds[];
   const int b = MODE == DS_WHOLE ? blockIdx.x : blockIdx.x / max_chunks, h = blockIdx.y;
-  const int KS = FOUR ? 4 : ks_lanes, TB = FOUR ? 16 : tb;
-  const int nw = FOUR ? 4 : blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int nw = blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int VC = 64 / KS, vc = lane % VC, ks = lane / VC;
   const int DKP = KS * KPL;                            // key channels with padding
   const int tile = nw * VC * VPL;                      // columns of the workgroup
@@ -201,7 +195,166 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
   float gprod[KPL];                                    // DS_LOCAL without the delta rule: the chunk's decays multiplied up
 #pragma unroll
   for (int i = 0; i < KPL; i++) gprod[i] = 1.f;
-  // a thread's share of a block's staged values, of which FOUR keeps the next block's in registers
+  for (int t0 = t_begin; t0 < t_end; t0 += TB) {
+    const int nb = min(TB, t_end - t0);
+    __syncthreads();                                   // the last block's staged values have been read
+    for (int idx = threadIdx.x; idx < nb * DKP; idx += blockDim.x) {      // only the block's tokens: a single token is one turn
+      const int tt = idx / DKP, c = idx % DKP;
+      const int t = t0 + min(tt, nb - 1), cc = min(c, dk - 1);
+      const bool in = tt < nb && c < dk;
+      const float kx = k[((size_t)t * KVH + kvh) * dk + cc];
+      const float qx = MODE == DS_LOCAL ? 0.f : q[((size_t)t * KVH + kvh) * dk + cc];
+      const float gx = g_channels ? g[((size_t)t * H + h) * dk + cc] : g[(size_t)t * H + h];
+      ks_[idx] = in ? kx : 0.f;
+      qs_[idx] = in ? qx : 0.f;
+      gs_[idx] = in ? gx : 1.f;
+    }
+    for (int idx = threadIdx.x; idx < nb * tile; idx += blockDim.x) {
+      const int tt = idx / tile, col = col0 + idx % tile;
+      const float x = load_f32(v + (size_t)(t0 + min(tt, nb - 1)) * ldv + (size_t)h * dv + min(col, dv - 1));
+      vs_[idx] = (tt < nb && col < dv) ? x : 0.f;       // the unit vectors' columns have values of zero
+    }
+    if ((int)threadIdx.x < TB) bs_[threadIdx.x] = beta[(size_t)(t0 + min((int)threadIdx.x, nb - 1)) * H + h];
+    __syncthreads();
+    for (int tt = 0; tt < nb; tt++) {
+      const float4* k4 = reinterpret_cast<const float4*>(ks_ + tt * DKP + c0);
+      const float4* g4 = reinterpret_cast<const float4*>(gs_ + tt * DKP + c0);
+      const float4* q4 = reinterpret_cast<const float4*>(qs_ + tt * DKP + c0);
+      const float bt = bs_[tt];
+      float kc[KPL], u[VPL];
+#pragma unroll
+      for (int j = 0; j < VPL; j++) u[j] = 0.f;
+#pragma unroll
+      for (int i = 0; i < KPL / 4; i++) {
+        const float4 kv = k4[i], gv = g4[i];
+        kc[4 * i] = kv.x; kc[4 * i + 1] = kv.y; kc[4 * i + 2] = kv.z; kc[4 * i + 3] = kv.w;
+        if (MODE == DS_LOCAL && !DELTA) { gprod[4 * i] *= gv.x; gprod[4 * i + 1] *= gv.y; gprod[4 * i + 2] *= gv.z; gprod[4 * i + 3] *= gv.w; }
+#pragma unroll
+        for (int j = 0; j < VPL; j++) {
+          S[j][4 * i] *= gv.x; S[j][4 * i + 1] *= gv.y; S[j][4 * i + 2] *= gv.z; S[j][4 * i + 3] *= gv.w;
+          if (DELTA) {
+            u[j] = fmaf(S[j][4 * i], kv.x, u[j]); u[j] = fmaf(S[j][4 * i + 1], kv.y, u[j]);
+            u[j] = fmaf(S[j][4 * i + 2], kv.z, u[j]); u[j] = fmaf(S[j][4 * i + 3], kv.w, u[j]);
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < VPL; j++) {
+        const float vt = vs_[tt * tile + lcol0 + j * VC];
+        if (DELTA) {
+          float sk = u[j];
+          for (int o = VC; o < 64; o <<= 1) sk += __shfl_xor(sk, o);
+          u[j] = bt * (vt - sk);
+        } else {
+          u[j] = bt * vt;
+        }
+      }
+      if (MODE == DS_LOCAL) {
+#pragma unroll
+        for (int j = 0; j < VPL; j++)
+#pragma unroll
+          for (int i = 0; i < KPL; i++) S[j][i] = fmaf(kc[i], u[j], S[j][i]);
+        continue;
+      }
+      float so[VPL];
+#pragma unroll
+      for (int j = 0; j < VPL; j++) so[j] = 0.f;
+#pragma unroll
+      for (int i = 0; i < KPL / 4; i++) {
+        const float4 qv = q4[i];
+#pragma unroll
+        for (int j = 0; j < VPL; j++) {
+          S[j][4 * i] = fmaf(kc[4 * i], u[j], S[j][4 * i]); so[j] = fmaf(S[j][4 * i], qv.x, so[j]);
+          S[j][4 * i + 1] = fmaf(kc[4 * i + 1], u[j], S[j][4 * i + 1]); so[j] = fmaf(S[j][4 * i + 1], qv.y, so[j]);
+          S[j][4 * i + 2] = fmaf(kc[4 * i + 2], u[j], S[j][4 * i + 2]); so[j] = fmaf(S[j][4 * i + 2], qv.z, so[j]);
+          S[j][4 * i + 3] = fmaf(kc[4 * i + 3], u[j], S[j][4 * i + 3]); so[j] = fmaf(S[j][4 * i + 3], qv.w, so[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < VPL; j++) {
+        float x = so[j];
+        for (int o = VC; o < 64; o <<= 1) x += __shfl_xor(x, o);
+        const int col = col0 + lcol0 + j * VC;
+        if (ks == 0 && col < dv) out[((size_t)(t0 + tt) * H + h) * dv + col] = x;
+      }
+    }
+  }
+  if (MODE == DS_FROM) return;
+#pragma unroll
+  for (int j = 0; j < VPL; j++) {
+    const int col = col0 + lcol0 + j * VC;
+    if (col >= ncols) continue;
+    if (col >= dv) {                                   // DS_LOCAL with the delta rule: column col - dv of P
+      float* pp = ws_P + (((size_t)blockIdx.x * H + h) * dk) * dk + (col - dv);
+#pragma unroll
+      for (int i = 0; i < KPL; i++)
+        if (c0 + i < dk) pp[(size_t)(c0 + i) * dk] = S[j][i];
+      continue;
+    }
+#pragma unroll
+    for (int i = 0; i < KPL; i++)
+      if (c0 + i < dk) sbase[(size_t)(c0 + i) * dv + col] = S[j][i];
+    if (MODE == DS_LOCAL && !DELTA && col == 0) {
+#pragma unroll
+      for (int i = 0; i < KPL; i++)
+        if (c0 + i < dk) ws_P[((size_t)blockIdx.x * H + h) * dk + c0 + i] = gprod[i];
+    }
+  }
+}
+
+// The two passes over chunks with four lanes a column, two columns a lane and four waves (DS_LOCAL and DS_FROM of the kernel above; the
+// same bits).  What a thread stages of the next block is asked for before this block's tokens are walked, and the sums over
+// key channels meet by lane swaps instead of through the LDS crossbar: a token is a chain, and with one or two waves a SIMD nothing
+// else hides its waits.  AHEAD: also a token's k, g and q are read from LDS under the token before; with 32 key channels a lane the
+// registers for that leave one wave a SIMD.  Microseconds of a call of 128, 700 and 2,052 tokens, general kernel / this one, 12 heads:
+// 64 keys and 128 values 130 / 67, 154 / 86, 190 / 129 (plain decays 87 / 55, 93 / 62, 112 / 79); 128 and 128 177 / 110, 228 / 150, 371 /
+// 273 (with AHEAD 113, 180, 353; plain 123 / 83, 140 / 92, 160 / 117, with AHEAD 88, 98, 187); 32 and 128 130 / 71, 210 / 153, 420 / 355.
+template <typename TV, int KPL, bool DELTA, int MODE>
+__global__ __launch_bounds__(256) void delta_scan4_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                          const TV* __restrict__ v, int ldv, const float* __restrict__ g,
+                                                          int g_channels, const float* __restrict__ beta,
+                                                          const int* __restrict__ cu_seqlens, const int* __restrict__ state_slots,
+                                                          float* __restrict__ out, int H, int KVH, int dk, int dv, int num_slots, int chunk,
+                                                          int max_chunks, float* __restrict__ ws_S, float* __restrict__ ws_P) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int b = blockIdx.x / max_chunks, h = blockIdx.y;
+  constexpr int KS = 4, TB = 16, VPL = 2, NW = 4, VC = 64 / KS, DKP = KS * KPL, tile = NW * VC * VPL;
+  constexpr bool AHEAD = KPL <= 16;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, vc = lane % VC, ks = lane / VC;
+  float* ks_ = lds;                                    // [TB][DKP]
+  float* qs_ = ks_ + TB * DKP;
+  float* gs_ = qs_ + TB * DKP;
+  float* vs_ = gs_ + TB * DKP;                         // [TB][tile]
+  float* bs_ = vs_ + TB * tile;                        // [TB]
+  const int t_begin = cu_seqlens[b] + (blockIdx.x % max_chunks) * chunk, t_end = min(cu_seqlens[b + 1], t_begin + chunk);
+  const int slot = state_slots[b];
+  if (slot < 0 || slot >= num_slots || t_end <= t_begin) return;          // the whole workgroup
+  const int ncols = (MODE == DS_LOCAL && DELTA) ? dv + dk : dv;           // the unit vectors' columns behind the values'
+  const int col0 = blockIdx.z * tile, lcol0 = wave * VC * VPL + vc;       // the tile's first column; this lane's first in the tile
+  const int c0 = ks * KPL;
+  const int kvh = h / (H / KVH);
+  float* sbase = ws_S + (((size_t)blockIdx.x * H + h) * dk) * dv;
+  float S[VPL][KPL];
+  if (MODE != DS_LOCAL) {
+#pragma unroll
+    for (int j = 0; j < VPL; j++)
+#pragma unroll
+      for (int i = 0; i < KPL; i++)
+        S[j][i] = sbase[(size_t)min(c0 + i, dk - 1) * dv + min(col0 + lcol0 + j * VC, dv - 1)];
+  }
+#pragma unroll
+  for (int j = 0; j < VPL; j++) {
+    const int col = col0 + lcol0 + j * VC;
+#pragma unroll
+    for (int i = 0; i < KPL; i++) {
+      if (MODE == DS_LOCAL) S[j][i] = (col >= dv && col < ncols && c0 + i == col - dv) ? 1.f : 0.f;
+      else S[j][i] = (c0 + i < dk && col < dv) ? S[j][i] : 0.f;
+    }
+  }
+  float gprod[KPL];                                    // DS_LOCAL without the delta rule: the chunk's decays multiplied up
+#pragma unroll
+  for (int i = 0; i < KPL; i++) gprod[i] = 1.f;
+  // a thread's share of a block's staged values; the next block's travel in registers
   constexpr int NK = KPL / 4, NV = 4 * VPL;
   float nk[NK], nq[NK], ng[NK], nv[NV], nbeta = 0.f;
   auto fetch = [&](int t0) {
@@ -236,61 +389,41 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
     }
     if (threadIdx.x < 16) bs_[threadIdx.x] = nbeta;
   };
-  // the sum over the lanes that share a column, in a fixed tree
-  auto across = [&](float x) {
-    if (FOUR) return sum_across_32(sum_across_16(x));
-    for (int o = VC; o < 64; o <<= 1) x += __shfl_xor(x, o);
-    return x;
-  };
   const bool idle = col0 + wave * VC * VPL >= ncols;               // the same for all lanes: a wave behind the last column
-  if (FOUR) fetch(t_begin);
+  fetch(t_begin);
   for (int t0 = t_begin; t0 < t_end; t0 += TB) {
     const int nb = min(TB, t_end - t0);
     __syncthreads();                                   // the last block's staged values have been read
-    if (FOUR) {
-      put();
-    } else {
-    for (int idx = threadIdx.x; idx < nb * DKP; idx += blockDim.x) {      // only the block's tokens: a single token is one turn
-      const int tt = idx / DKP, c = idx % DKP;
-      const int t = t0 + min(tt, nb - 1), cc = min(c, dk - 1);
-      const bool in = tt < nb && c < dk;
-      const float kx = k[((size_t)t * KVH + kvh) * dk + cc];
-      const float qx = MODE == DS_LOCAL ? 0.f : q[((size_t)t * KVH + kvh) * dk + cc];
-      const float gx = g_channels ? g[((size_t)t * H + h) * dk + cc] : g[(size_t)t * H + h];
-      ks_[idx] = in ? kx : 0.f;
-      qs_[idx] = in ? qx : 0.f;
-      gs_[idx] = in ? gx : 1.f;
-    }
-    for (int idx = threadIdx.x; idx < nb * tile; idx += blockDim.x) {
-      const int tt = idx / tile, col = col0 + idx % tile;
-      const float x = load_f32(v + (size_t)(t0 + min(tt, nb - 1)) * ldv + (size_t)h * dv + min(col, dv - 1));
-      vs_[idx] = (tt < nb && col < dv) ? x : 0.f;       // the unit vectors' columns have values of zero
-    }
-    if ((int)threadIdx.x < TB) bs_[threadIdx.x] = beta[(size_t)(t0 + min((int)threadIdx.x, nb - 1)) * H + h];
-    }
+    put();
     __syncthreads();
-    if (FOUR && t0 + TB < t_end) fetch(t0 + TB);
-    if (FOUR && idle) continue;
-    f32x4 kt[2][KPL / 4], gt[2][KPL / 4], qt[2][KPL / 4];
+    if (t0 + TB < t_end) fetch(t0 + TB);
+    if (idle) continue;
+    // AHEAD: a token's k, g and q, read under the token before
+    constexpr int SETS = AHEAD ? 2 : 1, HELD = AHEAD ? KPL / 4 : 1;
+    f32x4 kt[SETS][HELD], gt[SETS][HELD], qt[SETS][HELD];
     auto read = [&](int set, int tt) {
+      if (!AHEAD) return;
       const f32x4* k4 = reinterpret_cast<const f32x4*>(ks_ + tt * DKP + c0);
       const f32x4* g4 = reinterpret_cast<const f32x4*>(gs_ + tt * DKP + c0);
       const f32x4* q4 = reinterpret_cast<const f32x4*>(qs_ + tt * DKP + c0);
 #pragma unroll
-      for (int i = 0; i < KPL / 4; i++) {
+      for (int i = 0; i < HELD; i++) {
         kt[set][i] = k4[i];
         gt[set][i] = g4[i];
         if (MODE != DS_LOCAL) qt[set][i] = q4[i];
       }
     };
     auto token = [&](int set, int tt) {
+      const f32x4* k4 = reinterpret_cast<const f32x4*>(ks_ + tt * DKP + c0);
+      const f32x4* g4 = reinterpret_cast<const f32x4*>(gs_ + tt * DKP + c0);
+      const f32x4* q4 = reinterpret_cast<const f32x4*>(qs_ + tt * DKP + c0);
       const float bt = bs_[tt];
       float kc[KPL], u[VPL];
 #pragma unroll
       for (int j = 0; j < VPL; j++) u[j] = 0.f;
 #pragma unroll
       for (int i = 0; i < KPL / 4; i++) {
-        const f32x4 kv = kt[set][i], gv = gt[set][i];
+        const f32x4 kv = AHEAD ? kt[set][i % HELD] : k4[i], gv = AHEAD ? gt[set][i % HELD] : g4[i];
         kc[4 * i] = kv.x; kc[4 * i + 1] = kv.y; kc[4 * i + 2] = kv.z; kc[4 * i + 3] = kv.w;
         if (MODE == DS_LOCAL && !DELTA) { gprod[4 * i] *= gv.x; gprod[4 * i + 1] *= gv.y; gprod[4 * i + 2] *= gv.z; gprod[4 * i + 3] *= gv.w; }
 #pragma unroll
@@ -306,7 +439,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
       for (int j = 0; j < VPL; j++) {
         const float vt = vs_[tt * tile + lcol0 + j * VC];
         if (DELTA) {
-          u[j] = bt * (vt - across(u[j]));
+          u[j] = bt * (vt - sum_across_32(sum_across_16(u[j])));
         } else {
           u[j] = bt * vt;
         }
@@ -323,7 +456,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
       for (int j = 0; j < VPL; j++) so[j] = 0.f;
 #pragma unroll
       for (int i = 0; i < KPL / 4; i++) {
-        const f32x4 qv = qt[set][i];
+        const f32x4 qv = AHEAD ? qt[set][i % HELD] : q4[i];
 #pragma unroll
         for (int j = 0; j < VPL; j++) {
           S[j][4 * i] = fmaf(kc[4 * i], u[j], S[j][4 * i]); so[j] = fmaf(S[j][4 * i], qv.x, so[j]);
@@ -334,18 +467,22 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
       }
 #pragma unroll
       for (int j = 0; j < VPL; j++) {
-        const float x = across(so[j]);
+        const float x = sum_across_32(sum_across_16(so[j]));
         const int col = col0 + lcol0 + j * VC;
         if (ks == 0 && col < dv) out[((size_t)(t0 + tt) * H + h) * dv + col] = x;
       }
     };
+    if (!AHEAD) {
+      for (int tt = 0; tt < nb; tt++) token(0, tt);
+      continue;
+    }
     read(0, 0);
     for (int tt = 0; tt < nb; tt += 2) {
-      if (tt + 1 < nb) read(1, tt + 1);
+      if (tt + 1 < nb) read(SETS - 1, tt + 1);
       token(0, tt);
       if (tt + 1 >= nb) break;
       if (tt + 2 < nb) read(0, tt + 2);
-      token(1, tt + 1);
+      token(SETS - 1, tt + 1);
     }
   }
   if (MODE == DS_FROM) return;
@@ -617,18 +754,21 @@ extern "C" int pico_delta_scan(const float* q, const float* k, const void* v, in
                "pico_delta_scan: too many value channels");
 #define ARGS(TV) q, k, (const TV*)v, ldv, g, g_channels, beta, cu_seqlens, state_slots, state, out, H, KVH, dk, dv, KS, TB, num_slots, \
                  chunk, max_chunks, ws_S, ws_P
+#define ARGS4(TV) q, k, (const TV*)v, ldv, g, g_channels, beta, cu_seqlens, state_slots, out, H, KVH, dk, dv, num_slots, chunk, max_chunks, \
+                  ws_S, ws_P
 #define COMBINE(RB)                                                                                                          \
   delta_combine_mfma_kernel<RB><<<dim3(num_seqs, H, (dv + 15) / 16), 256, 0, stream>>>(cu_seqlens, state_slots, state, ws_S, ws_P, \
                                                                                        H, dv, num_slots, chunk, max_chunks)
-  // (fewer key channels a lane leave nothing to read ahead)
-  const bool four = chunk > 0 && KS == 4 && kpl >= 8 && vpl == 2 && nw_v == 4 && nw_l == 4 && TB == 16;
-#define FOUR_OK(KPL, VPL) (KPL >= 8 && VPL == 2)
+  // 17 to 128 key channels and more than 96 columns: eight key channels or more in each of four lanes, all four waves with columns
+  const bool four = KS == 4 && kpl >= 8 && vpl == 2 && nw_v == 4 && nw_l == 4;
+#define SCAN4(TV, KPL, D, MODE, COLS) \
+  delta_scan4_kernel<TV, KPL < 8 ? 8 : KPL, D, MODE><<<dim3(nblk, H, tiles(COLS, 4)), 256, lds_bytes(4), stream>>>(ARGS4(TV))
 #define GO(TV, KPL, VPL, D)                                                                                                  \
   do {                                                                                                                       \
     if (chunk == 0) {                                                                                                        \
       delta_scan_kernel<TV, KPL, VPL, D, DS_WHOLE><<<dim3(nblk, H, tiles(dv, nw_v)), 64 * nw_v, lds_bytes(nw_v), stream>>>(ARGS(TV)); \
     } else {                                                                                                                 \
-      if (FOUR_OK(KPL, VPL) && four) delta_scan_kernel<TV, KPL, VPL, D, DS_LOCAL, FOUR_OK(KPL, VPL)><<<dim3(nblk, H, tiles(cols_local, nw_l)), 256, lds_bytes(nw_l), stream>>>(ARGS(TV)); \
+      if (four) SCAN4(TV, KPL, D, DS_LOCAL, cols_local);                                                                     \
       else delta_scan_kernel<TV, KPL, VPL, D, DS_LOCAL><<<dim3(nblk, H, tiles(cols_local, nw_l)), 64 * nw_l, lds_bytes(nw_l), stream>>>(ARGS(TV)); \
       if (D && dk == 64) COMBINE(1);                                                                                         \
       else if (D && dk == 128) COMBINE(2);                                                                                   \
@@ -640,7 +780,7 @@ extern "C" int pico_delta_scan(const float* q, const float* k, const void* v, in
       else                                                                                                                   \
         decay_combine_kernel<<<dim3(num_seqs, H, (dk * dv + 255) / 256), 256, 0, stream>>>(                                  \
             cu_seqlens, state_slots, state, ws_S, ws_P, H, dk, dv, num_slots, chunk, max_chunks);                            \
-      if (FOUR_OK(KPL, VPL) && four) delta_scan_kernel<TV, KPL, VPL, D, DS_FROM, FOUR_OK(KPL, VPL)><<<dim3(nblk, H, tiles(dv, nw_v)), 256, lds_bytes(nw_v), stream>>>(ARGS(TV)); \
+      if (four) SCAN4(TV, KPL, D, DS_FROM, dv);                                                                              \
       else delta_scan_kernel<TV, KPL, VPL, D, DS_FROM><<<dim3(nblk, H, tiles(dv, nw_v)), 64 * nw_v, lds_bytes(nw_v), stream>>>(ARGS(TV)); \
     }                                                                                                                        \
   } while (0)
@@ -662,7 +802,8 @@ extern "C" int pico_delta_scan(const float* q, const float* k, const void* v, in
 #undef PICK
 #undef PICK2
 #undef GO
-#undef FOUR_OK
+#undef SCAN4
+#undef ARGS4
 #undef COMBINE
 #undef ARGS
   PICO_LAUNCH_CHECK();

@@ -1660,8 +1660,8 @@ def test_decay_chunks_keep_tokens_apart(K, H, G, dk, dv, varies):
             assert torch.equal(got[~hit], clean[~hit]) and torch.equal(st[~hit_state], left[~hit_state]), (what, at)
 
 
-@pytest.mark.parametrize("dk", [64, 96, 128, 192, 256])
-@pytest.mark.parametrize("lens,dv", [([1], 16), ([64, 65], 40), ([3, 700, 128], 72), ([130, 1, 80], 104), ([17, 64], 128)])
+@pytest.mark.parametrize("dk", [16, 17, 32, 64, 96, 128, 192, 256])
+@pytest.mark.parametrize("lens,dv", [([1], 16), ([64, 65], 40), ([3, 700, 128], 72), ([130, 1, 80], 104), ([70, 16], 96), ([100], 97), ([17, 64], 128)])
 def test_delta_chunks(K, dk, lens, dv):
     # the walk over the chunks' states on the matrix cores (key sizes of whole 64s) and without (96), value sizes that end inside
     # a tile of 16 columns, one and many chunks, a slot that no sequence holds, against the rule token by token in 64 bits
