@@ -115,8 +115,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define GLA_LOCAL 1
 #define GLA_FROM 2
 
-// FUSED: the decays are made inside the walk (log_decay is null) instead of read.  wide: the states' rows are whole aligned fours.
-template <typename T, int MODE, int NW, bool FUSED>
+// FUSED: the decays are made inside the walk (log_decay is null) instead of read.  FEW: blocks of two tokens.  wide: the states' rows are whole aligned fours.
+template <typename T, int MODE, int NW, bool FUSED, bool FEW = false>
 __global__ __launch_bounds__(64 * NW) void gla_scan_kernel(const T* __restrict__ x, int ldx, int q_col, int k_col, int v_col,
                                                        const float* __restrict__ log_decay,
                                                        const int* __restrict__ cu_seqlens,
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(64 * NW) void gla_scan_kernel(const T* __restrict__
                                                        float* __restrict__ ws_decay, const T* __restrict__ a2,
                                                        const float* __restrict__ a2_bias, int a_col, int R, float inv_tau,
                                                        const float* __restrict__ head_decay, int silu, int wide) {
-  constexpr int TB = NW <= 4 ? 16 : 8, CP = NW * GLA_CPT, NL = TB / 2, NV = TB / NW;
+  constexpr int TB = FEW ? 2 : NW <= 4 ? 16 : 8, CP = NW * GLA_CPT, NL = TB / 2, NV = TB / NW;
   __shared__ float qs[TB * CP], ks[TB * CP], as[TB * CP], vs[TB * 64], po[TB * NW * 64];
   // head_decay given: every key channel of head h decays by the constant head_decay[h] at every token (log_decay, a2
   // are not read); the decay is multiplied in as it is, no logarithm and exponential between
@@ -351,13 +351,18 @@ extern "C" int pico_gla_scan(const void* x, int ldx, int dtype, int q_col, int k
                               (long long)max_chunks * chunk >= T && (long long)num_seqs * max_chunks < (1ll << 31)),
                "pico_gla_scan: chunks need room for their states and must cover the step's tokens");
   if (num_seqs == 0 || T == 0) return 0;
+  // A step of few tokens with one wave a workgroup: blocks of two tokens, so that a thread fetches next to nothing for tokens that
+  // are not there.  (12 heads of 32 x 64, 8 requests of one token: 3.7 us, in blocks of 16 6.2; four waves of a workgroup share a
+  // block's values and gain nothing.)
+  const bool few = chunk == 0 && T <= 2 * num_seqs;
   const int wide = dv % 4 == 0 && ((uintptr_t)state | (uintptr_t)ws) % 16 == 0, vb = (dv + 63) / 64;
 #define GLA_ARGS(TT)                                                                                                       \
   (const TT*)x, ldx, q_col, k_col, v_col, log_decay, cu_seqlens, state_slots, state, out, H, dk, dv, qscale, num_slots,   \
       chunk, max_chunks, ws, ws_decay, (const TT*)a2, a2_bias, a_col, R, 1.0f / (tau > 0.f ? tau : 1.f), head_decay, silu, wide
 #define GLA_WAVES(TT, MODE, GX, FUSED)                                                                                     \
   do {                                                                                                                     \
-    if (dk <= 32) gla_scan_kernel<TT, MODE, 1, FUSED><<<dim3(GX, H, vb), 64, 0, stream>>>(GLA_ARGS(TT));                   \
+    if (dk <= 32 && few) gla_scan_kernel<TT, MODE, 1, FUSED, MODE == GLA_WHOLE><<<dim3(GX, H, vb), 64, 0, stream>>>(GLA_ARGS(TT)); \
+    else if (dk <= 32) gla_scan_kernel<TT, MODE, 1, FUSED><<<dim3(GX, H, vb), 64, 0, stream>>>(GLA_ARGS(TT));                   \
     else if (dk <= 64) gla_scan_kernel<TT, MODE, 2, FUSED><<<dim3(GX, H, vb), 128, 0, stream>>>(GLA_ARGS(TT));             \
     else if (dk <= 128) gla_scan_kernel<TT, MODE, 4, FUSED><<<dim3(GX, H, vb), 256, 0, stream>>>(GLA_ARGS(TT));            \
     else gla_scan_kernel<TT, MODE, 8, FUSED><<<dim3(GX, H, vb), 512, 0, stream>>>(GLA_ARGS(TT));                           \

@@ -424,6 +424,31 @@ def test_gla_kernels_in_portions_and_token_by_token(dtype, H, dk, dv, rank, tau)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dk,dv", [(1, 3), (24, 40), (32, 64), (32, 132), (33, 64)])
+@pytest.mark.parametrize("lens", [[1], [2, 2], [5, 1, 1, 1], [4, 1, 1], [1, 7, 0, 1, 1]])
+def test_few_tokens_have_the_bits_of_many(dtype, dk, dv, lens):
+    """Steps of up to two tokens a sequence walk in blocks of two, on both sides of the line and of the key size of a wave; decays read, made in
+    the walk and fixed: a sequence's outputs and state are those of its tokens beside enough others for the long blocks."""
+    from pico_vllm_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(dk + sum(lens))
+    H, R, more = 2, 5, [40]
+    T, offs = sum(lens) + 40, (2 * dk, 4 * dk, 4 * dk + 2 * dv)
+    x = torch.randn(T, offs[2] + R, device=DEV, generator=g).to(DT[dtype])
+    a2 = torch.randn(H * dk, R, device=DEV, generator=g).to(DT[dtype])
+    start, fixed = torch.randn(len(lens) + 1, H, dk, dv, device=DEV, generator=g), torch.tensor([0.9, 0.5], device=DEV)
+    ld = K.gla_decay(x, offs[2], a2, None, 2.0)
+    for how in ("read", "made", "fixed"):
+        got = []
+        for n in (lens, lens + more):
+            t, state = sum(n), start.clone()
+            o = K.gla_scan(x[:t], 0, offs[0], offs[1], ld[:t] if how == "read" else None, torch.tensor(np.cumsum([0] + n), dtype=torch.int32, device=DEV),
+                           torch.arange(len(n), dtype=torch.int32, device=DEV), state, len(n), H, dk, dv, 0.3,
+                           decay_from=(offs[2], a2, None, 2.0) if how == "made" else None, head_decay=fixed if how == "fixed" else None)
+            got.append((o[:sum(lens)], state[:len(lens)]))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), how
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,C,R", [(64, 256, 32), (71, 300, 5), (65, 1, 16), (130, 257, 1024), (64, 3, 1025)])
 def test_decays_of_many_tokens_are_those_of_one_at_a_time(dtype, T, C, R):
     """Blocks of tokens, rows of a2 in sixteens of bytes or entry by entry: the same sums in the same order, so the same bits."""
