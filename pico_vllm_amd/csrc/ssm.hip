@@ -44,13 +44,12 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(const T* __restrict__ 
   store_f32(out + (size_t)t * C + c, conv_act(acc, silu));
 }
 
-// The same for bfloat16 with four neighbouring channels (8-byte accesses; C and the row stride multiples of 4) and CONV_TOKENS
-// neighbouring tokens a thread: the taps' weights, twice the bytes of the inputs they meet, are read once a thread, and a row once
-// for all its taps, all of a thread's rows asked for at once.  grid (ceil(T / CONV_TOKENS), ceil(C / 4 / 64)).
+// The same for bfloat16 and up to four taps with four neighbouring channels (8-byte accesses; C and the row stride multiples of 4) and
+// CONV_TOKENS neighbouring tokens a thread: the taps' weights, twice the bytes of the inputs they meet, are read once a thread, and a
+// row once for all its taps, all of a thread's rows asked for at once.  grid (ceil(T / CONV_TOKENS), ceil(C / 4 / 64)).
 // Bound by that one latency and the silu; eight channels or eight tokens a thread leave half the waves to hide it.  Microseconds with the
-// history's launch, a token and eight channels a thread (one, where rows do not start on 16 bytes) / 8 channels, 8 tokens / 4, 8 / 4, 4:
-// 2,052 tokens of 3,328 channels 29 / 19 / 16 / 15; of 1,664 in rows of 3,212 25 / 11 / 11 / 10; 1,377 of 3,072 21 / 16 / 12 / 11; 16 of
-// 3,072 10 / 12 / 9 / 7.
+// history's launch, a token and eight channels a thread / 8 channels, 8 tokens / 4, 8 / 4, 4: 2,052 tokens of 3,328 channels 29 / 19 / 16 /
+// 15; 1,377 of 3,072 21 / 16 / 12 / 11.
 #define CONV_TOKENS 4
 template <int TAPS>
 __global__ __launch_bounds__(64) void causal_conv_rows_kernel(const bf16_t* __restrict__ x, int ldx, const float* __restrict__ w,
@@ -104,6 +103,45 @@ __global__ __launch_bounds__(64) void causal_conv_rows_kernel(const bf16_t* __re
     *reinterpret_cast<uint2*>(out + (size_t)t * C + c0) = make_uint2(pack2_bf16(conv_act(acc[0], silu), conv_act(acc[1], silu)),
                                                                     pack2_bf16(conv_act(acc[2], silu), conv_act(acc[3], silu)));
   }
+}
+
+// The same for bfloat16 with eight neighbouring channels a thread (16-byte accesses; C and the row stride multiples of 8).
+// grid (T, ceil(C / 8 / 256)).
+__global__ __launch_bounds__(256) void causal_conv8_kernel(const bf16_t* __restrict__ x, int ldx, const float* __restrict__ w,
+                                                           const float* __restrict__ bias, const int* __restrict__ token_seq,
+                                                           const int* __restrict__ cu_seqlens,
+                                                           const int* __restrict__ state_slots, const float* __restrict__ state,
+                                                           int num_slots, int C, int N, int taps, int silu, bf16_t* __restrict__ out) {
+  const int t = blockIdx.x, c0 = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
+  if (c0 >= C) return;
+  const int b = token_seq[t], first = cu_seqlens[b];
+  const int slot = min(max(state_slots[b], 0), num_slots - 1);
+  float acc[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) acc[i] = bias ? bias[c0 + i] : 0.f;
+  for (int j = 0; j < taps; j++) {
+    const int src = t - (taps - 1) + j;
+    float v[8];
+    if (src >= first) {
+      const uint4 r = *reinterpret_cast<const uint4*>(x + (size_t)src * ldx + c0);
+      v[0] = __uint_as_float(r.x << 16); v[1] = __uint_as_float(r.x & 0xffff0000u);
+      v[2] = __uint_as_float(r.y << 16); v[3] = __uint_as_float(r.y & 0xffff0000u);
+      v[4] = __uint_as_float(r.z << 16); v[5] = __uint_as_float(r.z & 0xffff0000u);
+      v[6] = __uint_as_float(r.w << 16); v[7] = __uint_as_float(r.w & 0xffff0000u);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[i] = state[((size_t)slot * C + c0 + i) * (N + taps - 1) + N + (taps - 1) + (src - first)];
+    }
+    const float4 w0 = *reinterpret_cast<const float4*>(w + (size_t)j * C + c0), w1 = *reinterpret_cast<const float4*>(w + (size_t)j * C + c0 + 4);
+    acc[0] = fmaf(w0.x, v[0], acc[0]); acc[1] = fmaf(w0.y, v[1], acc[1]); acc[2] = fmaf(w0.z, v[2], acc[2]); acc[3] = fmaf(w0.w, v[3], acc[3]);
+    acc[4] = fmaf(w1.x, v[4], acc[4]); acc[5] = fmaf(w1.y, v[5], acc[5]); acc[6] = fmaf(w1.z, v[6], acc[6]); acc[7] = fmaf(w1.w, v[7], acc[7]);
+  }
+  uint4 o;
+  o.x = pack2_bf16(conv_act(acc[0], silu), conv_act(acc[1], silu));
+  o.y = pack2_bf16(conv_act(acc[2], silu), conv_act(acc[3], silu));
+  o.z = pack2_bf16(conv_act(acc[4], silu), conv_act(acc[5], silu));
+  o.w = pack2_bf16(conv_act(acc[6], silu), conv_act(acc[7], silu));
+  *reinterpret_cast<uint4*>(out + (size_t)t * C + c0) = o;
 }
 
 // grid (sequences, ceil(C / 256)): the slot's history becomes the last taps - 1 inputs behind this step's tokens.
@@ -176,8 +214,14 @@ extern "C" int pico_causal_conv(const void* x, int ldx, int dtype, const float* 
     if (taps > 1)
       conv_history_kernel<float><<<dim3(B, cb), 256, 0, stream>>>((const float*)x, ldx, cu_seqlens, state_slots, state, num_slots, C, N, taps);
   } else if (dtype == PICO_DTYPE_BF16) {
-    // whole aligned fours of channels and few taps: the window stays in registers
-    if (C % 4 == 0 && ldx % 4 == 0 && taps >= 2 && taps <= 4 && ((uintptr_t)x | (uintptr_t)out) % 8 == 0 && (uintptr_t)w % 16 == 0) {
+    // Few entries are a thread's latency, which a token and a channel a thread keeps shortest: one chain of loads, and not four tokens
+    // one behind the other where sequences begin.  Microseconds, that / four tokens and channels, four taps: 8 requests of a token
+    // 5.4 / 8.6 (3,072 channels); 200 tokens of 3,072 7.3 / 7.3, 300 7.9 / 7.4, 700 14.9 / 8.5; 300 of 1,664 6.7 / 6.9, 500 7.6 / 7.0; 64 of
+    // 7,168 8.2 / 8.0, 96 8.5 / 7.6; 1,000 of 512 6.2 / 6.7, 1,377 7.2 / 6.6: they meet at 0.6 million entries.  More taps than four, that /
+    // eight channels a thread: 5 taps, 500 tokens of 3,072 12.1 / 14.6, 700 18.5 / 17.6, 1,377 34 / 23; 8 taps, 1,000 of 1,664 23 / 21, 700
+    // 14 / 17, 300 of 7,168 30 / 27; 12 taps, 1,377 of 3,072 61 / 40.
+    const long long entries = (long long)T * C;
+    if (entries >= 600000 && C % 4 == 0 && ldx % 4 == 0 && taps >= 2 && taps <= 4 && ((uintptr_t)x | (uintptr_t)out) % 8 == 0 && (uintptr_t)w % 16 == 0) {
       const dim3 grid((T + CONV_TOKENS - 1) / CONV_TOKENS, (C / 4 + 63) / 64);
       PICO_REQUIRE(grid.y <= 65535, "pico_causal_conv: too many channels");
 #define CONV_ROWS(TAPS) causal_conv_rows_kernel<TAPS><<<grid, 64, 0, stream>>>((const bf16_t*)x, ldx, w, bias, token_seq, cu_seqlens, state_slots, \
@@ -186,6 +230,9 @@ extern "C" int pico_causal_conv(const void* x, int ldx, int dtype, const float* 
       else if (taps == 3) CONV_ROWS(3);
       else CONV_ROWS(2);
 #undef CONV_ROWS
+    } else if (taps > 4 && entries >= (taps < 8 ? 2000000 : 1600000) && C % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x | (uintptr_t)out | (uintptr_t)w) % 16 == 0) {
+      causal_conv8_kernel<<<dim3(T, (C / 8 + 255) / 256), 256, 0, stream>>>((const bf16_t*)x, ldx, w, bias, token_seq, cu_seqlens,
+                                                                            state_slots, state, num_slots, C, N, taps, silu, (bf16_t*)out);
     } else {
       causal_conv_kernel<bf16_t><<<dim3(T, cb), 256, 0, stream>>>((const bf16_t*)x, ldx, w, bias, token_seq, cu_seqlens, state_slots,
                                                                   state, num_slots, C, N, taps, silu, (bf16_t*)out);

@@ -407,6 +407,31 @@ def test_a_convolution_without_bias_whose_state_is_its_last_inputs(dtype, C, tap
         assert float((state[0] - 7).abs().max()) == 0 and float((state[2] - 7).abs().max()) == 0 if taps > 1 else True
 
 
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5, 7, 8, 16])
+@pytest.mark.parametrize("C,lens", [(2048, [1, 3, 250, 0, 2, 37]), (4096, [1, 2, 1, 500, 5]), (4100, [1, 146]), (800, [749, 0, 1])])
+def test_a_convolution_has_the_same_bits_in_steps_of_any_size(C, lens, taps):
+    """Forms with four tokens or eight channels a thread where a step has many entries (600,000, beyond four taps 1.6 or 2 million) and its
+    rows are whole aligned fours or eights, a token and a channel a thread elsewhere: the same rows in a matrix whose rows begin anywhere."""
+    from pico_vllm_amd.ops import kernels
+    g = torch.Generator(device=DEV).manual_seed(C + taps)
+    T = sum(lens)
+    w, b = torch.randn(taps, C, device=DEV, generator=g), torch.randn(C, device=DEV, generator=g)
+    rows = torch.randn(T, C + 9, device=DEV, generator=g).to(torch.bfloat16)
+    start = torch.randn(len(lens) + 1, C, taps + 1, device=DEV, generator=g)
+    ctx = step_ctx(lens, [0] * len(lens), list(range(len(lens) - 1, -1, -1)))
+    got = []
+    for x in (rows[:, :C].contiguous(), rows[:, :C]):                # (C + 9: an odd row stride)
+        state = start.clone()
+        got.append((kernels.causal_conv(x, C, w, b, ctx, state, 2), state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    # one row in 64 bits: the first token of the longest sequence, whose taps are all history but one
+    s = max(range(len(lens)), key=lambda j: lens[j])
+    first, slot = sum(lens[:s]), len(lens) - 1 - s
+    hist = torch.cat([start[slot, :, 2:].double(), rows[first, :C].double()[:, None]], 1)
+    want = (hist * w.double().T).sum(1) + b.double()
+    close(got[0][0][first], (want * torch.sigmoid(want)).cpu(), "bfloat16")
+
+
 DELTA_SHAPES = [(3, 1, 12, 20), (4, 2, 32, 64), (2, 2, 16, 16), (2, 1, 136, 5), (1, 1, 4, 70), (4, 4, 64, 32), (2, 1, 300, 9)]
 
 
