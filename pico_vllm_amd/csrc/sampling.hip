@@ -29,8 +29,9 @@
 // on its inputs only.  e is the hardware's exponential (__expf: 2^(x log2 e)) in every launch alike: what a token weighs
 // must be the same bits wherever it is asked.
 // (Five rounds of 63 thresholds and float sums, each a launch that read the row, in place of 2 and the search of 4: the chain 62 us for 8 rows
-// of 151,936 logits with top_p < 1, 32 so; 64 rows 159, 65; one row 63, 30; 5,000 logits 34, 25.  Where a class holds most of a row
-// the last launch's one workgroup has it all: logits within a twentieth of each other 61, 47, all logits equal 63, 93.)
+// of 151,936 logits with top_p < 1, 32 so; 64 rows 159, 65; one row 63, 30; 5,000 logits 34, 24.  Where a class holds most of a row
+// the last launch's one workgroup has it all: logits within a twentieth of each other 61, 58.  Elements that are all alike are listed
+// once: all logits equal 28, one by one 93; logits rounded to halves 29, 38.)
 #include "common.h"
 
 #define SAMPLE_CHUNKS 32            // as ARGMAX_CHUNKS below: the two share the first launch
@@ -44,6 +45,7 @@
 #define SAMPLE_MID 9                // the last launch's classes: 2^(19 - 9) of 2^9 patterns, 2^9 of one
 #define SAMPLE_ONE 0x3f800000u      // the bit pattern of 1.0f
 #define SAMPLE_LISTED 4864          // elements of a class that a chunk lists (all of a chunk up to 155,648 tokens); more are read again
+#define SAMPLE_ALIKE 256            // from so many on a chunk looks whether they are one value, and then lists it once
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -224,7 +226,9 @@ __device__ __forceinline__ int block_prefix_i32(int v, int* wave_tot) {
 }
 
 // Per chunk: the sum (double) of the e above the row's class, and a list of those in it, a thread's behind the last thread's; the
-// number that there are.  Rows with top_p >= 1: the sum of all.
+// number that there are.  Where they are many and all alike (equal logits) one stands for them, and the number is its complement.
+// Rows with top_p >= 1: the sum of all.
+template <bool SEARCH>
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
     const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature, const float* __restrict__ top_p,
     const float* __restrict__ part_val, const unsigned long long* __restrict__ classes, int bits, double* __restrict__ fin_s,
@@ -233,8 +237,9 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
   __shared__ int cls;
   __shared__ double ws[SAMPLE_THREADS / 64];
   __shared__ int wn[SAMPLE_THREADS / 64];
+  __shared__ uint32_t ends[2][SAMPLE_THREADS / 64];
   const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
-  const float temp = temperature[row], tp = top_p != nullptr ? top_p[row] : 1.0f, mx = sample_row_max(part_val, row);
+  const float temp = temperature[row], tp = SEARCH ? top_p[row] : 1.0f, mx = sample_row_max(part_val, row);
   if (!(temp > 0.f)) return;
   const float* x = logits + (size_t)row * ld;
   const SampleChunk ch = sample_chunk(V, c);
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
     }
   }
   int above = -1;                                          // keep what is above this class, list what is in it
-  if (tp < 1.0f) {
+  if (SEARCH && tp < 1.0f) {
     constexpr int N = SAMPLE_CLASSES / SAMPLE_THREADS;
     unsigned long long h[N], own = 0, total;
 #pragma unroll
@@ -305,26 +310,45 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
       for (int k = 8 * g; k < 8 * g + 8; k++) mine[k] = __expf((mine[k] - mx) * inv_t);
     }
   }
-  if (above < 0) {
+  if (!SEARCH || above < 0) {
     each([&](float e) {
       if (e > 0.f) s += (double)e;
     });
   } else {
+    uint32_t lo = 0xffffffffu, hi = 0u;
     each([&](float e) {
-      const int k = (int)sample_class(__float_as_uint(e));
+      const uint32_t b = __float_as_uint(e);
+      const int k = (int)sample_class(b);
       if (k > above && e > 0.f) s += (double)e;
-      n += k == above;
+      if (k == above) n++, lo = min(lo, b), hi = max(hi, b);
     });
     const int before = block_prefix_i32<SAMPLE_THREADS>(n, wn);
     uint32_t* mylist = list + ((size_t)row * SAMPLE_CHUNKS + c) * SAMPLE_LISTED;
-    int at = before;
-    each([&](float e) {
-      if ((int)sample_class(__float_as_uint(e)) == above) {
-        if (at < SAMPLE_LISTED) mylist[at] = __float_as_uint(e);
-        at++;
+    int at = before, all = 0;
+#pragma unroll
+    for (int k = 0; k < SAMPLE_THREADS / 64; k++) all += wn[k];
+    bool alike = false;
+    if (all >= SAMPLE_ALIKE) {                             // the same for all threads
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, off, 64));
       }
-    });
-    if (tid == SAMPLE_THREADS - 1) fin_n[(size_t)row * SAMPLE_CHUNKS + c] = before + n;
+      if ((tid & 63) == 0) ends[0][tid >> 6] = lo, ends[1][tid >> 6] = hi;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < SAMPLE_THREADS / 64; k++) lo = min(lo, ends[0][k]), hi = max(hi, ends[1][k]);
+      alike = lo == hi;
+      if (alike && tid == 0) mylist[0] = lo;
+    }
+    if (!alike)
+      each([&](float e) {
+        if ((int)sample_class(__float_as_uint(e)) == above) {
+          if (at < SAMPLE_LISTED) mylist[at] = __float_as_uint(e);
+          at++;
+        }
+      });
+    if (tid == 0) fin_n[(size_t)row * SAMPLE_CHUNKS + c] = alike ? ~all : all;
   }
   s = wave_sum_f64(s);
   if ((tid & 63) == 0) ws[tid >> 6] = s;
@@ -372,16 +396,18 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
   int kept_n = 0;
   if constexpr (SEARCH) if (tp < 1.0f) {
     const SampleRow r = rows[row];
-    const int listed = fin_n[base + my_chunk];
+    const int number = fin_n[base + my_chunk], listed = number < 0 ? 1 : number;
     // the patterns of this chunk's elements of the class, PER threads side by side, four neighbours each: from the list, of which
     // each thread holds the first ones, or, where it did not have room for all, from the logits
     const u32x4* mylist = reinterpret_cast<const u32x4*>(list + (base + my_chunk) * SAMPLE_LISTED);
     const u32x4 held = 4 * part < listed ? mylist[part] : u32x4{0, 0, 0, 0};
-    auto entries = [&](auto use) {
-      if (listed <= SAMPLE_LISTED) {
+    auto entries = [&](auto use) {                        // use(pattern, how many of it)
+      if (number < 0) {
+        if (part == 0) use(held[0], ~number);
+      } else if (listed <= SAMPLE_LISTED) {
 #pragma unroll
         for (int j = 0; j < 4; j++)
-          if (4 * part + j < listed) use(held[j]);
+          if (4 * part + j < listed) use(held[j], 1);
         for (int k0 = part + PER; 4 * k0 < listed; k0 += 4 * PER) {
           u32x4 v[4];
 #pragma unroll
@@ -390,7 +416,7 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
           for (int k = 0; k < 4; k++)
 #pragma unroll
             for (int j = 0; j < 4; j++)
-              if (4 * (k0 + k * PER) + j < listed) use(v[k][j]);
+              if (4 * (k0 + k * PER) + j < listed) use(v[k][j], 1);
         }
       } else {
         const SampleChunk ch = sample_chunk(V, my_chunk);
@@ -401,7 +427,7 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
 #pragma unroll
           for (int k = 0; k < 16; k++) {
             const uint32_t b = __float_as_uint(__expf((v[k] - mx) * inv_t));
-            if (i0 + k * PER < ch.end && sample_class(b) == r.cls) use(b);
+            if (i0 + k * PER < ch.end && sample_class(b) == r.cls) use(b, 1);
           }
         }
       }
@@ -419,8 +445,8 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
       if (tid == 0) cls = -1;
       __syncthreads();
       SampleRun run{hist};
-      entries([&](uint32_t b) {
-        if (b >> (shift + width) == found) run.add((b >> shift) & ((1u << width) - 1), sample_fixed(b, bits));
+      entries([&](uint32_t b, int copies) {
+        if (b >> (shift + width) == found) run.add((b >> shift) & ((1u << width) - 1), sample_fixed(b, bits) * copies);
       });
       run.end();
       __syncthreads();
@@ -438,10 +464,10 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
     // the mass before them still is
     ties_kept = max(1, (int)ceilf((r.target - (float)((double)above / one)) / thr));
     double s = 0.0;
-    entries([&](uint32_t b) {
+    entries([&](uint32_t b, int copies) {
       const float e = __uint_as_float(b);
-      if (e > thr) s += (double)e;
-      kept_n += e == thr;
+      if (e > thr) s += (double)e * copies;
+      if (e == thr) kept_n += copies;
     });
 #pragma unroll
     for (int off = PER / 2; off > 0; off >>= 1) {
@@ -656,7 +682,8 @@ extern "C" int pico_sample(const float* logits, int ld, int R, int V, const floa
   argmax_part_kernel<<<grid, 256, 0, stream>>>(logits, ld, V, part_val, part_idx, top_p_rows ? classes : nullptr);
   const float* asked = top_p_rows ? top_p : nullptr;
   if (top_p_rows) sample_classes_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, top_p, part_val, classes, bits);
-  sample_collect_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, part_val, classes, bits, fin_s, fin_n, list, rows);
+  const auto collect = top_p_rows ? sample_collect_kernel<true> : sample_collect_kernel<false>;
+  collect<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, part_val, classes, bits, fin_s, fin_n, list, rows);
   if (top_p_rows)
     sample_pick_kernel<SAMPLE_PICK_THREADS, true><<<R, SAMPLE_PICK_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, u, part_val, part_idx,
                                                                                         fin_s, fin_n, list, rows, bits, out);

@@ -665,6 +665,28 @@ def test_sampling_searches_classes_of_any_size(K, V):
         assert float(p[out[r]]) > 0 or abs(float(us[r]) - 1) < 2e-6, (r, "a token outside the kept set")
 
 
+@pytest.mark.parametrize("V", [9000, 151936, 300001])
+def test_sampling_among_many_equal_logits(K, V):
+    # classes whose elements are one value (listed once), one value in some chunks and several in others, and one value but for a
+    # single element; every draw against the plain rule, in which tied tokens stay in vocabulary order
+    g = torch.Generator().manual_seed(V)
+    R = 10
+    logits = (torch.randn(R, V, generator=g) * 2).round() / 2
+    logits[3:6] = logits[3:6].clamp(min=1.0)                      # most of the row one value
+    logits[6:8] = 0.0
+    logits[8:] = 0.0
+    logits[8, V // 3], logits[9, V - 2] = -0.01, 0.02
+    top_ps = torch.tensor([0.3, 0.9, 0.999, 0.4, 0.8, 0.97, 0.51307, 0.98703, 0.70291, 0.01003])     # (no whole number of equal tokens)
+    us = torch.rand(R, generator=g)
+    out = K.sample(logits.to(DEV), torch.full((R,), 0.9).to(DEV), top_ps.to(DEV), us.to(DEV)).tolist()
+    for r in range(R):
+        p = P.top_p_probs(logits[r].double(), 0.9, float(top_ps[r]))
+        want, cum = P.inverse_cdf(p, float(us[r])), torch.cumsum(p, 0)
+        # as far from a boundary as sums of 32-bit exponentials are off
+        assert out[r] == want or abs(float(cum[min(out[r], want)]) - float(us[r])) < 2e-6, (r, out[r], want)
+        assert float(p[out[r]]) > 0 or abs(float(us[r]) - 1) < 2e-6, (r, "a token outside the kept set")
+
+
 def test_sampling_at_the_edges_of_its_options(K):
     # a nucleus so small that only the likeliest token fits, a temperature so low that it holds all the mass, one so high
     # that the distribution is flat, and a vocabulary smaller than the number of chunks a row is read in
