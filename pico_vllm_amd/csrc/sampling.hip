@@ -44,7 +44,8 @@
 #define SAMPLE_LOW 19
 #define SAMPLE_MID 9                // the last launch's classes: 2^(19 - 9) of 2^9 patterns, 2^9 of one
 #define SAMPLE_ONE 0x3f800000u      // the bit pattern of 1.0f
-#define SAMPLE_LISTED 4864          // elements of a class that a chunk lists (all of a chunk up to 155,648 tokens); more are read again
+#define SAMPLE_LISTED 4864          // elements of a class that a chunk lists at most (all of a chunk up to 155,648 tokens); more are read again
+#define SAMPLE_ROWS 256             // rows with a list at a time
 #define SAMPLE_ALIKE 256            // from so many on a chunk looks whether they are one value, and then lists it once
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -232,7 +233,7 @@ template <bool SEARCH>
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
     const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature, const float* __restrict__ top_p,
     const float* __restrict__ part_val, const unsigned long long* __restrict__ classes, int bits, double* __restrict__ fin_s,
-    int* __restrict__ fin_n, uint32_t* __restrict__ list, SampleRow* __restrict__ rows) {
+    int* __restrict__ fin_n, uint32_t* __restrict__ list, int room, SampleRow* __restrict__ rows) {
   __shared__ unsigned long long scratch[SAMPLE_THREADS / 64], mass;
   __shared__ int cls;
   __shared__ double ws[SAMPLE_THREADS / 64];
@@ -323,7 +324,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
       if (k == above) n++, lo = min(lo, b), hi = max(hi, b);
     });
     const int before = block_prefix_i32<SAMPLE_THREADS>(n, wn);
-    uint32_t* mylist = list + ((size_t)row * SAMPLE_CHUNKS + c) * SAMPLE_LISTED;
+    uint32_t* mylist = list + ((size_t)row * SAMPLE_CHUNKS + c) * room;
     int at = before, all = 0;
 #pragma unroll
     for (int k = 0; k < SAMPLE_THREADS / 64; k++) all += wn[k];
@@ -344,7 +345,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
     if (!alike)
       each([&](float e) {
         if ((int)sample_class(__float_as_uint(e)) == above) {
-          if (at < SAMPLE_LISTED) mylist[at] = __float_as_uint(e);
+          if (at < room) mylist[at] = __float_as_uint(e);
           at++;
         }
       });
@@ -363,7 +364,7 @@ template <int THREADS, bool SEARCH>
 __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
     const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature, const float* __restrict__ top_p,
     const float* __restrict__ u, const float* __restrict__ part_val, const int* __restrict__ part_idx,
-    const double* __restrict__ fin_s, const int* __restrict__ fin_n, const uint32_t* __restrict__ list,
+    const double* __restrict__ fin_s, const int* __restrict__ fin_n, const uint32_t* __restrict__ list, int room,
     const SampleRow* __restrict__ rows, int bits, int* __restrict__ out) {
   constexpr int WAVES = THREADS / 64, PER = THREADS / SAMPLE_CHUNKS, PIECE = SAMPLE_PIECE / THREADS;     // PER: threads a chunk
   __shared__ unsigned long long hist[SEARCH ? 1 << (SAMPLE_LOW - SAMPLE_MID) : 1], scratch[WAVES], mass;
@@ -399,12 +400,12 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
     const int number = fin_n[base + my_chunk], listed = number < 0 ? 1 : number;
     // the patterns of this chunk's elements of the class, PER threads side by side, four neighbours each: from the list, of which
     // each thread holds the first ones, or, where it did not have room for all, from the logits
-    const u32x4* mylist = reinterpret_cast<const u32x4*>(list + (base + my_chunk) * SAMPLE_LISTED);
+    const u32x4* mylist = reinterpret_cast<const u32x4*>(list + (base + my_chunk) * room);
     const u32x4 held = 4 * part < listed ? mylist[part] : u32x4{0, 0, 0, 0};
     auto entries = [&](auto use) {                        // use(pattern, how many of it)
       if (number < 0) {
         if (part == 0) use(held[0], ~number);
-      } else if (listed <= SAMPLE_LISTED) {
+      } else if (listed <= room) {
 #pragma unroll
         for (int j = 0; j < 4; j++)
           if (4 * part + j < listed) use(held[j], 1);
@@ -653,11 +654,20 @@ extern "C" int pico_argmax(const float* logits, int ld, int R, int V, float* par
   return 0;
 }
 
-// work: pico_sample_workspace_words(R) 4-byte words, 16-byte aligned.  top_p_rows == 0: no row has top_p < 1 (every
-// row is treated so), and the launch that looks for the threshold is left out.
-extern "C" long long pico_sample_workspace_words(int R) {
+// Words of a chunk's list: none are missing up to SAMPLE_LISTED elements a chunk.  (A class that is not listed whole is read again, three
+// times: nearly flat rows of 151,936 102 us in place of 58 with a list of half a chunk.)
+static int sample_room(int V) {
+  const long long len = ((long long)V + SAMPLE_CHUNKS - 1) / SAMPLE_CHUNKS;
+  return len < SAMPLE_LISTED ? (int)((len + 3) / 4 * 4) : SAMPLE_LISTED;
+}
+
+// work: pico_sample_workspace_words(R, V, top_p_rows) 4-byte words, 16-byte aligned: 640 bytes a row, and with top_p_rows for up to
+// SAMPLE_ROWS rows 16 KB of classes and a row's length of floats (at most 623 KB).  top_p_rows == 0: no row has top_p < 1
+// (every row is treated so), and the launch that looks for the threshold is left out.
+extern "C" long long pico_sample_workspace_words(int R, int V, int top_p_rows) {
   static_assert(sizeof(SampleRow) == 16, "four words a row");
-  return (long long)R * (2 * SAMPLE_CLASSES + 4 + SAMPLE_CHUNKS * (2 + 1 + 1 + 1 + SAMPLE_LISTED));
+  const long long at_once = R < SAMPLE_ROWS ? R : SAMPLE_ROWS;
+  return (long long)R * SAMPLE_CHUNKS * (2 + 1 + 1 + 1) + (top_p_rows ? at_once * (2 * SAMPLE_CLASSES + 4 + SAMPLE_CHUNKS * (long long)sample_room(V)) : 0);
 }
 
 extern "C" int pico_sample(const float* logits, int ld, int R, int V, const float* temperature, const float* top_p,
@@ -669,27 +679,36 @@ extern "C" int pico_sample(const float* logits, int ld, int R, int V, const floa
   // (every part of the workspace is a multiple of 16 bytes long)
   PICO_REQUIRE(work != nullptr && (uintptr_t)work % 16 == 0, "pico_sample: the workspace is missing or not 16-byte aligned");
   const size_t n = (size_t)R * SAMPLE_CHUNKS;
-  unsigned long long* classes = (unsigned long long*)work;
-  SampleRow* rows = (SampleRow*)(classes + (size_t)R * SAMPLE_CLASSES);
-  double* fin_s = (double*)(rows + R);
+  double* fin_s = (double*)work;
   float* part_val = (float*)(fin_s + n);
   int* part_idx = (int*)(part_val + n);
   int* fin_n = part_idx + n;
-  uint32_t* list = (uint32_t*)(fin_n + n);
+  unsigned long long* classes = (unsigned long long*)(fin_n + n);
+  const int room = sample_room(V), at_once = R < SAMPLE_ROWS ? R : SAMPLE_ROWS;
+  SampleRow* rows = (SampleRow*)(classes + (size_t)at_once * SAMPLE_CLASSES);
+  uint32_t* list = (uint32_t*)(rows + at_once);
   int bits = 40;                              // a row's sum of whole numbers of 2^-bits stays below 2^63
   while (bits > 31 && V > (1LL << (63 - bits))) bits--;
-  const dim3 grid(R, SAMPLE_CHUNKS);
-  argmax_part_kernel<<<grid, 256, 0, stream>>>(logits, ld, V, part_val, part_idx, top_p_rows ? classes : nullptr);
-  const float* asked = top_p_rows ? top_p : nullptr;
-  if (top_p_rows) sample_classes_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, top_p, part_val, classes, bits);
-  const auto collect = top_p_rows ? sample_collect_kernel<true> : sample_collect_kernel<false>;
-  collect<<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, part_val, classes, bits, fin_s, fin_n, list, rows);
-  if (top_p_rows)
-    sample_pick_kernel<SAMPLE_PICK_THREADS, true><<<R, SAMPLE_PICK_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, u, part_val, part_idx,
-                                                                                        fin_s, fin_n, list, rows, bits, out);
-  else
-    sample_pick_kernel<SAMPLE_THREADS, false><<<R, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, asked, u, part_val, part_idx,
-                                                                               fin_s, fin_n, list, rows, bits, out);
+  if (!top_p_rows) {
+    const dim3 grid(R, SAMPLE_CHUNKS);
+    argmax_part_kernel<<<grid, 256, 0, stream>>>(logits, ld, V, part_val, part_idx);
+    sample_collect_kernel<false><<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, nullptr, part_val, nullptr, bits, fin_s, fin_n,
+                                                                     nullptr, 0, nullptr);
+    sample_pick_kernel<SAMPLE_THREADS, false><<<R, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, nullptr, u, part_val, part_idx,
+                                                                               fin_s, fin_n, nullptr, 0, nullptr, bits, out);
+  }
+  for (int r = 0; top_p_rows && r < R; r += SAMPLE_ROWS) {     // rows with a list side by side; the next ones write it again behind them
+    const int m = R - r < SAMPLE_ROWS ? R - r : SAMPLE_ROWS;
+    const size_t c = (size_t)r * SAMPLE_CHUNKS;
+    const float* x = logits + (size_t)r * ld;
+    const dim3 grid(m, SAMPLE_CHUNKS);
+    argmax_part_kernel<<<grid, 256, 0, stream>>>(x, ld, V, part_val + c, part_idx + c, classes);
+    sample_classes_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(x, ld, V, temperature + r, top_p + r, part_val + c, classes, bits);
+    sample_collect_kernel<true><<<grid, SAMPLE_THREADS, 0, stream>>>(x, ld, V, temperature + r, top_p + r, part_val + c, classes, bits, fin_s + c,
+                                                                    fin_n + c, list, room, rows);
+    sample_pick_kernel<SAMPLE_PICK_THREADS, true><<<m, SAMPLE_PICK_THREADS, 0, stream>>>(x, ld, V, temperature + r, top_p + r, u + r, part_val + c,
+                                                                                        part_idx + c, fin_s + c, fin_n + c, list, room, rows, bits, out + r);
+  }
   PICO_LAUNCH_CHECK();
   return 0;
 }

@@ -43,11 +43,20 @@ class Sampler:
         self._dev = torch.zeros(3, max_rows, dtype=torch.float32, device=device)
         self._out = torch.zeros(max_rows, dtype=torch.int32, device=device)
         self._argmax_work = kernels.argmax_workspace(max_rows, device) if torch.cuda.is_available() else None
-        self._sample_work = kernels.sample_workspace(max_rows, device) if torch.cuda.is_available() else None
+        # of calls without top_p; what its search needs (as much as the logits of 256 rows) waits for the first call that has it
+        self._sample_work = kernels.sample_workspace(max_rows, device, top_p_rows=False) if torch.cuda.is_available() else None
+        self._top_p_work = None
         self._host_np = [h.numpy() for h in self._host]
         self._landing = [torch.zeros(max_rows, dtype=torch.int32, pin_memory=torch.cuda.is_available()) for _ in range(2)]
         self._landed = [torch.cuda.Event() if torch.cuda.is_available() else None for _ in range(2)]
         self._turn = 0
+
+    def _work(self, vocab: int) -> torch.Tensor:
+        """The workspace of a search, kept: all rows that the sampler was made for, of as many logits as have been seen."""
+        if self._top_p_work is None or vocab > self._top_p_work[0]:
+            self._top_p_work = None                          # (the smaller one goes first)
+            self._top_p_work = (vocab, kernels.sample_workspace(self.max_rows, self.device, vocab))
+        return self._top_p_work[1]
 
     def sample(self, logits: torch.Tensor, temperatures: Sequence[float], top_ps: Sequence[float],
                seeds: Sequence[int], indices: Sequence[int]) -> List[int]:
@@ -87,8 +96,9 @@ class Sampler:
             h[1, :R] = top_ps
             h[2, :R] = [uniform(s, i) if t > 0 else 0.0 for s, i, t in zip(seeds, indices, temperatures)]
             self._dev.copy_(self._host[self._turn], non_blocking=True)
-            kernels.sample(logits, self._dev[0], self._dev[1], self._dev[2], self._out, self._sample_work,
-                           top_p_rows=any(t > 0 and p < 1 for t, p in zip(temperatures, top_ps)))
+            searched = any(t > 0 and p < 1 for t, p in zip(temperatures, top_ps))
+            kernels.sample(logits, self._dev[0], self._dev[1], self._dev[2], self._out, self._work(logits.shape[1]) if searched else self._sample_work,
+                           top_p_rows=searched)
         turn = self._turn
         self._turn ^= 1
         self._landing[turn][:R].copy_(self._out[:R], non_blocking=True)

@@ -687,6 +687,36 @@ def test_sampling_among_many_equal_logits(K, V):
         assert float(p[out[r]]) > 0 or abs(float(us[r]) - 1) < 2e-6, (r, "a token outside the kept set")
 
 
+def test_sampling_of_more_rows_than_a_search_takes_at_a_time(K):
+    # 256 rows share the room for lists and classes, the next ones write it again; greedy, plain and top_p rows in turn
+    R, V = 515, 333
+    g = torch.Generator().manual_seed(5)
+    logits, us = (torch.randn(R, V, generator=g) * 2).to(DEV), torch.rand(R, generator=g).to(DEV)
+    temps, top_ps = torch.tensor([0.0, 0.8, 0.8, 1.3])[torch.arange(R) % 4].to(DEV), torch.tensor([1.0, 0.9, 1.0, 0.4])[torch.arange(R) % 4].to(DEV)
+    out = K.sample(logits, temps, top_ps, us)
+    alone = [K.sample(logits[r:r + 1], temps[r:r + 1], top_ps[r:r + 1], us[r:r + 1]) for r in (0, 1, 2, 3, 255, 256, 257, 258, 511, 512, 513, 514)]
+    assert out[[0, 1, 2, 3, 255, 256, 257, 258, 511, 512, 513, 514]].tolist() == [int(t[0]) for t in alone]
+    assert torch.equal(out, torch.cat([K.sample(logits[r:r + 103], temps[r:r + 103], top_ps[r:r + 103], us[r:r + 103]) for r in range(0, R, 103)]))
+
+
+def test_the_room_that_sampling_holds(K):
+    # bytes a row: 640, and what a search takes: classes, a row's length (rounded up a chunk) and at most 623 KB, for 256 rows at most
+    from pico_vllm_amd.sampling.sampler import Sampler
+    size = lambda *a, **k: 4 * K.sample_workspace(*a, **k).numel()
+    assert size(64, DEV, top_p_rows=False) == size(64, DEV, 151936, top_p_rows=False) == 640 * 64
+    assert size(1, DEV, 5000) == 640 + 16400 + 4 * 32 * 160
+    assert size(8, DEV, 151936) == 8 * (640 + 16400 + 4 * 151936 + 0) and size(8, DEV) == 8 * (640 + 16400 + 4 * 32 * 4864)
+    assert size(4096, DEV, 151936) == 4096 * 640 + 256 * (16400 + 4 * 151936)
+    sampler, logits = Sampler(torch.device(DEV), 64), torch.randn(2, 700, device=DEV)
+    for temps, top_ps in (([0.0, 0.0], [1.0, 1.0]), ([0.0, 0.7], [0.5, 1.0])):
+        sampler.sample(logits, temps, top_ps, [1, 2], [0, 0])
+    assert sampler._top_p_work is None
+    first = [sampler.sample(torch.cat([logits] * n, 1), [0.7, 0.0], [0.5, 1.0], [1, 2], [0, 0]) for n in (1, 3, 1)]
+    assert first[0] == first[2] and 4 * sampler._top_p_work[1].numel() == size(64, DEV, 2100)
+    with pytest.raises(K.KernelError, match="workspace"):
+        K.sample(logits, *(torch.full((2,), 0.5, device=DEV) for _ in range(3)), work=K.sample_workspace(2, DEV, top_p_rows=False))
+
+
 def test_sampling_at_the_edges_of_its_options(K):
     # a nucleus so small that only the likeliest token fits, a temperature so low that it holds all the mass, one so high
     # that the distribution is flat, and a vocabulary smaller than the number of chunks a row is read in
