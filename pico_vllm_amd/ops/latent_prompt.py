@@ -43,16 +43,22 @@ class LatentPrompt:
         self.slots = max(1, 2 * compute_units() // heads)      # workgroups a head: two a compute unit in all
         self.least = 4                                         # tiles of keys that a workgroup has at least
 
-    @staticmethod
-    def pays(tokens: int, keys: int, singles: int) -> bool:
-        """Whether a step's portions, of so many tokens that see so many keys, are served here.  What is paid here is a key's
-        product (12 heads: 27 us for 6,144 keys) and in the latent's space a query's.  Microseconds, latent's space / here, 12 heads of
-        128 + 64 and 128 and a latent of 256: 8 tokens behind 0, 1,000 and 8,000: 19 / 17, 25 / 29, 36 / 58; 32: 23 / 17, 29 / 31, 48 / 60;
-        48: 28 / 17, 33 / 31, 69 / 61; 64: 28 / 17, 37 / 31, 72 / 62; 128: 53 / 21, 69 / 34, 142 / 68 (28 heads cross at the same places).
-        With single tokens in front of the portions these need launches of their own (about 25 us), which 96 tokens earn."""
-        if singles:
-            return tokens >= 96
-        return tokens >= 48 or keys <= 16 * tokens
+    def gain(self, portions, singles: int) -> float:
+        """Microseconds that a step's portions, pairs (new tokens, context), are expected to take less here than in the latent's space.
+        Here a portion pays for its keys, whoever reads them: their way into memory and out of it, and products for whole tiles of
+        queries; there for its tokens' products and for every pair, and from 65 rows on for the batched products' launches and copies
+        and for the longest context, which few workgroups walk.  With single tokens in front of the portions these need launches of
+        their own.  A fit to 196 steps of seven sets of sizes (12 to 28 heads, latents of 32 to 256, 1 to 16 portions of 4 to 2,048 tokens
+        behind up to 8,000), of which it sends 11 the slower way, by 10 % at most; 4 of 140 drawn ones of five other sets, by 27 %.  Microseconds, latent's space / here, 12 heads of
+        128 + 64 and 128, latents of 256 and 64: 32 tokens 31 / 24 and 22 / 22, behind 8,000 56 / 68 and 35 / 56; 64 behind 8,000 85 / 72 and 49 /
+        60; six portions of 16 behind 8,000 154 / 234 and 87 / 207; 200 83 / 41 and 62 / 38; 2,048 behind 4,096 478 / 170 and 254 / 154."""
+        tokens, keys = sum(n for n, _ in portions), sum(c for _, c in portions)
+        pairs, tiles = sum(n * c for n, c in portions), sum(-(-n // QUERIES) * QUERIES * c for n, c in portions)
+        many = tokens + singles >= 65
+        H, outputs = self.heads, self.heads * (self.d + self.dv)
+        return ((23.0 + 4.0e-3 * max(c for _, c in portions) if many else 0.0) + 4.5e-8 * tokens * outputs * self.rank
+                + (5.6e-9 if many else 7.9e-9) * pairs * H * (2 * self.rank + self.r)
+                - 5.2e-7 * keys * outputs - 2.4e-9 * tiles * H * (self.d + self.r + self.dv) - (16.5 if singles else 0.0) - (2.0 if len(portions) > 1 else 0.0))
 
     def plan(self, ctx) -> Optional[tuple]:
         """(single tokens in front, room for tiles of keys) if the step's portions are served here, else None.  Decided on the
@@ -69,11 +75,10 @@ class LatentPrompt:
         real, lead = B - filler, 0
         while lead < real and cu[lead + 1] - cu[lead] == 1:
             lead += 1
-        contexts = [int(c) for c in ctx.host["context_lens"][lead:real]]
-        tokens = int(cu[real] - cu[lead])
-        if not contexts or not self.pays(tokens, sum(contexts), lead):
+        portions = [(int(cu[b + 1] - cu[b]), int(ctx.host["context_lens"][b])) for b in range(lead, real) if cu[b + 1] > cu[b]]
+        if not portions or self.gain(portions, lead) <= 0:
             return None
-        room = bucket(sum(-(-c // TILE) for c in contexts)) + (-(-ctx.num_tokens // TILE) if filler else 0)
+        room = bucket(sum(-(-int(c) // TILE) for c in ctx.host["context_lens"][lead:real])) + (-(-ctx.num_tokens // TILE) if filler else 0)
         fits = room * TILE * self.heads * (self.d + self.dv) * 2 <= MAX_BYTES and (ctx.num_tokens // QUERIES + B) * room < 1 << 30
         return (lead, room) if fits else None
 
