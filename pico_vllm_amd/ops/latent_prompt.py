@@ -21,12 +21,10 @@ def supported(dim: int, rot_dim: int, value_dim: int, rank: int) -> bool:
 
 
 def bucket(tiles: int) -> int:
-    """Room for so many tiles: the next of 2^k and 3 2^k, so that a recorded step serves contexts of a range of lengths."""
-    room = 16
+    """Room of a recorded step for so many tiles: the next of 64 4^k, so that three recordings serve contexts of up to 65,536 tokens."""
+    room = 64
     while room < tiles:
-        if room * 3 // 2 >= tiles:
-            return room * 3 // 2
-        room *= 2
+        room *= 4
     return room
 
 
@@ -78,9 +76,16 @@ class LatentPrompt:
         portions = [(int(cu[b + 1] - cu[b]), int(ctx.host["context_lens"][b])) for b in range(lead, real) if cu[b + 1] > cu[b]]
         if not portions or self.gain(portions, lead) <= 0:
             return None
-        room = bucket(sum(-(-int(c) // TILE) for c in ctx.host["context_lens"][lead:real])) + (-(-ctx.num_tokens // TILE) if filler else 0)
-        fits = room * TILE * self.heads * (self.d + self.dv) * 2 <= MAX_BYTES and (ctx.num_tokens // QUERIES + B) * room < 1 << 30
-        return (lead, room) if fits else None
+        need = sum(-(-int(c) // TILE) for c in ctx.host["context_lens"][lead:real])
+        behind = -(-ctx.num_tokens // TILE) if filler else 0
+        most = MAX_BYTES // self.tile_bytes - behind
+        room = (min(bucket(need), most) if filler else need) + behind
+        return (lead, room) if need <= most and (ctx.num_tokens // QUERIES + B) * room < 1 << 30 else None
+
+    @property
+    def tile_bytes(self) -> int:
+        """Keys and values of a tile."""
+        return TILE * (self.heads * (self.d + self.dv) + self.r) * 2
 
     def __call__(self, q: torch.Tensor, table: torch.Tensor, cache, block_table: torch.Tensor, ctx, plan: tuple, out: torch.Tensor,
                  gate: Optional[torch.Tensor] = None) -> torch.Tensor:
