@@ -127,7 +127,7 @@ class Linear:
             # this package's plain matrix-core product, in which a row's result does not depend on the other rows of
             # the step, as it does not in the weight-streaming kernel; the library's may
             return kernels.gemm_bf16(x, self.weight, self.bias_f32, torch.bfloat16)
-        parts = kernels.tiles_parts(x, self.weight)
+        parts = kernels.tiles_parts(x, self.weight, self.bias_f32)
         if parts > 1 and not _tuned(x.shape[0]):
             return kernels.gemm_tiles_split(x, self.weight, self.bias_f32, parts)
         _library_tuning(x.shape[0])

@@ -1815,3 +1815,15 @@ def test_the_layer_takes_a_long_inner_size_in_parts(K, M, N, K_):
     assert parts > 1
     assert torch.equal(Linear(w, b)(x), K.gemm_tiles_split(x, w, b.float(), parts))
     assert K.tiles_parts(x[:, :K_ - 4], w[:, :K_ - 4]) == 1 and K.tiles_parts(x[:, :6144], w[:, :6144]) == 1
+
+
+def test_the_layer_takes_a_bias_that_starts_anywhere(K):
+    # a float32 bias is kept where it lies: one that starts on no 16 bytes is the library's product's, as it was before there were parts
+    from pico_vllm_amd.ops.linear import Linear
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn(300, 8960, generator=g).bfloat16().to(DEV), torch.randn(1536, 8960, generator=g).bfloat16().to(DEV)
+    b = torch.randn(1537, generator=g).to(DEV)[1:]
+    assert K.tiles_parts(x, w, b) == 1 < K.tiles_parts(x, w, b.clone())
+    got, want = Linear(w, b)(x).double().cpu(), x.double().cpu() @ w.double().cpu().T + b.double().cpu()
+    # the bias and the result are rounded to bfloat16, and float32 sums of 8,960 terms
+    assert bool(((got - want).abs() <= 2.0 ** -8 * (want.abs() + b.double().cpu().abs()) + 8960 * 2.0 ** -24 * (x.double().cpu().abs() @ w.double().cpu().abs().T)).all())
