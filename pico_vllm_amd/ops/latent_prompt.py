@@ -36,7 +36,8 @@ class LatentPrompt:
         if tuple(uk.shape) != (heads * dim, rank) or tuple(uv.shape) != (heads * value_dim, rank) or uk.dtype != torch.bfloat16 \
                 or uv.dtype != torch.bfloat16 or not uk.is_contiguous() or not uv.is_contiguous():
             raise KernelError("latent prompt: the heads' matrices must be contiguous bfloat16 [heads * entries, latent]")
-        self.uk, self.uv = uk, uv
+        # (read in sixteens of bytes)
+        self.uk, self.uv = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (uk, uv))
         self.lib = library.latent_prompt_library(dim, rot_dim, value_dim, rank)
         self.slots = max(1, 2 * compute_units() // heads)      # workgroups a head: two a compute unit in all
         self.least = 4                                         # tiles of keys that a workgroup has at least

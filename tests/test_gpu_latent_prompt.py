@@ -145,3 +145,14 @@ def test_single_tokens_beside_portions_through_the_layer():
     new, old = run(True), run(False)
     assert (new[:2].float() - old[:2].float()).norm() <= TOL * old[:2].float().norm()
     assert (new.float() - old.float()).norm() <= 2 * TOL * old.float().norm()
+
+
+def test_matrices_of_the_heads_that_start_anywhere():
+    # a checkpoint's tensors may be views on the GPU: those that start on no 16 bytes are copied once
+    sizes, seqs = SIZES[1], [(40, 70)]
+    x = inputs(*sizes, seqs)
+    want = served(x, *sizes, seqs)
+    for name in ("uk", "uv"):
+        odd = torch.empty(x[name].numel() + 1, dtype=torch.bfloat16, device=DEV)[1:].view(x[name].shape)
+        x[name] = odd.copy_(x[name])
+    assert torch.equal(served(x, *sizes, seqs), want)
