@@ -68,6 +68,10 @@ class ModelRunner:
         self.storage = CacheStorage(self.manager, specs, model.dtype, self.device)
         self.max_pages = -(-max_seq_len // page_size)
         self.max_seq_len = max_seq_len
+        # with the cache laid out, what is left is for activations and workspaces alike: a prompt must not run out of memory for
+        # keys and values that are laid out only because that is faster
+        if self.device.type == "cuda":
+            model.limit_workspaces(torch.cuda.mem_get_info(self.device)[0] // 2)
         # a decode batch is padded to the power of two its graph was captured at: rows for that too
         # (and a recorded prompt step has a sequence of filler, and may have padded single tokens in front)
         padded = _bucket(min(max_seqs, max_graph_batch))

@@ -13,7 +13,7 @@ from .kernels import KernelError, _check, _check_cache2, _check_table, _ptr, _st
 c_float = ctypes.c_float
 TILE = 64                    # keys of a tile (csrc/latent_prompt.hip)
 QUERIES = 128                # queries of a workgroup
-MAX_BYTES = 1 << 31          # of the keys and values that a step lays out
+MAX_BYTES = 1 << 31          # of the keys and values that a step lays out, where memory for them is left (``LatentPrompt.limit``)
 
 
 def supported(dim: int, rot_dim: int, value_dim: int, rank: int) -> bool:
@@ -41,6 +41,7 @@ class LatentPrompt:
         self.lib = library.latent_prompt_library(dim, rot_dim, value_dim, rank)
         self.slots = max(1, 2 * compute_units() // heads)      # workgroups a head: two a compute unit in all
         self.least = 4                                         # tiles of keys that a workgroup has at least
+        self.limit: Optional[int] = None                       # bytes of a step's workspaces, if something limits them
 
     def gain(self, portions, singles: int) -> float:
         """Microseconds that a step's portions, pairs (new tokens, context), are expected to take less here than in the latent's space.
@@ -79,7 +80,7 @@ class LatentPrompt:
             return None
         need = sum(-(-int(c) // TILE) for c in ctx.host["context_lens"][lead:real])
         behind = -(-ctx.num_tokens // TILE) if filler else 0
-        most = MAX_BYTES // self.tile_bytes - behind
+        most = (MAX_BYTES if self.limit is None else max(0, min(MAX_BYTES, self.limit - self.part_bytes))) // self.tile_bytes - behind
         room = (min(bucket(need), most) if filler else need) + behind
         return (lead, room) if need <= most and (ctx.num_tokens // QUERIES + B) * room < 1 << 30 else None
 
@@ -87,6 +88,11 @@ class LatentPrompt:
     def tile_bytes(self) -> int:
         """Keys and values of a tile."""
         return TILE * (self.heads * (self.d + self.dv) + self.r) * 2
+
+    @property
+    def part_bytes(self) -> int:
+        """Sums of the tiles of queries whose keys several workgroups share."""
+        return self.heads * self.slots * 2 * QUERIES * (self.dv + 4) * 4
 
     def __call__(self, q: torch.Tensor, table: torch.Tensor, cache, block_table: torch.Tensor, ctx, plan: tuple, out: torch.Tensor,
                  gate: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -115,7 +121,7 @@ class LatentPrompt:
         kx = torch.empty(room * H * TILE * self.d, dtype=torch.bfloat16, device=dev)
         vx = torch.empty(room * H * TILE * self.dv, dtype=torch.bfloat16, device=dev)
         kr = torch.empty(room * TILE * self.r, dtype=torch.bfloat16, device=dev)
-        part = torch.empty(H * self.slots * 2 * QUERIES * (self.dv + 4), dtype=torch.float32, device=dev)
+        part = torch.empty(self.part_bytes // 4, dtype=torch.float32, device=dev)
         _check(self.lib, self.lib.pico_latent_prompt(
             _ptr(q), q.stride(0) if T > 1 else q.shape[1], _ptr(table), _ptr(k_cache), _ptr(self.uk), _ptr(self.uv), _ptr(block_table),
             block_table.shape[1], _ptr(cu_seqlens), _ptr(context_lens), num_seqs, first, T, _ptr(kx), _ptr(vx), _ptr(kr), room, _ptr(part),

@@ -120,6 +120,12 @@ class Part:
         return sum(m.weight.numel() * m.weight.element_size() if isinstance(m, Linear) else m.weight_bytes()
                    for m in self._members())
 
+    def limit_workspaces(self, nbytes: int) -> None:
+        """The most that a launch's workspaces may take, beside activations (a few rows a token), from here on: a part that trades
+        them for time keeps to it.  Said by whoever has given the rest of the memory away (``engine.step.ModelRunner``)."""
+        for p in self._sub_parts():
+            p.limit_workspaces(nbytes)
+
     def flops(self, tokens: int, pairs: int) -> float:
         """Floating-point operations of a step with ``tokens`` new tokens and ``pairs`` (query, key) pairs that
         attention looks at (a prompt of T tokens alone: T (T + 1) / 2): two per weight and token for the matrices

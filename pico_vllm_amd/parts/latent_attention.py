@@ -78,6 +78,11 @@ class LatentAttention(Mixer):
         per_head = 2.0 * tokens * H * self.kv_rank * (self.d + self.dv)
         return super().flops(tokens, pairs) + per_head + 2.0 * H * (self.dk + self.kv_rank) * pairs
 
+    def limit_workspaces(self, nbytes: int) -> None:
+        super().limit_workspaces(nbytes)
+        if self.prompt is not None:
+            self.prompt.limit = nbytes
+
     def weight_bytes(self) -> int:
         return super().weight_bytes() + sum(t.numel() * t.element_size() for t in (self.uk_t, self.uv_t))
 

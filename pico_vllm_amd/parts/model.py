@@ -166,6 +166,11 @@ class DecoderModel:
     def _all_parts(self):
         return self.layers + [self.final_norm] + [p for _, p in self.before + self.after + self.mix]
 
+    def limit_workspaces(self, nbytes: int) -> None:
+        """The most that the workspaces of a launch may take (``Part.limit_workspaces``)."""
+        for p in self._all_parts():
+            p.limit_workspaces(nbytes)
+
     def graph_variant(self, ctx) -> tuple:
         """The host-side choices of all parts for this step, each distinct one once (layers of one kind choose
         alike): part of the key under which a prompt step is recorded."""
