@@ -29,7 +29,10 @@ class LatentAttention(Mixer):
     (q'_h = [Wuk_h^T q_h[:d] | rot(q_h[d:])], ``kv_rank + r`` entries), attention runs with ONE key/value head whose key
     is [c | rot(kr)] and whose value is c, and a head's output (in the latent's space) goes through Wuv_h afterwards.
     That is attention with keys of kv_rank + r and values of kv_rank entries, which this package's attention kernels
-    serve (the value pages are laid out [dv, page], so c is stored a second time as the value column).
+    serve (the value pages are laid out [dv, page], so c is stored a second time as the value column).  Prompt portions
+    whose tokens earn it are served with the heads' own keys and values instead, made from the latents once a key for the
+    launch alone (``ops.latent_prompt``: bfloat16, sizes of whole 32s): d + r + dv multiplications a head and (query, key)
+    pair in place of 2 kv_rank + r.
     ``gate_heads``: head h's output is multiplied by sigmoid(Wg x)_h (in the latent's space, where the attention kernel
     does it: a number a head commutes with Wuv_h).
     Norms, angles, scores and softmax are float32.  ``names``: the tensors' names behind the part's prefix."""
@@ -75,8 +78,11 @@ class LatentAttention(Mixer):
 
     def flops(self, tokens: int, pairs: int) -> float:
         H = self.heads
+        # the heads' matrices meet every token once, be it as queries and outputs or as keys and values
         per_head = 2.0 * tokens * H * self.kv_rank * (self.d + self.dv)
-        return super().flops(tokens, pairs) + per_head + 2.0 * H * (self.dk + self.kv_rank) * pairs
+        # a prompt alone may be served with the heads' own keys and values; everything else counts as in the latent's space
+        own = self.prompt is not None and tokens > 1 and pairs == tokens * (tokens + 1) // 2 and self.prompt.gain([(tokens, tokens)], 0) > 0
+        return super().flops(tokens, pairs) + per_head + 2.0 * H * (self.d + self.r + self.dv if own else self.dk + self.kv_rank) * pairs
 
     def limit_workspaces(self, nbytes: int) -> None:
         super().limit_workspaces(nbytes)
