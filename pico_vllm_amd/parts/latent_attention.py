@@ -31,7 +31,7 @@ class LatentAttention(Mixer):
     That is attention with keys of kv_rank + r and values of kv_rank entries, which this package's attention kernels
     serve (the value pages are laid out [dv, page], so c is stored a second time as the value column).  Prompt portions
     whose tokens earn it are served with the heads' own keys and values instead, made from the latents once a key for the
-    launch alone (``ops.latent_prompt``: bfloat16, sizes of whole 32s): d + r + dv multiplications a head and (query, key)
+    launch alone (``ops.latent_prompt``: bfloat16; d, r and dv of 32, 64 or 128, latents of whole 32s up to 256): d + r + dv multiplications a head and (query, key)
     pair in place of 2 kv_rank + r.
     ``gate_heads``: head h's output is multiplied by sigmoid(Wg x)_h (in the latent's space, where the attention kernel
     does it: a number a head commutes with Wuv_h).

@@ -223,15 +223,21 @@ def test_gemm_tiles(K, M, N, K_, name):
     assert torch.equal(K.gemm_tiles(a[:(M + 1) // 2], w, b, epi, clip), out[:(M + 1) // 2])
 
 
-@pytest.mark.parametrize("tiles", [1, 7, 8, 9, 63, 255, 257, 511, 513, 520, 767, 1025, 1031])
+@pytest.mark.parametrize("tiles", [1, 7, 8, 9, 63, 255, 256, 257, 511, 512, 513, 519, 520, 521, 767, 768, 769, 1023, 1025, 1031])
 def test_gemm_tiles_deals_every_tile_once(K, tiles):
-    # grids of every remainder by eight, last rounds of one tile, of an eighth less one, of one tile a compute unit and more;
-    # a tile is made of exact sums (whole numbers), so a tile that is left out or written by another shows
+    # 100 rows and an inner size of one stage: so many tiles of 192 columns, the rows of one each, which the cost of a round gives to workgroups
+    # that a compute unit has to itself up to 256 of them and to two a unit beyond.  Grids of every remainder by eight, whole rounds of
+    # 512, last rounds of one tile, of an eighth less one, of one tile a compute unit and more, behind one round and two.  A tile
+    # is made of exact sums (whole numbers), so one that is left out or written by another shows
     g = torch.Generator(device=DEV).manual_seed(tiles)
+    N = 192 * tiles - 32
     a = torch.randint(-4, 5, (100, 64), device=DEV, generator=g).bfloat16()
-    w = torch.randint(-4, 5, (64 * tiles, 64), device=DEV, generator=g).bfloat16()
+    w = torch.randint(-4, 5, (N, 64), device=DEV, generator=g).bfloat16()
+    want = a.float() @ w.float().T
     for _ in range(2):
-        assert torch.equal(K.gemm_tiles(a, w, None, K.EPI_F32), a.float() @ w.float().T)
+        junk = torch.full((100, N), float("nan"), device=DEV)
+        del junk                                                  # (what the next tensor of this size finds in its memory)
+        assert torch.equal(K.gemm_tiles(a, w, None, K.EPI_F32), want)
 
 
 @pytest.mark.parametrize("M", [65, 700])
