@@ -24,9 +24,10 @@
 //   4. one workgroup a row finds t* among what is listed (classes of 2^9 patterns, then of one), then the chunk, the
 //      thread, and the token at which the running sum of the kept e passes u times their total, ties counted in
 //      vocabulary order (sample_pick_kernel).
-// The search sums e as whole numbers of 2^-40 (fewer bits from 2^23 tokens on): such sums are the same in any order, so they are
-// made with atomics, and off by 7e-8 of a row's mass at most.  All other sums run in a fixed order: a row's result depends
-// on its inputs only.  e is the hardware's exponential (__expf: 2^(x log2 e)) in every launch alike: what a token weighs
+// The search sums e as whole numbers of 2^-40 (fewer bits beyond 2^23 tokens): such sums are the same in any order, so they are
+// made with atomics.  Each term is rounded down by less than 2^-40 of the largest, which is 1: V tokens lose less than V 2^-40 of a mass
+// of 1 or more, 1.4e-7 at 151,936 tokens (7e-8 on average), 7.6e-6 at 2^23.  All other sums run in a fixed order: a row's result
+// depends on its inputs only.  e is the hardware's exponential (__expf: 2^(x log2 e)) in every launch alike: what a token weighs
 // must be the same bits wherever it is asked.
 // (Five rounds of 63 thresholds and float sums, each a launch that read the row, in place of 2 and the search of 4: the chain 62 us for 8 rows
 // of 151,936 logits with top_p < 1, 32 so; 64 rows 159, 65; one row 63, 30; 5,000 logits 34, 24.  Where a class holds most of a row
