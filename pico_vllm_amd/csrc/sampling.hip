@@ -31,8 +31,8 @@
 // must be the same bits wherever it is asked.
 // (Five rounds of 63 thresholds and float sums, each a launch that read the row, in place of 2 and the search of 4: the chain 62 us for 8 rows
 // of 151,936 logits with top_p < 1, 32 so; 64 rows 159, 65; one row 63, 30; 5,000 logits 34, 24.  Where a class holds most of a row
-// the last launch's one workgroup has it all: logits within a twentieth of each other 61, 58.  Elements that are all alike are listed
-// once: all logits equal 28, one by one 93; logits rounded to halves 29, 38.)
+// the last launch's one workgroup has it all: logits within a twentieth of each other 61, 58.  Where a chunk's elements are most of it
+// and all alike they are listed once: all logits equal 28, one by one 93.)
 #include "common.h"
 
 #define SAMPLE_CHUNKS 32            // as ARGMAX_CHUNKS below: the two share the first launch
@@ -47,7 +47,7 @@
 #define SAMPLE_ONE 0x3f800000u      // the bit pattern of 1.0f
 #define SAMPLE_LISTED 4864          // elements of a class that a chunk lists at most (all of a chunk up to 155,648 tokens); more are read again
 #define SAMPLE_ROWS 256             // rows with a list at a time
-#define SAMPLE_ALIKE 256            // from so many on a chunk looks whether they are one value, and then lists it once
+#define SAMPLE_ALIKE 256            // from so many on, and half of it, a chunk looks whether they are one value, and then lists it once
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -211,7 +211,7 @@ __device__ __forceinline__ double block_prefix_f64(double v, double* wave_tot, d
   return before + incl - v;
 }
 template <int THREADS>
-__device__ __forceinline__ int block_prefix_i32(int v, int* wave_tot) {
+__device__ __forceinline__ int block_prefix_i32(int v, int* wave_tot, int& total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int incl = v;
 #pragma unroll
@@ -223,7 +223,12 @@ __device__ __forceinline__ int block_prefix_i32(int v, int* wave_tot) {
   if (lane == 63) wave_tot[wave] = incl;
   __syncthreads();
   int before = 0;
-  for (int k = 0; k < wave; k++) before += wave_tot[k];
+  total = 0;
+#pragma unroll
+  for (int k = 0; k < THREADS / 64; k++) {
+    if (k < wave) before += wave_tot[k];
+    total += wave_tot[k];
+  }
   return before + incl - v;
 }
 
@@ -317,20 +322,22 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
       if (e > 0.f) s += (double)e;
     });
   } else {
-    uint32_t lo = 0xffffffffu, hi = 0u;
     each([&](float e) {
-      const uint32_t b = __float_as_uint(e);
-      const int k = (int)sample_class(b);
+      const int k = (int)sample_class(__float_as_uint(e));
       if (k > above && e > 0.f) s += (double)e;
-      if (k == above) n++, lo = min(lo, b), hi = max(hi, b);
+      n += k == above;
     });
-    const int before = block_prefix_i32<SAMPLE_THREADS>(n, wn);
+    int all;
+    const int before = block_prefix_i32<SAMPLE_THREADS>(n, wn, all);
     uint32_t* mylist = list + ((size_t)row * SAMPLE_CHUNKS + c) * room;
-    int at = before, all = 0;
-#pragma unroll
-    for (int k = 0; k < SAMPLE_THREADS / 64; k++) all += wn[k];
+    int at = before;
     bool alike = false;
-    if (all >= SAMPLE_ALIKE) {                             // the same for all threads
+    if (all >= SAMPLE_ALIKE && 2 * all >= ch.end - ch.begin) {      // the same for all threads; fewer are listed as fast as they are looked at
+      uint32_t lo = 0xffffffffu, hi = 0u;
+      each([&](float e) {
+        const uint32_t b = __float_as_uint(e);
+        if ((int)sample_class(b) == above) lo = min(lo, b), hi = max(hi, b);
+      });
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) {
         lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
@@ -398,28 +405,28 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
   int kept_n = 0;
   if constexpr (SEARCH) if (tp < 1.0f) {
     const SampleRow r = rows[row];
-    const int number = fin_n[base + my_chunk], listed = number < 0 ? 1 : number;
+    const int number = fin_n[base + my_chunk];
     // the patterns of this chunk's elements of the class, PER threads side by side, four neighbours each: from the list, of which
     // each thread holds the first ones, or, where it did not have room for all, from the logits
     const u32x4* mylist = reinterpret_cast<const u32x4*>(list + (base + my_chunk) * room);
-    const u32x4 held = 4 * part < listed ? mylist[part] : u32x4{0, 0, 0, 0};
+    const u32x4 held = 4 * part < number ? mylist[part] : u32x4{0, 0, 0, 0};
     auto entries = [&](auto use) {                        // use(pattern, how many of it)
-      if (number < 0) {
-        if (part == 0) use(held[0], ~number);
-      } else if (listed <= room) {
+      if ((uint32_t)number <= (uint32_t)room) {
 #pragma unroll
         for (int j = 0; j < 4; j++)
-          if (4 * part + j < listed) use(held[j], 1);
-        for (int k0 = part + PER; 4 * k0 < listed; k0 += 4 * PER) {
+          if (4 * part + j < number) use(held[j], 1);
+        for (int k0 = part + PER; 4 * k0 < number; k0 += 4 * PER) {
           u32x4 v[4];
 #pragma unroll
-          for (int k = 0; k < 4; k++) v[k] = 4 * (k0 + k * PER) < listed ? mylist[k0 + k * PER] : u32x4{0, 0, 0, 0};
+          for (int k = 0; k < 4; k++) v[k] = 4 * (k0 + k * PER) < number ? mylist[k0 + k * PER] : u32x4{0, 0, 0, 0};
 #pragma unroll
           for (int k = 0; k < 4; k++)
 #pragma unroll
             for (int j = 0; j < 4; j++)
-              if (4 * (k0 + k * PER) + j < listed) use(v[k][j], 1);
+              if (4 * (k0 + k * PER) + j < number) use(v[k][j], 1);
         }
+      } else if (number < 0) {
+        if (part == 0) use(mylist[0][0], ~number);
       } else {
         const SampleChunk ch = sample_chunk(V, my_chunk);
         for (int i0 = ch.begin + part; i0 < ch.end; i0 += 16 * PER) {
@@ -544,7 +551,8 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
   };
   int my_ties = 0;
   each([&](int, float e) { my_ties += e == thr; return true; });
-  const int ties_before = chosen_ties_before + block_prefix_i32<THREADS>(my_ties, wave_cnt);
+  int all_ties;
+  const int ties_before = chosen_ties_before + block_prefix_i32<THREADS>(my_ties, wave_cnt, all_ties);
   double s = 0.0;
   {
     int tie = ties_before;
