@@ -12,6 +12,7 @@
 #define GT_RELU2 3    // max(x W^T + bias, 0)^2
 #define GT_CLIPPED 5  // W = [gate rows; up rows]: g sigmoid(alpha g) (u + 1), g = min(gate, limit), u = up within -limit .. limit
 #define GT_GELU 7     // gelu(x W^T + bias) with the error function
+#define GT_PARTS 8    // float32 sums of a part of K (of the launches here alone)
 
 struct GemmArgs {
   const bf16_t* X;
@@ -21,12 +22,13 @@ struct GemmArgs {
   int M, cols, K, ldx, ldw, ldo;     // cols: output columns of this launch
   int up;                            // paired epilogues: from a gate row of W to the up row of the same column
   int m_tiles, n_tiles;
-  int splits, part;                  // of K: so many parts of `part` each, a part's sums in out + s M ldo (GT_F32; else one)
+  int splits, part;                  // of K: so many parts of `part` each, a part's sums in out + s M ldo (GT_PARTS; else one)
   float limit, alpha;
 };
 
 #define GT_COLS(NB, EPI) (gt_paired(EPI) ? 32 * (NB) : 64 * (NB))     // output columns of a tile
 constexpr bool gt_paired(int epi) { return epi == GT_SWIGLU || epi == GT_CLIPPED; }
+constexpr bool gt_float(int epi) { return epi == GT_F32 || epi == GT_PARTS; }
 
 // FEW: with the exponential of the weight-streaming product
 template <int EPI, bool FEW>
@@ -67,19 +69,19 @@ template <int MB, int NB, int EPI, int SETS>
 __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const GemmArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  typedef TileStream<MB, NB, SETS, EPI == GT_F32> TS;
+  typedef TileStream<MB, NB, SETS, EPI == GT_PARTS> TS;
   TS ts(smem);
   constexpr int TM = 64 * MB, TN = 64 * NB, COLS = gt_paired(EPI) ? TN / 2 : TN;      // output columns of a tile
-  const int tiles = a.m_tiles * a.n_tiles * (EPI == GT_F32 ? a.splits : 1);
+  const int tiles = a.m_tiles * a.n_tiles * (EPI == GT_PARTS ? a.splits : 1);
   if (ts_tile(0, tiles) < 0) return;
   TileRowsSource<MB> xs;
   TileRowsSource<NB> ws;
   auto aim = [&](int t) {
     int m, n;
-    ts_place(a.m_tiles, a.n_tiles * (EPI == GT_F32 ? a.splits : 1), t, m, n);
-    const int m0 = m * TM, s = EPI == GT_F32 ? n / a.n_tiles : 0, k0 = s * a.part, k = EPI == GT_F32 ? min(a.part, a.K - k0) : a.K;
+    ts_place(a.m_tiles, a.n_tiles * (EPI == GT_PARTS ? a.splits : 1), t, m, n);
+    const int m0 = m * TM, s = EPI == GT_PARTS ? n / a.n_tiles : 0, k0 = s * a.part, k = EPI == GT_PARTS ? min(a.part, a.K - k0) : a.K;
     n -= s * a.n_tiles;
-    if (EPI == GT_F32) ts.k_end = k;
+    if (EPI == GT_PARTS) ts.k_end = k;
     xs.rsrc = ts_buffer(a.X + (size_t)m0 * a.ldx + k0, ((long long)(a.M - m0 - 1) * a.ldx + k) * 2);
 #pragma unroll
     for (int j = 0; j < 2 * MB; j++) xs.off[j] = (uint32_t)(ts.row(j) * a.ldx) * 2;
@@ -99,17 +101,17 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
       for (int j = 0; j < 2 * NB; j++) ws.off[j] = (uint32_t)(ts.row(j) * a.ldw) * 2;
     }
   };
-  ts.run(tiles, EPI == GT_F32 ? a.part : a.K, xs, ws, aim, [&](int t) {
+  ts.run(tiles, EPI == GT_PARTS ? a.part : a.K, xs, ws, aim, [&](int t) {
     // lane (l, h): row l of a block of X, tile rows 8 (r / 4) + 4 h + r % 4 of a block of W in register r
     int mt, nt;
-    ts_place(a.m_tiles, a.n_tiles * (EPI == GT_F32 ? a.splits : 1), t, mt, nt);
-    const int split = EPI == GT_F32 ? nt / a.n_tiles : 0;
+    ts_place(a.m_tiles, a.n_tiles * (EPI == GT_PARTS ? a.splits : 1), t, mt, nt);
+    const int split = EPI == GT_PARTS ? nt / a.n_tiles : 0;
     nt -= split * a.n_tiles;
     const int l = ts.lane & 31, h = ts.lane >> 5;
     // of the bias what this lane adds, all of it asked for at once (a pair at a time between the outputs it was waited for each
     // time: 32 us of a call of 2,048 rows, 13,440 columns).  Not with float32 results, which do
     // little but store: of a 152,064 x 3,584 output matrix without a bias 740 rows took 943 us so, 762 to 805 without, 32 rows 221 and 211.
-    constexpr bool AHEAD = !gt_paired(EPI) && EPI != GT_F32;
+    constexpr bool AHEAD = !gt_paired(EPI) && !gt_float(EPI);
     gt_f32x4 bias[AHEAD ? NB : 1][4];
     if (AHEAD) {
 #pragma unroll
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
           }
         }
         const int blk = (ts.wave & 1) * NB + j;
-        if (EPI == GT_F32) {
+        if (gt_float(EPI)) {
           float* o = (float*)a.out + ((size_t)split * a.M + m) * a.ldo;
 #pragma unroll
           for (int q = 0; q < 4; q++) {
@@ -244,7 +246,7 @@ static int gt_run(GemmArgs a, hipStream_t stream) {
   if (rc || first == cols) return rc;
   a.W += (size_t)first * a.ldw;
   if (a.bias) a.bias += first;
-  a.out = (char*)a.out + (size_t)first * (EPI == GT_F32 ? 4 : 2);
+  a.out = (char*)a.out + (size_t)first * (gt_float(EPI) ? 4 : 2);
   a.cols = cols - first;
   return run(gt_choose(a.M, a.cols, stages, gt_paired(EPI), false, all, cost));
 }
@@ -348,7 +350,7 @@ extern "C" int pico_gemm_tiles_split(const void* X, const void* W, const float* 
   PICO_REQUIRE((long long)M * ldx < (1LL << 30) && (long long)N * ldw < (1LL << 30), "pico_gemm_tiles_split: an operand spans 2^31 bytes or more");
   if (M == 0) return 0;
   GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, nullptr, parts, M, N, K, ldx, ldw, N, 0, 0, 0, splits, gt_part(K, splits), 0.f, 0.f};
-  const int rc = gt_run<GT_F32>(a, stream);
+  const int rc = gt_run<GT_PARTS>(a, stream);
   if (rc) return rc;
   const long long eights = (long long)M * N / 8;
   gemm_join_kernel<<<(unsigned)((eights + 255) / 256), 256, 0, stream>>>(parts, splits, bias, (bf16_t*)out, eights, N);
