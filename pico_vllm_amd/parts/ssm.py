@@ -28,9 +28,8 @@ class SelectiveStateSpace(Mixer):
     graph_safe_prompts = True
 
     # In the bfloat16 engine a step with a prompt portion cuts its sequences into chunks of this many tokens that run
-    # side by side (``kernels.selective_scan``); decided from the step's shape alone.  (16 state elements: as many as
-    # ``kernels.scan_chunk`` says, from a dozen tokens on that are not a sequence's only one: 16 tokens of 3,072 channels 18 us, 28
-    # walked whole; 64: 21 and 91; 30 single tokens and 16: 34 and 36.)  The 32-bit engine walks every
+    # side by side (``kernels.selective_scan``); decided from the step's shape and its sequences' lengths.  (16 state elements: where
+    # ``kernels.scan_in_chunks`` says so, as many tokens as ``kernels.scan_chunk`` says.)  The 32-bit engine walks every
     # sequence whole, so that its sums do not depend on how a prompt was cut.
     CHUNK, CHUNKED_FROM = 64, 128
 
@@ -76,6 +75,16 @@ class SelectiveStateSpace(Mixer):
     def forward(self, x: torch.Tensor, ctx: StepContext, cache) -> torch.Tensor:
         return self.o.partial(self.mix(x, ctx, cache))
 
+    @staticmethod
+    def _longest(ctx: StepContext) -> int:
+        """Tokens of the step's longest sequence; of a recorded step, whose lengths another replay shares only in sum, what all but one
+        leave to it."""
+        if "longest_sequence" not in ctx.shared:
+            cu, B = ctx.host.get("cu_seqlens"), ctx.num_seqs
+            alone = cu is None or ctx.host.get("filler", 0)
+            ctx.shared["longest_sequence"] = ctx.num_tokens - B + 1 if alone else int(max(cu[b + 1] - cu[b] for b in range(B)))
+        return ctx.shared["longest_sequence"]
+
     def mix(self, x: torch.Tensor, ctx: StepContext, cache) -> torch.Tensor:
         """y * silu(z) [T, inner] in front of the output projection."""
         I, N, R = self.inner, self.state, self.dt_rank
@@ -85,7 +94,7 @@ class SelectiveStateSpace(Mixer):
         dt_pre = self.dt_proj(dbc[:, :R], out_dtype=torch.float32)                   # step sizes stay float32 from here on
         chunk = 0
         if kernels.scan_rows_held(N, self.act_dtype):
-            if not ctx.all_decode and ctx.num_tokens - ctx.num_seqs >= 12:
+            if not ctx.all_decode and kernels.scan_in_chunks(ctx.num_tokens, I, ctx.num_seqs, self._longest(ctx)):
                 chunk = kernels.scan_chunk(ctx.num_tokens, I, ctx.num_seqs)
         elif self.act_dtype == torch.bfloat16 and not ctx.all_decode and ctx.num_tokens >= self.CHUNKED_FROM:
             chunk = self.CHUNK
