@@ -352,8 +352,8 @@ extern "C" int pico_gla_scan(const void* x, int ldx, int dtype, int q_col, int k
                "pico_gla_scan: chunks need room for their states and must cover the step's tokens");
   if (num_seqs == 0 || T == 0) return 0;
   // A step of few tokens with one wave a workgroup: blocks of two tokens, so that a thread fetches next to nothing for tokens that
-  // are not there.  (12 heads of 32 x 64, 8 requests of one token: 3.7 us, in blocks of 16 6.2; four waves of a workgroup share a
-  // block's values and gain nothing.)
+  // are not there.  (12 heads of 32 x 64, 8 requests of one token: 3.7 us, in blocks of 16 6.2.  With more waves a thread's share of a block
+  // is smaller: 64 x 128 5.9, with a value and 32 keys a lane 6.1.)
   const bool few = chunk == 0 && T <= 2 * num_seqs;
   const int wide = dv % 4 == 0 && ((uintptr_t)state | (uintptr_t)ws) % 16 == 0, vb = (dv + 63) / 64;
 #define GLA_ARGS(TT)                                                                                                       \
