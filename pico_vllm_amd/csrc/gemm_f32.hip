@@ -1,24 +1,23 @@
-// True float32 matrix product C = A W^T (+ bias) on the float32 matrix instruction (v_mfma_f32_32x32x2_f32: products and
-// sums in float32, no reduced precision).  Every output element is accumulated in an order that depends on K alone, so a
-// row's result does not depend on how many other rows the call has, nor on how the work was dealt out.
+// True float32 matrix product C = A W^T (+ bias): every number is three bfloat16 pieces that hold all of its 24 bits, and the products
+// of the pieces run on the bfloat16 matrix instruction (split3.h; six instructions of 16 k are 6/16 of the float32 instruction's time).
+// Every output element is accumulated in an order that depends on K alone, so a row's result does not depend on how many
+// other rows the call has, nor on how the work was dealt out.
 //
-// The sum is a tree over k: 16 products one after the other (eight instructions on one accumulator), 16 such sums (256),
-// then the `ranges` of K, each of as many 256s as there are ranges (both about sqrt(K / 256)): four short chains in place
-// of one long one.  Error against 64 bits, in units of 2^-24 of the result's rms, measured: 1.93 at K = 1,536, 2.12 at
-// 8,960, 2.34 at 27,648 (plain FMA in a tree of radix 16 over four levels: 1.96, 2.28, 2.39; one running sum would give
-// 0.2 sqrt(K)).
+// The sum is a tree over k: 16 products an instruction, 16 instructions (256 k) on one accumulator, then the `ranges` of K, each of
+// as many 256s as there are ranges (both about sqrt(K / 256)); the small terms of a range are one sum beside that, 2^-8 of it.
+// A result that such products cannot give (split3.h) is made again on the float32 instruction, element by element, so that it
+// too depends on its own row and column alone.  Error against 64 bits, in units of 2^-24 of the result's rms, on the float32
+// instruction (16 products a sum, 16 sums) and so: 1.93 and 1.68 at K = 1,536, 2.13 and 1.90 at 8,960, 2.28 and 2.06 at 18,944 (one
+// running sum would give 0.2 sqrt(K)).
 //
-// Bound by the matrix instruction (157 TFLOP/s) from about 64 rows on, by the stream of W below.  A wave owns 32 x 32
-// outputs, so that the tree's four levels are 64 registers and three or four workgroups share a compute unit; its operands come
-// from LDS (64 of 128 B a cycle at most), stages of 32 k.  Tiles that read the same rows of W are neighbours on
-// one die.  Where the tiles alone leave the chip idle (less than two a compute unit) every range of K is a workgroup
-// of its own, its sum goes to a slab, and a second launch adds the slabs in the order in which one workgroup would have.
-// 320 rows, microseconds a call with plain FMA in 64 x 64 tiles and with this: 17,920 x 1,536 575 / 206 (86 TFLOP/s);
-// 1,536 x 8,960 1,421 / 104; 1,536 x 1,536 183 / 32.  2,048 rows of 17,920 x 1,536: 3,299 / 1,120 (101 TFLOP/s; the library's
-// product, which sums in one chain, 1,030).  One row of 151,936 x 1,536: 1,070 / 230 (4.1 TB/s).
-#include "common.h"
+// Over 32 rows bound by the vector instructions that take operands apart (45 % of the time) and by the matrix instruction (44 %), up
+// to there by the stream of W; with few tiles by the chain of a range's stages (0.8 us each).  Tiles that read the same rows
+// of W are neighbours on one die.  Where the tiles alone leave the chip idle (less than two a compute unit) every range of K is a
+// workgroup of its own, its sum goes to a slab, and a second launch adds the slabs in the order in which one workgroup would have.
+// Microseconds on the float32 instruction and so, in one process: 320 rows of 17,920 x 1,536 183 / 145, 1,536 x 8,960 103 / 88, 1,536
+// x 1,536 31 / 29; 2,048 rows of 17,920 x 1,536 1,060 / 785; one row of 151,936 x 1,536 212 / 183 (5.1 TB/s), 32 rows 230 / 206.
+#include "split3.h"
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define BK 32          // k of a stage
@@ -34,6 +33,13 @@ __host__ __device__ inline int f32_ranges(int K, int& len) {
   len = per * GROUP;
   return (groups + per - 1) / per;
 }
+
+#define F32_OUT 0x80000000u          // added to an offset: behind the end of any buffer (at most 2^31 - 1 bytes)
+#ifdef __HIP_DEVICE_COMPILE__
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t f32_rows(const float* base, long long rows, int ld, int K) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)min(((rows - 1) * ld + K) * 4, (long long)0x7fffffff), 0x00020000);
+}
+#endif
 
 __device__ __forceinline__ float4 zero_from(float4 v, int k, int K) {
   v.x = k < K ? v.x : 0.f; v.y = k + 1 < K ? v.y : 0.f; v.z = k + 2 < K ? v.z : 0.f; v.w = k + 3 < K ? v.w : 0.f;
@@ -58,11 +64,54 @@ __device__ __forceinline__ float4 fetch4(const bf16_t* row, int k, int K) {
                      bf16_to_f32(row[min(k + 2, K - 1)]), bf16_to_f32(row[min(k + 3, K - 1)]));
 }
 
+// A wave's 32 x 32 block over k_first .. k_end on the float32 instruction, straight from memory: lane (l, half) has row l of A and of
+// W (`a_row`, `w_row`) and of 16 k the half'th eight.
+template <typename TA>
+__device__ __forceinline__ s3_f32x16 plain_block(const TA* a_row, const float* w_row, int k_first, int k_end, int K, int half) {
+  s3_f32x16 sum = {}, group = {};
+  for (int k0 = k_first; k0 < k_end; k0 += 16) {
+    s3_f32x16 few = {};
+    const int k = k0 + 8 * half;
+    const float4 a0 = zero_from(fetch4<false>(a_row, k, K), k, K), a1 = zero_from(fetch4<false>(a_row, k + 4, K), k + 4, K);
+    const float4 w0 = zero_from(fetch4<false>(w_row, k, K), k, K), w1 = zero_from(fetch4<false>(w_row, k + 4, K), k + 4, K);
+    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, w0.x, few, 0, 0, 0);
+    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, w0.y, few, 0, 0, 0);
+    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.z, w0.z, few, 0, 0, 0);
+    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.w, w0.w, few, 0, 0, 0);
+    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, w1.x, few, 0, 0, 0);
+    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, w1.y, few, 0, 0, 0);
+    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, w1.z, few, 0, 0, 0);
+    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, w1.w, few, 0, 0, 0);
+    group += few;
+    if ((k0 - k_first) % GROUP == GROUP - 16) {
+      sum += group;
+      group = {};
+    }
+  }
+  return sum + group;
+}
+
+// What a range of K comes to: the sums of its large and of its small terms; results that split3.h says are made again.
+template <typename TA>
+__device__ __forceinline__ s3_f32x16 range_sum(const s3_f32x16& big, const s3_f32x16& small, const TA* a_row, const float* w_row, int k_first,
+                                               int k_end, int K, int half) {
+  s3_f32x16 sum = (big + small) * S3_BACK;
+  bool odd = false;
+#pragma unroll
+  for (int r = 0; r < 16; r++) odd = odd || s3_redo(sum[r]);
+  if (__any(odd)) {
+    const s3_f32x16 plain = plain_block(a_row, w_row, k_first, k_end, K, half);
+#pragma unroll
+    for (int r = 0; r < 16; r++) sum[r] = s3_redo(sum[r]) ? plain[r] : sum[r];
+  }
+  return sum;
+}
+
 // A [M, K] row stride lda; W [N, K] row stride ldw; C [M, N] row stride ldc.  TA is the storage type of A (float, or
 // bfloat16 bits that are widened on load).  WM x 2 waves of 32 x 32 outputs.  grid (8 ceil(n_tiles / 8) m_tiles, 1) with
 // `slabs` null, (.., ranges) with slabs [ranges, M, N].
 template <typename TA, int WM, bool VEC>
-__global__ __launch_bounds__(128 * WM, 4) void gemm_f32_kernel(const TA* __restrict__ A, const float* __restrict__ W,
+__global__ __launch_bounds__(128 * WM, 2) void gemm_f32_kernel(const TA* __restrict__ A, const float* __restrict__ W,
                                                                const float* __restrict__ bias, float* __restrict__ C,
                                                                float* __restrict__ slabs, int M, int N, int K, int lda,
                                                                int ldw, int ldc, int m_tiles) {
@@ -111,9 +160,10 @@ __global__ __launch_bounds__(128 * WM, 4) void gemm_f32_kernel(const TA* __restr
     for (int i = 0; i < NA; i++) *reinterpret_cast<float4*>(&As[b][a_at[i]]) = edge ? zero_from(av[i], k0 + kc, K) : av[i];
   };
 
-  f32x16 l1 = {}, l2 = {}, l3 = {};
-  const float* ap = &As[0][(32 * wm + l) * ST + 4 * half];
-  const float* wp = &Ws[0][(32 * wn + l) * ST + 4 * half];
+  s3_f32x16 big = {}, small = {}, l2 = {}, l3 = {};
+  const float* ap = &As[0][(32 * wm + l) * ST + 8 * half];
+  const float* wp = &Ws[0][(32 * wn + l) * ST + 8 * half];
+  const int n = n0 + 32 * wn + l;
   fetch(k_first);
   put(0, k_first);
   int buf = 0;
@@ -124,37 +174,24 @@ __global__ __launch_bounds__(128 * WM, 4) void gemm_f32_kernel(const TA* __restr
     const float* a = ap + buf * (TM * ST);
     const float* w = wp + buf * (TN * ST);
 #pragma unroll
-    for (int g = 0; g < BK; g += 16) {
-      // 16 k: this half of the lanes holds 0..3 and 8..11 (or 4..7 and 12..15) of them
-      const float4 a0 = *reinterpret_cast<const float4*>(a + g), a1 = *reinterpret_cast<const float4*>(a + g + 8);
-      const float4 w0 = *reinterpret_cast<const float4*>(w + g), w1 = *reinterpret_cast<const float4*>(w + g + 8);
-      f32x16 l0 = {};
-      l0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, w0.x, l0, 0, 0, 0);
-      l0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, w0.y, l0, 0, 0, 0);
-      l0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.z, w0.z, l0, 0, 0, 0);
-      l0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.w, w0.w, l0, 0, 0, 0);
-      l0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, w1.x, l0, 0, 0, 0);
-      l0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, w1.y, l0, 0, 0, 0);
-      l0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, w1.z, l0, 0, 0, 0);
-      l0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, w1.w, l0, 0, 0, 0);
-      l1 += l0;
-    }
+    for (int g = 0; g < BK; g += 16)                    // 16 k: this half of the lanes holds 0..7 (or 8..15) of them
+      split_multiply<sizeof(TA) == 2>(split8<true>(*reinterpret_cast<const float4*>(a + g), *reinterpret_cast<const float4*>(a + g + 4)),
+                                      split8<false>(*reinterpret_cast<const float4*>(w + g), *reinterpret_cast<const float4*>(w + g + 4)), big, small);
     if (more) put(buf ^ 1, k0 + BK);
     const int done = k0 + BK - k_first;
     if (done % GROUP == 0) {
-      l2 += l1;
-      l1 = {};
+      l2 += big;
+      big = {};
     }
-    if (!slabs && (done % len == 0 || !more)) {      // the same for all threads
-      l3 += l1 + l2;
-      l1 = {};
+    if (done % len == 0 || !more) {                      // the same for all threads
+      l3 += range_sum(l2 + big, small, A + (size_t)min(m0 + 32 * wm + l, M - 1) * lda, W + (size_t)min(n, N - 1) * ldw, k0 / len * len, min(K, k0 + BK), K, half);
+      big = {};
       l2 = {};
+      small = {};
     }
   }
-  const int n = n0 + 32 * wn + l;
   if (n >= N) return;
   const float b = !slabs && bias ? bias[n] : 0.f;
-  if (slabs) l3 = l1 + l2;
   float* out = slabs ? slabs + (size_t)blockIdx.y * M * N : C;
   const int ldo = slabs ? N : ldc;
 #pragma unroll
@@ -164,25 +201,103 @@ __global__ __launch_bounds__(128 * WM, 4) void gemm_f32_kernel(const TA* __restr
   }
 }
 
-// The same sums where both operands are float32 rows of whole aligned fours: a stage goes from memory straight to one of NBUF LDS
-// buffers (buffer_load .. lds, eight rows of 128 bytes an instruction, their sixteen-byte chunks xor-swizzled by the row so that the
-// operand reads of 16 rows meet every bank once).  The operands of 16 k are read under the products of the 16 before, and their sums
-// join the others under the products behind them; the one barrier of a stage stands where its last operands are in registers.
-// (Through registers, with every wave waiting for its operands and its sums in turn, the matrix instruction was busy 56 % of
-// the time at 320 rows and 67 % at 2,048.)  What lies outside a matrix (rows behind the last, k behind K) arrives as zeros.
-// Up to 32 rows the stream of W bounds a call and workgroups side by side count: two buffers (two 220, three 240, four 255 us, 1 row of
-// 151,936 x 1,536).  Microseconds through registers and so: 1 row of 151,936 x 1,536 268 and 230, 32 rows 283 and 266; 17,920 x 1,536
-// 100 rows 114 and 104, 320 211 and 206, 2,048 1,135 and 1,120; 1,536 x 8,960 33 rows 50 and 45, 320 108 and 104.
+// The same sums where both operands are float32 rows of whole aligned fours, up to 32 rows: the stream of W bounds a call.  A
+// stage of 32 k goes from memory straight to one of two LDS buffers (buffer_load .. lds, eight rows of 128 bytes an instruction,
+// their sixteen-byte chunks xor-swizzled by the row so that the operand reads of 16 rows meet every bank once); a wave has 32 x 32
+// outputs, and the one barrier of a stage stands where its operands are in registers.  What lies outside a matrix (rows
+// behind the last, k behind K) arrives as zeros.  (Three buffers instead of two 240 us, four 255, two 220: 1 row of 151,936 x 1,536 on
+// the float32 instruction.  Four where there are few tiles: 1,536 x 8,960 46 us, two 43: a stage's own chain, not memory.)
 // (The operands are read as native vectors: in front of a read of float4, a class, the compiler waits for all copies.)
-constexpr int fs_bytes(int WM) { return (32 * WM + 64) * BK * 4; }
-constexpr int fs_buffers(int WM) { return WM == 1 ? 2 : 3; }
-template <int WM>
-__global__ __launch_bounds__(128 * WM, 3) void gemm_f32_stream_kernel(const float* A, const float* W,
-                                                                      const float* bias, float* C,
-                                                                      float* slabs, int M, int N, int K, int lda,
-                                                                      int ldw, int ldc, int m_tiles) {
+#define FS_STAGE ((32 + 64) * BK * 4)
+__global__ __launch_bounds__(128, 3) void gemm_f32_stream_kernel(const float* A, const float* W, const float* bias, float* C, float* slabs, int M,
+                                                                 int N, int K, int lda, int ldw, int ldc) {
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
-  constexpr int TM = 32 * WM, TN = 64, WAVES = 2 * WM, COPIES = (TM + TN) / 8 / WAVES, NBUF = fs_buffers(WM), STAGE = fs_bytes(WM);
+  __shared__ __attribute__((aligned(1024))) char smem[2 * FS_STAGE];
+  const int n0 = blockIdx.x * 64;
+  int len;
+  f32_ranges(K, len);
+  const int k_first = slabs ? blockIdx.y * len : 0, k_end = slabs ? min(K, k_first + len) : K;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane & 31, half = lane >> 5;
+  const __amdgpu_buffer_rsrc_t as = f32_rows(A, M, lda, K), ws = f32_rows(W + (size_t)n0 * ldw, N - n0, ldw, K);
+  // copy j of this wave brings rows 8 (2 j + wave) .. + 7 of [A's tile | W's tile]; lane: row lane / 8, chunk lane % 8 there
+  uint32_t off[6];
+  const uint32_t kbyte = (uint32_t)(((lane & 7) ^ (4 * wave + (lane >> 4))) << 4);
+#pragma unroll
+  for (int j = 0; j < 6; j++) {
+    const int r = (j * 2 + wave) * 8 + (lane >> 3);
+    off[j] = (uint32_t)(r < 32 ? r * lda : (r - 32) * ldw) * 4;
+  }
+  auto ask = [&](int b, int k0) {
+    const uint32_t k = (uint32_t)k0 * 4 + kbyte, at = k < (uint32_t)K * 4 ? k : F32_OUT;
+#pragma unroll
+    for (int j = 0; j < 6; j++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(j < 2 ? as : ws, (__attribute__((address_space(3))) void*)(smem + b * FS_STAGE + (j * 2 + wave) * 1024), 16,
+                                               off[j] + at, 0, 0, 0);
+  };
+  const int sw = (l >> 1) & 7;                              // of row l and of row 32 + l
+  const char* ap = smem + l * 128;
+  const char* wp = smem + (32 + 32 * wave + l) * 128;
+  s3_f32x16 big = {}, small = {}, l2 = {}, l3 = {};
+  const int n = n0 + 32 * wave + l;
+  ask(0, k_first);
+  ask(1, k_first + BK);
+  int buf = 0;
+  for (int k0 = k_first; k0 < k_end; k0 += BK, buf ^= 1) {
+    // this wave's copies of this stage have landed; behind the barrier all waves'
+    __builtin_amdgcn_s_waitcnt(6 | (7 << 4) | (15 << 8));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 a[2][2], w[2][2];                                 // of 16 k this half of the lanes holds 0..7 (or 8..15)
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int c = ((4 * g + 2 * half + i) ^ sw) << 4;
+        a[g][i] = *reinterpret_cast<const f32x4*>(ap + buf * FS_STAGE + c);
+        w[g][i] = *reinterpret_cast<const f32x4*>(wp + buf * FS_STAGE + c);
+      }
+    // they are in registers, so the buffer may be filled again
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    ask(buf, k0 + 2 * BK);
+#pragma unroll
+    for (int g = 0; g < 2; g++) split_multiply(split8<true>(a[g][0], a[g][1]), split8<false>(w[g][0], w[g][1]), big, small);
+    const int done = k0 + BK - k_first;
+    if (done % GROUP == 0) {
+      l2 += big;
+      big = {};
+    }
+    if (done % len == 0 || k0 + BK >= k_end) {              // the same for all threads
+      l3 += range_sum(l2 + big, small, A + (size_t)min(l, M - 1) * lda, W + (size_t)min(n, N - 1) * ldw, k0 / len * len, min(K, k0 + BK), K, half);
+      big = {};
+      l2 = {};
+      small = {};
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);                        // the last copies (zeros) are in before LDS is given back
+  if (n >= N) return;
+  const float b = !slabs && bias ? bias[n] : 0.f;
+  float* out = slabs ? slabs + (size_t)blockIdx.y * M * N : C;
+  const int ldo = slabs ? N : ldc;
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int m = 8 * (r >> 2) + 4 * half + (r & 3);
+    if (m < M) out[(size_t)m * ldo + n] = slabs ? l3[r] : l3[r] + b;
+  }
+#endif
+}
+
+// The same sums over 32 rows: the operands are taken apart once a workgroup, on their way from memory through registers to LDS,
+// where a stage of 32 k lies as three planes of bfloat16 rows (64 bytes, their sixteen-byte chunks xor-swizzled by the row: reads of
+// eight rows and writes of two meet every bank once).  Four waves (2 x 2) of 32 x 32 NW outputs.  A stage's numbers are asked for
+// AHEAD stages ahead, lie in registers, and are taken apart under the products of the stage in front.
+constexpr int fp_plane(int NW) { return (64 + 64 * NW) * BK * 2; }
+template <int NW, int AHEAD>
+__global__ __launch_bounds__(256, NW == 1 && AHEAD == 2 ? 3 : 2) void gemm_f32_planes_kernel(const float* A, const float* W, const float* bias, float* C, float* slabs,
+                                                                               int M, int N, int K, int lda, int ldw, int ldc, int m_tiles) {
+#ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
+  constexpr int TM = 64, TN = 64 * NW, PLANE = fp_plane(NW), STAGE = 3 * PLANE, PIECES = (TM + TN) / 64;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   // dies take workgroups in turn: the tiles of one strip of W stay on one die
   const int die = blockIdx.x & 7, local = blockIdx.x >> 3;
@@ -193,111 +308,104 @@ __global__ __launch_bounds__(128 * WM, 3) void gemm_f32_stream_kernel(const floa
   const int k_first = slabs ? blockIdx.y * len : 0, k_end = slabs ? min(K, k_first + len) : K;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane & 31, half = lane >> 5;
   const int wm = wave >> 1, wn = wave & 1;
-
-  auto source = [](const float* base, long long rows, int ld, int K) {
-    const long long bytes = ((rows - 1) * ld + K) * 4;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)min(bytes, (long long)0x7fffffff), 0x00020000);
-  };
-  const __amdgpu_buffer_rsrc_t as = source(A + (size_t)m0 * lda, M - m0, lda, K), ws = source(W + (size_t)n0 * ldw, N - n0, ldw, K);
-  // copy j of this wave brings rows 8 (j WAVES + wave) .. + 7 of [A's tile | W's tile]; lane: row lane / 8, chunk lane % 8 there
-  uint32_t off[COPIES];
-  const uint32_t kbyte = (uint32_t)(((lane & 7) ^ (4 * (wave & 1) + (lane >> 4))) << 4);
+  const __amdgpu_buffer_rsrc_t as = f32_rows(A + (size_t)m0 * lda, M - m0, lda, K), ws = f32_rows(W + (size_t)n0 * ldw, N - n0, ldw, K);
+  // a thread's pieces: eight k (chunk threadIdx.x % 4 of a stage) of row threadIdx.x / 4 of A's tile, and of every 64 rows of W's
+  const int prow = threadIdx.x >> 2, chunk = threadIdx.x & 3;
+  uint32_t off[PIECES];
+  off[0] = (uint32_t)(prow * lda) * 4;
 #pragma unroll
-  for (int j = 0; j < COPIES; j++) {
-    const int r = (j * WAVES + wave) * 8 + (lane >> 3);
-    off[j] = (uint32_t)(r < TM ? r * lda : (r - TM) * ldw) * 4;
-  }
-  auto ask = [&](int b, int k0) {
-    const uint32_t k = (uint32_t)k0 * 4 + kbyte, at = k < (uint32_t)K * 4 ? k : 0x80000000u;
+  for (int j = 1; j < PIECES; j++) off[j] = (uint32_t)((prow + 64 * (j - 1)) * ldw) * 4;
+  char* put_at = smem + prow * 64 + ((chunk ^ ((prow >> 1) & 3)) << 4);
+  f32x4 raw[AHEAD][PIECES][2];
+  auto ask = [&](int set, int k0) {
+    const uint32_t k = (uint32_t)(k0 + 8 * chunk) * 4, end = (uint32_t)K * 4;
 #pragma unroll
-    for (int j = 0; j < COPIES; j++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(j * WAVES * 8 < TM ? as : ws, (__attribute__((address_space(3))) void*)(smem + b * STAGE + (j * WAVES + wave) * 1024),
-                                               16, off[j] + at, 0, 0, 0);
-  };
-  static_assert(TM % (8 * WAVES) == 0, "a copy of all waves is of one operand");
-  const int sw = (l >> 1) & 7;                              // of row l and of row 32 + l
-  const char* ap = smem + (32 * wm + l) * 128;
-  const char* wp = smem + (TM + 32 * wn + l) * 128;
-  // operands of 16 k: this half of the lanes holds 0..3 and 8..11 (or 4..7 and 12..15) of them
-  f32x4 a0[2], a1[2], w0[2], w1[2];
-  f32x16 l0[2], l1 = {}, l2 = {}, l3 = {};
-  auto read = [&](int b, int g) {
-    const int c0 = ((4 * g + half) ^ sw) << 4, c1 = ((4 * g + 2 + half) ^ sw) << 4;
-    a0[g] = *reinterpret_cast<const f32x4*>(ap + b * STAGE + c0);
-    w0[g] = *reinterpret_cast<const f32x4*>(wp + b * STAGE + c0);
-    a1[g] = *reinterpret_cast<const f32x4*>(ap + b * STAGE + c1);
-    w1[g] = *reinterpret_cast<const f32x4*>(wp + b * STAGE + c1);
-  };
-  // the products of group g, the sums of the group before joining theirs under them
-  auto multiply = [&](int g) {
-    l0[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[g].x, w0[g].x, f32x16{}, 0, 0, 0);
-    l0[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[g].y, w0[g].y, l0[g], 0, 0, 0);
-    l0[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[g].z, w0[g].z, l0[g], 0, 0, 0);
-    l0[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[g].w, w0[g].w, l0[g], 0, 0, 0);
-    l0[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[g].x, w1[g].x, l0[g], 0, 0, 0);
-    l0[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[g].y, w1[g].y, l0[g], 0, 0, 0);
-    l0[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[g].z, w1[g].z, l0[g], 0, 0, 0);
-    l0[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[g].w, w1[g].w, l0[g], 0, 0, 0);
-    l1 += l0[g ^ 1];
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    for (int j = 0; j < PIECES; j++)
 #pragma unroll
-    for (int i = 0; i < 6; i++) {
-      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < 2; i++)
+        raw[set][j][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(j == 0 ? as : ws, off[j] + (k + 16 * i < end ? k + 16 * i : F32_OUT), 0, 0));
   };
-  // what is summed up to k = done (all sums of the groups are in l1)
-  auto close = [&](int done) {
-    if (done % GROUP == 0) {
-      l2 += l1;
-      l1 = {};
-    }
-    if (!slabs && (done % len == 0 || k_first + done >= k_end)) {      // the same for all threads
-      l3 += l1 + l2;
-      l1 = {};
-      l2 = {};
+  auto put = [&](int set, int b) {
+#pragma unroll
+    for (int j = 0; j < PIECES; j++) {
+      const Split8 s = j == 0 ? split8<true>(raw[set][j][0], raw[set][j][1]) : split8<false>(raw[set][j][0], raw[set][j][1]);
+      char* dst = put_at + b * STAGE + j * (64 * 64);
+      *reinterpret_cast<s3_u32x4*>(dst) = s.h;
+      *reinterpret_cast<s3_u32x4*>(dst + PLANE) = s.m;
+      *reinterpret_cast<s3_u32x4*>(dst + 2 * PLANE) = s.l;
     }
   };
+  const int sw = (l >> 1) & 3;
+  const char* ap = smem + (32 * wm + l) * 64;
+  const char* wp = smem + (TM + 32 * NW * wn + l) * 64;
+  auto read = [&](const char* p, int b, int g) {
+    const char* at = p + b * STAGE + (((2 * g + half) ^ sw) << 4);
+    Split8 s;
+    s.h = *reinterpret_cast<const s3_u32x4*>(at);
+    s.m = *reinterpret_cast<const s3_u32x4*>(at + PLANE);
+    s.l = *reinterpret_cast<const s3_u32x4*>(at + 2 * PLANE);
+    return s;
+  };
+  s3_f32x16 big[NW], small[NW], l2[NW], l3[NW];
 #pragma unroll
-  for (int b = 0; b < NBUF - 1; b++) ask(b, k_first + b * BK);
-  l0[1] = {};
-  constexpr int LEFT = (NBUF - 2) * COPIES;                  // copies that may be on their way when a stage is begun
-  __builtin_amdgcn_s_waitcnt((LEFT & 15) | (LEFT >> 4 << 14) | (7 << 4) | (15 << 8));
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  ask(NBUF - 1, k_first + (NBUF - 1) * BK);
-  read(0, 0);
-  int buf = 0;
-  for (int k0 = k_first; k0 < k_end; k0 += BK) {
-    const int next = buf + 1 == NBUF ? 0 : buf + 1;
-    __builtin_amdgcn_sched_barrier(0);
-    read(buf, 1);
-    multiply(0);
-    if (k0 > k_first) close(k0 - k_first);
-    // this wave's copies of the next stage have landed and its reads of this one are done; behind the barrier all waves'
-    __builtin_amdgcn_s_waitcnt((LEFT & 15) | (LEFT >> 4 << 14) | (7 << 4));
+  for (int j = 0; j < NW; j++) big[j] = small[j] = l2[j] = l3[j] = s3_f32x16{};
+  auto stage = [&](int k0, int i) {                          // the i'th stage of AHEAD
+    const int b = i & 1, next = (i + 1) % AHEAD;
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));   // this wave's part of the stage is written; behind the barrier all waves'
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    ask(buf, k0 + NBUF * BK);
-    read(next, 0);
-    multiply(1);
-    buf = next;
-  }
-  l1 += l0[1];
-  close((k_end - k_first + BK - 1) / BK * BK);
-  __builtin_amdgcn_s_waitcnt(0x0070);                        // the last copies (zeros) are in before LDS is given back
-  const int n = n0 + 32 * wn + l;
-  if (n >= N) return;
-  const float b = !slabs && bias ? bias[n] : 0.f;
-  if (slabs) l3 = l1 + l2;
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+      const Split8 a = read(ap, b, g);
+      Split8 w[NW];
+#pragma unroll
+      for (int j = 0; j < NW; j++) w[j] = read(wp + j * (32 * 64), b, g);
+#pragma unroll
+      for (int j = 0; j < NW; j++) split_multiply(a, w[j], big[j], small[j]);
+      if (g == 0) {
+        put(next, b ^ 1);
+        ask(next, k0 + (AHEAD + 1) * BK);
+      }
+    }
+    const int done = k0 + BK - k_first;
+    if (done % GROUP == 0) {
+#pragma unroll
+      for (int j = 0; j < NW; j++) {
+        l2[j] += big[j];
+        big[j] = s3_f32x16{};
+      }
+    }
+    if (done % len == 0 || k0 + BK >= k_end) {              // the same for all threads
+#pragma unroll
+      for (int j = 0; j < NW; j++) {
+        const int n = n0 + 32 * (NW * wn + j) + l;
+        l3[j] += range_sum(l2[j] + big[j], small[j], A + (size_t)min(m0 + 32 * wm + l, M - 1) * lda, W + (size_t)min(n, N - 1) * ldw, k0 / len * len,
+                           min(K, k0 + BK), K, half);
+        big[j] = l2[j] = small[j] = s3_f32x16{};
+      }
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < AHEAD; i++) ask(i, k_first + i * BK);
+  put(0, 0);
+  ask(0, k_first + AHEAD * BK);
+  for (int k0 = k_first; k0 < k_end; k0 += AHEAD * BK)
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++)
+      if (k0 + i * BK < k_end) stage(k0 + i * BK, i);
   float* out = slabs ? slabs + (size_t)blockIdx.y * M * N : C;
   const int ldo = slabs ? N : ldc;
 #pragma unroll
-  for (int r = 0; r < 16; r++) {
-    const int m = m0 + 32 * wm + 8 * (r >> 2) + 4 * half + (r & 3);
-    if (m < M) out[(size_t)m * ldo + n] = slabs ? l3[r] : l3[r] + b;
+  for (int j = 0; j < NW; j++) {
+    const int n = n0 + 32 * (NW * wn + j) + l;
+    if (n >= N) continue;
+    const float b = !slabs && bias ? bias[n] : 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int m = m0 + 32 * wm + 8 * (r >> 2) + 4 * half + (r & 3);
+      if (m < M) out[(size_t)m * ldo + n] = slabs ? l3[j][r] : l3[j][r] + b;
+    }
   }
 #endif
 }
@@ -320,6 +428,10 @@ __global__ __launch_bounds__(256) void gemm_f32_join_kernel(const float* __restr
   C[(size_t)m * ldc + n] = sum + (bias ? bias[n] : 0.f);
 }
 
+// Tiles of 64 x 128 instead of 64 x 64: an operand is read from LDS for half as many products, so where they are more than the
+// chip holds at once (17,920 x 1,536: 700 tiles, 320 rows, 146 us, in tiles of 64 x 64 159; 560 tiles, 256 rows, 141 and 134).
+static bool f32_wide(int M, int N) { return (long long)((N + 127) / 128) * ((M + 63) / 64) >= 600; }
+
 // The number of slabs [M, N] that a call of these sizes wants as its workspace; 0: none.  Tiles of 64 x 64 (32 x 64 up to
 // 32 rows) and the ranges are the units of work; below two tiles a compute unit (four fit) the ranges are dealt out too.
 extern "C" int pico_gemm_f32_slabs(int M, int N, int K) {
@@ -330,26 +442,44 @@ extern "C" int pico_gemm_f32_slabs(int M, int N, int K) {
   return tiles < 512 && ranges > 1 ? ranges : 0;
 }
 
+template <int NW, int AHEAD>
+static bool launch_planes(const float* A, const float* W, const float* bias, float* C, float* slabs, int M, int N, int K, int lda, int ldw, int ldc,
+                          int ranges, hipStream_t stream) {
+  constexpr int bytes = 6 * fp_plane(NW);
+  static const hipError_t room = hipFuncSetAttribute((const void*)&gemm_f32_planes_kernel<NW, AHEAD>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (room != hipSuccess) return false;
+  const int m_tiles = (M + 63) / 64, n_tiles = (N + 64 * NW - 1) / (64 * NW);
+  gemm_f32_planes_kernel<NW, AHEAD>
+      <<<dim3((n_tiles + 7) / 8 * 8 * m_tiles, ranges), 256, bytes, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
+  return true;
+}
+
 template <typename TA, int WM>
 static void launch_gemm_f32(const TA* A, const float* W, const float* bias, float* C, float* slabs, int M, int N, int K,
                             int lda, int ldw, int ldc, hipStream_t stream) {
   const int m_tiles = (M + 32 * WM - 1) / (32 * WM), n_tiles = (N + 63) / 64;
   int len;
-  const int ranges = f32_ranges(K, len);
-  const dim3 grid((n_tiles + 7) / 8 * 8 * m_tiles, slabs ? ranges : 1);
+  const int all = f32_ranges(K, len), ranges = slabs ? all : 1;
+  const dim3 grid((n_tiles + 7) / 8 * 8 * m_tiles, ranges);
   const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % 16 == 0;
+  bool done = false;
   if constexpr (sizeof(TA) == 4) {
-    // (a tile's rows within 2^31 bytes of its first)
-    static const hipError_t room = hipFuncSetAttribute((const void*)&gemm_f32_stream_kernel<WM>, hipFuncAttributeMaxDynamicSharedMemorySize, fs_buffers(WM) * fs_bytes(WM));
-    if (vec && lda < (1 << 23) && ldw < (1 << 23) && room == hipSuccess)
-      gemm_f32_stream_kernel<WM><<<grid, 128 * WM, fs_buffers(WM) * fs_bytes(WM), stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
-    else
-      gemm_f32_kernel<TA, WM, false><<<grid, 128 * WM, 0, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
-  } else if (vec) {
-    gemm_f32_kernel<TA, WM, true><<<grid, 128 * WM, 0, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
-  } else {
-    gemm_f32_kernel<TA, WM, false><<<grid, 128 * WM, 0, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
+    if (vec && lda < (1 << 23) && ldw < (1 << 23)) {         // (a tile's rows within 2^31 bytes of its first)
+      if (WM == 1) {
+        gemm_f32_stream_kernel<<<dim3(n_tiles, ranges), 128, 0, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc);
+        done = true;
+      } else if (f32_wide(M, N) && ldw < (1 << 22)) {
+        done = launch_planes<2, 2>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, ranges, stream);
+      } else {                                               // few workgroups: reads ahead take the registers of a third one a unit
+        done = (long long)n_tiles * m_tiles * ranges <= 512 ? launch_planes<1, 4>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, ranges, stream)
+                                                            : launch_planes<1, 2>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, ranges, stream);
+      }
+    }
   }
+  if (!done && vec)
+    gemm_f32_kernel<TA, WM, true><<<grid, 128 * WM, 0, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
+  else if (!done)
+    gemm_f32_kernel<TA, WM, false><<<grid, 128 * WM, 0, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
   if (slabs) gemm_f32_join_kernel<<<dim3((N + 255) / 256, M), 256, 0, stream>>>(slabs, ranges, bias, C, M, N, ldc);
 }
 

@@ -5,8 +5,8 @@ steps; up to 256 for small matrices) the weight-streaming matrix-core kernel of 
 SwiGLU or float32 output as its epilogue (for shapes it refuses, this package's plain matrix-core product); with more rows this
 package's tiled product where an activation or a float32 result follows (``kernels.tiles_act_ok`` says where), else the library
 GEMM (hipBLASLt through torch), as the reference uses the library for every
-projection (pico_vllm/model.py:200,225,316,318).  float32 weights: this package's product on the float32 matrix
-instruction (products and sums in 32 bits, ``csrc/gemm_f32.hip``), never a library
+projection (pico_vllm/model.py:200,225,316,318).  float32 weights: this package's product of all 24 bits of
+both operands (in three bfloat16 pieces each, sums in 32 bits, ``csrc/gemm_f32.hip``), never a library
 call, so the 32-bit engine has no reduced-precision matrix mode anywhere; if
 the activations are bfloat16 (a tensor stored in 32 bit inside a bfloat16
 engine) they are widened on load and the result is rounded once.
