@@ -33,6 +33,8 @@
 // of 151,936 logits with top_p < 1, 32 so; 64 rows 159, 65; one row 63, 30; 5,000 logits 34, 24.  Where a class holds most of a row
 // the last launch's one workgroup has it all: logits within a twentieth of each other 61, 58.  Where a chunk's elements are most of it
 // and all alike they are listed once: all logits equal 28, one by one 93.)
+#include <chrono>
+
 #include "common.h"
 
 #define SAMPLE_CHUNKS 32            // as ARGMAX_CHUNKS below: the two share the first launch
@@ -368,12 +370,25 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
   }
 }
 
+// Where tokens go beside `out`: host memory that the GPU reaches, a word a row, the launch's stamp above the token (null: nowhere).
+// Written past the caches, so that the host sees a token a microsecond after it is chosen, without a copy, and knows by the
+// stamp whose it is, without an event.
+struct SampleLanding {
+  unsigned long long* words;
+  uint32_t stamp;
+};
+__device__ __forceinline__ void sample_leave(int token, int row, int* out, const SampleLanding& to) {
+  out[row] = token;
+  if (to.words != nullptr)
+    __hip_atomic_store(to.words + row, (unsigned long long)to.stamp << 32 | (uint32_t)token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <int THREADS, bool SEARCH>
 __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
     const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature, const float* __restrict__ top_p,
     const float* __restrict__ u, const float* __restrict__ part_val, const int* __restrict__ part_idx,
     const double* __restrict__ fin_s, const int* __restrict__ fin_n, const uint32_t* __restrict__ list, int room,
-    const SampleRow* __restrict__ rows, int bits, int* __restrict__ out) {
+    const SampleRow* __restrict__ rows, int bits, int* __restrict__ out, const SampleLanding landing) {
   constexpr int WAVES = THREADS / 64, PER = THREADS / SAMPLE_CHUNKS, PIECE = SAMPLE_PIECE / THREADS;     // PER: threads a chunk
   __shared__ unsigned long long hist[SEARCH ? 1 << (SAMPLE_LOW - SAMPLE_MID) : 1], scratch[WAVES], mass;
   __shared__ int cls;
@@ -392,7 +407,7 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
   const float temp = temperature[row], u_row = u[row];    // (asked for here: where it is used, one thread would wait for it)
   const float tp = SEARCH ? top_p[row] : 1.0f;
   if (!(temp > 0.f)) {
-    if (tid == 0) out[row] = mi;
+    if (tid == 0) sample_leave(mi, row, out, landing);
     return;
   }
   const float inv_t = 1.0f / temp;
@@ -582,7 +597,7 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
   }
   const int who = first != 0x7fffffff ? first : last;
   if (who < 0) {                              // nothing kept in the chunk (cannot be, but a token must come out)
-    if (tid == 0) out[row] = mi;
+    if (tid == 0) sample_leave(mi, row, out, landing);
     return;
   }
   if (tid == who) {
@@ -596,7 +611,7 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
       }
       return true;
     });
-    out[row] = pick >= 0 ? pick : last_kept;
+    sample_leave(pick >= 0 ? pick : last_kept, row, out, landing);
   }
 }
 
@@ -605,13 +620,26 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
 // one compute unit takes data in (19 us for 151,936 logits); ARGMAX_CHUNKS workgroups per row find the
 // first maximum of a chunk each, a second launch picks among them (the lowest index on a tie, as above).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void argmax_part_kernel(const float* __restrict__ logits, int ld, int V,
-                                                          float* __restrict__ part_val, int* __restrict__ part_idx,
-                                                          unsigned long long* __restrict__ clear = nullptr) {
+// What a step's rows are sampled with, as it travels with a launch: temperature, top_p, uniform number of up to N rows.
+template <int N>
+struct SampleGiven {
+  float v[3][N];
+};
+template <>
+struct SampleGiven<0> {};
+
+// N > 0: leaves the rows' options in params [3][stride] for the launches behind it.  clear: the classes of the second launch of sampling.
+template <int N>
+__global__ __launch_bounds__(256) void argmax_part_kernel(const float* __restrict__ logits, int ld, int V, float* __restrict__ part_val,
+                                                          int* __restrict__ part_idx, unsigned long long* __restrict__ clear,
+                                                          const SampleGiven<N> given, float* __restrict__ params, int stride) {
   __shared__ float vals[4];
   __shared__ int idxs[4];
   const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
-  constexpr int SHARE = SAMPLE_CLASSES / ARGMAX_CHUNKS;    // what the second launch of sampling adds to
+  constexpr int SHARE = SAMPLE_CLASSES / ARGMAX_CHUNKS;
+  if constexpr (N > 0) {
+    if (c == 0 && tid < 3) params[(size_t)tid * stride + row] = given.v[tid][row];
+  }
   if (clear != nullptr && tid < SHARE) clear[(size_t)row * SAMPLE_CLASSES + c * SHARE + tid] = 0ull;
   const float* x = logits + (size_t)row * ld;
   const int len = (V + ARGMAX_CHUNKS - 1) / ARGMAX_CHUNKS;
@@ -641,26 +669,68 @@ __global__ __launch_bounds__(256) void argmax_part_kernel(const float* __restric
 }
 
 __global__ __launch_bounds__(64) void argmax_final_kernel(const float* __restrict__ part_val, const int* __restrict__ part_idx,
-                                                          int* __restrict__ out) {
+                                                          int* __restrict__ out, const SampleLanding landing) {
   const int row = blockIdx.x, lane = threadIdx.x;
   float mx = lane < ARGMAX_CHUNKS ? part_val[row * ARGMAX_CHUNKS + lane] : -INFINITY;
   int mi = lane < ARGMAX_CHUNKS ? part_idx[row * ARGMAX_CHUNKS + lane] : 0x7fffffff;
   wave_first_max(mx, mi);
-  if (lane == 0) out[row] = mi;
+  if (lane == 0) sample_leave(mi, row, out, landing);
 }
 
 // part_val, part_idx: workspace of R * pico_argmax_chunks() entries each
 extern "C" int pico_argmax_chunks() { return ARGMAX_CHUNKS; }
 
-extern "C" int pico_argmax(const float* logits, int ld, int R, int V, float* part_val, int* part_idx, int* out,
-                           hipStream_t stream) {
+// landing, stamp: SampleLanding
+extern "C" int pico_argmax_rows(const float* logits, int ld, int R, int V, float* part_val, int* part_idx, int* out,
+                                unsigned long long* landing, uint32_t stamp, hipStream_t stream) {
   PICO_REQUIRE(R >= 0 && V > 0 && ld >= V, "pico_argmax: bad sizes R=%d V=%d ld=%d", R, V, ld);
   PICO_REQUIRE(R <= 65535, "pico_argmax: too many rows");
   if (R == 0) return 0;
-  argmax_part_kernel<<<dim3(R, ARGMAX_CHUNKS), 256, 0, stream>>>(logits, ld, V, part_val, part_idx);
-  argmax_final_kernel<<<R, 64, 0, stream>>>(part_val, part_idx, out);
+  argmax_part_kernel<0><<<dim3(R, ARGMAX_CHUNKS), 256, 0, stream>>>(logits, ld, V, part_val, part_idx, nullptr, SampleGiven<0>{}, nullptr, 0);
+  argmax_final_kernel<<<R, 64, 0, stream>>>(part_val, part_idx, out, SampleLanding{landing, stamp});
   PICO_LAUNCH_CHECK();
   return 0;
+}
+extern "C" int pico_argmax(const float* logits, int ld, int R, int V, float* part_val, int* part_idx, int* out, hipStream_t stream) {
+  return pico_argmax_rows(logits, ld, R, V, part_val, part_idx, out, nullptr, 0, stream);
+}
+
+// The address at which kernels reach pinned host memory; null: they do not.
+extern "C" void* pico_host_on_device(void* host) {
+  void* p = nullptr;
+  if (hipHostGetDevicePointer(&p, host, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return p;
+}
+
+// Waits on the host, for `limit_us` at most, until the n words of landing bear the stamp; their tokens.  0: they do not yet.
+extern "C" int pico_landed(const unsigned long long* landing, int n, uint32_t stamp, int* tokens, int limit_us) {
+  const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(limit_us);
+  for (int i = 0; i < n; i++) {
+    unsigned long long w;
+    for (int spins = 0; (uint32_t)((w = __atomic_load_n(landing + i, __ATOMIC_RELAXED)) >> 32) != stamp; spins++) {
+      if (spins % 64 == 63 && std::chrono::steady_clock::now() > end) return 0;
+      __builtin_ia32_pause();
+    }
+    tokens[i] = (int)(uint32_t)w;
+  }
+  return 1;
+}
+
+// The counter-based generator: u in [0, 1) of 24 random bits from (seed, index of the token in its request).
+static uint64_t splitmix64(uint64_t x) {
+  x += 0x9E3779B97F4A7C15ull;
+  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+  x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+  return x ^ (x >> 31);
+}
+static float sample_uniform(uint64_t seed, uint64_t index) {
+  return (float)(splitmix64(splitmix64(seed) ^ index * 0xD6E8FEB86659FD93ull) >> 40) / (float)(1 << 24);
+}
+extern "C" void pico_sample_uniforms(const uint64_t* seeds, const uint64_t* indices, int n, float* u) {
+  for (int i = 0; i < n; i++) u[i] = sample_uniform(seeds[i], indices[i]);
 }
 
 // Words of a chunk's list: none are missing up to SAMPLE_LISTED elements a chunk.  (A class that is not listed whole is read again, three
@@ -679,47 +749,100 @@ extern "C" long long pico_sample_workspace_words(int R, int V, int top_p_rows) {
   return (long long)R * SAMPLE_CHUNKS * (2 + 1 + 1 + 1) + (top_p_rows ? at_once * (2 * SAMPLE_CLASSES + 4 + SAMPLE_CHUNKS * (long long)sample_room(V)) : 0);
 }
 
-extern "C" int pico_sample(const float* logits, int ld, int R, int V, const float* temperature, const float* top_p,
-                           const float* u, int* out, void* work, int top_p_rows, hipStream_t stream) {
+// What the launches of a call share
+struct SampleCall {
+  const float* logits;
+  int ld, R, V;
+  const float *temperature, *top_p, *u;
+  int* out;
+  SampleLanding landing;
+  void* work;
+  int top_p_rows;
+  hipStream_t stream;
+};
+
+// first(row, rows, part_val, part_idx, classes or null): the first launch, for `most` rows at most
+template <typename First>
+static int sample_launches(const SampleCall& a, int most, First first) {
   static_assert(SAMPLE_CHUNKS == ARGMAX_CHUNKS, "the first launch is the argmax's");
-  PICO_REQUIRE(R >= 0 && V > 0 && ld >= V, "pico_sample: bad sizes R=%d V=%d ld=%d", R, V, ld);
-  PICO_REQUIRE(R <= 65535, "pico_sample: too many rows");
-  if (R == 0) return 0;
+  PICO_REQUIRE(a.R >= 0 && a.V > 0 && a.ld >= a.V, "pico_sample: bad sizes R=%d V=%d ld=%d", a.R, a.V, a.ld);
+  PICO_REQUIRE(a.R <= 65535, "pico_sample: too many rows");
+  if (a.R == 0) return 0;
   // (every part of the workspace is a multiple of 16 bytes long)
-  PICO_REQUIRE(work != nullptr && (uintptr_t)work % 16 == 0, "pico_sample: the workspace is missing or not 16-byte aligned");
-  const size_t n = (size_t)R * SAMPLE_CHUNKS;
-  double* fin_s = (double*)work;
+  PICO_REQUIRE(a.work != nullptr && (uintptr_t)a.work % 16 == 0, "pico_sample: the workspace is missing or not 16-byte aligned");
+  const size_t n = (size_t)a.R * SAMPLE_CHUNKS;
+  double* fin_s = (double*)a.work;
   float* part_val = (float*)(fin_s + n);
   int* part_idx = (int*)(part_val + n);
   int* fin_n = part_idx + n;
   unsigned long long* classes = (unsigned long long*)(fin_n + n);
-  const int room = sample_room(V), at_once = R < SAMPLE_ROWS ? R : SAMPLE_ROWS;
+  const int room = sample_room(a.V), at_once = a.R < SAMPLE_ROWS ? a.R : SAMPLE_ROWS;
   SampleRow* rows = (SampleRow*)(classes + (size_t)at_once * SAMPLE_CLASSES);
   uint32_t* list = (uint32_t*)(rows + at_once);
   int bits = 40;                              // a row's sum of whole numbers of 2^-bits stays below 2^63
-  while (bits > 31 && V > (1LL << (63 - bits))) bits--;
-  if (!top_p_rows) {
-    const dim3 grid(R, SAMPLE_CHUNKS);
-    argmax_part_kernel<<<grid, 256, 0, stream>>>(logits, ld, V, part_val, part_idx);
-    sample_collect_kernel<false><<<grid, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, nullptr, part_val, nullptr, bits, fin_s, fin_n,
-                                                                     nullptr, 0, nullptr);
-    sample_pick_kernel<SAMPLE_THREADS, false><<<R, SAMPLE_THREADS, 0, stream>>>(logits, ld, V, temperature, nullptr, u, part_val, part_idx,
-                                                                               fin_s, fin_n, nullptr, 0, nullptr, bits, out);
-  }
-  for (int r = 0; top_p_rows && r < R; r += SAMPLE_ROWS) {     // rows with a list side by side; the next ones write it again behind them
-    const int m = R - r < SAMPLE_ROWS ? R - r : SAMPLE_ROWS;
+  while (bits > 31 && a.V > (1LL << (63 - bits))) bits--;
+  for (int r = 0; r < a.R; r += most) {                        // rows with a list side by side; the next ones write it again behind them
+    const int m = a.R - r < most ? a.R - r : most;
     const size_t c = (size_t)r * SAMPLE_CHUNKS;
-    const float* x = logits + (size_t)r * ld;
+    const float* x = a.logits + (size_t)r * a.ld;
+    const SampleLanding landing{a.landing.words ? a.landing.words + r : nullptr, a.landing.stamp};
     const dim3 grid(m, SAMPLE_CHUNKS);
-    argmax_part_kernel<<<grid, 256, 0, stream>>>(x, ld, V, part_val + c, part_idx + c, classes);
-    sample_classes_kernel<<<grid, SAMPLE_THREADS, 0, stream>>>(x, ld, V, temperature + r, top_p + r, part_val + c, classes, bits);
-    sample_collect_kernel<true><<<grid, SAMPLE_THREADS, 0, stream>>>(x, ld, V, temperature + r, top_p + r, part_val + c, classes, bits, fin_s + c,
-                                                                    fin_n + c, list, room, rows);
-    sample_pick_kernel<SAMPLE_PICK_THREADS, true><<<m, SAMPLE_PICK_THREADS, 0, stream>>>(x, ld, V, temperature + r, top_p + r, u + r, part_val + c,
-                                                                                        part_idx + c, fin_s + c, fin_n + c, list, room, rows, bits, out + r);
+    first(r, m, part_val + c, part_idx + c, a.top_p_rows ? classes : nullptr);
+    if (!a.top_p_rows) {
+      sample_collect_kernel<false><<<grid, SAMPLE_THREADS, 0, a.stream>>>(x, a.ld, a.V, a.temperature + r, nullptr, part_val + c, nullptr, bits, fin_s + c,
+                                                                         fin_n + c, nullptr, 0, nullptr);
+      sample_pick_kernel<SAMPLE_THREADS, false><<<m, SAMPLE_THREADS, 0, a.stream>>>(x, a.ld, a.V, a.temperature + r, nullptr, a.u + r, part_val + c,
+                                                                                   part_idx + c, fin_s + c, fin_n + c, nullptr, 0, nullptr, bits, a.out + r,
+                                                                                   landing);
+      continue;
+    }
+    sample_classes_kernel<<<grid, SAMPLE_THREADS, 0, a.stream>>>(x, a.ld, a.V, a.temperature + r, a.top_p + r, part_val + c, classes, bits);
+    sample_collect_kernel<true><<<grid, SAMPLE_THREADS, 0, a.stream>>>(x, a.ld, a.V, a.temperature + r, a.top_p + r, part_val + c, classes, bits, fin_s + c,
+                                                                      fin_n + c, list, room, rows);
+    sample_pick_kernel<SAMPLE_PICK_THREADS, true><<<m, SAMPLE_PICK_THREADS, 0, a.stream>>>(x, a.ld, a.V, a.temperature + r, a.top_p + r, a.u + r,
+                                                                                          part_val + c, part_idx + c, fin_s + c, fin_n + c, list, room, rows,
+                                                                                          bits, a.out + r, landing);
   }
   PICO_LAUNCH_CHECK();
   return 0;
+}
+
+extern "C" int pico_sample(const float* logits, int ld, int R, int V, const float* temperature, const float* top_p,
+                           const float* u, int* out, void* work, int top_p_rows, hipStream_t stream) {
+  return sample_launches({logits, ld, R, V, temperature, top_p, u, out, {nullptr, 0}, work, top_p_rows, stream}, top_p_rows ? SAMPLE_ROWS : 65535,
+                         [&](int r, int m, float* val, int* idx, unsigned long long* classes) {
+                           argmax_part_kernel<0><<<dim3(m, SAMPLE_CHUNKS), 256, 0, stream>>>(logits + (size_t)r * ld, ld, V, val, idx, classes,
+                                                                                             SampleGiven<0>{}, nullptr, 0);
+                         });
+}
+
+template <int N>
+static void launch_given(const float* x, int ld, int V, float* val, int* idx, unsigned long long* classes, const float* temperature, const float* top_p,
+                         const uint64_t* seeds, const uint64_t* indices, int m, float* params, int stride, hipStream_t stream) {
+  SampleGiven<N> given;
+  for (int i = 0; i < m; i++) {
+    given.v[0][i] = temperature[i];
+    given.v[1][i] = top_p[i];
+    given.v[2][i] = temperature[i] > 0.f ? sample_uniform(seeds[i], indices[i]) : 0.f;
+  }
+  for (auto& row : given.v)
+    for (int i = m; i < N; i++) row[i] = 0.f;
+  argmax_part_kernel<N><<<dim3(m, SAMPLE_CHUNKS), 256, 0, stream>>>(x, ld, V, val, idx, classes, given, params, stride);
+}
+
+// The same with temperature, top_p, seeds and token indices [R] in ordinary host memory: they travel with the first launch, which leaves them in
+// params (float [3][stride], stride >= R, device memory), so there is no copy in front of it.  (8 rows, half of them with top_p: a step with its
+// copies and an event 63 us from call to tokens, so, and with landing, 48.)  A launch carries 768 bytes of options up to 64 rows, else 3 KB.
+extern "C" int pico_sample_rows(const float* logits, int ld, int R, int V, const float* temperature, const float* top_p, const uint64_t* seeds,
+                                const uint64_t* indices, float* params, int stride, int* out, unsigned long long* landing,
+                                uint32_t stamp, void* work, int top_p_rows, hipStream_t stream) {
+  PICO_REQUIRE(stride >= R && params && temperature && top_p && seeds && indices, "pico_sample_rows: room for %d rows' options, got %d", R, stride);
+  return sample_launches({logits, ld, R, V, params, params + stride, params + 2 * (size_t)stride, out, {landing, stamp}, work, top_p_rows, stream}, SAMPLE_ROWS,
+                         [&](int r, int m, float* val, int* idx, unsigned long long* classes) {
+                           const auto launch = m <= 64 ? launch_given<64> : launch_given<SAMPLE_ROWS>;
+                           launch(logits + (size_t)r * ld, ld, V, val, idx, classes, temperature + r, top_p + r, seeds + r, indices + r, m, params + r, stride,
+                                  stream);
+                         });
 }
 
 // ---------------------------------------------------------------------------
@@ -776,8 +899,8 @@ extern "C" int pico_argmax_noalloc(const float* logits, int ld, int R, int V, in
   float* part_val = reinterpret_cast<float*>(base);
   int* part_idx = reinterpret_cast<int*>(reinterpret_cast<unsigned char*>(base) + NOALLOC_ENTRIES * sizeof(float));
   // the first launch writes entries [0, R * ARGMAX_CHUNKS), the second reads exactly those: nothing to clear
-  argmax_part_kernel<<<dim3(R, ARGMAX_CHUNKS), 256, 0, stream>>>(logits, ld, V, part_val, part_idx);
-  argmax_final_kernel<<<R, 64, 0, stream>>>(part_val, part_idx, out);
+  argmax_part_kernel<0><<<dim3(R, ARGMAX_CHUNKS), 256, 0, stream>>>(logits, ld, V, part_val, part_idx, nullptr, SampleGiven<0>{}, nullptr, 0);
+  argmax_final_kernel<<<R, 64, 0, stream>>>(part_val, part_idx, out, SampleLanding{nullptr, 0});
   PICO_LAUNCH_CHECK();
   return 0;
 }

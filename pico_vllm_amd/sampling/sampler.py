@@ -4,12 +4,14 @@ Strategy per row as in pico_vllm/sampler.py:40-88 (greedy / temperature /
 temperature with top-p), but in one call with per-row parameters for the whole
 batch (a short chain of launches, several workgroups a row) instead of torch
 calls per group of equal parameters.  Randomness comes from
-a counter-based generator on the host: the uniform number of a draw depends
+a counter-based generator on the host (``uniform`` here; the launch makes the same numbers in
+native code): the uniform number of a draw depends
 only on (seed, index of the token in its request), so a request samples the
 same tokens whatever else is in the batch.
 """
 from __future__ import annotations
 
+import weakref
 from typing import List, Sequence
 
 import torch
@@ -17,6 +19,7 @@ import torch
 from ..ops import kernels
 
 _MASK = (1 << 64) - 1
+POLL_US = 2000
 
 
 def _splitmix64(x: int) -> int:
@@ -33,23 +36,34 @@ def uniform(seed: int, index: int) -> float:
     return (z >> 40) / float(1 << 24)
 
 
+def _outlive(landing, landed) -> None:
+    """The host memory ``landing`` is held until what writes there is done."""
+    for event in landed:
+        if event is not None:
+            event.synchronize()
+
+
 class Sampler:
     def __init__(self, device: torch.device, max_rows: int):
         self.device = device
         self.max_rows = max_rows
-        # two sets of host buffers, used in turn: a step's tokens may be read, and its parameters
-        # may still wait for their copy, after the next step was launched
-        self._host = [torch.zeros(3, max_rows, dtype=torch.float32, pin_memory=torch.cuda.is_available()) for _ in range(2)]
+        self._options = kernels.SampleOptions(max_rows)
         self._dev = torch.zeros(3, max_rows, dtype=torch.float32, device=device)
         self._out = torch.zeros(max_rows, dtype=torch.int32, device=device)
         self._argmax_work = kernels.argmax_workspace(max_rows, device) if torch.cuda.is_available() else None
         # of calls without top_p; what its search needs (as much as the logits of 256 rows) waits for the first call that has it
         self._sample_work = kernels.sample_workspace(max_rows, device, top_p_rows=False) if torch.cuda.is_available() else None
         self._top_p_work = None
-        self._host_np = [h.numpy() for h in self._host]
-        self._landing = [torch.zeros(max_rows, dtype=torch.int32, pin_memory=torch.cuda.is_available()) for _ in range(2)]
+        # two sets, used in turn: a step's tokens may be read after the next step was launched.  The last launch writes them there itself,
+        # a word a row: the launch's stamp above the token, so that words of a launch that nobody read are not taken for another's
+        self._landing = [torch.zeros(max_rows, dtype=torch.int64, pin_memory=torch.cuda.is_available()) for _ in range(2)]
+        self._stamps, self._stamp = [0, 0], 1
+        self._tokens = [torch.zeros(max_rows, dtype=torch.int32) for _ in range(2)]
+        self._landing_at = [kernels.host_on_device(t) if torch.cuda.is_available() and max_rows else 0 for t in self._landing]
         self._landed = [torch.cuda.Event() if torch.cuda.is_available() else None for _ in range(2)]
         self._turn = 0
+        # a launch that is never read still writes there
+        weakref.finalize(self, _outlive, self._landing, self._landed).atexit = False
 
     def _work(self, vocab: int) -> torch.Tensor:
         """The workspace of a search, kept: all rows that the sampler was made for, of as many logits as have been seen."""
@@ -73,8 +87,17 @@ class Sampler:
         turn, R = ticket
         if R == 0:
             return []
-        self._landed[turn].synchronize()
-        return self._landing[turn][:R].tolist()
+        if not self._landing_at[turn]:
+            self._landed[turn].synchronize()
+            return self._landing[turn][:R].tolist()
+        # the host sees a word some 6 us before it would see the event behind it (8 rows: 48 us from call to tokens, 54 so); of a wait so
+        # long that this does not count the rest is the event's
+        tokens = self._tokens[turn]
+        if not kernels.landed(self._landing[turn], R, self._stamps[turn], tokens, POLL_US):
+            self._landed[turn].synchronize()
+            if not kernels.landed(self._landing[turn], R, self._stamps[turn], tokens, POLL_US):
+                raise RuntimeError("the step's tokens did not arrive")
+        return tokens[:R].tolist()
 
     def launch(self, logits: torch.Tensor, temperatures: Sequence[float], top_ps: Sequence[float],
                seeds: Sequence[int], indices: Sequence[int]):
@@ -87,20 +110,20 @@ class Sampler:
             raise ValueError(f"{R} rows to sample, the sampler was made for {self.max_rows}")
         if R == 0:
             return (0, 0)
-        if not any(temperatures):
-            # all rows greedy: nothing to upload, and the argmax alone spreads a row over several workgroups
-            kernels.argmax(logits, self._out, self._argmax_work)
-        else:
-            h = self._host_np[self._turn]
-            h[0, :R] = temperatures
-            h[1, :R] = top_ps
-            h[2, :R] = [uniform(s, i) if t > 0 else 0.0 for s, i, t in zip(seeds, indices, temperatures)]
-            self._dev.copy_(self._host[self._turn], non_blocking=True)
-            searched = any(t > 0 and p < 1 for t, p in zip(temperatures, top_ps))
-            kernels.sample(logits, self._dev[0], self._dev[1], self._dev[2], self._out, self._work(logits.shape[1]) if searched else self._sample_work,
-                           top_p_rows=searched)
         turn = self._turn
+        landing, stamp = self._landing_at[turn], self._stamp
+        self._stamp = stamp % 0xffffffff + 1
+        self._stamps[turn] = stamp
+        if not any(temperatures):
+            # all rows greedy: no options, and the argmax alone spreads a row over several workgroups
+            kernels.argmax(logits, self._out, self._argmax_work, landing, stamp)
+        else:
+            self._options.fill(temperatures, top_ps, seeds, indices)
+            searched = any(t > 0 and p < 1 for t, p in zip(temperatures, top_ps))
+            work = self._work(logits.shape[1]) if searched else self._sample_work
+            kernels.sample_rows(logits, self._options, self._dev, self._out, work, searched, landing, stamp)
         self._turn ^= 1
-        self._landing[turn][:R].copy_(self._out[:R], non_blocking=True)
+        if not landing:
+            self._landing[turn][:R].copy_(self._out[:R], non_blocking=True)
         self._landed[turn].record()
         return (turn, R)

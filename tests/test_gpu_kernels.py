@@ -746,6 +746,29 @@ def test_the_room_that_sampling_holds(K):
         K.sample(logits, *(torch.full((2,), 0.5, device=DEV) for _ in range(3)), work=K.sample_workspace(2, DEV, top_p_rows=False))
 
 
+@pytest.mark.parametrize("R", [1, 63, 64, 65, 256, 257, 300])
+def test_options_that_travel_with_the_launch(K, R):
+    # the sampler's rows against the launches that read them from the GPU, at the edges of how many travel with one launch; two launches
+    # unread at a time
+    from pico_vllm_amd.sampling.sampler import Sampler, uniform
+    g = torch.Generator().manual_seed(R)
+    seeds = torch.randint(-2 ** 62, 2 ** 62, (R,), generator=g).tolist()
+    seeds[0] = 2 ** 70 + 5
+    at = torch.randint(0, 5000, (R,), generator=g).tolist()
+    assert K.sample_uniforms(seeds, at).tolist() == [uniform(s, i) for s, i in zip(seeds, at)]
+    temps, top_ps = [[0.0, 0.7, 1.0, 0.8][i % 4] for i in range(R)], [[1.0, 0.9, 1.0, 0.95][i % 4] for i in range(R)]
+    sampler = Sampler(torch.device(DEV), R + 3)
+    tickets, want = [], []
+    for step, (t, p) in enumerate([(temps, top_ps), ([0.0] * R, top_ps), (temps, [1.0] * R), (temps[::-1], top_ps)]):
+        logits = torch.randn(R, 3000, generator=g).to(DEV) * 2.5
+        us = [uniform(s, i + step) if x > 0 else 0.0 for s, i, x in zip(seeds, at, t)]
+        want.append(K.sample(logits, *(torch.tensor(x, device=DEV) for x in (t, p, us))).tolist())
+        tickets.append(sampler.launch(logits, t, p, [s if x > 0 else None for s, x in zip(seeds, t)], [i + step for i in at]))
+        assert sampler.device_tokens[:R].tolist() == want[-1]
+        if step % 2:
+            assert [sampler.read(x) for x in tickets[-2:]] == want[-2:]
+
+
 def test_sampling_at_the_edges_of_its_options(K):
     # a nucleus so small that only the likeliest token fits, a temperature so low that it holds all the mass, one so high
     # that the distribution is flat, and a vocabulary smaller than the number of chunks a row is read in
