@@ -36,7 +36,7 @@ __device__ __forceinline__ float gt_pair(float g, float u, const GemmArgs& a) {
   if (EPI == GT_SWIGLU) return FEW ? g / (1.0f + __expf(-g)) * u : silu_f(g) * u;
   g = fminf(g, a.limit);
   u = fminf(fmaxf(u, -a.limit), a.limit);
-  return g / (1.0f + (FEW ? __expf(-a.alpha * g) : expf(-a.alpha * g))) * (u + 1.0f);
+  return (FEW ? g / (1.0f + __expf(-a.alpha * g)) : times_sigmoid(g, a.alpha * g)) * (u + 1.0f);
 }
 // z times the normal distribution's share below z, without a branch: a thread has up to 144 of them in a row, and erff has two
 // branches, both taken by every wave.  13,440 outputs with a bias, K 1,536, microseconds with erff and the bias read between the

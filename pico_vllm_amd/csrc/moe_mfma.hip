@@ -19,11 +19,11 @@
 // mode 0: the clipped activation, the row's weight w on its input; mode 1: w silu(g) u (the weight on the expert's
 // output, taken in front of the linear second product); mode 2: w times the clipped activation
 __device__ __forceinline__ float moe_act(float g, float u, float limit, float alpha, int mode, float w) {
-  if (mode == 1) return w * (g / (1.0f + expf(-g))) * u;
+  if (mode == 1) return w * silu_f(g) * u;
   if (mode == 0) { g *= w; u *= w; }
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return (mode == 2 ? w : 1.0f) * (g / (1.0f + expf(-alpha * g)) * (u + 1.0f));
+  return (mode == 2 ? w : 1.0f) * (times_sigmoid(g, alpha * g) * (u + 1.0f));
 }
 
 __device__ __forceinline__ void unpack8(const uint4& v, float* f) {

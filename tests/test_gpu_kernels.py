@@ -256,6 +256,26 @@ def test_gemm_tiles_gelu_over_its_range(K, M):
     assert bool((out[:, -2] == float("inf")).all()) and bool(out[:, -1].isnan().all())
 
 
+@pytest.mark.parametrize("name", ["swiglu", "clipped"])
+def test_activation_of_the_tiled_product_over_all_numbers(K, name):
+    # a gate that is one number of the row, an up that is 1 (0, for the clipped form's u + 1): every bfloat16 number through the
+    # activation, which is then rounded to bfloat16 (2^-8 of it) from what is within 2^-21 of the quotient in 64 bits (results below 2^-119, of z
+    # under -87.3, may be zero)
+    x = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    a = torch.zeros(65536, 16, dtype=torch.bfloat16)
+    a[:, 0], a[:, 1] = x, 1
+    w = torch.zeros(16, 16, dtype=torch.bfloat16)
+    w[:8, 0], w[8:, 1] = 1, 1 if name == "swiglu" else 0
+    alpha = 1.0 if name == "swiglu" else 1.702
+    out = K.gemm_tiles(a.to(DEV), w.to(DEV), None, K.EPI_SWIGLU if name == "swiglu" else K.EPI_CLIPPED, clip=(float("inf"), alpha)).cpu()
+    g = x.double()
+    want = g / (1 + torch.exp(-(x.float() * alpha).double()))
+    bad = ~torch.isfinite(g)                                # (an infinite gate times the up rows' zero is NaN)
+    assert bool((out == out[:, :1])[~bad].all())
+    got, want = out[:, 0][~bad].double(), want[~bad]
+    assert bool(((got - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -21) + 2.0 ** -119).all())      # (eight bits: half of the last is 2^-8 of 1)
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,name", [(66000, "f32"), (65536, "f32"), (65600, "swiglu"), (33024, "clipped"), (65536, "swiglu")])
 def test_few_rows_of_a_large_matrix(K, M, N, name):
