@@ -65,15 +65,38 @@ __device__ __forceinline__ float gt_one(float v) {
 }
 typedef float gt_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int MB, int NB, int EPI, int SETS>
-__global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const GemmArgs a) {
+#ifdef __HIP_DEVICE_COMPILE__
+// A workgroup without a tile reads its share of W's rows, in the order in which the tiles want their k, once: the memory-side cache
+// then has them.  Where a single round of tiles waits for memory stage after stage, W comes from there in half the time.
+__device__ __forceinline__ void gt_bring(const GemmArgs& a, int worker, int workers, char* lds) {
+  const int rows = (a.cols + workers - 1) / workers, r0 = worker * rows, r1 = min(a.cols, r0 + rows);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const __amdgpu_buffer_rsrc_t w = ts_buffer(a.W, ((long long)(a.cols - 1) * a.ldw + a.K) * 2);
+  for (int k = 0; k < a.K; k += TS_BK)
+    for (int r = r0 + 8 * wave; r < r1; r += 32) {                 // eight rows of 128 bytes a copy; its place in LDS is nobody's
+      const int row = r + (lane >> 3), col = k + (lane & 7) * 8;
+      const uint32_t at = row < r1 && col < a.K ? (uint32_t)(row * a.ldw + col) * 2 : TS_OUT;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w, (__attribute__((address_space(3))) void*)(lds + wave * 1024), 16, at, 0, 0, 0);
+    }
+  __builtin_amdgcn_s_waitcnt(ts_wait(0, true));
+}
+#endif
+
+// BRING: workgroups without a tile read W ahead for the others (gt_bring; the grid has some)
+template <int MB, int NB, int EPI, int SETS, int SHARE, int BUFS, bool BRING>
+__global__ __launch_bounds__(256, SHARE) void gemm_tiles_kernel(const GemmArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  typedef TileStream<MB, NB, SETS, EPI == GT_PARTS> TS;
+  typedef TileStream<MB, NB, SETS, EPI == GT_PARTS, BUFS> TS;
   TS ts(smem);
   constexpr int TM = 64 * MB, TN = 64 * NB, COLS = gt_paired(EPI) ? TN / 2 : TN;      // output columns of a tile
   const int tiles = a.m_tiles * a.n_tiles * (EPI == GT_PARTS ? a.splits : 1);
-  if (ts_tile(0, tiles) < 0) return;
+  if (ts_tile(0, tiles) < 0) {
+    // (a single round: the first `busy` places of a die have its tiles)
+    const int busy = (tiles + 7) >> 3;
+    if (BRING && (int)(blockIdx.x >> 3) >= busy) gt_bring(a, (int)blockIdx.x - 8 * busy, (int)gridDim.x - 8 * busy, smem);
+    return;
+  }
   TileRowsSource<MB> xs;
   TileRowsSource<NB> ws;
   auto aim = [&](int t) {
@@ -182,16 +205,17 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void gemm_tiles_kernel(const
 #endif
 }
 
-template <int MB, int NB, int EPI, int SETS = 1>
+template <int MB, int NB, int EPI, int SETS = 1, int SHARE = ts_share(MB, NB), int BUFS = ts_buffers(MB, NB), bool BRING = false>
 static int gt_launch(GemmArgs a, hipStream_t stream) {
-  static const hipError_t room = hipFuncSetAttribute((const void*)&gemm_tiles_kernel<MB, NB, EPI, SETS>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, ts_lds_bytes(MB, NB));
+  constexpr int bytes = ts_stage_bytes(MB, NB) * BUFS;
+  const auto kernel = gemm_tiles_kernel<MB, NB, EPI, SETS, SHARE, BUFS, BRING>;
+  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   PICO_REQUIRE(room == hipSuccess, "pico_gemm_tiles: %s", hipGetErrorString(room));
   a.m_tiles = (a.M + 64 * MB - 1) / (64 * MB);
   a.n_tiles = (a.cols + GT_COLS(NB, EPI) - 1) / GT_COLS(NB, EPI);
   const long long tiles = (long long)a.m_tiles * a.n_tiles * a.splits;
   PICO_REQUIRE(tiles < (1LL << 30), "pico_gemm_tiles: %d x %d outputs are too many for one launch", a.M, a.cols);
-  gemm_tiles_kernel<MB, NB, EPI, SETS><<<ts_grid(tiles, 256 * ts_share(MB, NB)), 256, ts_lds_bytes(MB, NB), stream>>>(a);
+  kernel<<<BRING ? 256 * SHARE : ts_grid(tiles, 256 * SHARE), 256, bytes, stream>>>(a);
   PICO_LAUNCH_CHECK();
   return 0;
 }
@@ -251,6 +275,33 @@ static int gt_run(GemmArgs a, hipStream_t stream) {
   return run(gt_choose(a.M, a.cols, stages, gt_paired(EPI), false, all, cost));
 }
 
+// Plain products that are a single round of small tiles.  What such a call takes is the stages' latency from memory, so its
+// workgroups have a compute unit each and as many stages on their way as LDS holds (128 x 128, K 1,536, 192 tiles: two buffers
+// and two workgroups a unit 21.3 us, three, four, five buffers 15.5, 15.5, 16.3), and where an eighth of the units has no tile
+// those read the matrix ahead (gt_bring).  Microseconds, library / so (with W read ahead): 2,048 rows of 1,536 x 1,536 17.2 / 15.1,
+// 1,536 x 4,480 35.1 / 32.9, 1,536 x 8,960 70.5 / 74.1 (63.2); 1,377 rows 15.3 / 14.3, 31.3 / 30.3 (29.8), 67.0 / 71.6 (55.7); 832 rows of
+// 4,608 x 3,584 37.6 / 33.1, 3,584 x 3,584 26.8 / 27.4 (28.0), 640 rows of 3,584 x 4,736 40.0 / 44.1 (32.8), x 7,168 54.5 / 57.2 (47.2).  Of up to
+// 128 such tiles 128 x 64 are a single round too; each is as long a chain as the larger, so they pay for short K alone and from
+// where the library's fewer, longer workgroups run out: 700 rows of 1,536 x 1,536 12.8 / 11.1 (640 10.2 / 11.4), 400 of 3,072 x 1,536 13.0 /
+// 11.5, 300 of 4,608 x 1,536 14.0 / 11.6, 832 of 2,048 x 2,048 15.2 / 14.2, of 1,536 x 2,240 16.5 / 14.7, of 1,536 x 3,072 17.8 / 18.9.  Of 191
+// points of 38 matrices in these ranges the geometric mean is 9 % ahead of the library, the worst 13 % behind.
+#define GT_ROUND 256
+#define GT_NARROW 144                                // the library is as fast up to so many tiles of 128 x 64
+#define GT_NARROW_K 2560
+#define GT_BRING (4 << 20)                           // elements of W from which it pays to read ahead
+#define GT_BRING_EACH (1 << 18)                      // and at most for each who does (300 rows of 9,472 x 3,584, a million each: 44 us, 30 without)
+static int gt_small(int M, int N, int mb, int nb) { return ((M + 64 * mb - 1) / (64 * mb)) * ((N + 64 * nb - 1) / (64 * nb)); }
+// 0: more or fewer tiles than that; 1: tiles of 128 x 64; 2: of 128 x 128; 3: of 128 x 128 with W read ahead by the idle workgroups (not
+// with next to no rows in the last tiles, which wait for W alone and so read ahead themselves: 2,052 rows of 1,536 x 8,960 62 us either way)
+extern "C" int pico_gemm_tiles_round(int M, int N, int K) {
+  if (M <= 64 || N <= 0 || K <= 0 || (long long)M * N > (long long)GT_ROUND * 128 * 128) return 0;
+  const int narrow = gt_small(M, N, 2, 1), square = gt_small(M, N, 2, 2), last = (M - 1) % 128 + 1;
+  if (narrow <= GT_ROUND) return K <= GT_NARROW_K && narrow > GT_NARROW ? 1 : 0;
+  if (square > GT_ROUND || square <= GT_ROUND / 2) return 0;
+  const int idle = GT_ROUND - (square + 7) / 8 * 8;
+  return idle >= GT_ROUND / 8 && (long long)N * K >= GT_BRING && (long long)N * K <= (long long)idle * GT_BRING_EACH && last > 32 ? 3 : 2;
+}
+
 // Up to 64 rows of a large matrix: the stream of W bounds a call, and tiles of 64 rows carry it.  32 rows of a 152,064 x 3,584
 // output matrix in float32 203 us (5.4 TB/s; the weight-streaming product 244), of 28,416 pairs, K 3,584, 74 (89).  A row must not
 // depend on how many others the call has, and fewer rows or a smaller matrix go through the weight-streaming product: so its
@@ -287,7 +338,13 @@ extern "C" int pico_gemm_tiles(const void* X, const void* W, const float* bias, 
     PICO_REQUIRE(false, "pico_gemm_tiles: no epilogue %d for few rows", epi);
   }
   switch (epi) {
-    case GT_BF16: return gt_run<GT_BF16>(a, stream);
+    case GT_BF16:
+      switch (pico_gemm_tiles_round(M, N, K)) {
+        case 1: return gt_launch<2, 1, GT_BF16>(a, stream);
+        case 2: return gt_launch<2, 2, GT_BF16, 1, 1, 4>(a, stream);
+        case 3: return gt_launch<2, 2, GT_BF16, 1, 1, 4, true>(a, stream);
+      }
+      return gt_run<GT_BF16>(a, stream);
     case GT_F32: return gt_run<GT_F32>(a, stream);
     case GT_SWIGLU: return gt_run<GT_SWIGLU>(a, stream);
     case GT_RELU2: return gt_run<GT_RELU2>(a, stream);

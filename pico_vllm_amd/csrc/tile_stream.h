@@ -66,10 +66,10 @@ __device__ __forceinline__ int ts_tile(int r, int tiles) {
 
 template <int FROM, int TO> struct Range { static constexpr int from = FROM, to = TO; };
 
-// ENDS: tiles end at a k of their own (k_end).
-template <int MB, int NB, int SETS = 1, bool ENDS = false>
+// ENDS: tiles end at a k of their own (k_end).  BUFS: buffers of a stage each, all but one of them on their way.
+template <int MB, int NB, int SETS = 1, bool ENDS = false, int BUFS = ts_buffers(MB, NB)>
 struct TileStream {
-  static constexpr int NBUF = ts_buffers(MB, NB), STAGE = ts_stage_bytes(MB, NB), LOADS = 2 * (MB + NB);
+  static constexpr int NBUF = BUFS, STAGE = ts_stage_bytes(MB, NB), LOADS = 2 * (MB + NB);
   char* lds;
   int wave, lane;
   int k_end;                            // ENDS: k from here on is asked for as zeros, set by `aim` (at most `run`'s K)
@@ -151,8 +151,8 @@ struct TileStream {
     }
   }
   // The copies that take the place of a finished stage go out in PARTS quarters from its last one on: all four where there
-  // is a third buffer, else three, so that the last has a quarter to land.
-  static constexpr int PARTS = NBUF == 3 ? 4 : 3;
+  // are three buffers, else three, so that the last has a quarter to land.
+  static constexpr int PARTS = NBUF >= 3 ? 4 : 3;
   static constexpr int part(int i) { return LOADS * i / PARTS; }
   // The products of the stage in buffer b, whose first operands are in set 0; leaves the first operands of the stage in
   // buffer `next` there.  `copies` is called with the numbers of the copies to ask for: first what is left of those that

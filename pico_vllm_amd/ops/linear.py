@@ -3,7 +3,8 @@
 bfloat16 weights: with up to 64 rows of activations (decode, small mixed
 steps; up to 256 for small matrices) the weight-streaming matrix-core kernel of this package, with bias,
 SwiGLU or float32 output as its epilogue (for shapes it refuses, this package's plain matrix-core product); with more rows this
-package's tiled product where an activation or a float32 result follows (``kernels.tiles_act_ok`` says where), else the library
+package's tiled product where an activation or a float32 result follows (``kernels.tiles_act_ok`` says where), where a long inner size is cut
+into parts, and where the product is a single round of small tiles (``kernels.tiles_round_ok``), else the library
 GEMM (hipBLASLt through torch), as the reference uses the library for every
 projection (pico_vllm/model.py:200,225,316,318).  float32 weights: this package's product of all 24 bits of
 both operands (in three bfloat16 pieces each, sums in 32 bits, ``csrc/gemm_f32.hip``), never a library
@@ -130,6 +131,8 @@ class Linear:
         parts = kernels.tiles_parts(x, self.weight, self.bias_f32)
         if parts > 1 and not _tuned(x.shape[0]):
             return kernels.gemm_tiles_split(x, self.weight, self.bias_f32, parts)
+        if kernels.tiles_round_ok(x, self.weight) and not _tuned(x.shape[0]):
+            return kernels.gemm_tiles(x, self.weight, self.bias_f32, kernels.EPI_BF16)
         _library_tuning(x.shape[0])
         if self.bias is not None:
             return torch.addmm(self.bias, x, self.weight.t())

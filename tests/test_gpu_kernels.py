@@ -256,6 +256,27 @@ def test_gemm_tiles_gelu_over_its_range(K, M):
     assert bool((out[:, -2] == float("inf")).all()) and bool(out[:, -1].isnan().all())
 
 
+@pytest.mark.parametrize("M,N,K_", [(1024, 1168, 8), (700, 1552, 200), (641, 1600, 2560), (1025, 2064, 72), (1920, 2048, 64), (2048, 2048, 328), (1377, 1536, 2736),
+                                    (1568, 1680, 2504), (1569, 1680, 2504), (1570, 1664, 3000)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_products_of_a_single_round(K, M, N, K_, bias):
+    # the smallest and largest numbers of tiles, ends inside a tile and a stage, with and without workgroups that read the matrix ahead
+    # (the last four), next to no rows in the last tile (1,569 and 1,570: one row more than 32 decides)
+    assert K.library.core().pico_gemm_tiles_round(M, N, K_) == (1 if -(-M // 128) * -(-N // 64) <= 256 else 3 if N * K_ >= 4 << 20 and (M - 1) % 128 >= 32 else 2)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    a, w = torch.full((M, K_ + 8), float("nan"), device=DEV, dtype=torch.bfloat16), torch.full((N, K_ + 16), float("nan"), device=DEV, dtype=torch.bfloat16)
+    a[:, :K_], w[:, :K_] = torch.randn(M, K_, device=DEV, generator=g), torch.randn(N, K_, device=DEV, generator=g)
+    b = torch.randn(N, device=DEV, generator=g) if bias else None
+    a, w = a[:, :K_], w[:, :K_]
+    assert K.tiles_round_ok(a, w)
+    out = K.gemm_tiles(a, w, b)
+    want = a.double() @ w.double().T + (b.double() if bias else 0.0)
+    # float32 sums (a chain of K / 16 additions, 2^-24 of a partial sum each: under 1e-5 of a row's size), rounded to eight bits
+    assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-5 * K_ ** 0.5 * 4).all())
+    rows = slice(M - 70, M)                              # a row's result does not depend on which tiles it is in
+    assert torch.equal(out[rows], K.gemm_tiles(a[rows].contiguous(), w, b))
+
+
 @pytest.mark.parametrize("name", ["swiglu", "clipped"])
 def test_activation_of_the_tiled_product_over_all_numbers(K, name):
     # a gate that is one number of the row, an up that is 1 (0, for the clipped form's u + 1): every bfloat16 number through the
