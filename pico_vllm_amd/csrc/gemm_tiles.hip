@@ -22,6 +22,7 @@ struct GemmArgs {
   int M, cols, K, ldx, ldw, ldo;     // cols: output columns of this launch
   int up;                            // paired epilogues: from a gate row of W to the up row of the same column
   int m_tiles, n_tiles;
+  int bring;                         // so much of every part's k is read ahead by workgroups without a tile (unpaired; the grid has some)
   int splits, part;                  // of K: so many parts of `part` each, a part's sums in out + s M ldo (GT_PARTS; else one)
   float limit, alpha;
 };
@@ -65,25 +66,7 @@ __device__ __forceinline__ float gt_one(float v) {
 }
 typedef float gt_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 
-#ifdef __HIP_DEVICE_COMPILE__
-// A workgroup without a tile reads its share of W's rows, in the order in which the tiles want their k, once: the memory-side cache
-// then has them.  Where a single round of tiles waits for memory stage after stage, W comes from there in half the time.
-__device__ __forceinline__ void gt_bring(const GemmArgs& a, int worker, int workers, char* lds) {
-  const int rows = (a.cols + workers - 1) / workers, r0 = worker * rows, r1 = min(a.cols, r0 + rows);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const __amdgpu_buffer_rsrc_t w = ts_buffer(a.W, ((long long)(a.cols - 1) * a.ldw + a.K) * 2);
-  for (int k = 0; k < a.K; k += TS_BK)
-    for (int r = r0 + 8 * wave; r < r1; r += 32) {                 // eight rows of 128 bytes a copy; its place in LDS is nobody's
-      const int row = r + (lane >> 3), col = k + (lane & 7) * 8;
-      const uint32_t at = row < r1 && col < a.K ? (uint32_t)(row * a.ldw + col) * 2 : TS_OUT;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w, (__attribute__((address_space(3))) void*)(lds + wave * 1024), 16, at, 0, 0, 0);
-    }
-  __builtin_amdgcn_s_waitcnt(ts_wait(0, true));
-}
-#endif
-
-// BRING: workgroups without a tile read W ahead for the others (gt_bring; the grid has some)
-template <int MB, int NB, int EPI, int SETS, int SHARE, int BUFS, bool BRING>
+template <int MB, int NB, int EPI, int SETS, int SHARE, int BUFS>
 __global__ __launch_bounds__(256, SHARE) void gemm_tiles_kernel(const GemmArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -94,7 +77,8 @@ __global__ __launch_bounds__(256, SHARE) void gemm_tiles_kernel(const GemmArgs a
   if (ts_tile(0, tiles) < 0) {
     // (a single round: the first `busy` places of a die have its tiles)
     const int busy = (tiles + 7) >> 3;
-    if (BRING && (int)(blockIdx.x >> 3) >= busy) gt_bring(a, (int)blockIdx.x - 8 * busy, (int)gridDim.x - 8 * busy, smem);
+    if (a.bring > 0 && (int)(blockIdx.x >> 3) >= busy)
+      ts_bring(a.W, a.cols, a.ldw, a.K, a.splits, a.part, a.bring, (int)blockIdx.x - 8 * busy, (int)gridDim.x - 8 * busy, smem);
     return;
   }
   TileRowsSource<MB> xs;
@@ -205,17 +189,31 @@ __global__ __launch_bounds__(256, SHARE) void gemm_tiles_kernel(const GemmArgs a
 #endif
 }
 
-template <int MB, int NB, int EPI, int SETS = 1, int SHARE = ts_share(MB, NB), int BUFS = ts_buffers(MB, NB), bool BRING = false>
+// Of a single round that leaves an eighth of its places idle: how much of every part's k the workgroups there read ahead, all of it or
+// what each of them can while a tile reads GT_BRING times as much (their one wave of copies a SIMD waits for itself); 0: nothing.
+// Few elements are there before it pays to look ahead, and tiles with next to no rows wait for W alone and so read ahead themselves
+// (2,052 rows of 1,536 x 8,960 62 us either way).
+#define GT_BRING 0.4f
+#define GT_BRING_LEAST (4 << 20)
+static int gt_bring(const GemmArgs& a, long long tiles, int slots, int mb, int nb) {
+  const long long idle = slots - (tiles + 7) / 8 * 8;
+  if (idle < slots / 8 || (long long)a.cols * a.K < GT_BRING_LEAST || (a.M - 1) % (64 * mb) < 32) return 0;
+  const float each = (float)a.cols / idle * a.splits / (64 * (mb + nb));
+  return each <= GT_BRING ? a.part : (int)(a.part * GT_BRING / each) / TS_BK * TS_BK;
+}
+
+template <int MB, int NB, int EPI, int SETS = 1, int SHARE = ts_share(MB, NB), int BUFS = ts_buffers(MB, NB)>
 static int gt_launch(GemmArgs a, hipStream_t stream) {
   constexpr int bytes = ts_stage_bytes(MB, NB) * BUFS;
-  const auto kernel = gemm_tiles_kernel<MB, NB, EPI, SETS, SHARE, BUFS, BRING>;
+  const auto kernel = gemm_tiles_kernel<MB, NB, EPI, SETS, SHARE, BUFS>;
   static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   PICO_REQUIRE(room == hipSuccess, "pico_gemm_tiles: %s", hipGetErrorString(room));
   a.m_tiles = (a.M + 64 * MB - 1) / (64 * MB);
   a.n_tiles = (a.cols + GT_COLS(NB, EPI) - 1) / GT_COLS(NB, EPI);
   const long long tiles = (long long)a.m_tiles * a.n_tiles * a.splits;
   PICO_REQUIRE(tiles < (1LL << 30), "pico_gemm_tiles: %d x %d outputs are too many for one launch", a.M, a.cols);
-  kernel<<<BRING ? 256 * SHARE : ts_grid(tiles, 256 * SHARE), 256, bytes, stream>>>(a);
+  a.bring = gt_paired(EPI) ? 0 : gt_bring(a, tiles, 256 * SHARE, MB, NB);
+  kernel<<<a.bring ? 256 * SHARE : ts_grid(tiles, 256 * SHARE), 256, bytes, stream>>>(a);
   PICO_LAUNCH_CHECK();
   return 0;
 }
@@ -288,18 +286,13 @@ static int gt_run(GemmArgs a, hipStream_t stream) {
 #define GT_ROUND 256
 #define GT_NARROW 144                                // the library is as fast up to so many tiles of 128 x 64
 #define GT_NARROW_K 2560
-#define GT_BRING (4 << 20)                           // elements of W from which it pays to read ahead
-#define GT_BRING_EACH (1 << 18)                      // and at most for each who does (300 rows of 9,472 x 3,584, a million each: 44 us, 30 without)
 static int gt_small(int M, int N, int mb, int nb) { return ((M + 64 * mb - 1) / (64 * mb)) * ((N + 64 * nb - 1) / (64 * nb)); }
-// 0: more or fewer tiles than that; 1: tiles of 128 x 64; 2: of 128 x 128; 3: of 128 x 128 with W read ahead by the idle workgroups (not
-// with next to no rows in the last tiles, which wait for W alone and so read ahead themselves: 2,052 rows of 1,536 x 8,960 62 us either way)
+// 0: more or fewer tiles than that; 1: tiles of 128 x 64; 2: of 128 x 128
 extern "C" int pico_gemm_tiles_round(int M, int N, int K) {
   if (M <= 64 || N <= 0 || K <= 0 || (long long)M * N > (long long)GT_ROUND * 128 * 128) return 0;
-  const int narrow = gt_small(M, N, 2, 1), square = gt_small(M, N, 2, 2), last = (M - 1) % 128 + 1;
+  const int narrow = gt_small(M, N, 2, 1), square = gt_small(M, N, 2, 2);
   if (narrow <= GT_ROUND) return K <= GT_NARROW_K && narrow > GT_NARROW ? 1 : 0;
-  if (square > GT_ROUND || square <= GT_ROUND / 2) return 0;
-  const int idle = GT_ROUND - (square + 7) / 8 * 8;
-  return idle >= GT_ROUND / 8 && (long long)N * K >= GT_BRING && (long long)N * K <= (long long)idle * GT_BRING_EACH && last > 32 ? 3 : 2;
+  return square <= GT_ROUND && square > GT_ROUND / 2 ? 2 : 0;
 }
 
 // Up to 64 rows of a large matrix: the stream of W bounds a call, and tiles of 64 rows carry it.  32 rows of a 152,064 x 3,584
@@ -327,7 +320,7 @@ extern "C" int pico_gemm_tiles(const void* X, const void* W, const float* bias, 
   PICO_REQUIRE((long long)M * ldx < (1LL << 30) && (long long)N * ldw < (1LL << 30), "pico_gemm_tiles: an operand spans 2^31 bytes or more");
   PICO_REQUIRE(!bias || !gt_paired(epi), "pico_gemm_tiles: the paired epilogues take no bias");
   if (M == 0) return 0;
-  GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, bias, out, M, cols, K, ldx, ldw, ldo, N - cols, 0, 0, 1, K, limit, alpha};
+  GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, bias, out, M, cols, K, ldx, ldw, ldo, N - cols, 0, 0, 0, 1, K, limit, alpha};
   if (few) {
     PICO_REQUIRE(M <= 64, "pico_gemm_tiles: %d rows are not few", M);
     switch (epi) {
@@ -342,7 +335,6 @@ extern "C" int pico_gemm_tiles(const void* X, const void* W, const float* bias, 
       switch (pico_gemm_tiles_round(M, N, K)) {
         case 1: return gt_launch<2, 1, GT_BF16>(a, stream);
         case 2: return gt_launch<2, 2, GT_BF16, 1, 1, 4>(a, stream);
-        case 3: return gt_launch<2, 2, GT_BF16, 1, 1, 4, true>(a, stream);
       }
       return gt_run<GT_BF16>(a, stream);
     case GT_F32: return gt_run<GT_F32>(a, stream);
@@ -406,7 +398,7 @@ extern "C" int pico_gemm_tiles_split(const void* X, const void* W, const float* 
   PICO_REQUIRE(((uintptr_t)X | (uintptr_t)W | (uintptr_t)out | (uintptr_t)parts | (uintptr_t)bias) % 16 == 0, "pico_gemm_tiles_split: operands must start on 16 bytes");
   PICO_REQUIRE((long long)M * ldx < (1LL << 30) && (long long)N * ldw < (1LL << 30), "pico_gemm_tiles_split: an operand spans 2^31 bytes or more");
   if (M == 0) return 0;
-  GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, nullptr, parts, M, N, K, ldx, ldw, N, 0, 0, 0, splits, gt_part(K, splits), 0.f, 0.f};
+  GemmArgs a{(const bf16_t*)X, (const bf16_t*)W, nullptr, parts, M, N, K, ldx, ldw, N, 0, 0, 0, 0, splits, gt_part(K, splits), 0.f, 0.f};
   const int rc = gt_run<GT_PARTS>(a, stream);
   if (rc) return rc;
   const long long eights = (long long)M * N / 8;

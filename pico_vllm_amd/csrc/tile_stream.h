@@ -234,6 +234,23 @@ struct TileStream {
   }
 };
 
+// Copies of the rows worker, worker + workers, .. (eights of them) of `rows` rows of stride ld, k from `parts` starts `part` apart on side
+// by side, `most` of each, to nobody's place in LDS: the memory-side cache then has them.  Tiles that wait for memory stage after stage
+// get theirs from there in half the time, so workgroups without a tile do this for the others' matrix, in the order in which those want it.
+__device__ __forceinline__ void ts_bring(const bf16_t* base, int rows, int ld, int K, int parts, int part, int most, int worker, int workers, char* lds) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const __amdgpu_buffer_rsrc_t r = ts_buffer(base, ((long long)(rows - 1) * ld + K) * 2);
+  const int each = ((rows + workers - 1) / workers + 7) / 8 * 8, r0 = worker * each, r1 = min(rows, r0 + each);
+  for (int k = 0; k < most; k += TS_BK)
+    for (int p = 0; p < parts; p++)
+      for (int i = r0 + 8 * wave; i < r1; i += 32) {               // eight rows of 128 bytes a copy
+        const int row = i + (lane >> 3), at = k + (lane & 7) * 8, col = p * part + at;
+        const uint32_t off = row < r1 && at < part && col < K ? (uint32_t)(row * ld + col) * 2 : TS_OUT;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(lds + wave * 1024), 16, off, 0, 0, 0);
+      }
+  __builtin_amdgcn_s_waitcnt(ts_wait(0, true));
+}
+
 // Tile t of the order in which tiles are dealt out: strips of up to 8 tiles of rows, inside a strip column by column, so
 // that the 32 tiles a die works on at a time are about 8 x 4 and share their operands in its L2.
 __device__ __forceinline__ void ts_place(int m_tiles, int n_tiles, int t, int& m, int& n) {
