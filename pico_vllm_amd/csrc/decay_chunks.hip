@@ -9,23 +9,25 @@
 //   S_n = g^n S0 + L,   L = sum_j g^(n - 1 - j) k_j v_j^T
 //
 // Three launches: every chunk's L from zero; a walk over a sequence's chunks that turns the L's into the states in front
-// of the chunks and leaves the slot's new state; every chunk's outputs.  The operands are bfloat16 rows (optionally through
-// z sigmoid(z) as they are read); from there on everything is float32, the products included (v_mfma_f32_32x32x2_f32), so
-// state, decays and sums are what the walk's are, in another order.
+// of the chunks and leaves the slot's new state; every chunk's outputs.  The operands are bfloat16 rows; state, decays and sums are
+// float32 as the walk's are, in another order, and nothing is rounded to less on the way (decay_pieces_*: what is multiplied with
+// the rows is taken apart).  Rows that go through z sigmoid(z) as they are read are float32 numbers on both sides of a product: those run
+// on v_mfma_f32_32x32x2_f32 (decay_chunk_*).
 //
 // VAR: the decay changes from token to token (one number a head), g^(i - j) becomes the product of the decays behind j up to
 // i, a written key has a factor, and heads share queries and keys (a state-space duality layer).
 //
-// 2,048 tokens of 48 heads of 128 x 64 over two heads of queries and keys: 128 us against 366 for the walk in chunks on the
-// vector units, 300 tokens 35 against 151; error against 64 bits 1.0e-7 against 1.3e-7.  Bound by the states' traffic (52 MB
-// written, walked and read) and by LDS, which lets one workgroup of the outputs onto a compute unit at 128 key channels.
+// 2,048 tokens of 48 heads of 128 x 64 over two heads of queries and keys: 71 us; 125 with all products on the float32 instruction, 366
+// for the walk in chunks on the vector units; 300 tokens 26, 31 and 151; error against 64 bits 0.86e-7, 1.05e-7 and 1.3e-7.  12 heads of
+// 64 x 128 with a constant decay: 1,377 tokens 31 us and 40, error 2.2e-7 and 2.7e-7.  Bound by the states' traffic (52 MB written,
+// walked and read), the float32 instruction by itself and by LDS, which lets one of its workgroups onto a compute unit at 128 key channels.
 //
-// A workgroup (four waves) owns one chunk, one head and 32 NBLK value columns; its rows lie in LDS as float32.  An operand
+// decay_chunk_*: a workgroup (four waves) owns one chunk, one head and 32 NBLK value columns; its rows lie in LDS as float32.  An operand
 // tile of the products is 32 rows (lane % 32) by 2 k (lane / 32); which k a step takes is free as long as both operands
 // agree, so lane half h takes k = 8 b + 4 h + 0..3 over four steps: four contiguous floats where k runs along a row.
-#include "common.h"
+#include "split3.h"
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef s3_f32x16 f32x16;
 
 #define DC_CHUNK 64
 
@@ -152,28 +154,21 @@ __device__ __forceinline__ bool chunk_tokens(const ChunkArgs& a, int& t0, int& n
 
 // L of every chunk into ws.  Wave w: value columns 32 (w % NBLK) .. of the workgroup's; with fewer than four column blocks
 // the waves of one share the key channels.
-template <int DKP, int NBLK, bool VAR>
+template <int DKP, int NBLK>
 __global__ __launch_bounds__(256) void decay_chunk_state_kernel(const ChunkArgs a) {
   constexpr int KS = DKP + 4, NB = 32 * NBLK, VS = NB + 8, CB = DKP / 32, SHARE = 4 / NBLK;
-  __shared__ double lc[VAR ? DC_CHUNK : 1];
-  __shared__ float be[VAR ? DC_CHUNK : 1];
   __shared__ __attribute__((aligned(16))) float ks[DC_CHUNK * KS];
   __shared__ __attribute__((aligned(16))) float vs[DC_CHUNK * VS];
   int t0, n;
   if (!chunk_tokens(a, t0, n)) return;
   const int h = blockIdx.y, n0 = blockIdx.z * NB, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane & 31, half = lane >> 5;
-  const float lg = VAR ? 0.f : log2f(a.decay[h]);
+  const float lg = log2f(a.decay[h]);
   const bf16_t* row = a.x + (size_t)t0 * a.ld;
   Rows<DKP> k;
   Rows<NB> v;
-  k.fetch(row + a.k_col + (VAR ? h / a.share : h) * a.dk, a.ld, n, a.dk);
+  k.fetch(row + a.k_col + h * a.dk, a.ld, n, a.dk);
   v.fetch(row + a.v_col + h * a.dv + n0, a.ld, n, a.dv - n0);
-  if (VAR) {
-    chunk_decays(a, t0, n, h, lc, be);
-    __syncthreads();
-    if (threadIdx.x == 0 && n0 == 0) a.ws_decay[(size_t)blockIdx.x * a.H + h] = exp2f((float)lc[n - 1]);
-  }
-  k.put(ks, KS, n, a.dk, a.silu, [&](int r) { return VAR ? be[r] * between(lc[r], lc[n - 1]) : decay_power(lg, n - 1 - r); });
+  k.put(ks, KS, n, a.dk, a.silu, [&](int r) { return decay_power(lg, n - 1 - r); });
   v.put(vs, VS, n, a.dv - n0, a.silu, [&](int) { return 1.0f; });
   __syncthreads();
   const int nb = wave % NBLK, c_first = wave / NBLK;
@@ -268,10 +263,8 @@ __global__ __launch_bounds__(256) void decay_chunk_walk_kernel(const ChunkArgs a
 //
 // A token's weight on a later one is 0, and 0 * Inf is NaN: the products see an Inf or NaN among the values as zero, and
 // where there is one it is added afterwards to the tokens from its own on.
-template <int DKP, int NBLK, bool VAR>
+template <int DKP, int NBLK>
 __global__ __launch_bounds__(256) void decay_chunk_out_kernel(const ChunkArgs a) {
-  __shared__ double lc[VAR ? DC_CHUNK : 1];
-  __shared__ float be[VAR ? DC_CHUNK : 1];
   __shared__ bool odd_values[4];
   constexpr int KS = DKP + 4, PS = DC_CHUNK + 4, NB = 32 * NBLK, VS = NB + 8, IB = NBLK == 4 ? 2 : 1;
   extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -282,13 +275,12 @@ __global__ __launch_bounds__(256) void decay_chunk_out_kernel(const ChunkArgs a)
   if (!chunk_tokens(a, t0, n)) return;
   const int h = blockIdx.y, n0 = blockIdx.z * NB, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane & 31, half = lane >> 5;
   const int nb = wave % NBLK, ib0 = NBLK == 4 ? 0 : wave / NBLK, col = n0 + 32 * nb + l;
-  const float lg = VAR ? 0.f : log2f(a.decay[h]);
+  const float lg = log2f(a.decay[h]);
   const bf16_t* row = a.x + (size_t)t0 * a.ld;
-  const int hk = VAR ? h / a.share : h;
   Rows<DKP> q, k;
   Rows<NB> v;
-  q.fetch(row + a.q_col + hk * a.dk, a.ld, n, a.dk);
-  k.fetch(row + a.k_col + hk * a.dk, a.ld, n, a.dk);
+  q.fetch(row + a.q_col + h * a.dk, a.ld, n, a.dk);
+  k.fetch(row + a.k_col + h * a.dk, a.ld, n, a.dk);
   v.fetch(row + a.v_col + h * a.dv + n0, a.ld, n, a.dv - n0);
   // the state in front of the chunk as an operand: rows 8 b + 4 half + 0..3, this lane's column
   float s0[DKP / 2];
@@ -301,7 +293,6 @@ __global__ __launch_bounds__(256) void decay_chunk_out_kernel(const ChunkArgs a)
   k.put(ks, KS, n, a.dk, a.silu, [&](int) { return 1.0f; });
   const bool odd = __any(v.template put<true>(vs, VS, n, a.dv - n0, a.silu, [&](int) { return 1.0f; }));
   if (lane == 0) odd_values[wave] = odd;
-  if (VAR) chunk_decays(a, t0, n, h, lc, be);
   __syncthreads();
   // queries and keys: wave 0 block (0, 0), wave 1 (1, 0), wave 2 (1, 1)
   const int pi = wave == 0 ? 0 : 1, pj = wave == 2 ? 1 : 0;
@@ -346,14 +337,14 @@ __global__ __launch_bounds__(256) void decay_chunk_out_kernel(const ChunkArgs a)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const int t = 32 * (ib0 + i) + 8 * (r >> 2) + 4 * half + (r & 3);
-      acc[i][r] = (acc[i][r] + half_sum[i][r]) * (VAR ? exp2f((float)lc[t]) : decay_power(lg, t + 1));
+      acc[i][r] = (acc[i][r] + half_sum[i][r]) * decay_power(lg, t + 1);
     }
   __syncthreads();                                       // every wave is done with the keys
   if (wave < 3) {
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const int i = 32 * pi + 8 * (r >> 2) + 4 * half + (r & 3), j = 32 * pj + l;
-      ks[i * PS + j] = j <= i ? p[r] * (VAR ? be[j] * between(lc[j], lc[i]) : decay_power(lg, i - j)) : 0.f;
+      ks[i * PS + j] = j <= i ? p[r] * decay_power(lg, i - j) : 0.f;
     }
   }
   __syncthreads();
@@ -396,23 +387,320 @@ __global__ __launch_bounds__(256) void decay_chunk_out_kernel(const ChunkArgs a)
     }
 }
 
-template <int DKP, int NBLK, bool VAR>
-static int launch_chunks(const ChunkArgs& a, int num_seqs, hipStream_t stream) {
-  constexpr int KS = DKP + 4, PS = DC_CHUNK + 4, VS = 32 * NBLK + 8;
-  constexpr int bytes = DC_CHUNK * (KS + (KS > PS ? KS : PS) + VS) * (int)sizeof(float);
-  static bool raised = false;
-  if (!raised) {
-    PICO_REQUIRE(hipFuncSetAttribute((const void*)decay_chunk_out_kernel<DKP, NBLK, VAR>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess,
-                 "pico_decay_chunks: %d bytes of LDS refused", bytes);
-    raised = true;
+// ---------------------------------------------------------------------------
+// Rows that are read as they stand (no z sigmoid(z)): q, k and v are bfloat16 numbers, and what they are multiplied with, state, weighted
+// values and weighted products, is taken apart into three of them (split3.h; three instructions of 16 k, 3/16 of the float32
+// instruction's time).  Products of queries and keys are the bfloat16 instruction's own.  All of a tile in LDS is bfloat16: a
+// third of the bytes, so that three workgroups share a compute unit.  Pieces of numbers below 2^-110 end at 2^-133.
+// ---------------------------------------------------------------------------
+#define DC_TS (DC_CHUNK + 8)             // row stride of [channel][token] and [token][token] planes: 16-byte reads of rows meet every bank once
+
+// Two numbers' pieces; what is not finite (or rounds to it) is its own upper piece.
+__device__ __forceinline__ void split2_any(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = pack2_bf16(a, b);
+  const float ha = s3_low(h), hb = s3_high(h);
+  a = fabsf(ha) < INFINITY ? a - ha : 0.f;
+  b = fabsf(hb) < INFINITY ? b - hb : 0.f;
+  m = pack2_bf16(a, b);
+  l = pack2_bf16(a - s3_low(m), b - s3_high(m));
+}
+
+// 64 rows x COLS columns on their way to LDS turned around: a thread has two neighbouring rows of eight columns.
+template <int COLS>
+struct Turned {
+  static constexpr int UNITS = 32 * COLS / 8, N = (UNITS + 255) / 256;
+  uint4 v[N][2];
+  __device__ __forceinline__ int pair(int i) const { return (threadIdx.x + 256 * i) % 32; }
+  __device__ __forceinline__ int col(int i) const { return (threadIdx.x + 256 * i) / 32 * 8; }
+  __device__ __forceinline__ void fetch(const bf16_t* src, int ld, int n, int cols) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const int c = col(i) < cols ? col(i) : 0;
+#pragma unroll
+      for (int k = 0; k < 2; k++) v[i][k] = *reinterpret_cast<const uint4*>(src + (size_t)min(2 * pair(i) + k, n - 1) * ld + c);
+    }
   }
-  const dim3 grid(a.chunks, a.H, (a.dv + 32 * NBLK - 1) / (32 * NBLK));
-  decay_chunk_state_kernel<DKP, NBLK, VAR><<<grid, 256, 0, stream>>>(a);
+  // use(column, row pair, word of the two rows' numbers in it): rows from n on and columns from `cols` on are zero
+  template <typename F>
+  __device__ __forceinline__ void each(int n, int cols, F use) const {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      if (COLS % 64 != 0 && (int)threadIdx.x + 256 * i >= UNITS) break;
+      const int r = 2 * pair(i);
+      const uint32_t a[4] = {v[i][0].x, v[i][0].y, v[i][0].z, v[i][0].w}, b[4] = {v[i][1].x, v[i][1].y, v[i][1].z, v[i][1].w};
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int c = col(i) + j;
+        const uint32_t lo = (j & 1) ? a[j / 2] >> 16 : a[j / 2] & 0xffffu, hi = (j & 1) ? b[j / 2] & 0xffff0000u : b[j / 2] << 16;
+        use(c, r, c < cols ? (r < n ? lo : 0u) | (r + 1 < n ? hi : 0u) : 0u);
+      }
+    }
+  }
+};
+
+__device__ __forceinline__ s3_u32x4 dc_read(const bf16_t* p) { return *reinterpret_cast<const s3_u32x4*>(p); }
+
+template <int DKP, int NBLK>
+constexpr int dc_state_bytes() { return (DKP + 3 * 32 * NBLK) * DC_TS * 2; }
+template <int DKP, int NBLK>
+constexpr int dc_out_bytes() {
+  const int rows = 2 * DC_CHUNK * (DKP + 8), planes = 3 * DC_CHUNK * DC_TS;
+  return ((rows > planes ? rows : planes) + 32 * NBLK * DC_TS) * 2;
+}
+
+// L of every chunk into ws, as decay_chunk_state_kernel; the weights on the values.
+template <int DKP, int NBLK, bool VAR>
+__global__ __launch_bounds__(256, 2) void decay_pieces_state_kernel(const ChunkArgs a) {
+  constexpr int NB = 32 * NBLK, CB = DKP / 32, SHARE = 4 / NBLK, PLANE = NB * DC_TS;
+  __shared__ double lc[VAR ? DC_CHUNK : 1];
+  __shared__ float be[VAR ? DC_CHUNK : 1];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  bf16_t* kt = reinterpret_cast<bf16_t*>(lds);                // [DKP][DC_TS]
+  bf16_t* vt = kt + DKP * DC_TS;                              // three planes of [NB][DC_TS]
+  int t0, n;
+  if (!chunk_tokens(a, t0, n)) return;
+  const int h = blockIdx.y, n0 = blockIdx.z * NB, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane & 31, half = lane >> 5;
+  const float lg = VAR ? 0.f : log2f(a.decay[h]);
+  const bf16_t* row = a.x + (size_t)t0 * a.ld;
+  Turned<DKP> k;
+  Turned<NB> v;
+  k.fetch(row + a.k_col + (VAR ? h / a.share : h) * a.dk, a.ld, n, a.dk);
+  v.fetch(row + a.v_col + h * a.dv + n0, a.ld, n, a.dv - n0);
+  if (VAR) {
+    chunk_decays(a, t0, n, h, lc, be);
+    __syncthreads();
+    if (threadIdx.x == 0 && n0 == 0) a.ws_decay[(size_t)blockIdx.x * a.H + h] = exp2f((float)lc[n - 1]);
+  }
+  k.each(n, a.dk, [&](int c, int r, uint32_t w) { *reinterpret_cast<uint32_t*>(kt + c * DC_TS + r) = w; });
+  const int pair = 2 * (threadIdx.x % 32);                    // this thread's rows (of every unit)
+  float f[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) f[i] = pair + i < n ? (VAR ? be[pair + i] * between(lc[pair + i], lc[n - 1]) : decay_power(lg, n - 1 - pair - i)) : 0.f;
+  v.each(n, a.dv - n0, [&](int c, int r, uint32_t w) {
+    uint32_t p[3];
+    split2_any(r < n ? s3_low(w) * f[0] : 0.f, r + 1 < n ? s3_high(w) * f[1] : 0.f, p[0], p[1], p[2]);
+#pragma unroll
+    for (int i = 0; i < 3; i++) *reinterpret_cast<uint32_t*>(vt + i * PLANE + c * DC_TS + r) = p[i];
+  });
+  __syncthreads();
+  const int nb = wave % NBLK, c_first = wave / NBLK;
+  f32x16 acc[(CB + SHARE - 1) / SHARE];
+#pragma unroll
+  for (int i = 0; i < (CB + SHARE - 1) / SHARE; i++) acc[i] = zero16();
+#pragma unroll
+  for (int j = 0; j < DC_CHUNK; j += 16) {
+    if (j >= n) break;                                        // (rows from n on are zero)
+    const bf16_t* vp = vt + (32 * nb + l) * DC_TS + j + 8 * half;
+    const s3_u32x4 vl = dc_read(vp + 2 * PLANE), vm = dc_read(vp + PLANE), vh = dc_read(vp);
+#pragma unroll
+    for (int i = 0; i < (CB + SHARE - 1) / SHARE; i++) {
+      const s3_u32x4 kk = dc_read(kt + (32 * min(c_first + i * SHARE, CB - 1) + l) * DC_TS + j + 8 * half);
+      acc[i] = mfma16(kk, vl, acc[i]);
+      acc[i] = mfma16(kk, vm, acc[i]);
+      acc[i] = mfma16(kk, vh, acc[i]);
+    }
+  }
+  float* ws = a.ws + ((size_t)blockIdx.x * a.H + h) * a.dk * a.dv;
+  const int col = n0 + 32 * nb + l;
+  if (col >= a.dv) return;
+#pragma unroll
+  for (int i = 0; i < (CB + SHARE - 1) / SHARE; i++) {
+    const int cb = c_first + i * SHARE;
+    if (cb >= CB) break;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int c = 32 * cb + 8 * (r >> 2) + 4 * half + (r & 3);
+      if (c < a.dk) ws[(size_t)c * a.dv + col] = acc[i][r];
+    }
+  }
+}
+
+// The outputs of every chunk, as decay_chunk_out_kernel.  The products of queries and keys are made turned around (a lane has
+// a query, a register a key), so that a lane writes four neighbouring keys' pieces at a time.
+template <int DKP, int NBLK, bool VAR>
+__global__ __launch_bounds__(256, 2) void decay_pieces_out_kernel(const ChunkArgs a) {
+  constexpr int QS = DKP + 8, NB = 32 * NBLK, IB = NBLK == 4 ? 2 : 1, PLANE = DC_CHUNK * DC_TS, UNITS = DC_CHUNK * DKP / 8 / 256;
+  static_assert(UNITS >= 1, "at least one piece a thread");
+  __shared__ double lc[VAR ? DC_CHUNK : 1];
+  __shared__ float be[VAR ? DC_CHUNK : 1];
+  __shared__ bool odd_values[4];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  bf16_t* qs = reinterpret_cast<bf16_t*>(lds);                // [64][QS], then the weighted products' planes [64][DC_TS]
+  bf16_t* ks = qs + DC_CHUNK * QS;
+  bf16_t* ps = qs;
+  bf16_t* vt = qs + (2 * DC_CHUNK * QS > 3 * PLANE ? 2 * DC_CHUNK * QS : 3 * PLANE);      // [NB][DC_TS]
+  int t0, n;
+  if (!chunk_tokens(a, t0, n)) return;
+  const int h = blockIdx.y, n0 = blockIdx.z * NB, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane & 31, half = lane >> 5;
+  const int nb = wave % NBLK, ib0 = NBLK == 4 ? 0 : wave / NBLK, col = n0 + 32 * nb + l;
+  const float lg = VAR ? 0.f : log2f(a.decay[h]);
+  const bf16_t* row = a.x + (size_t)t0 * a.ld;
+  const bf16_t* qrow = row + a.q_col + (VAR ? h / a.share : h) * a.dk;
+  const bf16_t* krow = row + a.k_col + (VAR ? h / a.share : h) * a.dk;
+  uint4 qv[UNITS], kv[UNITS];
+#pragma unroll
+  for (int i = 0; i < UNITS; i++) {
+    const int u = threadIdx.x + 256 * i, r = u / (DKP / 8), c = u % (DKP / 8) * 8;
+    const size_t at = (size_t)min(r, n - 1) * a.ld + (c < a.dk ? c : 0);
+    qv[i] = *reinterpret_cast<const uint4*>(qrow + at);
+    kv[i] = *reinterpret_cast<const uint4*>(krow + at);
+  }
+  Turned<NB> v;
+  v.fetch(row + a.v_col + h * a.dv + n0, a.ld, n, a.dv - n0);
+  // the state in front of the chunk as an operand: of 16 channels the half'th eight, this lane's column
+  float s0[DKP / 2];
+  {
+    const float* sp = a.ws + ((size_t)blockIdx.x * a.H + h) * a.dk * a.dv + min(col, a.dv - 1);
+#pragma unroll
+    for (int i = 0; i < DKP / 2; i++) s0[i] = sp[(size_t)min(i / 8 * 16 + 8 * half + i % 8, a.dk - 1) * a.dv];
+  }
+#pragma unroll
+  for (int i = 0; i < UNITS; i++) {
+    const int u = threadIdx.x + 256 * i, r = u / (DKP / 8), c = u % (DKP / 8) * 8;
+    const bool in = r < n && c < a.dk;
+    *reinterpret_cast<uint4*>(qs + r * QS + c) = in ? qv[i] : make_uint4(0, 0, 0, 0);
+    *reinterpret_cast<uint4*>(ks + r * QS + c) = in ? kv[i] : make_uint4(0, 0, 0, 0);
+  }
+  bool odd = false;                                           // an Inf or NaN among the values is written as zero
+  v.each(n, a.dv - n0, [&](int c, int r, uint32_t w) {
+    const bool lo = (w & 0x7f80u) == 0x7f80u, hi = (w & 0x7f800000u) == 0x7f800000u;
+    odd = odd || lo || hi;
+    *reinterpret_cast<uint32_t*>(vt + c * DC_TS + r) = (lo ? 0u : w & 0xffffu) | (hi ? 0u : w & 0xffff0000u);
+  });
+  odd = __any(odd);
+  if (lane == 0) odd_values[wave] = odd;
+  if (VAR) chunk_decays(a, t0, n, h, lc, be);
+  __syncthreads();
+  // keys by queries: wave 0 queries 0 .. 31 and keys 0 .. 31, wave 1 the later queries, wave 2 the later of both
+  const int pi = wave == 0 ? 0 : 1, pj = wave == 2 ? 1 : 0;
+  f32x16 p = zero16();
+  if (wave < 3) {
+#pragma unroll
+    for (int c = 0; c < DKP; c += 16)
+      p = mfma16(dc_read(ks + (32 * pj + l) * QS + c + 8 * half), dc_read(qs + (32 * pi + l) * QS + c + 8 * half), p);
+  }
+  // what the state contributes
+  f32x16 acc[IB];
+#pragma unroll
+  for (int i = 0; i < IB; i++) acc[i] = zero16();
+#pragma unroll
+  for (int c = 0; c < DKP; c += 16) {
+    s3_u32x4 sh, sm, sl;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      uint32_t x, y, z;
+      split2_any(s0[c / 2 + 2 * w], s0[c / 2 + 2 * w + 1], x, y, z);
+      sh[w] = x; sm[w] = y; sl[w] = z;
+    }
+#pragma unroll
+    for (int i = 0; i < IB; i++) {
+      // (rows of the state from dk on stand beside zeros of q; they are another row's numbers, finite as the state is)
+      const s3_u32x4 qq = dc_read(qs + (32 * (ib0 + i) + l) * QS + c + 8 * half);
+      acc[i] = mfma16(qq, sl, acc[i]);
+      acc[i] = mfma16(qq, sm, acc[i]);
+      acc[i] = mfma16(qq, sh, acc[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < IB; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int t = 32 * (ib0 + i) + 8 * (r >> 2) + 4 * half + (r & 3);
+      acc[i][r] *= (VAR ? exp2f((float)lc[t]) : decay_power(lg, t + 1)) * a.qscale;
+    }
+  __syncthreads();                                            // every wave is done with the queries and keys
+  if (wave < 3) {
+    const int i = 32 * pi + l;
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) {
+      const int j0 = 32 * pj + 2 * r + 4 * half;
+      float w[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int j = j0 + e;
+        w[e] = j <= i ? p[r + e] * a.qscale * (VAR ? be[j] * between(lc[j], lc[i]) : decay_power(lg, i - j)) : 0.f;
+      }
+      uint32_t x[3], y[3];
+      split2_any(w[0], w[1], x[0], x[1], x[2]);
+      split2_any(w[2], w[3], y[0], y[1], y[2]);
+#pragma unroll
+      for (int e = 0; e < 3; e++) *reinterpret_cast<uint2*>(ps + e * PLANE + i * DC_TS + j0) = make_uint2(x[e], y[e]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < IB; i++) {
+    const int ib = ib0 + i;
+    const bf16_t* pp = ps + (32 * ib + l) * DC_TS + 8 * half;
+#pragma unroll
+    for (int j = 0; j < DC_CHUNK; j += 16) {
+      if (j >= 32 * (ib + 1)) break;
+      const s3_u32x4 vv = dc_read(vt + (32 * nb + l) * DC_TS + j + 8 * half);
+      acc[i] = mfma16(dc_read(pp + 2 * PLANE + j), vv, acc[i]);
+      acc[i] = mfma16(dc_read(pp + PLANE + j), vv, acc[i]);
+      acc[i] = mfma16(dc_read(pp + j), vv, acc[i]);
+    }
+  }
+  if (col >= a.dv) return;
+  if (odd_values[0] || odd_values[1] || odd_values[2] || odd_values[3]) {
+    const bf16_t* vcol = row + a.v_col + h * a.dv + col;
+#pragma unroll 1
+    for (int j = 0; j < n; j++) {
+      const float x = bf16_to_f32(vcol[(size_t)j * a.ld]);
+      if (fabsf(x) < INFINITY) continue;
+#pragma unroll
+      for (int i = 0; i < IB; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int t = 32 * (ib0 + i) + 8 * (r >> 2) + 4 * half + (r & 3);
+          const bf16_t* w = ps + t * DC_TS + j;
+          // (the block of later keys and earlier queries is not written)
+          if (t >= j) acc[i][r] = fmaf(bf16_to_f32(w[0]) + (bf16_to_f32(w[PLANE]) + bf16_to_f32(w[2 * PLANE])), x, acc[i][r]);
+        }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < IB; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int t = 32 * (ib0 + i) + 8 * (r >> 2) + 4 * half + (r & 3);
+      if (t < n) a.out[(size_t)(t0 + t) * a.H * a.dv + (size_t)h * a.dv + col] = acc[i][r];
+    }
+}
+
+// The walk between the chunks' two launches
+template <bool VAR>
+static void launch_walk(const ChunkArgs& a, int num_seqs, hipStream_t stream) {
   if (num_seqs > 4 && (uintptr_t)a.state % 16 == 0 && (uintptr_t)a.ws % 16 == 0)       // (dv is a multiple of 8)
     decay_chunk_walk_kernel<VAR, 4><<<dim3(num_seqs, a.H, (a.dk * a.dv + 1023) / 1024), 256, 0, stream>>>(a);
   else
     decay_chunk_walk_kernel<VAR, 1><<<dim3(num_seqs, a.H, (a.dk * a.dv + 255) / 256), 256, 0, stream>>>(a);
-  decay_chunk_out_kernel<DKP, NBLK, VAR><<<grid, 256, bytes, stream>>>(a);
+}
+
+template <int DKP, int NBLK>
+static int launch_chunks(const ChunkArgs& a, int num_seqs, hipStream_t stream) {
+  constexpr int KS = DKP + 4, PS = DC_CHUNK + 4, VS = 32 * NBLK + 8;
+  constexpr int bytes = DC_CHUNK * (KS + (KS > PS ? KS : PS) + VS) * (int)sizeof(float);
+  static const hipError_t room = hipFuncSetAttribute((const void*)decay_chunk_out_kernel<DKP, NBLK>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  PICO_REQUIRE(room == hipSuccess, "pico_decay_chunks: %d bytes of LDS refused", bytes);
+  const dim3 grid(a.chunks, a.H, (a.dv + 32 * NBLK - 1) / (32 * NBLK));
+  decay_chunk_state_kernel<DKP, NBLK><<<grid, 256, 0, stream>>>(a);
+  launch_walk<false>(a, num_seqs, stream);
+  decay_chunk_out_kernel<DKP, NBLK><<<grid, 256, bytes, stream>>>(a);
+  PICO_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int DKP, int NBLK, bool VAR>
+static int launch_pieces(const ChunkArgs& a, int num_seqs, hipStream_t stream) {
+  constexpr int first = dc_state_bytes<DKP, NBLK>(), last = dc_out_bytes<DKP, NBLK>();
+  static const hipError_t room1 = hipFuncSetAttribute((const void*)decay_pieces_state_kernel<DKP, NBLK, VAR>, hipFuncAttributeMaxDynamicSharedMemorySize, first);
+  static const hipError_t room2 = hipFuncSetAttribute((const void*)decay_pieces_out_kernel<DKP, NBLK, VAR>, hipFuncAttributeMaxDynamicSharedMemorySize, last);
+  PICO_REQUIRE(room1 == hipSuccess && room2 == hipSuccess, "pico_decay_chunks: %d and %d bytes of LDS refused", first, last);
+  const dim3 grid(a.chunks, a.H, (a.dv + 32 * NBLK - 1) / (32 * NBLK));
+  decay_pieces_state_kernel<DKP, NBLK, VAR><<<grid, 256, first, stream>>>(a);
+  launch_walk<VAR>(a, num_seqs, stream);
+  decay_pieces_out_kernel<DKP, NBLK, VAR><<<grid, 256, last, stream>>>(a);
   PICO_LAUNCH_CHECK();
   return 0;
 }
@@ -420,7 +708,11 @@ static int launch_chunks(const ChunkArgs& a, int num_seqs, hipStream_t stream) {
 template <bool VAR>
 static int pick_chunks(const ChunkArgs& a, int num_seqs, hipStream_t stream) {
   const bool wide = a.dv > 64;
-#define PICK(DKP) return wide ? launch_chunks<DKP, 4, VAR>(a, num_seqs, stream) : launch_chunks<DKP, 2, VAR>(a, num_seqs, stream)
+#define PICK(DKP)                                                                                                                \
+  do {                                                                                                                           \
+    if (!VAR && a.silu) return wide ? launch_chunks<DKP, 4>(a, num_seqs, stream) : launch_chunks<DKP, 2>(a, num_seqs, stream);    \
+    return wide ? launch_pieces<DKP, 4, VAR>(a, num_seqs, stream) : launch_pieces<DKP, 2, VAR>(a, num_seqs, stream);              \
+  } while (0)
   if (a.dk <= 32) PICK(32);
   if (a.dk <= 64) PICK(64);
   if (a.dk <= 96) PICK(96);

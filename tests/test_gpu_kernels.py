@@ -1727,6 +1727,37 @@ def test_ssd_chunks(K, H, G, dk, dv, lens, steps):
     assert torch.equal(st[0].cpu(), state[0])       # a slot that no sequence holds
 
 
+@pytest.mark.parametrize("dk,dv", [(32, 64), (40, 72), (96, 128), (128, 200)])
+@pytest.mark.parametrize("n", [1, 31, 64, 150])
+def test_decay_chunks_scale_and_odd_states(K, dk, dv, n):
+    # a constant decay with a scale on the queries against the walk in 64 bits; an infinite element of the state and an Inf among the
+    # values stay in their columns (and, of the value, in its own and later tokens)
+    g = torch.Generator().manual_seed(dk + n)
+    H = 3
+    x, fixed, state = torch.randn(n, 2 * H * dk + H * dv, generator=g).bfloat16(), torch.tensor([0.6, 0.97, 1.0]), torch.randn(1, H, dk, dv, generator=g)
+    cu, slots = torch.tensor([0, n], dtype=torch.int32).to(DEV), torch.zeros(1, dtype=torch.int32, device=DEV)
+
+    def run(rows, start):
+        st = start.to(DEV)
+        return K.gla_scan(rows.to(DEV), 0, H * dk, 2 * H * dk, None, cu, slots, st, 1, H, dk, dv, 0.3, 64, head_decay=fixed.to(DEV)).view(n, H, dv).cpu(), st.cpu()
+    out, st = run(x, state)
+    q, k, v = x[:, :H * dk].double().view(n, H, dk), x[:, H * dk:2 * H * dk].double().view(n, H, dk), x[:, 2 * H * dk:].double().view(n, H, dv)
+    S = state[0].double()
+    size = S.abs()
+    for t in range(n):
+        add, w = k[t].unsqueeze(-1) * v[t].unsqueeze(1), fixed.double().view(H, 1, 1)
+        S, size = w * S + add, w * size + add.abs()
+        # (test_ssd_chunks' bound, and powers of the decay that are made from its float32 logarithm: 2^-24 of an exponent of up to 64 a chunk)
+        assert bool(((out[t].double() - 0.3 * (S * q[t].unsqueeze(-1)).sum(1)).abs() <= (20 + 64) * 2.0 ** -24 * 0.3 * (size * q[t].abs().unsqueeze(-1)).sum(1)).all())
+    odd_state, odd_x = state.clone(), x.clone()
+    odd_state[0, 1, 5, 3], odd_x[n // 2, 2 * H * dk + 7] = float("inf"), float("-inf")
+    got, st2 = run(odd_x, odd_state)
+    hit = torch.zeros(n, H, dv, dtype=torch.bool)
+    hit[:, 1, 3], hit[n // 2:, 0, 7] = True, True
+    assert torch.equal(got[~hit], out[~hit]) and not torch.isfinite(got[hit]).any()
+    assert torch.equal(st2[0, 2], st[0, 2]) and st2[0, 1, 5, 3] == float("inf") and torch.isinf(st2[0, 0, :, 7]).all()
+
+
 @pytest.mark.parametrize("H,G,dk,dv", [(4, 2, 128, 64), (6, 1, 40, 72), (3, 3, 8, 8)])
 @pytest.mark.parametrize("lens", [[1] * 70 + [130, 17, 64], [33, 0, 1, 32, 8, 200], [9] * 5])
 def test_decay_chunks_of_many_sequences(K, H, G, dk, dv, lens):
