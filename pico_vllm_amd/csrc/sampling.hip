@@ -62,10 +62,10 @@ __device__ __forceinline__ SampleChunk sample_chunk(int V, int c) {
   return {begin, min(V, begin + len)};
 }
 
-// the row's maximum from the chunks' maxima; every lane of every wave gets it
-__device__ __forceinline__ float sample_row_max(const float* __restrict__ part_val, int row) {
-  const int lane = threadIdx.x & 63;
-  return wave_max(lane < SAMPLE_CHUNKS ? part_val[row * SAMPLE_CHUNKS + lane] : -INFINITY);
+// a lane's of the row's chunks' maxima (each stands in two lanes): the row's is their wave_max, in every lane of every wave
+__device__ __forceinline__ float sample_chunk_max(const float* __restrict__ part_val, int row) {
+  static_assert(SAMPLE_CHUNKS == 32, "a chunk in two lanes");
+  return part_val[row * SAMPLE_CHUNKS + (threadIdx.x & 31)];
 }
 
 // e as a whole number of 2^-bits, rounded down
@@ -141,35 +141,35 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_classes_kernel(
     const float* __restrict__ part_val, unsigned long long* __restrict__ classes, int bits) {
   __shared__ unsigned long long hist[SAMPLE_CLASSES];
   const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
-  // everything the workgroup needs from memory is asked for at once, whatever it turns out to need: what the launch
-  // before wrote comes from memory, a microsecond or two away, and asking one after the other would add them up
-  const float temp = temperature[row], tp = top_p[row], mx = sample_row_max(part_val, row);
+  // everything the workgroup needs from memory is asked for at once, whatever it turns out to need, without branches and
+  // before anything is waited for: what the launch before wrote comes from memory, a microsecond or two away, and asking one after
+  // the other would add them up
+  const float mine = sample_chunk_max(part_val, row), temp = temperature[row], tp = top_p[row];
   const float* x = logits + (size_t)row * ld;
   const SampleChunk ch = sample_chunk(V, c);
-  auto fetch = [&](int i0, float (&v)[8]) {
+  constexpr int AT_ONCE = 24;                              // elements of a thread: all of a chunk up to vocabularies of 196,608
+  float v[AT_ONCE];
+  auto fetch = [&](int i0) {
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int i = i0 + k * SAMPLE_THREADS;
-      v[k] = i < ch.end ? x[i] : -INFINITY;                // exp(-inf) = 0 adds nothing
-    }
+    for (int k = 0; k < AT_ONCE; k++) v[k] = x[min(i0 + k * SAMPLE_THREADS, V - 1)];
   };
-  float v[8], ahead[8];
-  fetch(ch.begin + tid, v);
+  fetch(ch.begin + tid);
+  const float mx = wave_max(mine);
   if (!(temp > 0.f) || !(tp < 1.0f)) return;
   const float inv_t = 1.0f / temp;
 #pragma unroll
   for (int j = 0; j < SAMPLE_CLASSES / SAMPLE_THREADS; j++) hist[j * SAMPLE_THREADS + tid] = 0ull;
   __syncthreads();
   SampleRun run{hist};
-  for (int i0 = ch.begin + tid; i0 < ch.end; i0 += 8 * SAMPLE_THREADS) {
-    fetch(i0 + 8 * SAMPLE_THREADS, ahead);
+  for (int i0 = ch.begin + tid;;) {
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const float e = __expf((v[k] - mx) * inv_t);
+    for (int k = 0; k < AT_ONCE; k++) {
+      const float e = i0 + k * SAMPLE_THREADS < ch.end ? __expf((v[k] - mx) * inv_t) : 0.f;
       if (e > 0.f) run.add(sample_class(__float_as_uint(e)), sample_fixed(__float_as_uint(e), bits));
     }
-#pragma unroll
-    for (int k = 0; k < 8; k++) v[k] = ahead[k];
+    i0 += AT_ONCE * SAMPLE_THREADS;
+    if (i0 >= ch.end) break;
+    fetch(i0);
   }
   run.end();
   __syncthreads();
@@ -248,13 +248,12 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
   __shared__ int wn[SAMPLE_THREADS / 64];
   __shared__ uint32_t ends[2][SAMPLE_THREADS / 64];
   const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
-  const float temp = temperature[row], tp = SEARCH ? top_p[row] : 1.0f, mx = sample_row_max(part_val, row);
-  if (!(temp > 0.f)) return;
+  // (asked for at once and without branches, as in the launch before)
+  const float own_max = sample_chunk_max(part_val, row), temp = temperature[row], tp = SEARCH ? top_p[row] : 1.0f;
   const float* x = logits + (size_t)row * ld;
   const SampleChunk ch = sample_chunk(V, c);
   // the terms of the elements begin + thread, begin + thread + SAMPLE_THREADS, .., all asked for at once: one load at a
   // time, each used at once, is a chain of memory latencies (6 us for the 19 elements a thread has of a chunk of 151,936 logits)
-  const float inv_t = 1.0f / temp;
   const bool held = ch.end - ch.begin <= SAMPLE_HELD * SAMPLE_THREADS;     // the same for all threads
   const int rounds = held ? (ch.end - ch.begin + 8 * SAMPLE_THREADS - 1) / (8 * SAMPLE_THREADS) : 0;      // of eight elements a thread
   float mine[SAMPLE_HELD];
@@ -262,26 +261,26 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_collect_kernel(
   for (int g = 0; g < SAMPLE_HELD / 8; g++) {
     if (g < rounds) {
 #pragma unroll
-      for (int k = 8 * g; k < 8 * g + 8; k++) {
-        const int i = ch.begin + tid + k * SAMPLE_THREADS;
-        mine[k] = i < ch.end ? x[i] : 0.f;
-      }
+      for (int k = 8 * g; k < 8 * g + 8; k++) mine[k] = x[min(ch.begin + tid + k * SAMPLE_THREADS, V - 1)];
     }
   }
+  constexpr int OWN = SEARCH ? SAMPLE_CLASSES / SAMPLE_THREADS : 1;
+  unsigned long long h[OWN];                               // the row's classes that this thread looks at
+#pragma unroll
+  for (int j = 0; SEARCH && j < OWN; j++) h[j] = classes[(size_t)row * SAMPLE_CLASSES + tid * OWN + j];
+  const float mx = wave_max(own_max);
+  if (!(temp > 0.f)) return;
+  const float inv_t = 1.0f / temp;
   int above = -1;                                          // keep what is above this class, list what is in it
   if (SEARCH && tp < 1.0f) {
-    constexpr int N = SAMPLE_CLASSES / SAMPLE_THREADS;
-    unsigned long long h[N], own = 0, total;
+    unsigned long long own = 0, total;
 #pragma unroll
-    for (int j = 0; j < N; j++) {
-      h[j] = classes[(size_t)row * SAMPLE_CLASSES + tid * N + j];
-      own += h[j];
-    }
+    for (int j = 0; j < OWN; j++) own += h[j];
     if (tid == 0) cls = SAMPLE_ONE >> SAMPLE_LOW, mass = 0;                // (a target that is not above zero: the largest alone)
     const unsigned long long behind = block_behind(own, scratch, SAMPLE_THREADS / 64, total);
     const double one = (double)(1ull << bits);
     const float target = tp * (float)((double)total / one);
-    sample_cross(h, behind, (double)target * one, tid * N, &cls, &mass);
+    sample_cross(h, behind, (double)target * one, tid * OWN, &cls, &mass);
     __syncthreads();
     above = cls;
     if (c == 0 && tid == 0) rows[row] = {mass, target, (uint32_t)above};
@@ -400,31 +399,39 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(
   __shared__ double chunk_s[SAMPLE_CHUNKS];
   __shared__ double chosen_before, chosen_target;
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-  // the row's first maximum: what a greedy row gives, and what a draw falls back on
-  float mx = lane < SAMPLE_CHUNKS ? part_val[row * SAMPLE_CHUNKS + lane] : -INFINITY;
-  int mi = lane < SAMPLE_CHUNKS ? part_idx[row * SAMPLE_CHUNKS + lane] : 0x7fffffff;
-  wave_first_max(mx, mi);
-  const float temp = temperature[row], u_row = u[row];    // (asked for here: where it is used, one thread would wait for it)
+  // (asked for at once and without branches, as in the launches before; rows without a search find in `r`, `number` and `head` what they do
+  // not look at)
+  const size_t base = (size_t)row * SAMPLE_CHUNKS;
+  const int my_chunk = tid / PER, part = tid % PER;
+  float mx = part_val[base + (lane & 31)];
+  int mi = part_idx[base + (lane & 31)];
+  const float temp = temperature[row], u_row = u[row];
   const float tp = SEARCH ? top_p[row] : 1.0f;
+  double kept_s = fin_s[base + my_chunk];
+  SampleRow r{};
+  int number = 0;
+  u32x4 head{0, 0, 0, 0};
+  if (SEARCH) {
+    r = rows[row];
+    number = fin_n[base + my_chunk];
+    head = reinterpret_cast<const u32x4*>(list + (base + my_chunk) * room)[min(part, room / 4 - 1)];
+  }
+  // the row's first maximum: what a greedy row gives, and what a draw falls back on
+  wave_first_max(mx, mi);
   if (!(temp > 0.f)) {
     if (tid == 0) sample_leave(mi, row, out, landing);
     return;
   }
   const float inv_t = 1.0f / temp;
   const float* x = logits + (size_t)row * ld;
-  const size_t base = (size_t)row * SAMPLE_CHUNKS;
   float thr = 0.f;                            // keep e > thr, and the first `ties_kept` tokens with e == thr
   int ties_kept = 0x7fffffff;
-  const int my_chunk = tid / PER, part = tid % PER;
-  double kept_s = fin_s[base + my_chunk];
   int kept_n = 0;
   if constexpr (SEARCH) if (tp < 1.0f) {
-    const SampleRow r = rows[row];
-    const int number = fin_n[base + my_chunk];
     // the patterns of this chunk's elements of the class, PER threads side by side, four neighbours each: from the list, of which
     // each thread holds the first ones, or, where it did not have room for all, from the logits
     const u32x4* mylist = reinterpret_cast<const u32x4*>(list + (base + my_chunk) * room);
-    const u32x4 held = 4 * part < number ? mylist[part] : u32x4{0, 0, 0, 0};
+    const u32x4 held = 4 * part < number ? head : u32x4{0, 0, 0, 0};
     auto entries = [&](auto use) {                        // use(pattern, how many of it)
       if ((uint32_t)number <= (uint32_t)room) {
 #pragma unroll
