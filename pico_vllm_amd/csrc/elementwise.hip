@@ -317,6 +317,19 @@ __global__ void gated_act_kernel(const T* __restrict__ gu, T* __restrict__ out, 
   store_f32(out + idx, gated_act<ACT>(g, u, limit, alpha));
 }
 
+// float32 rows whose halves start on 16 bytes (I % 4 == 0): four elements a thread, a row a line of the grid, so that nothing is divided in
+// 64 bits (300 rows of 8,960 7.7 us one a thread, 5.6 so).
+template <int ACT>
+__global__ __launch_bounds__(256) void gated_act_f32x4_kernel(const float* __restrict__ gu, float* __restrict__ out, int I, float limit, float alpha) {
+  const int col = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (col >= I) return;
+  const float* row = gu + (size_t)blockIdx.y * 2 * I + col;
+  const float4 g = *reinterpret_cast<const float4*>(row), u = *reinterpret_cast<const float4*>(row + I);
+  *reinterpret_cast<float4*>(out + (size_t)blockIdx.y * I + col) =
+      make_float4(gated_act<ACT>(g.x, u.x, limit, alpha), gated_act<ACT>(g.y, u.y, limit, alpha), gated_act<ACT>(g.z, u.z, limit, alpha),
+                  gated_act<ACT>(g.w, u.w, limit, alpha));
+}
+
 // bfloat16 rows whose halves start on 16 bytes (I % 8 == 0): eight elements per thread, 16-byte loads and stores
 template <int ACT>
 __global__ void gated_act_bf16x8_kernel(const bf16_t* __restrict__ gu, bf16_t* __restrict__ out, int I8, size_t total8, float limit,
@@ -346,6 +359,11 @@ static int gated_act_launch(const void* gu, void* out, int dtype, int T, int I, 
   if (dtype == PICO_DTYPE_BF16 && I % 8 == 0 && (uintptr_t)gu % 16 == 0 && (uintptr_t)out % 16 == 0) {
     const size_t total8 = total / 8;
     gated_act_bf16x8_kernel<ACT><<<(unsigned)((total8 + 255) / 256), 256, 0, stream>>>((const bf16_t*)gu, (bf16_t*)out, I / 8, total8, limit, alpha);
+    PICO_LAUNCH_CHECK();
+    return 0;
+  }
+  if (dtype == PICO_DTYPE_F32 && I % 4 == 0 && T <= 65535 && ((uintptr_t)gu | (uintptr_t)out) % 16 == 0) {
+    gated_act_f32x4_kernel<ACT><<<dim3((I / 4 + 255) / 256, T), 256, 0, stream>>>((const float*)gu, (float*)out, I, limit, alpha);
     PICO_LAUNCH_CHECK();
     return 0;
   }

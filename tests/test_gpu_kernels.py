@@ -89,6 +89,18 @@ def test_swiglu(K, dtype):
         close(K.swiglu(gu.to(DEV)), P.swiglu(gu), dtype)
 
 
+@pytest.mark.parametrize("T,I", [(1, 4), (3, 1020), (7, 1028), (300, 8960), (65536, 4)])
+def test_swiglu_of_float32_rows(K, T, I):
+    # four elements a thread at the edges of a workgroup and of the grid; the same bits as rows that start elsewhere, one element a thread
+    gu = torch.randn(T, 2 * I, device=DEV)
+    odd = torch.empty(2 * I * T + 1, device=DEV)[1:].view(T, 2 * I)
+    odd.copy_(gu)
+    out = K.swiglu(gu)
+    assert torch.equal(out, K.swiglu(odd))
+    want = F.silu(gu[:, :I].double()) * gu[:, I:].double()
+    assert bool(((out.double() - want).abs() <= 2.0 ** -21 * want.abs() + 1e-30).all())     # exponential, sum, quotient, product: under 8 roundings of 2^-24
+
+
 @pytest.mark.parametrize("counts,D,F_", [([0, 1, 63, 64, 65], 72, 40), ([129, 0, 48, 2], 64, 264), ([1, 127, 128, 129, 700], 136, 1000),
                                          ([0, 1100], 328, 200), ([0, 0, 5], 1536, 8)])
 @pytest.mark.parametrize("mode", [0, 1, 2])
