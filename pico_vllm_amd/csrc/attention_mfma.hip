@@ -1130,17 +1130,24 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int KS16 = D / 32;   // contraction steps of a 16-key tile
 constexpr int DT16 = D / 16;   // 16-wide tiles of the output's head dimension
 
-template <bool CUT>
-__global__ __launch_bounds__(256, 2) void decode16_kernel(const bf16_t* __restrict__ q, int q_stride,
+// WHOLE: a sequence's keys are one split, and its workgroup (WAVES waves) leaves the output itself, without a merging launch: short
+// contexts are two latencies either way, and the merge a third.
+constexpr int WHOLE_WAVES = 8;
+constexpr int XS = D + 4;      // floats of a wave's output a head in LDS
+constexpr int whole_lds() { return WHOLE_WAVES * 16 * (XS + 2) * (int)sizeof(float); }
+template <bool CUT, bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? 64 * WHOLE_WAVES : 256, 2) void decode16_kernel(const bf16_t* __restrict__ q, int q_stride,
                                                           const bf16_t* __restrict__ k_cache,
                                                           const bf16_t* __restrict__ v_cache,
                                                           const int* __restrict__ block_table, int max_pages,
                                                           const int* __restrict__ context_lens,
                                                           float* __restrict__ part, int nsplit, int nq, int nkv, int P,
                                                           int num_pages, float scale, int reach, const int4* __restrict__ plan,
-                                                          int num_seqs) {
-  __shared__ float xo[3][D][16];     // outputs of waves 1..3 for the final merge
-  __shared__ float xml[3][2][16];
+                                                          int num_seqs, bf16_t* __restrict__ out) {
+  constexpr int WAVES = WHOLE ? WHOLE_WAVES : 4, TURN = 32 * WAVES;
+  __shared__ float xo[WHOLE ? 1 : 3][WHOLE ? 1 : D][16];     // outputs of waves 1..3 for the final merge
+  __shared__ float xml[WHOLE ? 1 : 3][2][16];
+  extern __shared__ __attribute__((aligned(16))) float whole[];     // WHOLE: of all waves [wave][head][XS], then m and l [wave][2][16]
   const int g = blockIdx.y;
   const int G = nq / nkv;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, kq = lane >> 4;
@@ -1186,7 +1193,7 @@ __global__ __launch_bounds__(256, 2) void decode16_kernel(const bf16_t* __restri
   const int first = k_begin + 32 * wave;
   const int pshift = 31 - __clz(P);                             // page sizes are powers of two
   if (first < k_end) {
-    const int last = first + (k_end - 1 - first) / 128 * 128;   // this wave's last block
+    const int last = first + (k_end - 1 - first) / TURN * TURN;   // this wave's last block
     const int last_key = k_end - 1, last_group = last_key / 8 * 8;
     const int row_key = 8 * (col >> 2) + (col & 3);             // key of this lane's row in tile 0; tile 1: 4 more
     uint4 kr[2][KS16];
@@ -1214,8 +1221,8 @@ __global__ __launch_bounds__(256, 2) void decode16_kernel(const bf16_t* __restri
     __builtin_amdgcn_sched_barrier(0);       // keys before values, as in the loop, so the waits there stay partial
     load_v(first);
     __builtin_amdgcn_sched_barrier(0);
-    for (int key0 = first;; key0 += 128) {
-      const int next = min(key0 + 128, last);
+    for (int key0 = first;; key0 += TURN) {
+      const int next = min(key0 + TURN, last);
       f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
       for (int st = 0; st < KS16; st++) {
@@ -1277,6 +1284,29 @@ __global__ __launch_bounds__(256, 2) void decode16_kernel(const bf16_t* __restri
       load_v(next);
       __builtin_amdgcn_sched_barrier(0);
     }
+  }
+  if constexpr (WHOLE) {
+    float* ml = whole + WAVES * 16 * XS;
+    float* mine = whole + (wave * 16 + col) * XS + 4 * kq;
+#pragma unroll
+    for (int tt = 0; tt < DT16; tt++) *reinterpret_cast<f32x4*>(mine + 16 * tt) = o[tt];
+    if (kq == 0) { ml[wave * 32 + col] = m; ml[wave * 32 + 16 + col] = l; }
+    __syncthreads();
+    for (int e = threadIdx.x; e < G * D; e += 64 * WAVES) {
+      const int c = e / D, dim = e % D;
+      float M = -INFINITY, L = 0.f, acc = 0.f;
+#pragma unroll
+      for (int w = 0; w < WAVES; w++) M = fmaxf(M, ml[w * 32 + c]);
+      const float m_use = M == -INFINITY ? 0.f : M;             // an empty row (padding of a captured batch) is zero
+#pragma unroll
+      for (int w = 0; w < WAVES; w++) {
+        const float f = __expf(ml[w * 32 + c] - m_use);
+        L = fmaf(ml[w * 32 + 16 + c], f, L);
+        acc = fmaf(whole[(w * 16 + c) * XS + dim], f, acc);
+      }
+      out[((size_t)b * nq + g * G + c) * D + dim] = f32_to_bf16(M == -INFINITY ? 0.f : acc / L);
+    }
+    return;
   }
   // merge the four waves; lane (col, kq) of wave 0 holds head dimensions 16 tt + 4 kq + r of head `col`
   if (wave > 0) {
@@ -1662,8 +1692,15 @@ extern "C" int pico_attn_decode(const void* q, int q_stride, const void* k_cache
                     part, nsplit, nq, nkv, P, num_pages, scale, reach, cut, num_seqs
 #if PICO_HEAD_DIM % 32 == 0 && PICO_HEAD_DIM <= 128
   if (direct) {
-    if (cut != nullptr) decode16_kernel<true><<<grid, 256, 0, stream>>>(DECODE_ARGS);
-    else decode16_kernel<false><<<grid, 256, 0, stream>>>(DECODE_ARGS);
+    if (cut == nullptr && nsplit == 1) {
+      static const hipError_t room = hipFuncSetAttribute((const void*)&decode16_kernel<false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, whole_lds());
+      PICO_REQUIRE(room == hipSuccess, "pico_attn_decode: %s", hipGetErrorString(room));
+      decode16_kernel<false, true><<<grid, 64 * WHOLE_WAVES, whole_lds(), stream>>>(DECODE_ARGS, (bf16_t*)out);
+      PICO_LAUNCH_CHECK();
+      return 0;
+    }
+    if (cut != nullptr) decode16_kernel<true, false><<<grid, 256, 0, stream>>>(DECODE_ARGS, nullptr);
+    else decode16_kernel<false, false><<<grid, 256, 0, stream>>>(DECODE_ARGS, nullptr);
   }
 #endif
   if (!direct) {

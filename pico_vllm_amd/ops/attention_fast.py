@@ -49,6 +49,22 @@ class FastAttention:
             by_len = max(64, -(-keys // 128))
         return max(1, min(by_fill, by_len, 256))
 
+    def step_splits(self, num_seqs: int, max_context: int) -> int:
+        """How many splits a step's contexts are read in: one up to ``whole_keys``, else ``num_splits``."""
+        keys = min(max_context, self.window + 31) if self.window else max_context
+        return 1 if keys <= self.whole_keys(self.padded(num_seqs)) else self.num_splits(num_seqs, max_context)
+
+    def whole_keys(self, padded: int) -> int:
+        """Up to how many keys a sequence is read whole, by a workgroup that leaves the output itself and saves the merging launch; the more
+        (sequence, kv head) pairs there are, the longer that pays.  Microseconds split and merged / whole at 128, 256, 384, 512, 1,024
+        keys, heads of 128: 2 pairs 7.5 / 5.3, 7.5 / 7.0, 7.6 / 8.7; 16 pairs 7.6 / 5.4, 8.1 / 7.6, 8.4 / 9.2; 64 pairs 8.7 / 6.2, 9.2 / 8.0,
+        10.1 / 9.6, 11.0 / 11.6; 128 pairs 10.9 / 6.5, 13.0 / 8.7, 15.0 / 10.6, 16.5 / 11.8, 21.1 / 18.2; 256 pairs 14.6 / 7.6, 17.8 / 10.6,
+        19.8 / 12.6, 22.6 / 15.3, 31.0 / 23.8."""
+        if self.d % 32 or self.d > 128 or self.nq // self.nkv > 16:        # head shapes whose kernel has no such form
+            return 0
+        pairs = padded * self.nkv
+        return 1024 if pairs >= 256 else 512 if pairs >= 128 else 384 if pairs >= 64 else 256
+
     @staticmethod
     def padded(num_seqs: int) -> int:
         """The power of two that a recorded decode step of so many sequences is padded to."""
@@ -277,7 +293,7 @@ class FastAttention:
         B = ctx.num_seqs
         grouped = self.nq // self.nkv <= 32
         if ctx.all_decode and grouped:
-            nsplit = self.num_splits(B, ctx.max_context)
+            nsplit = self.step_splits(B, ctx.max_context)
             cut, build = self._step_cut(ctx, B, nsplit, qkv.device)
             return self.decode(qkv, cache.k, cache.v, block_table, ctx.context_lens, B, scale, nsplit, cut=cut, cut_build=build)
         teams, lead, chunk_len, max_chunks = self.plan(ctx)
@@ -297,7 +313,7 @@ class FastAttention:
         # 0 .. lead - 1) go through the decode kernel, which reads keys and values once for all query heads of
         # a group; the prompt portions behind them through the prefill kernel, whose offsets are absolute.
         out = torch.empty(qkv.shape[0], self.nq * self.d, dtype=torch.bfloat16, device=qkv.device)
-        nsplit = self.num_splits(lead, ctx.max_context)
+        nsplit = self.step_splits(lead, ctx.max_context)
         cut, cut_build = self._step_cut(ctx, lead, nsplit, qkv.device)
         self.decode(qkv[:lead], cache.k, cache.v, block_table[:lead], ctx.context_lens[:lead], lead, scale, nsplit, out=out[:lead],
                     cut=cut, cut_build=cut_build)

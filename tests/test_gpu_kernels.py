@@ -1251,6 +1251,22 @@ def test_fast_decode(K, nq, nkv, d, Pg, nsplit):
     close(out, want, torch.bfloat16)
 
 
+@pytest.mark.parametrize("nq,nkv,d", [(1, 1, 32), (12, 2, 128), (16, 1, 96), (32, 2, 64), (30, 2, 128)])
+@pytest.mark.parametrize("window", [0, 40])
+def test_fast_decode_of_whole_sequences(K, nq, nkv, d, window):
+    # one split: no merging launch.  Contexts at the edges of blocks of 32 keys and of the turns of the workgroup's eight waves, groups of
+    # one to sixteen heads; a sequence without a context (the padding of a recorded step) is left zero and no other is touched
+    from pico_vllm_amd.ops.attention_fast import FastAttention
+    out, want = _fast_case([1] * 8, [0, 30, 31, 32, 255, 256, 511, 700], nq, nkv, d, 16, seed=nq + d, decode=True, nsplit=1, window=window)
+    close(out, want, torch.bfloat16)
+    fa = FastAttention(nq, nkv, d, window)
+    kc, vc = torch.randn(4, nkv, 16, d, device=DEV).bfloat16(), torch.randn(4, nkv, d, 16, device=DEV).bfloat16()
+    q, bt = torch.randn(3, nq * d, device=DEV).bfloat16(), torch.arange(4, dtype=torch.int32, device=DEV).view(1, 4).repeat(3, 1)
+    some = fa.decode(q, kc, vc, bt, torch.tensor([50, 0, 64], dtype=torch.int32, device=DEV), 3, d ** -0.5, 1)
+    alone = fa.decode(q[2:], kc, vc, bt[2:], torch.tensor([64], dtype=torch.int32, device=DEV), 1, d ** -0.5, 1)
+    assert not some[1].any() and torch.equal(some[2:], alone)
+
+
 def test_fast_kernels_find_one_far_key_among_hundreds(K):
     for far in (0, 15, 16, 31, 32, 63, 64, 127, 128, 200, 511, 596):
         def boost(qs, ks, vs, far=far):
