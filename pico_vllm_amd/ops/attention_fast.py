@@ -50,9 +50,11 @@ class FastAttention:
         return max(1, min(by_fill, by_len, 256))
 
     def step_splits(self, num_seqs: int, max_context: int) -> int:
-        """How many splits a step's contexts are read in: one up to ``whole_keys``, else ``num_splits``."""
+        """How many splits a step's contexts are read in: one up to ``whole_keys``, else ``num_splits``.  Many sequences keep theirs: they are
+        cut into pieces of one length over all (``decode_cut``), which unequal contexts need."""
+        padded = self.padded(num_seqs)
         keys = min(max_context, self.window + 31) if self.window else max_context
-        return 1 if keys <= self.whole_keys(self.padded(num_seqs)) else self.num_splits(num_seqs, max_context)
+        return 1 if padded < self.CUT_FROM and keys <= self.whole_keys(padded) else self.num_splits(num_seqs, max_context)
 
     def whole_keys(self, padded: int) -> int:
         """Up to how many keys a sequence is read whole, by a workgroup that leaves the output itself and saves the merging launch; the more

@@ -54,11 +54,11 @@ def test_the_splits_of_a_decode_step(num_seqs, context, want):
 
 
 @pytest.mark.parametrize("fa,num_seqs,context,want", [
-    (plan(12), 1, 256, 1), (plan(12), 1, 257, 5), (plan(12), 17, 384, 1), (plan(12), 16, 384, 6), (plan(12), 64, 512, 1), (plan(12), 64, 513, 4),
-    (plan(28, 4), 64, 1024, 1), (plan(28, 4), 64, 1025, 2), (plan(12, window=200), 1, 9000, 1), (plan(5, 5, 48), 1, 256, 4), (plan(40, 2), 1, 256, 4)])
+    (plan(12), 1, 256, 1), (plan(12), 1, 257, 5), (plan(12), 16, 384, 6), (plan(28, 4), 16, 384, 1), (plan(28, 4), 16, 385, 7), (plan(64, 16), 16, 1024, 1),
+    (plan(64, 16), 16, 1025, 2), (plan(12), 17, 256, 4), (plan(12, window=200), 1, 9000, 1), (plan(5, 5, 48), 1, 256, 4), (plan(40, 2), 1, 256, 4)])
 def test_short_contexts_are_read_whole(fa, num_seqs, context, want):
     # by a workgroup that leaves the output itself: the more (sequence, kv head) pairs, padded as a recorded step is, the longer; not for
-    # head sizes and groups that the kernel without LDS staging does not serve
+    # head sizes and groups that the kernel without LDS staging does not serve, nor where contexts are cut over all sequences
     assert fa.step_splits(num_seqs, context) == want
 
 
