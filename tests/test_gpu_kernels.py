@@ -133,6 +133,25 @@ def test_moe_grouped(K, counts, D, F_, mode):
         assert bool(((got[at] - want).abs() <= slack).all())
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_experts_activation_has_the_same_bits_by_every_kernel(K, mode):
+    # a gate that is one number of the row and an up that is another: every finite bfloat16 number through the activation by the grouped products,
+    # the kernel that streams matrices and the plain one.  All other sums are exact, so the bits are the activation's: a last bit here sends
+    # later tokens to other experts
+    x = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x = x[torch.isfinite(x.float())]
+    T = x.numel()
+    h = torch.zeros(T, 16, dtype=torch.bfloat16)
+    h[:, 0], h[:, 1] = x, (torch.arange(T) % 13 - 6) / 8
+    gate_up, down = torch.zeros(1, 16, 16, dtype=torch.bfloat16), torch.zeros(1, 16, 8, dtype=torch.bfloat16)
+    gate_up[0, :8, 0], gate_up[0, 8:, 1], down[0, :8] = 1, 1, torch.eye(8)
+    which, wt = torch.zeros(T, 1, dtype=torch.int32), torch.full((T, 1), 1.0 if mode == 0 else 0.3)
+    args = [t.to(DEV) for t in (h, gate_up, down, which, wt)]
+    plain = K.moe_experts_plain(*args, 7.0, 1.702, mode=mode)
+    for grouped in (True, False):
+        assert torch.equal(K.moe_experts(*args, 7.0, 1.702, grouped=grouped, mode=mode), plain)
+
+
 def test_moe_experts_of_operands_beyond_the_grouped_products_reach(K):
     # activations that span 2^31 bytes and more, and an expert of as many
     g = torch.Generator(device=DEV).manual_seed(1)
