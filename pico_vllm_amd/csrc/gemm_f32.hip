@@ -175,8 +175,8 @@ __global__ __launch_bounds__(128 * WM, 2) void gemm_f32_kernel(const TA* __restr
     const float* w = wp + buf * (TN * ST);
 #pragma unroll
     for (int g = 0; g < BK; g += 16)                    // 16 k: this half of the lanes holds 0..7 (or 8..15) of them
-      split_multiply<sizeof(TA) == 2>(split8<true>(*reinterpret_cast<const float4*>(a + g), *reinterpret_cast<const float4*>(a + g + 4)),
-                                      split8<false>(*reinterpret_cast<const float4*>(w + g), *reinterpret_cast<const float4*>(w + g + 4)), big, small);
+      split_multiply<sizeof(TA) == 2>(split8(*reinterpret_cast<const float4*>(a + g), *reinterpret_cast<const float4*>(a + g + 4)),
+                                      split8(*reinterpret_cast<const float4*>(w + g), *reinterpret_cast<const float4*>(w + g + 4)), big, small);
     if (more) put(buf ^ 1, k0 + BK);
     const int done = k0 + BK - k_first;
     if (done % GROUP == 0) {
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(128, 3) void gemm_f32_stream_kernel(const float* A,
     __builtin_amdgcn_sched_barrier(0);
     ask(buf, k0 + 2 * BK);
 #pragma unroll
-    for (int g = 0; g < 2; g++) split_multiply(split8<true>(a[g][0], a[g][1]), split8<false>(w[g][0], w[g][1]), big, small);
+    for (int g = 0; g < 2; g++) split_multiply(split8(a[g][0], a[g][1]), split8(w[g][0], w[g][1]), big, small);
     const int done = k0 + BK - k_first;
     if (done % GROUP == 0) {
       l2 += big;
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256, NW == 1 && AHEAD == 2 ? 3 : 2) void gemm_f32_p
   auto put = [&](int set, int b) {
 #pragma unroll
     for (int j = 0; j < PIECES; j++) {
-      const Split8 s = j == 0 ? split8<true>(raw[set][j][0], raw[set][j][1]) : split8<false>(raw[set][j][0], raw[set][j][1]);
+      const Split8 s = split8(raw[set][j][0], raw[set][j][1]);
       char* dst = put_at + b * STAGE + j * (64 * 64);
       *reinterpret_cast<s3_u32x4*>(dst) = s.h;
       *reinterpret_cast<s3_u32x4*>(dst + PLANE) = s.m;

@@ -7,11 +7,10 @@
 // with the last three, 2^-26 of the product and less, left out: a float32 sum rounds by more at every addition.  The small terms
 // are summed apart from ah wh, where their rounding is 2^-8 of its.
 //
-// bfloat16 has float32's exponents, so the lower pieces of numbers below 2^-110 would end at the smallest number that there is.
-// The left operand is therefore taken 2^96 times as large, where all of float32's numbers below 2^32 have their 24 bits in the pieces,
-// and the sums are scaled back; the right one's pieces are then off by 2^-126 at most, a product by 2^-94.  A larger number on the
-// left, a sum of 2^32 and more, infinities and NaN on either side make the sum not finite.  Such sums, and what lies below 2^-56
-// (2^25 times what a range of 8,192 products is off), are made again in float32 by who uses this (s3_redo).
+// bfloat16 has float32's exponents, so the lower pieces of numbers below 2^-110 would end at the smallest number that there is, and a number
+// below 2^-134 would have none at all.  Both operands are therefore taken 2^48 times as large, where all of float32's numbers below 2^80 have their
+// 24 bits in the pieces, and the sums are scaled back.  A larger number, a sum of 2^32 and more, infinities and NaN make the sum not
+// finite.  Such sums are made again in float32 by who uses this (s3_redo).
 #pragma once
 #include "common.h"
 
@@ -23,20 +22,17 @@ struct Split8 {
   s3_u32x4 h, m, l;                    // eight numbers' pieces
 };
 
-constexpr float S3_LEFT = 0x1p96f, S3_BACK = 0x1p-96f;
+constexpr float S3_SCALE = 0x1p48f, S3_BACK = 0x1p-96f;
 
 // A sum (scaled back) that has to be made again in float32
-__device__ __forceinline__ bool s3_redo(float sum) { return !(fabsf(sum) < INFINITY) || (sum != 0.f && fabsf(sum) < 0x1p-56f); }
+__device__ __forceinline__ bool s3_redo(float sum) { return !(fabsf(sum) < INFINITY); }
 
 __device__ __forceinline__ float s3_low(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float s3_high(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
 
-template <bool LEFT>                   // of the product's left operand: scaled
 __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-  if (LEFT) {
-    a *= S3_LEFT;
-    b *= S3_LEFT;
-  }
+  a *= S3_SCALE;
+  b *= S3_SCALE;
   h = pack2_bf16(a, b);
   a -= s3_low(h);
   b -= s3_high(h);
@@ -44,14 +40,14 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& 
   l = pack2_bf16(a - s3_low(m), b - s3_high(m));
 }
 
-template <bool LEFT, typename V>       // V: four floats
+template <typename V>                  // V: four floats
 __device__ __forceinline__ Split8 split8(const V& a, const V& b) {
   Split8 s;
   uint32_t h, m, l;
-  split2<LEFT>(a.x, a.y, h, m, l); s.h[0] = h; s.m[0] = m; s.l[0] = l;
-  split2<LEFT>(a.z, a.w, h, m, l); s.h[1] = h; s.m[1] = m; s.l[1] = l;
-  split2<LEFT>(b.x, b.y, h, m, l); s.h[2] = h; s.m[2] = m; s.l[2] = l;
-  split2<LEFT>(b.z, b.w, h, m, l); s.h[3] = h; s.m[3] = m; s.l[3] = l;
+  split2(a.x, a.y, h, m, l); s.h[0] = h; s.m[0] = m; s.l[0] = l;
+  split2(a.z, a.w, h, m, l); s.h[1] = h; s.m[1] = m; s.l[1] = l;
+  split2(b.x, b.y, h, m, l); s.h[2] = h; s.m[2] = m; s.l[2] = l;
+  split2(b.z, b.w, h, m, l); s.h[3] = h; s.m[3] = m; s.l[3] = l;
   return s;
 }
 
