@@ -5,8 +5,9 @@
 //
 // The sum is a tree over k: 16 products an instruction, 16 instructions (256 k) on one accumulator, then the `ranges` of K, each of
 // as many 256s as there are ranges (both about sqrt(K / 256)); the small terms of a range are one sum beside that, 2^-8 of it.
-// A result that such products cannot give (split3.h) is made again on the float32 instruction, element by element, so that it
-// too depends on its own row and column alone.  Error against 64 bits, in units of 2^-24 of the result's rms, on the float32
+// A result that is not finite (split3.h) is made again on the float32 instruction, element by element, so that it
+// too depends on its own row and column alone: one infinite number in 320 rows of 17,920 x 1,536 141 and 182 us, in 1 of 1,536 x 1,536 18
+// and 34.  Error against 64 bits, in units of 2^-24 of the result's rms, on the float32
 // instruction (16 products a sum, 16 sums) and so: 1.93 and 1.68 at K = 1,536, 2.13 and 1.90 at 8,960, 2.28 and 2.06 at 18,944 (one
 // running sum would give 0.2 sqrt(K)).
 //
@@ -14,8 +15,8 @@
 // to there by the stream of W; with few tiles by the chain of a range's stages (0.8 us each).  Tiles that read the same rows
 // of W are neighbours on one die.  Where the tiles alone leave the chip idle (less than two a compute unit) every range of K is a
 // workgroup of its own, its sum goes to a slab, and a second launch adds the slabs in the order in which one workgroup would have.
-// Microseconds on the float32 instruction and so, in one process: 320 rows of 17,920 x 1,536 183 / 145, 1,536 x 8,960 103 / 88, 1,536
-// x 1,536 31 / 29; 2,048 rows of 17,920 x 1,536 1,060 / 785; one row of 151,936 x 1,536 212 / 183 (5.1 TB/s), 32 rows 230 / 206.
+// Microseconds on the float32 instruction and so, in one process: 320 rows of 17,920 x 1,536 184 / 140, 1,536 x 8,960 98 / 85, 1,536
+// x 1,536 31 / 28; 2,048 rows of 17,920 x 1,536 1,060 / 785; one row of 151,936 x 1,536 212 / 183 (5.1 TB/s), 32 rows 230 / 206.
 #include "split3.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -64,24 +65,36 @@ __device__ __forceinline__ float4 fetch4(const bf16_t* row, int k, int K) {
                      bf16_to_f32(row[min(k + 2, K - 1)]), bf16_to_f32(row[min(k + 3, K - 1)]));
 }
 
+// Eight k of a row, in loads of four where they all lie in it
+typedef float f32_four __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void fetch8(const float* row, int k, int K, float (&v)[8]) {
+  if (k + 8 <= K) {
+    const f32_four a = *reinterpret_cast<const f32_four*>(row + k), b = *reinterpret_cast<const f32_four*>(row + k + 4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) { v[i] = a[i]; v[4 + i] = b[i]; }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = k + i < K ? row[k + i] : 0.f;
+}
+__device__ __forceinline__ void fetch8(const bf16_t* row, int k, int K, float (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = k + i < K ? bf16_to_f32(row[k + i]) : 0.f;
+}
+
 // A wave's 32 x 32 block over k_first .. k_end on the float32 instruction, straight from memory: lane (l, half) has row l of A and of
 // W (`a_row`, `w_row`) and of 16 k the half'th eight.
 template <typename TA>
 __device__ __forceinline__ s3_f32x16 plain_block(const TA* a_row, const float* w_row, int k_first, int k_end, int K, int half) {
   s3_f32x16 sum = {}, group = {};
+#pragma unroll 1
   for (int k0 = k_first; k0 < k_end; k0 += 16) {
     s3_f32x16 few = {};
-    const int k = k0 + 8 * half;
-    const float4 a0 = zero_from(fetch4<false>(a_row, k, K), k, K), a1 = zero_from(fetch4<false>(a_row, k + 4, K), k + 4, K);
-    const float4 w0 = zero_from(fetch4<false>(w_row, k, K), k, K), w1 = zero_from(fetch4<false>(w_row, k + 4, K), k + 4, K);
-    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, w0.x, few, 0, 0, 0);
-    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, w0.y, few, 0, 0, 0);
-    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.z, w0.z, few, 0, 0, 0);
-    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.w, w0.w, few, 0, 0, 0);
-    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, w1.x, few, 0, 0, 0);
-    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, w1.y, few, 0, 0, 0);
-    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, w1.z, few, 0, 0, 0);
-    few = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, w1.w, few, 0, 0, 0);
+    float a[8], w[8];
+    fetch8(a_row, k0 + 8 * half, K, a);
+    fetch8(w_row, k0 + 8 * half, K, w);
+#pragma unroll
+    for (int i = 0; i < 8; i++) few = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], w[i], few, 0, 0, 0);
     group += few;
     if ((k0 - k_first) % GROUP == GROUP - 16) {
       sum += group;
@@ -293,7 +306,10 @@ __global__ __launch_bounds__(128, 3) void gemm_f32_stream_kernel(const float* A,
 // eight rows and writes of two meet every bank once).  Four waves (2 x 2) of 32 x 32 NW outputs.  A stage's numbers are asked for
 // AHEAD stages ahead, lie in registers, and are taken apart under the products of the stage in front.
 constexpr int fp_plane(int NW) { return (64 + 64 * NW) * BK * 2; }
-template <int NW, int AHEAD>
+// Rows may start anywhere: a load of four to registers needs no more alignment than one.  (Through gemm_f32_kernel, where every wave takes its
+// operands apart by itself, 64 such rows of 32,000 x 1,024 95 us and so 64, 320 of 17,920 x 1,536 262 and 145.)  EVEN: whole fours; else
+// the four numbers that K ends in are asked for one by one.
+template <int NW, int AHEAD, bool EVEN>
 __global__ __launch_bounds__(256, NW == 1 && AHEAD == 2 ? 3 : 2) void gemm_f32_planes_kernel(const float* A, const float* W, const float* bias, float* C, float* slabs,
                                                                                int M, int N, int K, int lda, int ldw, int ldc, int m_tiles) {
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
@@ -319,6 +335,14 @@ __global__ __launch_bounds__(256, NW == 1 && AHEAD == 2 ? 3 : 2) void gemm_f32_p
   f32x4 raw[AHEAD][PIECES][2];
   auto ask = [&](int set, int k0) {
     const uint32_t k = (uint32_t)(k0 + 8 * chunk) * 4, end = (uint32_t)K * 4;
+    if (!EVEN && k0 + BK > K) {
+#pragma unroll
+      for (int j = 0; j < PIECES; j++)
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          raw[set][j][i / 4][i % 4] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(j == 0 ? as : ws, off[j] + (k + 4 * i < end ? k + 4 * i : F32_OUT), 0, 0));
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < PIECES; j++)
 #pragma unroll
@@ -442,16 +466,22 @@ extern "C" int pico_gemm_f32_slabs(int M, int N, int K) {
   return tiles < 512 && ranges > 1 ? ranges : 0;
 }
 
+template <int NW, int AHEAD, bool EVEN>
+static bool launch_planes_of(const float* A, const float* W, const float* bias, float* C, float* slabs, int M, int N, int K, int lda, int ldw, int ldc,
+                          int ranges, hipStream_t stream) {
+  constexpr int bytes = 6 * fp_plane(NW);
+  static const hipError_t room = hipFuncSetAttribute((const void*)&gemm_f32_planes_kernel<NW, AHEAD, EVEN>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (room != hipSuccess) return false;
+  const int m_tiles = (M + 63) / 64, n_tiles = (N + 64 * NW - 1) / (64 * NW);
+  gemm_f32_planes_kernel<NW, AHEAD, EVEN>
+      <<<dim3((n_tiles + 7) / 8 * 8 * m_tiles, ranges), 256, bytes, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
+  return true;
+}
 template <int NW, int AHEAD>
 static bool launch_planes(const float* A, const float* W, const float* bias, float* C, float* slabs, int M, int N, int K, int lda, int ldw, int ldc,
                           int ranges, hipStream_t stream) {
-  constexpr int bytes = 6 * fp_plane(NW);
-  static const hipError_t room = hipFuncSetAttribute((const void*)&gemm_f32_planes_kernel<NW, AHEAD>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (room != hipSuccess) return false;
-  const int m_tiles = (M + 63) / 64, n_tiles = (N + 64 * NW - 1) / (64 * NW);
-  gemm_f32_planes_kernel<NW, AHEAD>
-      <<<dim3((n_tiles + 7) / 8 * 8 * m_tiles, ranges), 256, bytes, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, m_tiles);
-  return true;
+  return K % 4 == 0 ? launch_planes_of<NW, AHEAD, true>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, ranges, stream)
+                    : launch_planes_of<NW, AHEAD, false>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc, ranges, stream);
 }
 
 template <typename TA, int WM>
@@ -464,7 +494,8 @@ static void launch_gemm_f32(const TA* A, const float* W, const float* bias, floa
   const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % 16 == 0;
   bool done = false;
   if constexpr (sizeof(TA) == 4) {
-    if (vec && lda < (1 << 23) && ldw < (1 << 23)) {         // (a tile's rows within 2^31 bytes of its first)
+    // (a tile's rows within 2^31 bytes of its first; copies to LDS want whole aligned fours)
+    if ((vec || WM == 2) && lda < (1 << 23) && ldw < (1 << 23)) {
       if (WM == 1) {
         gemm_f32_stream_kernel<<<dim3(n_tiles, ranges), 128, 0, stream>>>(A, W, bias, C, slabs, M, N, K, lda, ldw, ldc);
         done = true;

@@ -729,6 +729,23 @@ def test_gemm_f32_at_the_limits_of_its_numbers(K, M, N, K_, ea, ew):
     assert torch.equal(K.gemm_f32(torch.zeros_like(a), w[cols]), torch.zeros(M, N - 1, device=DEV))
 
 
+@pytest.mark.parametrize("M,N,K_", [(33, 65, 1), (64, 63, 255), (65, 2050, 517), (200, 200, 2051), (300, 33000, 66), (300, 15403, 515), (31, 64, 37)])
+def test_gemm_f32_of_rows_that_end_anywhere(K, M, N, K_):
+    # no multiple of four: the bits are those of the same rows with zeros up to whole fours, whatever stands behind a row
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    even = (K_ + 3) // 4 * 4
+    out = []
+    for width, cols, fill in ((even, even, 0.0), (K_ + 2, K_, float("nan"))):
+        g.manual_seed(M + N)
+        a, w = (torch.full((r, width), fill, device=DEV) for r in (M, N))
+        for t in (a, w):
+            t[:, :K_] = torch.randn(t.shape[0], K_, device=DEV, generator=g)
+        out.append(K.gemm_f32(a[:, :cols], w[:, :cols]))
+    assert torch.equal(*out)
+    a[1, 0] = float("inf")                                  # and those that are made again
+    assert torch.equal(K.gemm_f32(a[:, :K_], w[:, :K_])[2:], out[0][2:])
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 70, 4), (1, 5000, 1540), (31, 64, 36), (32, 130, 256), (33, 65, 288), (64, 63, 260), (65, 2050, 512),
                                     (200, 200, 2052), (300, 33000, 68)])
 def test_gemm_f32_has_the_same_bits_by_copies_and_through_registers(K, M, N, K_):
