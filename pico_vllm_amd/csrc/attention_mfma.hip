@@ -1658,10 +1658,12 @@ static int attn_prefill(const void* q, int q_stride, const void* k_cache, const 
 // plan (may be null): 4 * plan_slots + 2 * num_seqs integers; the contexts of all sequences are then cut into pieces of
 // one length, at most plan_slots >= num_seqs of them in all (pico_attn_decode_plan writes the cut when plan_build is
 // set, the first layer of a step; the other layers find it there), and part holds plan_slots * nq * (D + 2) floats.
+// whole: every sequence's keys are read by one workgroup (WHOLE); one split, no plan, head sizes in steps of 32 up to 128 and up to 16
+// query heads a kv head; part may be null.
 extern "C" int pico_attn_decode(const void* q, int q_stride, const void* k_cache, const void* v_cache,
                                 const int* block_table, int max_pages, const int* context_lens, int num_seqs,
                                 void* out, float* part, int nsplit, int nq, int nkv, int d, int P, int num_pages,
-                                float scale, int window, int* plan, int plan_slots, int plan_build, hipStream_t stream) {
+                                float scale, int window, int* plan, int plan_slots, int plan_build, int whole, hipStream_t stream) {
   if (check_common("pico_attn_decode", nq, nkv, d, P, max_pages, num_pages, q_stride)) return -1;
   PICO_REQUIRE(window >= 0 && window < NO_WINDOW, "pico_attn_decode: bad window %d", window);
   const int reach = window > 0 ? window : NO_WINDOW;
@@ -1673,6 +1675,9 @@ extern "C" int pico_attn_decode(const void* q, int q_stride, const void* k_cache
 #if PICO_HEAD_DIM % 32 == 0 && PICO_HEAD_DIM <= 128
   direct = nq / nkv <= 16;
 #endif
+  PICO_REQUIRE(!whole || (direct && nsplit == 1 && plan == nullptr), "pico_attn_decode: %d splits of %d query heads of %d a kv head are not read whole",
+               nsplit, nq / nkv, d);
+  PICO_REQUIRE(whole || part != nullptr, "pico_attn_decode: the workspace is missing");
   const int4* cut = nullptr;
   const int2* rows = nullptr;
   if (plan != nullptr) {
@@ -1692,7 +1697,7 @@ extern "C" int pico_attn_decode(const void* q, int q_stride, const void* k_cache
                     part, nsplit, nq, nkv, P, num_pages, scale, reach, cut, num_seqs
 #if PICO_HEAD_DIM % 32 == 0 && PICO_HEAD_DIM <= 128
   if (direct) {
-    if (cut == nullptr && nsplit == 1) {
+    if (whole) {
       static const hipError_t room = hipFuncSetAttribute((const void*)&decode16_kernel<false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, whole_lds());
       PICO_REQUIRE(room == hipSuccess, "pico_attn_decode: %s", hipGetErrorString(room));
       decode16_kernel<false, true><<<grid, 64 * WHOLE_WAVES, whole_lds(), stream>>>(DECODE_ARGS, (bf16_t*)out);

@@ -49,19 +49,27 @@ class FastAttention:
             by_len = max(64, -(-keys // 128))
         return max(1, min(by_fill, by_len, 256))
 
-    def step_splits(self, num_seqs: int, max_context: int) -> int:
-        """How many splits a step's contexts are read in: one up to ``whole_keys``, else ``num_splits``.  Many sequences keep theirs: they are
-        cut into pieces of one length over all (``decode_cut``), which unequal contexts need."""
+    def step_whole(self, num_seqs: int, max_context: int) -> bool:
+        """Whether a step's contexts are read whole (``decode(whole=True)``): up to ``whole_keys``.  Many sequences keep their splits: they are
+        cut into pieces of one length over all (``decode_cut``), which unequal contexts need.  Where every sequence is a single split anyway
+        (512 pairs and more) there is no such cut; longer contexts gain 2 to 5 % if the pairs fill the workgroups' places, and lose up to
+        10 % if they do not (33 sequences of 8 kv heads, 8,192 keys, 270 / 292 us), so these keep the other form too."""
         padded = self.padded(num_seqs)
         keys = min(max_context, self.window + 31) if self.window else max_context
-        return 1 if padded < self.CUT_FROM and keys <= self.whole_keys(padded) else self.num_splits(num_seqs, max_context)
+        return keys <= self.whole_keys(padded) and (padded < self.CUT_FROM or self.num_splits(num_seqs, max_context) == 1)
+
+    def step_splits(self, num_seqs: int, max_context: int) -> int:
+        """How many splits a step's contexts are read in: one if they are read whole, else ``num_splits``."""
+        return 1 if self.step_whole(num_seqs, max_context) else self.num_splits(num_seqs, max_context)
 
     def whole_keys(self, padded: int) -> int:
         """Up to how many keys a sequence is read whole, by a workgroup that leaves the output itself and saves the merging launch; the more
         (sequence, kv head) pairs there are, the longer that pays.  Microseconds split and merged / whole at 128, 256, 384, 512, 1,024
         keys, heads of 128: 2 pairs 7.5 / 5.3, 7.5 / 7.0, 7.6 / 8.7; 16 pairs 7.6 / 5.4, 8.1 / 7.6, 8.4 / 9.2; 64 pairs 8.7 / 6.2, 9.2 / 8.0,
         10.1 / 9.6, 11.0 / 11.6; 128 pairs 10.9 / 6.5, 13.0 / 8.7, 15.0 / 10.6, 16.5 / 11.8, 21.1 / 18.2; 256 pairs 14.6 / 7.6, 17.8 / 10.6,
-        19.8 / 12.6, 22.6 / 15.3, 31.0 / 23.8."""
+        19.8 / 12.6, 22.6 / 15.3, 31.0 / 23.8; 512 in one split and merged / whole 23.2 / 20.1, 35.4 / 29.5 at 512, 51 / 47 at 1,024, 264 of them
+        17.5 / 15.7, 24.7 / 24.5, 37.3 / 38.0.  The contexts are those that the engine allows (``max_seq_len``), so that all steps of a request
+        are read alike."""
         if self.d % 32 or self.d > 128 or self.nq // self.nkv > 16:        # head shapes whose kernel has no such form
             return 0
         pairs = padded * self.nkv
@@ -222,10 +230,11 @@ class FastAttention:
 
     def decode(self, q: torch.Tensor, k_cache, v_cache, block_table, context_lens, num_seqs: int, scale: float,
                nsplit: int, out: Optional[torch.Tensor] = None, cut: Optional[tuple] = None,
-               cut_build: bool = True) -> torch.Tensor:
+               cut_build: bool = True, whole: bool = False) -> torch.Tensor:
         """One query token per sequence: q [B, >= nq*d]; returns [B, nq*d].  cut: ``decode_cut(...)``, where the
         kernel writes (``cut_build``) or finds (the other layers of a step) the pieces of one length that the contexts
-        of all sequences are cut into; without it every sequence is cut into ``nsplit`` splits of its own."""
+        of all sequences are cut into; without it every sequence is cut into ``nsplit`` splits of its own.  whole: a workgroup reads a
+        sequence's keys (of a kv head) whole and leaves the output itself; one split, no cut, ``whole_keys`` above 0."""
         nq, nkv, d = self.nq, self.nkv, self.d
         if q.shape[0] != num_seqs:
             raise KernelError("decode attention wants exactly one query token per sequence")
@@ -237,11 +246,11 @@ class FastAttention:
         if out is None:
             out = torch.empty(num_seqs, nq * d, dtype=torch.bfloat16, device=q.device)
         plan, slots = cut if cut is not None else (None, 0)
-        part = torch.empty(max(num_seqs * nsplit, slots) * nq * (d + 2), dtype=torch.float32, device=q.device)
+        part = None if whole else torch.empty(max(num_seqs * nsplit, slots) * nq * (d + 2), dtype=torch.float32, device=q.device)
         _check(self.lib, self.lib.pico_attn_decode(
             _ptr(q), q.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1],
             _ptr(context_lens), num_seqs, _ptr(out), _ptr(part), nsplit, nq, nkv, d, P, pages, c_float(scale),
-            self.window, _ptr(plan), slots, 1 if cut_build else 0, _stream()))
+            self.window, _ptr(plan), slots, 1 if cut_build else 0, 1 if whole else 0, _stream()))
         return out
 
     def _step_cut(self, ctx, num_seqs: int, nsplit: int, device):
@@ -297,7 +306,8 @@ class FastAttention:
         if ctx.all_decode and grouped:
             nsplit = self.step_splits(B, ctx.max_context)
             cut, build = self._step_cut(ctx, B, nsplit, qkv.device)
-            return self.decode(qkv, cache.k, cache.v, block_table, ctx.context_lens, B, scale, nsplit, cut=cut, cut_build=build)
+            return self.decode(qkv, cache.k, cache.v, block_table, ctx.context_lens, B, scale, nsplit, cut=cut, cut_build=build,
+                               whole=self.step_whole(B, ctx.max_context))
         teams, lead, chunk_len, max_chunks = self.plan(ctx)
         if not grouped:
             lead = 0
@@ -318,7 +328,7 @@ class FastAttention:
         nsplit = self.step_splits(lead, ctx.max_context)
         cut, cut_build = self._step_cut(ctx, lead, nsplit, qkv.device)
         self.decode(qkv[:lead], cache.k, cache.v, block_table[:lead], ctx.context_lens[:lead], lead, scale, nsplit, out=out[:lead],
-                    cut=cut, cut_build=cut_build)
+                    cut=cut, cut_build=cut_build, whole=self.step_whole(lead, ctx.max_context))
         if lead < B:
             self.prefill(qkv, cache.k, cache.v, block_table[lead:], ctx.cu_seqlens[lead:], ctx.context_lens[lead:],
                          B - lead, scale, out=out, teams=teams, chunk_len=chunk_len, max_chunks=max_chunks, order=order,

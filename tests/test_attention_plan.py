@@ -62,6 +62,15 @@ def test_short_contexts_are_read_whole(fa, num_seqs, context, want):
     assert fa.step_splits(num_seqs, context) == want
 
 
+@pytest.mark.parametrize("fa,num_seqs,context,splits,whole", [
+    (plan(64, 8), 64, 32768, 1, False), (plan(32, 8), 33, 4096, 1, False), (plan(28, 4), 128, 4096, 1, False), (plan(64, 8), 64, 1024, 1, True),
+    (plan(64, 8), 64, 1025, 1, False), (plan(64, 8), 32, 1024, 2, False), (plan(12), 1, 256, 1, True), (plan(12), 1, 257, 5, False),
+    (plan(16, 8, 48), 64, 256, 1, False), (plan(32, 8, window=900), 64, 32768, 1, True)])
+def test_a_single_split_is_not_read_whole_at_any_length(fa, num_seqs, context, splits, whole):
+    # so many pairs of sequence and kv head that every sequence is one split: up to the length that was measured
+    assert fa.step_splits(num_seqs, context) == splits and fa.step_whole(num_seqs, context) is whole
+
+
 def test_a_window_bounds_the_splits():
     assert plan(12, window=100).num_splits(1, 32768) == 3                # 131 keys at most
 

@@ -935,7 +935,7 @@ def test_sampling_top_p(K):
 
 # ---- matrix-core attention (bfloat16) ----------------------------------------------------------
 def _fast_case(new_lens, prefix_lens, nq, nkv, d, Pg, seed=0, boost=None, decode=False, nsplit=1, teams=0, as_step=False,
-               window=0, chunk_len=0, max_chunks=0, order=None, cut=None):
+               window=0, chunk_len=0, max_chunks=0, order=None, cut=None, whole=False):
     from pico_vllm_amd.ops.attention_fast import FastAttention
     dtype = torch.bfloat16
     g = torch.Generator().manual_seed(seed)
@@ -964,7 +964,7 @@ def _fast_case(new_lens, prefix_lens, nq, nkv, d, Pg, seed=0, boost=None, decode
     elif decode:
         if cut is not None:             # a cut to fill: the contexts of all sequences in pieces of one length
             cut.append(fa.decode_cut(B, nsplit, DEV))
-        out = fa.decode(wide, kc, vc, bt, ctxl, B, scale, nsplit, cut=cut[0] if cut is not None else None)
+        out = fa.decode(wide, kc, vc, bt, ctxl, B, scale, nsplit, cut=cut[0] if cut is not None else None, whole=whole)
     else:
         if order is not None:           # a list to fill: the query tiles of all sequences longest first
             order.append(fa.order_list(T, B, DEV))
@@ -1295,14 +1295,16 @@ def test_fast_decode_of_whole_sequences(K, nq, nkv, d, window):
     # one split: no merging launch.  Contexts at the edges of blocks of 32 keys and of the turns of the workgroup's eight waves, groups of
     # one to sixteen heads; a sequence without a context (the padding of a recorded step) is left zero and no other is touched
     from pico_vllm_amd.ops.attention_fast import FastAttention
-    out, want = _fast_case([1] * 8, [0, 30, 31, 32, 255, 256, 511, 700], nq, nkv, d, 16, seed=nq + d, decode=True, nsplit=1, window=window)
+    out, want = _fast_case([1] * 8, [0, 30, 31, 32, 255, 256, 511, 700], nq, nkv, d, 16, seed=nq + d, decode=True, nsplit=1, window=window, whole=True)
     close(out, want, torch.bfloat16)
     fa = FastAttention(nq, nkv, d, window)
     kc, vc = torch.randn(4, nkv, 16, d, device=DEV).bfloat16(), torch.randn(4, nkv, d, 16, device=DEV).bfloat16()
     q, bt = torch.randn(3, nq * d, device=DEV).bfloat16(), torch.arange(4, dtype=torch.int32, device=DEV).view(1, 4).repeat(3, 1)
-    some = fa.decode(q, kc, vc, bt, torch.tensor([50, 0, 64], dtype=torch.int32, device=DEV), 3, d ** -0.5, 1)
-    alone = fa.decode(q[2:], kc, vc, bt[2:], torch.tensor([64], dtype=torch.int32, device=DEV), 1, d ** -0.5, 1)
+    some = fa.decode(q, kc, vc, bt, torch.tensor([50, 0, 64], dtype=torch.int32, device=DEV), 3, d ** -0.5, 1, whole=True)
+    alone = fa.decode(q[2:], kc, vc, bt[2:], torch.tensor([64], dtype=torch.int32, device=DEV), 1, d ** -0.5, 1, whole=True)
     assert not some[1].any() and torch.equal(some[2:], alone)
+    with pytest.raises(K.KernelError, match="not read whole"):
+        fa.decode(q, kc, vc, bt, torch.tensor([50, 0, 64], dtype=torch.int32, device=DEV), 3, d ** -0.5, 2, whole=True)
 
 
 def test_fast_kernels_find_one_far_key_among_hundreds(K):
