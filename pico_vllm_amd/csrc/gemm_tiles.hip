@@ -22,7 +22,7 @@ struct GemmArgs {
   int M, cols, K, ldx, ldw, ldo;     // cols: output columns of this launch
   int up;                            // paired epilogues: from a gate row of W to the up row of the same column
   int m_tiles, n_tiles;
-  int bring;                         // so much of every part's k is read ahead by workgroups without a tile (unpaired; the grid has some)
+  int bring;                         // so much of k is read ahead by workgroups without a tile (unpaired, whole K; the grid has some)
   int splits, part;                  // of K: so many parts of `part` each, a part's sums in out + s M ldo (GT_PARTS; else one)
   float limit, alpha;
 };
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256, SHARE) void gemm_tiles_kernel(const GemmArgs a
     // (a single round: the first `busy` places of a die have its tiles)
     const int busy = (tiles + 7) >> 3;
     if (a.bring > 0 && (int)(blockIdx.x >> 3) >= busy)
-      ts_bring(a.W, a.cols, a.ldw, a.K, a.splits, a.part, a.bring, (int)blockIdx.x - 8 * busy, (int)gridDim.x - 8 * busy, smem);
+      ts_bring(a.W, a.cols, a.ldw, a.bring, (int)blockIdx.x - 8 * busy, (int)gridDim.x - 8 * busy, smem);
     return;
   }
   TileRowsSource<MB> xs;
@@ -189,17 +189,34 @@ __global__ __launch_bounds__(256, SHARE) void gemm_tiles_kernel(const GemmArgs a
 #endif
 }
 
-// Of a single round that leaves an eighth of its places idle: how much of every part's k the workgroups there read ahead, all of it or
-// what each of them can while a tile reads GT_BRING times as much (their one wave of copies a SIMD waits for itself); 0: nothing.
-// Few elements are there before it pays to look ahead, and tiles with next to no rows wait for W alone and so read ahead themselves
-// (2,052 rows of 1,536 x 8,960 62 us either way).
+// Of a single round that leaves an eighth of its places idle: how much of k the workgroups there read ahead, all of it or what each of
+// them can while a tile reads GT_BRING times as much (their one wave of copies a SIMD waits for itself); 0: nothing.  That pays where the
+// tiles wait for memory and several of them want the same rows of W; where the flow into the compute units is the bound it only adds to
+// it.  So, microseconds without and with (recorded launches, matrices from memory):
+// * not for parts of K (65 rows of 1,536 x 13,440 21.2 / 27.1, 256 28.2 / 31.0, 832 of 3,584 x 18,944 135 / 134) nor tiles of 192 or 256 rows
+//   (832 rows of 6,144 x 1,536 with gelu 26.8 / 28.3, 352 of 18,944 x 3,584 60 / 66),
+// * a single tile of rows up to GT_BRING_LONE tiles (96 rows, gelu: 6,144 x 1,536 15.2 / 13.4, 8,960 15.9 / 15.4, 13,440 17.0 / 17.9),
+// * not what two share some units for, if K is long (1,700 rows of 1,536 x 13,440 to float32 118 / 133),
+// * where a helper gets through most of its rows of W (384 rows of 7,168 x 3,584 36.6 / 32.3, 300 of 8,960 x 1,536, with a helper's rows in two
+//   fifths of the time, 17.3 / 18.6),
+// * from few elements on, and not where the last tiles have next to no rows, which wait for W alone and so read ahead themselves (2,052 rows of
+//   1,536 x 8,960 62 either way).
+// Of 420 points drawn over the single rounds below 196 are left: 11 % faster in the geometric mean, the slowest 2 % behind; the others
+// the same.
 #define GT_BRING 0.4f
+#define GT_BRING_MOST 0.5f
+#define GT_BRING_LONE 160
+#define GT_BRING_K 4096
 #define GT_BRING_LEAST (4 << 20)
-static int gt_bring(const GemmArgs& a, long long tiles, int slots, int mb, int nb) {
-  const long long idle = slots - (tiles + 7) / 8 * 8;
-  if (idle < slots / 8 || (long long)a.cols * a.K < GT_BRING_LEAST || (a.M - 1) % (64 * mb) < 32) return 0;
-  const float each = (float)a.cols / idle * a.splits / (64 * (mb + nb));
-  return each <= GT_BRING ? a.part : (int)(a.part * GT_BRING / each) / TS_BK * TS_BK;
+extern "C" int pico_gemm_tiles_ahead(int M, int cols, int K, int splits, int mb, int nb, int share) {
+  const int m_tiles = (M + 64 * mb - 1) / (64 * mb), slots = 256 * share, last = (M - 1) % (64 * mb);
+  const long long tiles = (long long)m_tiles * ((cols + 64 * nb - 1) / (64 * nb)), idle = slots - (tiles + 7) / 8 * 8;
+  if (splits > 1 || mb != 2 || idle < slots / 8 || (long long)cols * K < GT_BRING_LEAST) return 0;
+  if (last < 32) return 0;
+  if ((m_tiles == 1 && tiles > GT_BRING_LONE) || (tiles > 256 && K > GT_BRING_K)) return 0;
+  const float each = (float)ts_bring_rows(cols, (int)idle) / (64 * (mb + nb));
+  if (each > GT_BRING_MOST) return 0;
+  return each <= GT_BRING ? K : (int)(K * GT_BRING / each) / TS_BK * TS_BK;
 }
 
 template <int MB, int NB, int EPI, int SETS = 1, int SHARE = ts_share(MB, NB), int BUFS = ts_buffers(MB, NB)>
@@ -212,7 +229,7 @@ static int gt_launch(GemmArgs a, hipStream_t stream) {
   a.n_tiles = (a.cols + GT_COLS(NB, EPI) - 1) / GT_COLS(NB, EPI);
   const long long tiles = (long long)a.m_tiles * a.n_tiles * a.splits;
   PICO_REQUIRE(tiles < (1LL << 30), "pico_gemm_tiles: %d x %d outputs are too many for one launch", a.M, a.cols);
-  a.bring = gt_paired(EPI) ? 0 : gt_bring(a, tiles, 256 * SHARE, MB, NB);
+  a.bring = gt_paired(EPI) ? 0 : pico_gemm_tiles_ahead(a.M, a.cols, a.K, a.splits, MB, NB, SHARE);
   kernel<<<a.bring ? 256 * SHARE : ts_grid(tiles, 256 * SHARE), 256, bytes, stream>>>(a);
   PICO_LAUNCH_CHECK();
   return 0;
@@ -276,13 +293,14 @@ static int gt_run(GemmArgs a, hipStream_t stream) {
 // Plain products that are a single round of small tiles.  What such a call takes is the stages' latency from memory, so its
 // workgroups have a compute unit each and as many stages on their way as LDS holds (128 x 128, K 1,536, 192 tiles: two buffers
 // and two workgroups a unit 21.3 us, three, four, five buffers 15.5, 15.5, 16.3), and where an eighth of the units has no tile
-// those read the matrix ahead (gt_bring).  Microseconds, library / so (with W read ahead): 2,048 rows of 1,536 x 1,536 17.2 / 15.1,
-// 1,536 x 4,480 35.1 / 32.9, 1,536 x 8,960 70.5 / 74.1 (63.2); 1,377 rows 15.3 / 14.3, 31.3 / 30.3 (29.8), 67.0 / 71.6 (55.7); 832 rows of
-// 4,608 x 3,584 37.6 / 33.1, 3,584 x 3,584 26.8 / 27.4 (28.0), 640 rows of 3,584 x 4,736 40.0 / 44.1 (32.8), x 7,168 54.5 / 57.2 (47.2).  Of up to
+// those read the matrix ahead (pico_gemm_tiles_ahead).  Microseconds, library / so without / with W read ahead, matrices from memory: 2,048 rows of
+// 1,536 x 1,536 15.8 / 13.4, x 4,480 37.5 / 39.4 / 31.8, x 8,960 71.2 / 74.8 / 65.4; 640 rows of 3,584 x 4,736 40.5 / 44.3 / 34.1, 832 38.4 / 39.8,
+// of 3,584 x 3,584 31.0 / 30.7; 352 of 7,168 x 3,584 34.9 / 35.0 / 30.3.  Of up to
 // 128 such tiles 128 x 64 are a single round too; each is as long a chain as the larger, so they pay for short K alone and from
 // where the library's fewer, longer workgroups run out: 700 rows of 1,536 x 1,536 12.8 / 11.1 (640 10.2 / 11.4), 400 of 3,072 x 1,536 13.0 /
-// 11.5, 300 of 4,608 x 1,536 14.0 / 11.6, 832 of 2,048 x 2,048 15.2 / 14.2, of 1,536 x 2,240 16.5 / 14.7, of 1,536 x 3,072 17.8 / 18.9.  Of 191
-// points of 38 matrices in these ranges the geometric mean is 9 % ahead of the library, the worst 13 % behind.
+// 11.5, 300 of 4,608 x 1,536 14.0 / 11.6, 832 of 2,048 x 2,048 15.2 / 14.2, of 1,536 x 2,240 16.5 / 14.7, of 1,536 x 3,072 17.8 / 18.9.  Of 420
+// points drawn over these ranges the geometric mean is 12 % ahead of the library; 44 are behind it, most of them with up to 32 rows in
+// the last tiles, where it depends on how the library's come out (129 rows of 5,120 x 2,560 16.1 / 20.2, the worst, of 6,144 x 2,048 21.5 / 16.8).
 #define GT_ROUND 256
 #define GT_NARROW 144                                // the library is as fast up to so many tiles of 128 x 64
 #define GT_NARROW_K 2560

@@ -15,7 +15,7 @@
 //
 // What bounds it, measured: operands that the L2 holds, a 256 x 128 stage takes 1,290 cycles (1,024 of products, 1,175 for
 // its 48 KB at the 41 bytes a cycle at which a compute unit takes in lines), a 256 x 256 one 2,230 (2,048); from memory the
-// latency of a copy shows, because LDS holds two or three stages: 0.8 to 0.9 us a 256 x 128 stage.  Lines asked for
+// latency of a copy shows, because LDS holds two or three stages (four of a 128 x 128 tile, BUFS): 0.8 to 0.9 us a 256 x 128 stage.  Lines asked for
 // further ahead (four bytes each into the L2, 2 to 6 stages before their copies) made it slower (113 to 117 us and 122 to
 // 145): the copies' counter retires in order, behind the far lines.
 #pragma once
@@ -38,6 +38,9 @@ constexpr int ts_wait(int n, bool lds) { return (n & 15) | ((n >> 4) << 14) | (7
 
 // workgroups for so many tiles where `most` run at once
 constexpr int ts_grid(long long tiles, int most) { return tiles < most ? (int)((tiles + 7) / 8 * 8) : most; }
+
+// Of `rows` rows dealt out in blocks of whole eights to `workers` workgroups: how many a block has (the last workgroups may have none).
+__host__ __device__ inline int ts_bring_rows(int rows, int workers) { return ((rows + workers - 1) / workers + 7) / 8 * 8; }
 
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources exist on the device only)
 // The rows of one operand of a tile, as what a lane asks for: `rsrc` over the matrix from the tile's first row on, and the
@@ -234,20 +237,19 @@ struct TileStream {
   }
 };
 
-// Copies of the rows worker, worker + workers, .. (eights of them) of `rows` rows of stride ld, k from `parts` starts `part` apart on side
-// by side, `most` of each, to nobody's place in LDS: the memory-side cache then has them.  Tiles that wait for memory stage after stage
-// get theirs from there in half the time, so workgroups without a tile do this for the others' matrix, in the order in which those want it.
-__device__ __forceinline__ void ts_bring(const bf16_t* base, int rows, int ld, int K, int parts, int part, int most, int worker, int workers, char* lds) {
+// Copies of this worker's block of rows of stride ld, their first `most` k, to nobody's place in LDS: the memory-side cache then
+// has them.  Tiles that wait for memory stage after stage get theirs from there in half the time, so workgroups without a tile do this for the
+// others' matrix, in the order in which those want it.
+__device__ __forceinline__ void ts_bring(const bf16_t* base, int rows, int ld, int most, int worker, int workers, char* lds) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const __amdgpu_buffer_rsrc_t r = ts_buffer(base, ((long long)(rows - 1) * ld + K) * 2);
-  const int each = ((rows + workers - 1) / workers + 7) / 8 * 8, r0 = worker * each, r1 = min(rows, r0 + each);
+  const __amdgpu_buffer_rsrc_t r = ts_buffer(base, ((long long)(rows - 1) * ld + most) * 2);
+  const int each = ts_bring_rows(rows, workers), r0 = worker * each, r1 = min(rows, r0 + each);
   for (int k = 0; k < most; k += TS_BK)
-    for (int p = 0; p < parts; p++)
-      for (int i = r0 + 8 * wave; i < r1; i += 32) {               // eight rows of 128 bytes a copy
-        const int row = i + (lane >> 3), at = k + (lane & 7) * 8, col = p * part + at;
-        const uint32_t off = row < r1 && at < part && col < K ? (uint32_t)(row * ld + col) * 2 : TS_OUT;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(lds + wave * 1024), 16, off, 0, 0, 0);
-      }
+    for (int i = r0 + 8 * wave; i < r1; i += 32) {                 // eight rows of 128 bytes a copy
+      const int row = i + (lane >> 3), col = k + (lane & 7) * 8;
+      const uint32_t off = row < r1 && col < most ? (uint32_t)(row * ld + col) * 2 : TS_OUT;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(lds + wave * 1024), 16, off, 0, 0, 0);
+    }
   __builtin_amdgcn_s_waitcnt(ts_wait(0, true));
 }
 

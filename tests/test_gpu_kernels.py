@@ -308,6 +308,16 @@ def test_products_of_a_single_round(K, M, N, K_, bias):
     assert torch.equal(out[rows], K.gemm_tiles(a[rows].contiguous(), w, b))
 
 
+@pytest.mark.parametrize("M,N,K_,parts,mb,nb,share,want", [
+    (65, 13440, 1536, 1, 2, 1, 2, 0), (128, 8960, 1536, 1, 2, 1, 2, 1536), (96, 1536, 13440, 8, 2, 1, 2, 0), (832, 3584, 18944, 2, 4, 2, 1, 0), (352, 18944, 3584, 1, 3, 3, 1, 0),
+    (300, 7168, 3584, 1, 2, 2, 1, 3584), (352, 7168, 3584, 1, 2, 2, 1, 3584), (300, 6144, 1536, 1, 2, 1, 2, 1536), (320, 8960, 1536, 1, 2, 2, 1, 0), (768, 4608, 3584, 1, 2, 2, 1, 3008),
+    (1700, 1536, 13440, 1, 2, 1, 2, 0), (1024, 1536, 13440, 1, 2, 1, 2, 13440), (2048, 1536, 8960, 1, 2, 2, 1, 8960), (2052, 1536, 8960, 1, 2, 2, 1, 0), (512, 1024, 1536, 1, 2, 1, 2, 0)])
+def test_what_is_read_ahead_of_a_product(K, M, N, K_, parts, mb, nb, share, want):
+    # both sides of every line of the rule, at points where it was measured: no parts, no large tiles, no matrix that a single row of many tiles
+    # reads, no helper with more rows than it gets through
+    assert K.library.core().pico_gemm_tiles_ahead(M, N, K_, parts, mb, nb, share) == want
+
+
 @pytest.mark.parametrize("name", ["swiglu", "clipped"])
 def test_activation_of_the_tiled_product_over_all_numbers(K, name):
     # a gate that is one number of the row, an up that is 1 (0, for the clipped form's u + 1): every bfloat16 number through the
