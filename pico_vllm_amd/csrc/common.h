@@ -59,15 +59,16 @@ __device__ __forceinline__ float gelu_tanh_f(float z) {
 // 0.5 z (1 + erf(z / sqrt 2))
 __device__ __forceinline__ float gelu_erf_f(float z) { return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f)); }
 
-// n sigmoid(z) = n / (1 + exp(-z)) from the hardware's exponential and reciprocal: 13 instructions and those two, where expf and
+// n sigmoid(z) = n / (1 + exp(-z)) from the hardware's exponential and reciprocal: 15 instructions and those two, where expf and
 // a division are 25 and two (up to 280 of them a thread behind a tiled product: 2,048 rows of 4,480 pairs, K 1,536, 65 us and 60 so).  What
 // the exponent loses in its rounding is put back as a factor, what the sum 1 + e loses is kept in `low`, and one step of
-// refinement makes the quotient; its fixup takes zeros, infinities and NaN.  Error against 64 bits in units of 2^-24 of the rms, z = n
-// normal, 4 times that, -20 .. 20: 0.46, 0.43, 0.39 (0.66, 0.71, 0.55 with expf and a division).  Below z = -87.3 the result is zero.
+// refinement makes the quotient; its fixup takes zeros, infinities and NaN.  The reciprocal is of a quarter of the sum, as it gives zero for
+// sums over 2^126 (z < -87.3).  Error against 64 bits in units of 2^-24 of the rms, z = n
+// normal, 4 times that, -20 .. 20: 0.46, 0.43, 0.39 (0.66, 0.71, 0.55 with expf and a division).  Below z = -88.7 the result is zero, as theirs.
 __device__ __forceinline__ float times_sigmoid(float n, float z) {
   const float zc = __builtin_amdgcn_fmed3f(z, -1000.0f, 128.0f), y = zc * -1.44269504f;                  // -z log2(e) = y + off
   const float off = fmaf(zc, -1.925963033e-8f, fmaf(zc, -1.44269504f, -y)), e = __builtin_amdgcn_exp2f(y), c = fmaf(off, 0.693147181f, 1.0f);
-  const float d = fmaf(e, c, 1.0f), low = fmaf(e, c, 1.0f - d), r = __builtin_amdgcn_rcpf(d), q = n * r;
+  const float d = fmaf(e, c, 1.0f), low = fmaf(e, c, 1.0f - d), r = __builtin_amdgcn_rcpf(d * 0.25f) * 0.25f, q = n * r;
   return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-low, q, fmaf(-d, q, n)), r, q), d, n);
 }
 // z sigmoid(z)

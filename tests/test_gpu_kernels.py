@@ -322,7 +322,7 @@ def test_what_is_read_ahead_of_a_product(K, M, N, K_, parts, mb, nb, share, want
 def test_activation_of_the_tiled_product_over_all_numbers(K, name):
     # a gate that is one number of the row, an up that is 1 (0, for the clipped form's u + 1): every bfloat16 number through the
     # activation, which is then rounded to bfloat16 (2^-8 of it) from what is within 2^-21 of the quotient in 64 bits (results below 2^-119, of z
-    # under -87.3, may be zero)
+    # under -88.7, may be zero)
     x = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
     a = torch.zeros(65536, 16, dtype=torch.bfloat16)
     a[:, 0], a[:, 1] = x, 1
@@ -336,6 +336,21 @@ def test_activation_of_the_tiled_product_over_all_numbers(K, name):
     assert bool((out == out[:, :1])[~bad].all())
     got, want = out[:, 0][~bad].double(), want[~bad]
     assert bool(((got - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -21) + 2.0 ** -119).all())      # (eight bits: half of the last is 2^-8 of 1)
+
+
+@pytest.mark.parametrize("name,gates", [("swiglu", [-86.0, -87.0, -87.5, -88.0, -88.5]), ("clipped", [-51.0, -51.25, -51.5, -51.75, -52.0])])
+def test_activation_of_the_tiled_product_keeps_its_smallest_results(K, name, gates):
+    # gates at which 1 + exp(-z) is between 2^126 and the largest number: results of about 5e-37 are normal numbers, rounded to eight bits (from
+    # within 2^-17 of the quotient: in float32 the exponent alpha g is off by up to 88 2^-24)
+    x = torch.tensor(gates).repeat(20).bfloat16()
+    a = torch.zeros(x.numel(), 16, dtype=torch.bfloat16)
+    a[:, 0], a[:, 1] = x, 1
+    w = torch.zeros(16, 16, dtype=torch.bfloat16)
+    w[:8, 0], w[8:, 1] = 1, 1 if name == "swiglu" else 0
+    alpha = 1.0 if name == "swiglu" else 1.702
+    out = K.gemm_tiles(a.to(DEV), w.to(DEV), None, K.EPI_SWIGLU if name == "swiglu" else K.EPI_CLIPPED, clip=(float("inf"), alpha)).cpu().double()
+    want = (x.double() / (1 + torch.exp(-alpha * x.double()))).view(-1, 1)
+    assert bool(((out - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -17)).all())
 
 
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
