@@ -885,6 +885,20 @@ def test_options_that_travel_with_the_launch(K, R):
             assert [sampler.read(x) for x in tickets[-2:]] == want[-2:]
 
 
+@pytest.mark.parametrize("V", [40, 2049, 65535, 65537, 131073, 196608, 196641, 262145])
+def test_sampling_finds_every_element_of_a_chunk(K, V):
+    # likely tokens at the edges of a row's 32 chunks and of what a thread reads of one at a time, all others next to impossible: each is drawn
+    # where its share of the row lies
+    step = -(-V // 32)
+    at = sorted({c * step + o for c in (0, 13, 31) for o in (0, 255, 256, 2047, 2048, 4095, 4096, 6143, 6144, 8191, step - 1) if o < step and c * step + o < V})
+    n = len(at)
+    logits = torch.full((n, V), -40.0)
+    logits[:, at] = 3.0
+    u = (torch.arange(n) + 0.5) / n
+    got = K.sample(logits.to(DEV), torch.ones(n, device=DEV), torch.full((n,), 0.999, device=DEV), u.to(DEV))
+    assert got.tolist() == at
+
+
 def test_sampling_at_the_edges_of_its_options(K):
     # a nucleus so small that only the likeliest token fits, a temperature so low that it holds all the mass, one so high
     # that the distribution is flat, and a vocabulary smaller than the number of chunks a row is read in
