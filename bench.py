@@ -371,21 +371,20 @@ def attention_point(cfg, nseq, new_len, prefix, shape=0, reps=20, chunk_len=0):
 
 
 def sampling_point(cfg, rows, top_p, reps=50):
-    """The sampling call alone on ``rows`` rows of float32 logits of the shape's vocabulary: greedy, temperature 0.8,
-    and temperature 0.8 with ``top_p``; microseconds a call."""
+    """A step's sampling launches alone (as ``Sampler.launch`` makes them, behind one another, nobody waiting for the tokens) on ``rows`` rows of
+    float32 logits of the shape's vocabulary: greedy, temperature 0.8, and temperature 0.8 with ``top_p``; microseconds a call."""
     import torch
     from pico_vllm_amd.ops import kernels
     dev, V = "cuda", describe(cfg)[2].vocab_size
     g = torch.Generator(device=dev).manual_seed(0)
     logits = torch.randn(rows, V, device=dev, generator=g) * 3.0
-    u = torch.rand(rows, device=dev, generator=g)
     out = torch.empty(rows, dtype=torch.int32, device=dev)
-    work = kernels.sample_workspace(rows, dev)
+    work, chunk_work = kernels.sample_workspace(rows, dev), kernels.argmax_workspace(rows, dev)
+    options, params = kernels.SampleOptions(rows), torch.empty(3, rows, dtype=torch.float32, device=dev)
     res = {}
     for name, temp, p in (("greedy", 0.0, 1.0), ("temperature", 0.8, 1.0), ("top_p", 0.8, top_p)):
-        t = torch.full((rows,), temp, device=dev)
-        pp = torch.full((rows,), p, device=dev)
-        run = lambda: kernels.sample(logits, t, pp, u, out=out, work=work, top_p_rows=temp > 0 and p < 1)
+        options.fill([temp] * rows, [p] * rows, range(rows), range(rows))
+        run = lambda: kernels.sample_rows(logits, options, params, out, work, p < 1) if temp else kernels.argmax(logits, out, chunk_work)
         for _ in range(5):
             run()
         torch.cuda.synchronize()

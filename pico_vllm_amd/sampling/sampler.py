@@ -31,7 +31,8 @@ def _splitmix64(x: int) -> int:
 
 
 def uniform(seed: int, index: int) -> float:
-    """A number in [0, 1) with 24 random bits, a pure function of (seed, index)."""
+    """A number in [0, 1) with 24 random bits, a pure function of (seed, index): the generator in its plain form, which launches make
+    natively (``kernels.sample_uniforms``) and tests hold them to."""
     z = _splitmix64(_splitmix64(seed & _MASK) ^ ((index * 0xD6E8FEB86659FD93) & _MASK))
     return (z >> 40) / float(1 << 24)
 
