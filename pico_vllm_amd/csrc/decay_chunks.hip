@@ -10,8 +10,8 @@
 //
 // Three launches: every chunk's L from zero; a walk over a sequence's chunks that turns the L's into the states in front
 // of the chunks and leaves the slot's new state; every chunk's outputs.  The operands are bfloat16 rows; state, decays and sums are
-// float32 as the walk's are, in another order, and nothing is rounded to less on the way (decay_pieces_*: what is multiplied with
-// the rows is taken apart).  Rows that go through z sigmoid(z) as they are read are float32 numbers on both sides of a product: those run
+// float32 as the walk's are, in another order, and keep their 24 bits on the way (decay_pieces_*: what is multiplied with
+// the rows is taken apart; of numbers below 2^-110 what is above 2^-134 is left).  Rows that go through z sigmoid(z) as they are read are float32 numbers on both sides of a product: those run
 // on v_mfma_f32_32x32x2_f32 (decay_chunk_*).
 //
 // VAR: the decay changes from token to token (one number a head), g^(i - j) becomes the product of the decays behind j up to
@@ -391,7 +391,8 @@ __global__ __launch_bounds__(256) void decay_chunk_out_kernel(const ChunkArgs a)
 // Rows that are read as they stand (no z sigmoid(z)): q, k and v are bfloat16 numbers, and what they are multiplied with, state, weighted
 // values and weighted products, is taken apart into three of them (split3.h; three instructions of 16 k, 3/16 of the float32
 // instruction's time).  Products of queries and keys are the bfloat16 instruction's own.  All of a tile in LDS is bfloat16: a
-// third of the bytes, so that three workgroups share a compute unit.  Pieces of numbers below 2^-110 end at 2^-133.
+// third of the bytes, so that three workgroups share a compute unit.  Pieces of numbers below 2^-110 end at 2^-133 (scaled, as in
+// split3.h, states of 2^80 and more would not be numbers).
 // ---------------------------------------------------------------------------
 #define DC_TS (DC_CHUNK + 8)             // row stride of [channel][token] and [token][token] planes: 16-byte reads of rows meet every bank once
 

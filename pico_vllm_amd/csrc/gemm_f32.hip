@@ -11,12 +11,12 @@
 // instruction (16 products a sum, 16 sums) and so: 1.93 and 1.68 at K = 1,536, 2.13 and 1.90 at 8,960, 2.28 and 2.06 at 18,944 (one
 // running sum would give 0.2 sqrt(K)).
 //
-// Over 32 rows bound by the vector instructions that take operands apart (45 % of the time) and by the matrix instruction (44 %), up
+// Over 32 rows bound by the vector instructions that take operands apart and by the matrix instruction, about as much by either, up
 // to there by the stream of W; with few tiles by the chain of a range's stages (0.8 us each).  Tiles that read the same rows
 // of W are neighbours on one die.  Where the tiles alone leave the chip idle (less than two a compute unit) every range of K is a
 // workgroup of its own, its sum goes to a slab, and a second launch adds the slabs in the order in which one workgroup would have.
 // Microseconds on the float32 instruction and so, in one process: 320 rows of 17,920 x 1,536 184 / 140, 1,536 x 8,960 98 / 85, 1,536
-// x 1,536 31 / 28; 2,048 rows of 17,920 x 1,536 1,060 / 785; one row of 151,936 x 1,536 212 / 183 (5.1 TB/s), 32 rows 230 / 206.
+// x 1,536 31 / 28; 2,048 rows of 17,920 x 1,536 1,060 / 761; one row of 151,936 x 1,536 212 / 187 (5.0 TB/s), 32 rows 230 / 208.
 #include "split3.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(256) void gemm_f32_join_kernel(const float* __restr
 }
 
 // Tiles of 64 x 128 instead of 64 x 64: an operand is read from LDS for half as many products, so where they are more than the
-// chip holds at once (17,920 x 1,536: 700 tiles, 320 rows, 146 us, in tiles of 64 x 64 159; 560 tiles, 256 rows, 141 and 134).
+// chip holds at once (17,920 x 1,536: 700 tiles, 320 rows, 138 us, in tiles of 64 x 64 153; 560 tiles, 256 rows, 135 and 128).
 static bool f32_wide(int M, int N) { return (long long)((N + 127) / 128) * ((M + 63) / 64) >= 600; }
 
 // The number of slabs [M, N] that a call of these sizes wants as its workspace; 0: none.  Tiles of 64 x 64 (32 x 64 up to
