@@ -14,6 +14,7 @@ from .kernels import KernelError, _check, _check_cache2, _ptr, _stream
 c_float = ctypes.c_float
 MAX_CHUNKS = 32
 PROMPT_KERNEL_FROM = 64      # tokens of a step from which the prompt kernel serves it (a tile of its workgroups)
+DECODE_TILE_KEYS, DECODE_TILE_PAIRS = 136, 128      # single tokens that it serves too: keys, and (sequence, kv head) pairs, at most
 
 
 def supported(key_dim: int, value_dim: int) -> bool:
@@ -58,20 +59,27 @@ class FastBiasAttention:
         blocks = -(-num_tokens // max(1, 16 // R)) * -(-R // 16) * self.nkv
         return blocks < 8 * self.cus
 
-    def chunks(self, num_tokens: int, num_seqs: int) -> int:
+    def chunks(self, num_tokens: int, num_seqs: int, max_keys: int = 0) -> int:
         """Into how many pieces every block's keys are cut, each piece a workgroup of its own (their parts are put
         together by a second launch): as many as bring the step to two workgroups a compute unit, at most MAX_CHUNKS.
         Decided from the step's size alone; a piece is a whole number of 128 keys, found on the device from the block's
-        own range of keys."""
+        own range of keys.  max_keys (of steps of single tokens: what the engine's contexts may reach): no more pieces than those have, the
+        others would be empty."""
         if not self.split(num_tokens):
             return 1
         R = self.nq // self.nkv
         blocks = (-(-num_tokens // max(1, 16 // R)) + num_seqs) * -(-R // 16) * self.nkv
-        return max(1, min(MAX_CHUNKS, -(-2 * self.cus // blocks)))
+        most = MAX_CHUNKS if not max_keys else min(MAX_CHUNKS, -(-max_keys // 128))
+        return max(1, min(most, -(-2 * self.cus // blocks)))
 
     def prompt_shape(self, ctx) -> int:
-        """The shape of the prompt kernel's workgroups for this step (0: that kernel does not serve it)."""
+        """The shape of the prompt kernel's workgroups for this step (0: that kernel does not serve it).  A step of single tokens leaves it 63 of
+        a tile's 64 queries idle; it serves those of few (sequence, kv head) pairs and contexts of a tile or two, where it needs no second
+        launch.  Microseconds a step by the prompt kernel / by blocks of columns, four layers: 64 sequences of 2 kv heads, 560 keys 799 / 720, 250 keys
+        713 / 701, 120 keys 687 / 688, 32 keys 661 / 672; of 4 kv heads 2,156 / 1,955, 32 keys 1,867 / 1,863."""
         if self.tuned is None or ctx.num_tokens < PROMPT_KERNEL_FROM:
+            return 0
+        if ctx.all_decode and (ctx.max_context > DECODE_TILE_KEYS or ctx.num_seqs * self.nkv > DECODE_TILE_PAIRS):
             return 0
         key = ("bias_attention_shape", self.nq, self.nkv, self.dk, self.window)
         if key not in ctx.shared:
@@ -84,8 +92,13 @@ class FastBiasAttention:
             ctx.shared[key] = shape
         return ctx.shared[key]
 
+    def decode_keys(self, ctx) -> int:
+        """The most keys that a single token of this step may see, in any step that is recorded as this one."""
+        return min(ctx.max_context, self.window + 31) if self.window else ctx.max_context
+
     def plan(self, ctx) -> tuple:
-        return (bool(self.split(ctx.num_tokens)), self.chunks(ctx.num_tokens, ctx.num_seqs), self.prompt_shape(ctx))
+        keys = self.decode_keys(ctx) if ctx.all_decode else 0
+        return (bool(self.split(ctx.num_tokens)), self.chunks(ctx.num_tokens, ctx.num_seqs, keys), self.prompt_shape(ctx))
 
     def run(self, q: torch.Tensor, k_cache, v_cache, block_table, cu_seqlens, positions, num_seqs: int,
             split: Optional[bool] = None, out: Optional[torch.Tensor] = None, chunks: Optional[int] = None,

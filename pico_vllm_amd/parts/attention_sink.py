@@ -106,9 +106,10 @@ class SinkAttention(OpenMixer):
         if not (isinstance(other, LightningAttention) and self.fast is not None and cache.k.dtype == torch.bfloat16 and ctx.all_decode
                 and ctx.num_tokens == ctx.num_seqs and other.heads * other.dv <= kernels.PAIR_MAX_ROW):
             return False
-        split, pieces, shape = self.fast.plan(ctx)
-        if shape or not split or not 2 <= pieces <= kernels.PAIR_MAX_PIECES:
+        split, pieces, _ = self.fast.plan(ctx)
+        if not split or pieces > kernels.PAIR_MAX_PIECES:
             return False
+        pieces = max(2, pieces)             # (short contexts too: their second piece is empty, the launches saved are worth more)
         table = self.angles.table(ctx) if self.angles is not None else None
         q, o = kernels.pair_open(
             y, (col, col + self.k_col, col + self.v_col, self.nq, self.nkv, self.dk, self.dv), self.norm_eps, table,

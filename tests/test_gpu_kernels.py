@@ -2058,3 +2058,28 @@ def test_the_layer_takes_a_bias_that_starts_anywhere(K):
     got, want = Linear(w, b)(x).double().cpu(), x.double().cpu() @ w.double().cpu().T + b.double().cpu()
     # the bias and the result are rounded to bfloat16, and float32 sums of 8,960 terms
     assert bool(((got - want).abs() <= 2.0 ** -8 * (want.abs() + b.double().cpu().abs()) + 8960 * 2.0 ** -24 * (x.double().cpu().abs() @ w.double().cpu().abs().T)).all())
+
+
+@pytest.mark.parametrize("nq,nkv,dk,dv,more", [(12, 2, 128, 128, {"window": 300, "slope_span": 8.0}), (6, 2, 64, 128, {"window": 50, "keep_first": 5, "softcap": 20.0}),
+                                               (5, 5, 128, 16, {"chunk": 64, "sink": True}), (12, 1, 320, 256, {})])
+@pytest.mark.parametrize("most", [128, 129, 384, 600])
+def test_bias_attention_of_single_tokens_in_as_many_pieces_as_keys(nq, nkv, dk, dv, more, most):
+    # the pieces that contexts up to `most` keys have, against the most there are (the rest of them empty): the same keys a piece, so the same bits
+    # but for a single piece, which is rounded once without a merge
+    from pico_vllm_amd.ops.attention_bias_fast import MAX_CHUNKS, FastBiasAttention
+    fast = FastBiasAttention(nq, nkv, dk, dv, dk ** -0.5, **more)
+    g = torch.Generator(device=DEV).manual_seed(most)
+    contexts = [n for n in (1, 31, 127, 128, 129, 256, 257, 383, 600) if n <= most]
+    B, per = len(contexts), -(-most // 16)
+    kc, vc = (torch.randn(B * per, nkv, *s, device=DEV, generator=g).bfloat16() for s in ((16, dk), (dv, 16)))
+    bt = torch.randperm(B * per, device=DEV, generator=g).int().reshape(B, per).contiguous()
+    q = torch.randn(B, nq * dk, device=DEV, generator=g).bfloat16()
+    cu, pos = torch.arange(B + 1, dtype=torch.int32, device=DEV), torch.tensor(contexts, dtype=torch.int32, device=DEV) - 1
+    keys = min(most, fast.window + 31) if fast.window else most
+    pieces = fast.chunks(B, B, keys)
+    assert pieces == min(-(-keys // 128), fast.chunks(B, B))
+    got, want = (fast.run(q, kc, vc, bt, cu, pos, B, split=True, chunks=n) for n in (pieces, MAX_CHUNKS))
+    if pieces > 1:
+        assert torch.equal(got, want)
+    else:
+        assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -9)        # an ulp of bfloat16 where the last bit of the sum differs
