@@ -1,6 +1,6 @@
 // A routed feed-forward in bfloat16: the kernels that serve it.
 //
-// Few rows (a row is one (token, chosen expert) pair; single tokens and small steps): every row streams its expert's
+// Few rows (a row is one (token, chosen expert) pair; single tokens and small steps): every expert that they chose streams its
 // matrices once, 16 bytes a lane, sixteen lanes to an output element.
 //
 // More rows: they are sorted by expert on the device (nothing comes back to the host), every expert's rows padded to whole
@@ -55,78 +55,178 @@ __device__ __forceinline__ float row16_sum(float v) {
 }
 
 // ---------------------------------------------------------------------------
-// Few rows, first half.  grid (rows, ceil(F / 16)); 4 waves; a row of 16 lanes makes one f (its gate and its up).
+// Few rows, SHARED: an expert's matrices are streamed once for all of its rows.  Workgroup (tile, j) looks the rows' experts over and takes the j-th
+// that occurs for the first time; the last workgroups of a grid for as many experts as rows find none.  Tiles run along the grid's first
+// index, so that an expert's workgroups go to all dies at one time.  The sums of a row are made as if it were alone.  Bound by the matrices' stream.
+// Otherwise a row streams its expert's matrices itself, rows along the grid's first index: up to three tokens, whose experts seldom meet, and
+// more rows than a wave has lanes.  Microseconds for both halves, every row for itself / shared / shared with a quarter of the tokens
+// padding, by tokens: two of 16 experts of 2,240 x 1,536 at 2 18.2 / 18.6, 4 31.4 / 29.6 / 26.6, 8 53.0 / 47.4 / 42.5; of 4,480 x 1,536 4 55.2 / 51.8 / 42.5,
+// 8 99.8 / 82.0 / 68.4; four of 32 of 4,736 x 3,584 1 78.1 / 80.3, 2 132 / 135, 4 235 / 226 / 195, of 2,368 x 3,584 2 77.1 / 81.1, 4 125.9 / 124.6 / 100.4.
+// live (or null): the context of every token; a token without one pads a recorded step: where rows share, its rows choose no expert
+// and come out as zeros.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void moe_up_rows_kernel(const bf16_t* __restrict__ h, int ldh,
-                                                          const bf16_t* __restrict__ gate_up,
-                                                          const int* __restrict__ experts, const float* __restrict__ weights,
-                                                          bf16_t* __restrict__ y, int top, int E, int F, int D, float limit,
-                                                          float alpha, int mode) {
-  const int r = blockIdx.x, sub = threadIdx.x & 15;
-  const int f = blockIdx.y * 16 + (threadIdx.x >> 4);
-  const int e = experts[r];
-  if (e < 0 || e >= E || f >= F) return;
-  const float w = weights[r];
-  const bf16_t* x = h + (size_t)(r / top) * ldh;
-  const bf16_t* wg = gate_up + ((size_t)e * 2 * F + f) * D;
-  const bf16_t* wu = wg + (size_t)F * D;
-  float g = 0.f, u = 0.f;
-#pragma unroll 2
-  for (int k = sub * 8; k < D; k += 128) {
-    const uint4 xv = *reinterpret_cast<const uint4*>(x + k);
-    const uint4 gv = *reinterpret_cast<const uint4*>(wg + k);
-    const uint4 uv = *reinterpret_cast<const uint4*>(wu + k);
-    float xf[8];
-    unpack8(xv, xf);
-    g = dot8(gv, xf, g);
-    u = dot8(uv, xf, u);
+#define MOE_LANES 64
+struct MoeRows {
+  unsigned long long mask;                            // row numbers: base + the bits' numbers
+  unsigned long long dead;                            // rows of padding, of whoever is the first of a tile
+  int base, expert, tile;                             // expert < 0: nothing to do
+};
+template <bool SHARED>
+__device__ __forceinline__ MoeRows moe_rows_of(const int* __restrict__ experts, const int* __restrict__ live, int R, int top, int E) {
+  MoeRows m;
+  m.dead = 0;
+  if (!SHARED) {
+    m.base = blockIdx.x; m.tile = blockIdx.y; m.mask = 1;
+    const int e = experts[m.base];
+    m.expert = e < E ? e : -1;
+    return m;
   }
-  g = row16_sum(g);
-  u = row16_sum(u);
-  if (sub == 0) y[(size_t)r * F + f] = f32_to_bf16(moe_act(g, u, limit, alpha, mode, w));
+  const int lane = threadIdx.x & 63;
+  int e = lane < R ? experts[lane] : -1;
+  const bool there = lane >= R || !live || live[lane / top] > 0;
+  if (e >= E || !there) e = -1;
+  bool leads = e >= 0;
+  for (int i = 0; i < R - 1; i++) leads = leads && !(i < lane && __builtin_amdgcn_readlane(e, i) == e);
+  unsigned long long leaders = __ballot(leads);
+  m.base = 0; m.tile = blockIdx.x;
+  if (blockIdx.y == 0) m.dead = __ballot(!there);
+  for (int j = blockIdx.y; j > 0; j--) leaders &= leaders - 1;
+  m.expert = leaders ? __builtin_amdgcn_readlane(e, __builtin_ctzll(leaders)) : -1;
+  m.mask = __ballot(e == m.expert);
+  return m;
+}
+// the next M rows of the mask; the last one again where there are fewer
+template <int M>
+__device__ __forceinline__ void moe_next_rows(unsigned long long& mask, int base, int (&r)[M]) {
+#pragma unroll
+  for (int i = 0; i < M; i++) {
+    r[i] = base + __builtin_ctzll(mask);
+    if (mask & (mask - 1)) mask &= mask - 1;
+  }
 }
 
-// ---------------------------------------------------------------------------
-// Few rows, second half: out[slot][t][n] = down_e[n] . y[(t, slot)] (a slab a slot; whoever reads it adds the slabs up).  A
-// wave makes MOE_DOWN_OUT neighbouring outputs of a row with all its lanes along k, so that a launch of one token still has a
-// few hundred workgroups and a lane several loads on their way.  grid (rows, ceil(D / (4 MOE_DOWN_OUT))).
-// ---------------------------------------------------------------------------
-#define MOE_DOWN_OUT 2
-__global__ __launch_bounds__(256) void moe_down_rows_kernel(const bf16_t* __restrict__ y, const bf16_t* __restrict__ down,
-                                                            const int* __restrict__ experts, float* __restrict__ out,
-                                                            int top, int E, int F, int D) {
-  const int r = blockIdx.x, lane = threadIdx.x & 63;
-  const int n = (blockIdx.y * 4 + (threadIdx.x >> 6)) * MOE_DOWN_OUT;
-  const int e = experts[r];
-  if (e < 0 || e >= E || n >= D) return;
-  const bf16_t* wd[MOE_DOWN_OUT];
-  float s[MOE_DOWN_OUT];
+constexpr int moe_up_out(bool shared) { return shared ? 8 : 16; }
+// First half: 16 lanes make one f (its gate and its up) of M rows.
+template <int M>
+__device__ __forceinline__ void moe_up_some(const bf16_t* __restrict__ h, int ldh, const bf16_t* __restrict__ wg, const bf16_t* __restrict__ wu,
+                                            const float* __restrict__ weights, bf16_t* __restrict__ y, unsigned long long& mask, int base,
+                                            int top, int F, int D, int f, float limit, float alpha, int mode) {
+  const int sub = threadIdx.x & 15, n = min(M, (int)__popcll(mask));
+  int r[M];
+  moe_next_rows(mask, base, r);
+  const bf16_t* x[M];
+  float g[M], u[M], w[M];
 #pragma unroll
-  for (int i = 0; i < MOE_DOWN_OUT; i++) {
-    wd[i] = down + ((size_t)e * D + min(n + i, D - 1)) * F;
-    s[i] = 0.f;
+  for (int i = 0; i < M; i++) {
+    x[i] = h + (size_t)(r[i] / top) * ldh;
+    w[i] = weights[r[i]];
+    g[i] = u[i] = 0.f;
   }
-  const bf16_t* yr = y + (size_t)r * F;
+#pragma unroll 2
+  for (int k = sub * 8; k < D; k += 128) {
+    const uint4 gv = *reinterpret_cast<const uint4*>(wg + k);
+    const uint4 uv = *reinterpret_cast<const uint4*>(wu + k);
+    uint4 xv[M];
+#pragma unroll
+    for (int i = 0; i < M; i++) xv[i] = *reinterpret_cast<const uint4*>(x[i] + k);
+#pragma unroll
+    for (int i = 0; i < M; i++) {
+      float xf[8];
+      unpack8(xv[i], xf);
+      g[i] = dot8(gv, xf, g[i]);
+      u[i] = dot8(uv, xf, u[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < M; i++) {
+    g[i] = row16_sum(g[i]);
+    u[i] = row16_sum(u[i]);
+    if (sub == 0 && i < n) y[(size_t)r[i] * F + f] = f32_to_bf16(moe_act(g[i], u[i], limit, alpha, mode, w[i]));
+  }
+}
+template <bool SHARED>
+__global__ __launch_bounds__(16 * moe_up_out(SHARED)) void moe_up_rows_kernel(const bf16_t* __restrict__ h, int ldh, const bf16_t* __restrict__ gate_up,
+                                                          const int* __restrict__ experts, const float* __restrict__ weights,
+                                                          const int* __restrict__ live, bf16_t* __restrict__ y, int R, int top, int E,
+                                                          int F, int D, float limit, float alpha, int mode) {
+  MoeRows m = moe_rows_of<SHARED>(experts, live, R, top, E);
+  const int f = m.tile * moe_up_out(SHARED) + (threadIdx.x >> 4);
+  if (m.expert < 0 || f >= F) return;
+  const bf16_t* wg = gate_up + ((size_t)m.expert * 2 * F + f) * D;
+  const bf16_t* wu = wg + (size_t)F * D;
+  if (!SHARED) return moe_up_some<1>(h, ldh, wg, wu, weights, y, m.mask, m.base, top, F, D, f, limit, alpha, mode);
+  for (int left = __popcll(m.mask); left > 0; left -= 4) {
+    if (left == 1) moe_up_some<1>(h, ldh, wg, wu, weights, y, m.mask, m.base, top, F, D, f, limit, alpha, mode);
+    else if (left == 2) moe_up_some<2>(h, ldh, wg, wu, weights, y, m.mask, m.base, top, F, D, f, limit, alpha, mode);
+    else moe_up_some<4>(h, ldh, wg, wu, weights, y, m.mask, m.base, top, F, D, f, limit, alpha, mode);
+  }
+}
+
+// Second half: out[slot][t][n] = down_e[n] . y[(t, slot)] (a slab a slot; whoever reads it adds the slabs up).  A
+// wave makes MOE_DOWN_OUT neighbouring outputs of M rows with all its lanes along k, so that a launch of one token still has a
+// few hundred workgroups and a lane several loads on their way.
+#define MOE_DOWN_OUT 2
+template <int M>
+__device__ __forceinline__ void moe_down_some(const bf16_t* __restrict__ y, const bf16_t* const (&wd)[MOE_DOWN_OUT], float* __restrict__ out,
+                                              unsigned long long& mask, int base, int T, int top, int F, int D, int n) {
+  const int lane = threadIdx.x & 63, rows = min(M, (int)__popcll(mask));
+  int r[M];
+  moe_next_rows(mask, base, r);
+  float s[M][MOE_DOWN_OUT];
+#pragma unroll
+  for (int m = 0; m < M; m++)
+#pragma unroll
+    for (int i = 0; i < MOE_DOWN_OUT; i++) s[m][i] = 0.f;
 #pragma unroll 3
   for (int j = lane * 8; j < F; j += 512) {
-    uint4 wv[MOE_DOWN_OUT];
+    uint4 wv[MOE_DOWN_OUT], yv[M];
 #pragma unroll
     for (int i = 0; i < MOE_DOWN_OUT; i++) wv[i] = *reinterpret_cast<const uint4*>(wd[i] + j);
-    float yf[8];
-    unpack8(*reinterpret_cast<const uint4*>(yr + j), yf);
 #pragma unroll
-    for (int i = 0; i < MOE_DOWN_OUT; i++) s[i] = dot8(wv[i], yf, s[i]);
+    for (int m = 0; m < M; m++) yv[m] = *reinterpret_cast<const uint4*>(y + (size_t)r[m] * F + j);
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+      float yf[8];
+      unpack8(yv[m], yf);
+#pragma unroll
+      for (int i = 0; i < MOE_DOWN_OUT; i++) s[m][i] = dot8(wv[i], yf, s[m][i]);
+    }
   }
-  float* o = out + ((size_t)(r % top) * (gridDim.x / top) + r / top) * D + n;
 #pragma unroll
-  for (int i = 0; i < MOE_DOWN_OUT; i++) {
-    const float total = wave_sum(s[i]);
-    if (lane == 0 && n + i < D) o[i] = total;
+  for (int m = 0; m < M; m++) {
+    float* o = out + ((size_t)(r[m] % top) * T + r[m] / top) * D + n;
+#pragma unroll
+    for (int i = 0; i < MOE_DOWN_OUT; i++) {
+      const float total = wave_sum(s[m][i]);
+      if (lane == 0 && n + i < D && m < rows) o[i] = total;
+    }
+  }
+}
+template <bool SHARED>
+__global__ __launch_bounds__(256) void moe_down_rows_kernel(const bf16_t* __restrict__ y, const bf16_t* __restrict__ down,
+                                                            const int* __restrict__ experts, const int* __restrict__ live,
+                                                            float* __restrict__ out, int T, int top, int E, int F, int D) {
+  MoeRows m = moe_rows_of<SHARED>(experts, live, T * top, top, E);
+  const int n = (m.tile * 4 + (threadIdx.x >> 6)) * MOE_DOWN_OUT;
+  if (n >= D) return;
+  for (; m.dead; m.dead &= m.dead - 1) {
+    const int r = __builtin_ctzll(m.dead), i = threadIdx.x & 63;
+    if (i < MOE_DOWN_OUT && n + i < D) out[((size_t)(r % top) * T + r / top) * D + n + i] = 0.f;
+  }
+  if (m.expert < 0) return;
+  const bf16_t* wd[MOE_DOWN_OUT];
+#pragma unroll
+  for (int i = 0; i < MOE_DOWN_OUT; i++) wd[i] = down + ((size_t)m.expert * D + min(n + i, D - 1)) * F;
+  if (!SHARED) return moe_down_some<1>(y, wd, out, m.mask, m.base, T, top, F, D, n);
+  for (int left = __popcll(m.mask); left > 0; left -= 4) {
+    if (left == 1) moe_down_some<1>(y, wd, out, m.mask, m.base, T, top, F, D, n);
+    else if (left == 2) moe_down_some<2>(y, wd, out, m.mask, m.base, T, top, F, D, n);
+    else moe_down_some<4>(y, wd, out, m.mask, m.base, T, top, F, D, n);
   }
 }
 
 extern "C" int pico_moe_experts_rows(const void* h, int ldh, const void* gate_up, const void* down, const int* experts,
-                                     const float* weights, void* y, float* out, int T, int top, int E, int F, int D,
+                                     const float* weights, const int* live, void* y, float* out, int T, int top, int E, int F, int D,
                                      float limit, float alpha, int mode, hipStream_t stream) {
   PICO_REQUIRE(T >= 0 && top > 0 && E > 0 && F > 0 && D > 0 && ldh >= D, "pico_moe_experts_rows: bad sizes");
   PICO_REQUIRE(mode >= 0 && mode <= 2, "pico_moe_experts_rows: unknown mode %d", mode);
@@ -134,11 +234,18 @@ extern "C" int pico_moe_experts_rows(const void* h, int ldh, const void* gate_up
   PICO_REQUIRE(((uintptr_t)h | (uintptr_t)gate_up | (uintptr_t)down | (uintptr_t)y) % 16 == 0,
                "pico_moe_experts_rows: operands must start on 16 bytes");
   if (T == 0) return 0;
-  const dim3 g1(T * top, (F + 15) / 16), g2(T * top, (D + 4 * MOE_DOWN_OUT - 1) / (4 * MOE_DOWN_OUT));
-  PICO_REQUIRE(g1.y <= 65535 && g2.y <= 65535, "pico_moe_experts_rows: sizes beyond the grid");
-  moe_up_rows_kernel<<<g1, 256, 0, stream>>>((const bf16_t*)h, ldh, (const bf16_t*)gate_up, experts, weights, (bf16_t*)y,
-                                             top, E, F, D, limit, alpha, mode);
-  moe_down_rows_kernel<<<g2, 256, 0, stream>>>((const bf16_t*)y, (const bf16_t*)down, experts, out, top, E, F, D);
+  const long long R = (long long)T * top;
+  const bool shared = T > 3 && R <= MOE_LANES;
+  const unsigned out_up = moe_up_out(shared), up = (F + out_up - 1) / out_up, dn = (D + 4 * MOE_DOWN_OUT - 1) / (4 * MOE_DOWN_OUT);
+  PICO_REQUIRE(R < (1ll << 30) && up <= 65535 && dn <= 65535, "pico_moe_experts_rows: sizes beyond the grid");
+  const unsigned met = (unsigned)min(R, (long long)E);
+  const dim3 g1 = shared ? dim3(up, met) : dim3((unsigned)R, up), g2 = shared ? dim3(dn, met) : dim3((unsigned)R, dn);
+#define LAUNCH(SHARED)                                                                                                                             \
+  moe_up_rows_kernel<SHARED><<<g1, 16 * moe_up_out(SHARED), 0, stream>>>((const bf16_t*)h, ldh, (const bf16_t*)gate_up, experts, weights, live,      \
+                                                                         (bf16_t*)y, (int)R, top, E, F, D, limit, alpha, mode);                    \
+  moe_down_rows_kernel<SHARED><<<g2, 256, 0, stream>>>((const bf16_t*)y, (const bf16_t*)down, experts, live, out, T, top, E, F, D)
+  if (shared) { LAUNCH(true); } else { LAUNCH(false); }
+#undef LAUNCH
   PICO_LAUNCH_CHECK();
   return 0;
 }
@@ -159,16 +266,33 @@ extern "C" int pico_moe_experts_rows(const void* h, int ldh, const void* gate_up
 __global__ __launch_bounds__(MOE_SORT_THREADS) void moe_sort_kernel(const int* __restrict__ experts,
                                                                     const float* __restrict__ weights, int R, int E, int bm,
                                                                     int tiles_cap, int* __restrict__ sorted,
-                                                                    float* __restrict__ sorted_w, int* __restrict__ tiles_out) {
+                                                                    float* __restrict__ sorted_w, int* __restrict__ tiles_out,
+                                                                    const int* __restrict__ live, int top, float* __restrict__ out, int T, int D) {
   __shared__ int hist[MOE_SORT_MAX_E];
   __shared__ int wave_count[MOE_SORT_THREADS / 64];
   __shared__ int base_tiles;
   const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = MOE_SORT_THREADS / 64;
+  // (a token without a context pads a recorded step: its rows, of MOE_LANES, have no expert and come out as zeros)
+  auto expert = [&](int r) {
+    const int x = experts[r];
+    return (live ? live[r / top] : 1) > 0 ? x : -1;
+  };
+  if (live) {
+    int turn = 0;
+    for (unsigned long long dead = __ballot(lane < R && live[min(lane, R - 1) / top] <= 0); dead; dead &= dead - 1) {
+      if (turn == e) {
+        const int r = __builtin_ctzll(dead);
+        float* o = out + ((size_t)(r % top) * T + r / top) * D;
+        for (int n = tid; n < D; n += MOE_SORT_THREADS) o[n] = 0.f;
+      }
+      turn = turn + 1 == E ? 0 : turn + 1;
+    }
+  }
   for (int i = tid; i < E; i += MOE_SORT_THREADS) hist[i] = 0;
   if (tid == 0) base_tiles = 0;
   __syncthreads();
   for (int r = tid; r < R; r += MOE_SORT_THREADS) {
-    const int x = experts[r];
+    const int x = expert(r);
     if (x >= 0 && x < E) atomicAdd(&hist[x], 1);
   }
   __syncthreads();
@@ -188,7 +312,7 @@ __global__ __launch_bounds__(MOE_SORT_THREADS) void moe_sort_kernel(const int* _
   int mine = 0;
   for (int r0 = lo; r0 < hi; r0 += 64) {
     const int r = r0 + lane;
-    const bool is = r < hi && experts[r] == e;
+    const bool is = r < hi && expert(r) == e;
     mine += __popcll(__ballot(is));
   }
   if (lane == 0) wave_count[wave] = mine;
@@ -199,7 +323,7 @@ __global__ __launch_bounds__(MOE_SORT_THREADS) void moe_sort_kernel(const int* _
   float* dst_w = sorted_w + (size_t)base * bm;
   for (int r0 = lo; r0 < hi; r0 += 64) {
     const int r = r0 + lane;
-    const bool is = r < hi && experts[r] == e;
+    const bool is = r < hi && expert(r) == e;
     const unsigned long long m = __ballot(is);
     if (is) {
       const int to = at + __popcll(m & ((1ull << lane) - 1ull));
@@ -391,7 +515,7 @@ static int moe_product(int bm, int E, const MoeArgs& a, hipStream_t stream) {
 
 // sorted: int32 [2 tiles_cap bm] (row numbers, then weights), tiles: int32 [2 tiles_cap + 1]
 extern "C" int pico_moe_experts_grouped(const void* h, int ldh, const void* gate_up, const void* down, const int* experts,
-                                        const float* weights, int* sorted, int* tiles, int tiles_cap, int bm, void* y,
+                                        const float* weights, const int* live, int* sorted, int* tiles, int tiles_cap, int bm, void* y,
                                         float* out, int T, int top, int E, int F, int D, float limit, float alpha,
                                         int mode, hipStream_t stream) {
   PICO_REQUIRE(mode >= 0 && mode <= 2, "pico_moe_experts_grouped: unknown mode %d", mode);
@@ -409,7 +533,9 @@ extern "C" int pico_moe_experts_grouped(const void* h, int ldh, const void* gate
   const long long need = (R + (long long)E * (bm - 1)) / bm;
   PICO_REQUIRE(tiles_cap >= need, "pico_moe_experts_grouped: room for %d tiles, %lld may be needed", tiles_cap, need);
   float* sorted_w = (float*)sorted + (size_t)tiles_cap * bm;
-  moe_sort_kernel<<<E, MOE_SORT_THREADS, 0, stream>>>(experts, weights, (int)R, E, bm, tiles_cap, sorted, sorted_w, tiles);
+  // (with more rows every expert has some either way, and to look for padding takes longer than it gives)
+  if (R > MOE_LANES || R > 2 * E) live = nullptr;
+  moe_sort_kernel<<<E, MOE_SORT_THREADS, 0, stream>>>(experts, weights, (int)R, E, bm, tiles_cap, sorted, sorted_w, tiles, live, top, out, T, D);
   const MoeArgs up{(const bf16_t*)h, (const bf16_t*)gate_up, sorted, sorted_w, tiles, (bf16_t*)y, nullptr, tiles_cap, ldh, T, top, F, D, 0, mode, limit, alpha};
   MoeArgs dn = up;
   dn.X = (const bf16_t*)y; dn.W = (const bf16_t*)down; dn.out = out;

@@ -15,6 +15,11 @@ from .spec import ParamSpec
 ACT_ALPHA = 1.702
 
 
+def _live(ctx: Optional[StepContext]) -> Optional[torch.Tensor]:
+    """The contexts of a step of single tokens: the rows that pad a recorded one have none, and read no expert."""
+    return ctx.context_lens if ctx is not None and ctx.all_decode and ctx.num_tokens == ctx.num_seqs else None
+
+
 @register_part("feed_forward", "routed_experts")
 class RoutedExperts(FeedForward):
     """Router: z = x Wr^T in float32, scores s = sigmoid(z); a token's ``top`` experts are those with the largest
@@ -84,7 +89,7 @@ class RoutedExperts(FeedForward):
         if kernels.moe_fast_ok(x, gate_up, down):
             # few rows stream their experts' matrices; many are sorted by expert and go to the matrix cores.  The
             # second gives one float32 slab a slot: the next norm adds them up
-            return kernels.moe_experts(x, gate_up, down, experts, weights, self.limit, self.act_alpha, mode=self.MODE)
+            return kernels.moe_experts(x, gate_up, down, experts, weights, self.limit, self.act_alpha, mode=self.MODE, live=_live(ctx))
         return kernels.moe_experts_plain(x, gate_up, down, experts, weights, self.limit, self.act_alpha, mode=self.MODE)
 
     def graph_variant(self, ctx: StepContext) -> tuple:
@@ -186,7 +191,7 @@ class SoftmaxRoutedExperts(FeedForward):
         return 2.0 * tokens * (self.outputs * D + self.top * 3 * F * D) + (self.shared.flops(tokens, pairs) if self.shared is not None else 0.0)
 
     def forward(self, x: torch.Tensor, ctx: StepContext):
-        out = self._routed(x)
+        out = self._routed(x, ctx)
         if self.shared is None:
             return out
         return [self.shared.forward(x, ctx), out]
@@ -196,16 +201,16 @@ class SoftmaxRoutedExperts(FeedForward):
         step); the routed sum is returned, for the next norm's launch to add."""
         if self.shared is not None:
             self.shared.down.add_into(self.shared.gate_up.swiglu(x), resid)
-        return self._routed(x)
+        return self._routed(x, ctx)
 
-    def _routed(self, x: torch.Tensor) -> torch.Tensor:
+    def _routed(self, x: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         E, F, D = self.num_experts, self.expert_size, self.hidden_size
         experts, weights = kernels.moe_router_softmax(x, self.router.weight, self.correction, self.top, self.scale)
         gate_up = self.gate_up.weight.view(E, 2 * F, D)
         down = self.down.weight.view(E, D, F)
         xe = x if x.dtype == gate_up.dtype else x.to(gate_up.dtype)
         if kernels.moe_fast_ok(xe, gate_up, down):
-            out = kernels.moe_experts(xe, gate_up, down, experts, weights, 0.0, 0.0, mode=kernels.MOE_SWIGLU)
+            out = kernels.moe_experts(xe, gate_up, down, experts, weights, 0.0, 0.0, mode=kernels.MOE_SWIGLU, live=_live(ctx))
         else:
             out = kernels.moe_experts_plain(xe, gate_up, down, experts, weights, 0.0, 0.0, mode=kernels.MOE_SWIGLU)
         if self.identity:
@@ -261,7 +266,7 @@ class TopSoftmaxRoutedExperts(SoftmaxRoutedExperts):
         down = self.down.weight.view(E, D, F)
         xe = x if x.dtype == gate_up.dtype else x.to(gate_up.dtype)
         if kernels.moe_fast_ok(xe, gate_up, down):
-            routed = kernels.moe_experts(xe, gate_up, down, experts, weights, 0.0, 0.0, mode=kernels.MOE_SWIGLU)
+            routed = kernels.moe_experts(xe, gate_up, down, experts, weights, 0.0, 0.0, mode=kernels.MOE_SWIGLU, live=_live(ctx))
         else:
             routed = kernels.moe_experts_plain(xe, gate_up, down, experts, weights, 0.0, 0.0, mode=kernels.MOE_SWIGLU)
         if self.shared is None:

@@ -152,6 +152,33 @@ def test_experts_activation_has_the_same_bits_by_every_kernel(K, mode):
         assert torch.equal(K.moe_experts(*args, 7.0, 1.702, grouped=grouped, mode=mode), plain)
 
 
+@pytest.mark.parametrize("T,top,E,F,D", [(4, 2, 16, 2240, 1536), (5, 4, 7, 24, 40), (8, 2, 2, 200, 72), (16, 1, 3, 136, 520), (16, 4, 40, 64, 64), (17, 4, 6, 48, 56), (64, 1, 64, 32, 8)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_rows_that_share_an_expert_have_the_bits_of_rows_alone(K, T, top, E, F, D, mode):
+    # a wave's 64 rows and more, experts that all rows and that none chose, a slot without an expert (from E on: left as it is), padding tokens
+    g = torch.Generator(device=DEV).manual_seed(T * top + E)
+    h = torch.randn(T, D, device=DEV, generator=g).bfloat16()
+    gate_up = torch.randn(E, 2 * F, D, device=DEV, generator=g).mul(D ** -0.5).bfloat16()
+    down = torch.randn(E, D, F, device=DEV, generator=g).mul(F ** -0.5).bfloat16()
+    which = torch.stack([torch.randperm(E + 1, device=DEV, generator=g)[:top] for _ in range(T)]).int()
+    wt = torch.rand(T, top, device=DEV, generator=g)
+    live = torch.randint(0, 3, (T,), device=DEV, generator=g).int()
+    live[-1] = 5
+    slabs = lambda t: t.reshape(top, -1, D)
+    alone = torch.cat([slabs(K.moe_experts(h[t:t + 1], gate_up, down, which[t:t + 1], wt[t:t + 1], 0.7, 1.702, grouped=False, mode=mode)) for t in range(T)], 1)
+    got = slabs(K.moe_experts(h, gate_up, down, which, wt, 0.7, 1.702, grouped=False, mode=mode))
+    padded = slabs(K.moe_experts(h, gate_up, down, which, wt, 0.7, 1.702, grouped=False, mode=mode, live=live))
+    there = (which < E).t()                       # a slot without an expert is not written
+    assert torch.equal(got[there], alone[there])
+    keep = there & (live > 0)
+    assert torch.equal(padded[keep], alone[keep])
+    if 3 < T and T * top <= 64:
+        assert float(padded[:, live == 0].abs().sum()) == 0
+    # sorted by expert: what padding tokens would read and write is left out, the others' rows keep their bits
+    sort = [slabs(K.moe_experts(h, gate_up, down, which, wt, 0.7, 1.702, grouped=True, mode=mode, live=x)) for x in (None, live)]
+    assert torch.equal(sort[1][keep], sort[0][keep]) and (T * top > min(64, 2 * E) or float(sort[1][:, live == 0].abs().sum()) == 0)
+
+
 def test_moe_experts_of_operands_beyond_the_grouped_products_reach(K):
     # activations that span 2^31 bytes and more, and an expert of as many
     g = torch.Generator(device=DEV).manual_seed(1)
