@@ -371,11 +371,11 @@ __device__ __forceinline__ void moe_place(const MoeArgs& a, int t, int& m, int& 
 }
 #endif
 
-template <int MB, int NB, bool UP>
-__global__ __launch_bounds__(256, ts_share(MB, NB)) void moe_grouped_kernel(const MoeArgs a) {
+template <int MB, int NB, bool UP, int SHARE = ts_share(MB, NB), int BUFS = ts_buffers(MB, NB)>
+__global__ __launch_bounds__(256, SHARE) void moe_grouped_kernel(const MoeArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  typedef TileStream<MB, NB> TS;
+  typedef TileStream<MB, NB, 1, false, BUFS> TS;
   TS ts(smem);
   constexpr int TM = 64 * MB, TN = 64 * NB, COLS = UP ? TN / 2 : TN;
   const int K = UP ? a.D : a.F, tiles = moe_scalar(a.tiles + 2 * a.tiles_cap) * a.n_tiles;
@@ -463,16 +463,17 @@ __global__ __launch_bounds__(256, ts_share(MB, NB)) void moe_grouped_kernel(cons
 #endif
 }
 
-template <int MB, int NB, bool UP>
+template <int MB, int NB, bool UP, int SHARE = ts_share(MB, NB), int BUFS = ts_buffers(MB, NB)>
 static int moe_launch(MoeArgs a, hipStream_t stream) {
-  static const hipError_t room = hipFuncSetAttribute((const void*)&moe_grouped_kernel<MB, NB, UP>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, ts_lds_bytes(MB, NB));
+  constexpr int bytes = ts_stage_bytes(MB, NB) * BUFS;
+  static const hipError_t room = hipFuncSetAttribute((const void*)&moe_grouped_kernel<MB, NB, UP, SHARE, BUFS>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   PICO_REQUIRE(room == hipSuccess, "pico_moe_experts_grouped: %s", hipGetErrorString(room));
   const int cols = UP ? 32 * NB : 64 * NB, n = UP ? a.F : a.D;
   a.n_tiles = (n + cols - 1) / cols;
   const long long tiles = (long long)a.tiles_cap * a.n_tiles;
   PICO_REQUIRE(tiles < (1LL << 30), "pico_moe_experts_grouped: sizes beyond one launch");
-  moe_grouped_kernel<MB, NB, UP><<<ts_grid(tiles, 256 * ts_share(MB, NB)), 256, ts_lds_bytes(MB, NB), stream>>>(a);
+  moe_grouped_kernel<MB, NB, UP, SHARE, BUFS><<<ts_grid(tiles, 256 * SHARE), 256, bytes, stream>>>(a);
   return 0;
 }
 
@@ -498,9 +499,28 @@ static double moe_live(double rows, int E, int bm) {           // tiles that are
   return tiles;
 }
 
+// The second product where its tiles of 128 or 192 columns are a single round: its rows are read as they lie and its ends are stores alone, so a unit is
+// better left to one workgroup with three or four stages on their way (the first product's activations hide behind the other workgroup of a
+// unit: 2,754 rows 84 us, with one 86).  0: no; else the blocks of 64 columns, by the number of stages: microseconds as two workgroups of 192 columns / one
+// of 256, two stages on their way / of 192, three / of 128, four: 16 experts of 2,240 x 1,536, 1,400 rows 46 / 41 / 36 / 34, 2,754 47 / 44 / 39 / 50 (two
+// rounds), 4,096 61 / 47 / 60 / 52 (two rounds of both); of 4,480 x 1,536 89 / 78 / 68 / 58, 92 / 77 / 69 / 97, 112 / 80 / 114 / 98.  If some experts are chosen more
+// than others half a tile an expert is empty, which may be more tiles than rows at random make: the round is to hold either.
+extern "C" int pico_moe_down_round(long long rows, int E, int D) {
+  const double live = ceil(fmax(moe_live((double)rows, E, 128), rows / 128.0 + 0.5 * E));
+  for (int nb = 2; nb <= 3; nb++)
+    if (live * ((D + 64 * nb - 1) / (64 * nb)) <= 256) return nb;
+  return 0;
+}
+
 template <bool UP>
 static int moe_product(int bm, int E, const MoeArgs& a, hipStream_t stream) {
-  const double live = moe_live((double)a.T * a.top, E, bm);
+  const long long rows = (long long)a.T * a.top;
+  if (!UP && bm == 128) {
+    const int round = pico_moe_down_round(rows, E, a.D);
+    if (round == 2) return moe_launch<2, 2, false, 1, 5>(a, stream);
+    if (round == 3) return moe_launch<2, 3, false, 1, 4>(a, stream);
+  }
+  const double live = moe_live((double)rows, E, bm);
   double cost[2];
   for (int i = 0; i < 2; i++) {
     const MoeTile& t = moe_tiles[bm == 128][i];
