@@ -302,9 +302,11 @@ __global__ __launch_bounds__(128, 3) void gemm_f32_stream_kernel(const float* A,
 }
 
 // The same sums over 32 rows: the operands are taken apart once a workgroup, on their way from memory through registers to LDS,
-// where a stage of 32 k lies as three planes of bfloat16 rows (64 bytes, their sixteen-byte chunks xor-swizzled by the row: reads of
-// eight rows and writes of two meet every bank once).  Four waves (2 x 2) of 32 x 32 NW outputs.  A stage's numbers are asked for
-// AHEAD stages ahead, lie in registers, and are taken apart under the products of the stage in front.
+// where a stage of 32 k lies as three planes of bfloat16 rows of 64 bytes, their sixteen-byte chunks xor-swizzled by a quarter of the
+// row: LDS serves sixteen lanes of a read or write at a time, and sixteen rows of one chunk, or four rows whole, so meet every bank
+// once (swizzled by half of the row, which is right for eight lanes, two lanes met in each bank: 300 rows of 17,920 x 1,536 148 us and
+// so 143, 100 rows 84 and 78).  Four waves (2 x 2) of 32 x 32 NW outputs.  A stage's numbers are asked for AHEAD stages ahead, lie in
+// registers, and are taken apart under the products of the stage in front.
 constexpr int fp_plane(int NW) { return (64 + 64 * NW) * BK * 2; }
 // Rows may start anywhere: a load of four to registers needs no more alignment than one.  (Through gemm_f32_kernel, where every wave takes its
 // operands apart by itself, 64 such rows of 32,000 x 1,024 95 us and so 64, 320 of 17,920 x 1,536 262 and 145.)  EVEN: whole fours; else
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(256, NW == 1 && AHEAD == 2 ? 3 : 2) void gemm_f32_p
   off[0] = (uint32_t)(prow * lda) * 4;
 #pragma unroll
   for (int j = 1; j < PIECES; j++) off[j] = (uint32_t)((prow + 64 * (j - 1)) * ldw) * 4;
-  char* put_at = smem + prow * 64 + ((chunk ^ ((prow >> 1) & 3)) << 4);
+  char* put_at = smem + prow * 64 + ((chunk ^ ((prow >> 2) & 3)) << 4);
   f32x4 raw[AHEAD][PIECES][2];
   auto ask = [&](int set, int k0) {
     const uint32_t k = (uint32_t)(k0 + 8 * chunk) * 4, end = (uint32_t)K * 4;
@@ -359,7 +361,7 @@ __global__ __launch_bounds__(256, NW == 1 && AHEAD == 2 ? 3 : 2) void gemm_f32_p
       *reinterpret_cast<s3_u32x4*>(dst + 2 * PLANE) = s.l;
     }
   };
-  const int sw = (l >> 1) & 3;
+  const int sw = (l >> 2) & 3;
   const char* ap = smem + (32 * wm + l) * 64;
   const char* wp = smem + (TM + 32 * NW * wn + l) * 64;
   auto read = [&](const char* p, int b, int g) {
