@@ -169,6 +169,22 @@ def test_layer_norm_with_a_scaled_sum_in_front(dtype, T, H, slabs, scaled):
     close(kernels.add_layernorm(flat, None, w.to(DEV), b.to(DEV), 1e-5, torch.float32), b.double()[None], "float32")
 
 
+@pytest.mark.parametrize("H", [4, 252, 256, 260, 1536, 4092, 4096, 4100, 15360])
+@pytest.mark.parametrize("slabs,scaled", [(0, False), (1, True), (3, False)])
+def test_layer_norm_of_rows_up_to_and_beyond_a_group_of_four_a_thread(H, slabs, scaled):
+    # a thread's entries of a row: none for some, four for all (4,096), several; the float32 sums over H entries of a workgroup of
+    # tens of threads in a row lose no more than 64 roundings of the largest, 64 x 2^-24 = 4e-6 of it, below what `close` allows
+    from pico_vllm_amd.ops import kernels
+    g = torch.Generator().manual_seed(H + slabs)
+    resid, delta = torch.randn(3, H, generator=g) * 2 - 0.5, torch.randn(max(slabs, 1), 3, H, generator=g)
+    w, b, s = 1 + 0.3 * torch.randn(H, generator=g), 0.2 * torch.randn(H, generator=g), 0.5 + torch.rand(H, generator=g)
+    x = resid.double() + ((s.double() if scaled else 1.0) * delta.double().sum(0) if slabs else 0.0)
+    r, d = resid.to(DEV), None if not slabs else delta.to(DEV) if slabs > 1 else delta[0].to(DEV)
+    got = kernels.add_layernorm(r, d, w.to(DEV), b.to(DEV), 1e-5, torch.float32, None, s.to(DEV) if scaled else None)
+    close(got, P.layer_norm(x, w.double(), b.double(), 1e-5), "float32")
+    close(r, x, "float32")
+
+
 def test_pair_rows_in_portions_with_the_previous_token_in_the_state():
     from pico_vllm_amd.ops import kernels
     big = {"buckets": 13, "mul_prev": 40000, "mul_cur": 70001}
