@@ -269,22 +269,38 @@ extern "C" int pico_add_rmsnorm2(float* resid, const void* delta, int delta_dtyp
 }
 
 // resid[t] += delta[t] without a norm (for an arrangement that ends on an add)
-template <typename TD>
-__global__ void residual_add_kernel(float* __restrict__ resid, const TD* __restrict__ delta, size_t n) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) resid[i] += load_f32(delta + i);
+// V entries a thread: four where the addresses allow it, the last thread what is left.  Memory bounds it: 2,048 rows of 1,536 with a
+// bfloat16 addend 7.5 us with one, 6.3 with four (31 MB, 5.0 TB/s).
+template <typename TD, int V>
+__global__ __launch_bounds__(256) void residual_add_kernel(float* __restrict__ resid, const TD* __restrict__ delta, size_t n) {
+  size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
+  if (V == 4 && i + 4 <= n) {
+    float4 x = *reinterpret_cast<const float4*>(resid + i);
+    const float4 d = load4_f32(delta + i);
+    x.x += d.x; x.y += d.y; x.z += d.z; x.w += d.w;
+    *reinterpret_cast<float4*>(resid + i) = x;
+    return;
+  }
+  for (; i < n; i++) {
+    resid[i] += load_f32(delta + i);
+    if (V == 1) break;
+  }
 }
 
 extern "C" int pico_residual_add(float* resid, const void* delta, int delta_dtype, long long n, hipStream_t stream) {
   PICO_REQUIRE(n >= 0, "pico_residual_add: bad size");
   if (n == 0) return 0;
-  const unsigned blocks = (unsigned)((n + 255) / 256);
-  if (delta_dtype == PICO_DTYPE_F32)
-    residual_add_kernel<float><<<blocks, 256, 0, stream>>>(resid, (const float*)delta, (size_t)n);
-  else if (delta_dtype == PICO_DTYPE_BF16)
-    residual_add_kernel<bf16_t><<<blocks, 256, 0, stream>>>(resid, (const bf16_t*)delta, (size_t)n);
-  else
-    PICO_REQUIRE(false, "pico_residual_add: unknown dtype %d", delta_dtype);
+  const bool four = ((uintptr_t)resid | (uintptr_t)delta) % 16 == 0;
+  const unsigned blocks = (unsigned)(((four ? (n + 3) / 4 : n) + 255) / 256);
+#define LAUNCH(TD)                                                                                          \
+  do {                                                                                                      \
+    if (four) residual_add_kernel<TD, 4><<<blocks, 256, 0, stream>>>(resid, (const TD*)delta, (size_t)n);   \
+    else residual_add_kernel<TD, 1><<<blocks, 256, 0, stream>>>(resid, (const TD*)delta, (size_t)n);        \
+  } while (0)
+  if (delta_dtype == PICO_DTYPE_F32) LAUNCH(float);
+  else if (delta_dtype == PICO_DTYPE_BF16) LAUNCH(bf16_t);
+  else PICO_REQUIRE(false, "pico_residual_add: unknown dtype %d", delta_dtype);
+#undef LAUNCH
   PICO_LAUNCH_CHECK();
   return 0;
 }

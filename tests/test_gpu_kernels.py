@@ -71,6 +71,19 @@ def test_residual_add(K, dtype):
     assert torch.equal(r.cpu(), resid + delta.float())
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1027])
+def test_residual_add_in_fours_and_what_is_left(K, dtype, n):
+    # whole fours, what they leave, and rows that start on no sixteen bytes: one float32 sum an entry, so exact
+    resid, delta = torch.randn(n + 3) * 3, torch.randn(n + 3).to(dtype)
+    for at in (0, 1):
+        r, d = resid.clone().to(DEV), delta.to(DEV)
+        K.residual_add(r[at:at + n], d[at:at + n])
+        want = resid.clone()
+        want[at:at + n] += delta[at:at + n].float()
+        assert torch.equal(r.cpu(), want)
+
+
 def test_rmsnorm_eps_is_inside_the_root(K):
     x = torch.full((1, 64), 1e-4)
     out = K.add_rmsnorm(x.to(DEV), None, torch.ones(64, device=DEV), 1e-2, torch.float32)
