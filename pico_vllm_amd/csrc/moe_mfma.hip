@@ -85,14 +85,16 @@ __device__ __forceinline__ MoeRows moe_rows_of(const int* __restrict__ experts, 
   int e = lane < R ? experts[lane] : -1;
   const bool there = lane >= R || !live || live[lane / top] > 0;
   if (e >= E || !there) e = -1;
-  bool leads = e >= 0;
-  for (int i = 0; i < R - 1; i++) leads = leads && !(i < lane && __builtin_amdgcn_readlane(e, i) == e);
-  unsigned long long leaders = __ballot(leads);
-  m.base = 0; m.tile = blockIdx.x;
+  m.base = 0; m.tile = blockIdx.x; m.expert = -1; m.mask = 0;
   if (blockIdx.y == 0) m.dead = __ballot(!there);
-  for (int j = blockIdx.y; j > 0; j--) leaders &= leaders - 1;
-  m.expert = leaders ? __builtin_amdgcn_readlane(e, __builtin_ctzll(leaders)) : -1;
-  m.mask = __ballot(e == m.expert);
+  // (the walk is the same for all lanes: a lane is read while all of them are on, as what one holds that is off is nobody's promise)
+  unsigned long long left = __ballot(e >= 0);
+  for (int j = blockIdx.y; left; j--) {
+    const int next = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
+    const unsigned long long same = __ballot(e == next);
+    if (j == 0) { m.expert = next; m.mask = same; break; }
+    left &= ~same;
+  }
   return m;
 }
 // the next M rows of the mask; the last one again where there are fewer

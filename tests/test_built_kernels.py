@@ -37,3 +37,23 @@ def test_staged_keys_travel_in_registers(tmp_path, dk, dv):
     path = library.build_library(f"pico_attnb_k{dk}_v{dv}", library.ATTN_BIAS_SOURCES, (f"-DPICO_DK={dk}", f"-DPICO_DV={dv}"))
     found = {n: b for n, b in kernels_of(path, tmp_path).items() if "attn_bias_staged_kernel" in n}
     assert len(found) == 1 and set(found.values()) == {0}, found
+
+
+def test_rows_of_an_expert_are_looked_up_with_all_lanes_on(tmp_path):
+    # a lane that is off while another reads it need not hold its value: an expert would be missed, or taken twice
+    out = str(tmp_path / "moe_mfma.s")
+    subprocess.run([library._hipcc(), *library.HIP_FLAGS, "-I", library.CSRC, "--cuda-device-only", "-S",
+                    os.path.join(library.CSRC, "moe_mfma.hip"), "-o", out], check=True, capture_output=True)
+    with open(out) as f:
+        bodies = re.findall(r"^_Z\d+moe_(?:up|down)_rows_kernelILb1E\S*:(.*?)s_endpgm", f.read(), re.M | re.S)
+    assert len(bodies) == 2
+    for body in bodies:
+        reads = 0
+        for block in re.split(r"^\.LBB\S+:|s_or_b64 exec, exec", body, flags=re.M):       # (where lanes come back on, or another way joins)
+            saved = False
+            for line in block.splitlines():
+                saved = saved or "saveexec" in line
+                if "v_readlane" in line:
+                    reads += 1
+                    assert not saved, block
+        assert reads
