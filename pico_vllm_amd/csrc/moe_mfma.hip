@@ -239,7 +239,9 @@ extern "C" int pico_moe_experts_rows(const void* h, int ldh, const void* gate_up
   const long long R = (long long)T * top;
   const bool shared = T > 3 && R <= MOE_LANES;
   const unsigned out_up = moe_up_out(shared), up = (F + out_up - 1) / out_up, dn = (D + 4 * MOE_DOWN_OUT - 1) / (4 * MOE_DOWN_OUT);
-  PICO_REQUIRE(R < (1ll << 30) && up <= 65535 && dn <= 65535, "pico_moe_experts_rows: sizes beyond the grid");
+  // (tiles lie along the grid's first index where rows share: 2^32 threads there, 65,535 workgroups along the second)
+  const unsigned most = shared ? 1u << 24 : 65536u;
+  PICO_REQUIRE(R < (1ll << 30) && up < most && dn < most, "pico_moe_experts_rows: sizes beyond the grid");
   const unsigned met = (unsigned)min(R, (long long)E);
   const dim3 g1 = shared ? dim3(up, met) : dim3((unsigned)R, up), g2 = shared ? dim3(dn, met) : dim3((unsigned)R, dn);
 #define LAUNCH(SHARED)                                                                                                                             \

@@ -194,6 +194,17 @@ def test_rows_that_share_an_expert_have_the_bits_of_rows_alone(K, T, top, E, F, 
     assert torch.equal(sort[1][keep], sort[0][keep]) and (T * top > min(64, 2 * E) or float(sort[1][:, live == 0].abs().sum()) == 0)
 
 
+@pytest.mark.parametrize("F", [524280, 524288, 1048560])
+def test_experts_of_few_rows_and_very_many_columns(K, F):
+    # 65,535 tiles of sixteen columns a row alone, of eight where rows share an expert, and beyond
+    g = torch.Generator(device=DEV).manual_seed(F)
+    h, gate_up = torch.randn(4, 8, device=DEV, generator=g).bfloat16(), torch.randn(1, 2 * F, 8, device=DEV, generator=g).bfloat16()
+    down, wt = torch.randn(1, 8, F, device=DEV, generator=g).mul(F ** -0.5).bfloat16(), torch.rand(4, 1, device=DEV, generator=g)
+    which = torch.zeros(4, 1, dtype=torch.int32, device=DEV)
+    alone = torch.cat([K.moe_experts(h[t:t + 1], gate_up, down, which[t:t + 1], wt[t:t + 1], 0.7, 1.702, grouped=False) for t in range(4)])
+    assert torch.equal(K.moe_experts(h, gate_up, down, which, wt, 0.7, 1.702, grouped=False), alone)
+
+
 def test_moe_experts_of_operands_beyond_the_grouped_products_reach(K):
     # activations that span 2^31 bytes and more, and an expert of as many
     g = torch.Generator(device=DEV).manual_seed(1)
