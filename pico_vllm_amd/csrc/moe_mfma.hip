@@ -1,7 +1,7 @@
 // A routed feed-forward in bfloat16: the kernels that serve it.
 //
-// Few rows (a row is one (token, chosen expert) pair; single tokens and small steps): every expert that they chose streams its
-// matrices once, 16 bytes a lane, sixteen lanes to an output element.
+// Few rows (a row is one (token, chosen expert) pair; single tokens and small steps): the matrices of the experts that they chose are
+// streamed, once an expert where enough rows meet in one, 16 bytes a lane, sixteen lanes to an output element.
 //
 // More rows: they are sorted by expert on the device (nothing comes back to the host), every expert's rows padded to whole
 // tiles, and two grouped products run on the matrix cores, tiles as tile_stream.h has them:
@@ -58,17 +58,13 @@ __device__ __forceinline__ float row16_sum(float v) {
 // Few rows, SHARED: an expert's matrices are streamed once for all of its rows.  Workgroup (tile, j) looks the rows' experts over and takes the j-th
 // that occurs for the first time; the last workgroups of a grid for as many experts as rows find none.  Tiles run along the grid's first
 // index, so that an expert's workgroups go to all dies at one time.  The sums of a row are made as if it were alone.  Bound by the matrices' stream.
-// Otherwise a row streams its expert's matrices itself, rows along the grid's first index: up to three tokens, whose experts seldom meet, and
-// more rows than a wave has lanes.  Microseconds for both halves, every row for itself / shared / shared with a quarter of the tokens
-// padding, by tokens: two of 16 experts of 2,240 x 1,536 at 2 18.2 / 18.6, 4 31.4 / 29.6 / 26.6, 8 53.0 / 47.4 / 42.5; of 4,480 x 1,536 4 55.2 / 51.8 / 42.5,
-// 8 99.8 / 82.0 / 68.4; four of 32 of 4,736 x 3,584 1 78.1 / 80.3, 2 132 / 135, 4 235 / 226 / 195, of 2,368 x 3,584 2 77.1 / 81.1, 4 125.9 / 124.6 / 100.4.
-// live (or null): the context of every token; a token without one pads a recorded step: where rows share, its rows choose no expert
-// and come out as zeros.
+// Otherwise a row streams its expert's matrices itself, rows along the grid's first index (pico_moe_rows_shared says which).
+// live (or null): the context of every token; a token without one pads a recorded step: its rows choose no expert and come out as zeros.
 // ---------------------------------------------------------------------------
 #define MOE_LANES 64
 struct MoeRows {
   unsigned long long mask;                            // row numbers: base + the bits' numbers
-  unsigned long long dead;                            // rows of padding, of whoever is the first of a tile
+  unsigned long long dead;                            // rows of padding, of whoever is to write their zeros
   int base, expert, tile;                             // expert < 0: nothing to do
 };
 template <bool SHARED>
@@ -78,7 +74,9 @@ __device__ __forceinline__ MoeRows moe_rows_of(const int* __restrict__ experts, 
   if (!SHARED) {
     m.base = blockIdx.x; m.tile = blockIdx.y; m.mask = 1;
     const int e = experts[m.base];
-    m.expert = e < E ? e : -1;
+    const bool there = !live || live[m.base / top] > 0;
+    m.dead = there ? 0 : 1;
+    m.expert = there && e < E ? e : -1;
     return m;
   }
   const int lane = threadIdx.x & 63;
@@ -212,7 +210,7 @@ __global__ __launch_bounds__(256) void moe_down_rows_kernel(const bf16_t* __rest
   const int n = (m.tile * 4 + (threadIdx.x >> 6)) * MOE_DOWN_OUT;
   if (n >= D) return;
   for (; m.dead; m.dead &= m.dead - 1) {
-    const int r = __builtin_ctzll(m.dead), i = threadIdx.x & 63;
+    const int r = m.base + __builtin_ctzll(m.dead), i = threadIdx.x & 63;
     if (i < MOE_DOWN_OUT && n + i < D) out[((size_t)(r % top) * T + r / top) * D + n + i] = 0.f;
   }
   if (m.expert < 0) return;
@@ -227,9 +225,23 @@ __global__ __launch_bounds__(256) void moe_down_rows_kernel(const bf16_t* __rest
   }
 }
 
+// Whether rows share their experts' streams: from four tokens on, as far as a wave has lanes, where T tokens that choose at random name an
+// expert again so often that 80 MB less are asked for, of matrices (what is met at all) that the dies' L2s do not hold anyway.  To look
+// the experts over takes 0.5 us a launch, and the rows of one workgroup more registers.  Microseconds for both halves, every row for itself / shared, by
+// tokens x chosen experts: 16 experts of 2,240 x 1,536 4x2 31.9 / 30.3 (29 MB again), 8x2 54.9 / 53.1 (114 MB); of 4,480 x 1,536 4x2 56.9 / 55.4 (57 MB),
+// 8x2 100.1 / 85.4 (227); 32 of 2,368 x 3,584 4x2 66.0 / 69.2 (37), 8x1 72.8 / 76.2 (42), 4x4 122.1 / 115.4 (140); 64 of 704 x 2,048 16x1 29.2 / 34.3 (15); eight
+// of 704 x 2,048 16x1 26.0 / 27.4 (77); four of 1,536 x 1,536 8x2 35.3 / 25.2 (170); two of 512 x 1,024 8x2 11.4 / 16.2 (44, of 6 MB).  Over 321
+// such sizes 10 % less in the mean than every row for itself, and at most 1.5 % more.
+extern "C" int pico_moe_rows_shared(int T, int top, int E, int F, int D) {
+  const double rows = (double)T * top, bytes = 6.0 * F * D;
+  const double met = E * (1.0 - pow(1.0 - fmin(1.0, (double)top / E), T));
+  return T > 3 && rows <= MOE_LANES && (rows - met) * bytes >= 80e6 && met * bytes >= 32e6;
+}
+
+// share: 1 or 0, or as pico_moe_rows_shared says (-1)
 extern "C" int pico_moe_experts_rows(const void* h, int ldh, const void* gate_up, const void* down, const int* experts,
                                      const float* weights, const int* live, void* y, float* out, int T, int top, int E, int F, int D,
-                                     float limit, float alpha, int mode, hipStream_t stream) {
+                                     float limit, float alpha, int mode, int share, hipStream_t stream) {
   PICO_REQUIRE(T >= 0 && top > 0 && E > 0 && F > 0 && D > 0 && ldh >= D, "pico_moe_experts_rows: bad sizes");
   PICO_REQUIRE(mode >= 0 && mode <= 2, "pico_moe_experts_rows: unknown mode %d", mode);
   PICO_REQUIRE(F % 8 == 0 && D % 8 == 0 && ldh % 8 == 0, "pico_moe_experts_rows: sizes must be multiples of 8");
@@ -237,7 +249,8 @@ extern "C" int pico_moe_experts_rows(const void* h, int ldh, const void* gate_up
                "pico_moe_experts_rows: operands must start on 16 bytes");
   if (T == 0) return 0;
   const long long R = (long long)T * top;
-  const bool shared = T > 3 && R <= MOE_LANES;
+  PICO_REQUIRE(share <= 0 || R <= MOE_LANES, "pico_moe_experts_rows: up to %d rows share", MOE_LANES);
+  const bool shared = share < 0 ? pico_moe_rows_shared(T, top, E, F, D) : share;
   const unsigned out_up = moe_up_out(shared), up = (F + out_up - 1) / out_up, dn = (D + 4 * MOE_DOWN_OUT - 1) / (4 * MOE_DOWN_OUT);
   // (tiles lie along the grid's first index where rows share: 2^32 threads there, 65,535 workgroups along the second)
   const unsigned most = shared ? 1u << 24 : 65536u;

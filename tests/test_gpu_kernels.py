@@ -202,7 +202,30 @@ def test_experts_of_few_rows_and_very_many_columns(K, F):
     down, wt = torch.randn(1, 8, F, device=DEV, generator=g).mul(F ** -0.5).bfloat16(), torch.rand(4, 1, device=DEV, generator=g)
     which = torch.zeros(4, 1, dtype=torch.int32, device=DEV)
     alone = torch.cat([K.moe_experts(h[t:t + 1], gate_up, down, which[t:t + 1], wt[t:t + 1], 0.7, 1.702, grouped=False) for t in range(4)])
-    assert torch.equal(K.moe_experts(h, gate_up, down, which, wt, 0.7, 1.702, grouped=False), alone)
+    for share in (None, True):
+        assert torch.equal(K.moe_experts(h, gate_up, down, which, wt, 0.7, 1.702, grouped=False, share=share), alone)
+
+
+@pytest.mark.parametrize("T,top,E,F,D", [(1, 1, 1, 8, 8), (3, 4, 4, 40, 24), (4, 2, 16, 2240, 1536), (5, 4, 7, 24, 40), (8, 2, 2, 200, 72), (16, 1, 3, 136, 520),
+                                         (16, 4, 40, 64, 64), (64, 1, 64, 32, 8), (8, 2, 16, 2240, 1536)])
+@pytest.mark.parametrize("share", [True, False])
+def test_rows_that_share_a_stream_and_rows_that_do_not(K, T, top, E, F, D, share):
+    # either way the bits of rows one by one, a slot without an expert left as it is, padding tokens zero; as the rule has it in the last
+    g = torch.Generator(device=DEV).manual_seed(T * top + F)
+    h = torch.randn(T, D, device=DEV, generator=g).bfloat16()
+    gate_up = torch.randn(E, 2 * F, D, device=DEV, generator=g).mul(D ** -0.5).bfloat16()
+    down = torch.randn(E, D, F, device=DEV, generator=g).mul(F ** -0.5).bfloat16()
+    which = torch.stack([torch.randperm(E + 1, device=DEV, generator=g)[:top] for _ in range(T)]).int()
+    wt = torch.rand(T, top, device=DEV, generator=g)
+    live = torch.randint(0, 2, (T,), device=DEV, generator=g).int()
+    run = lambda rows, **more: K.moe_experts(h[rows], gate_up, down, which[rows], wt[rows], 7.0, 1.702, grouped=False, **more).reshape(top, -1, D)
+    alone = torch.cat([run(slice(t, t + 1), share=False) for t in range(T)], 1)
+    there = (which < E).t()
+    every = slice(None)
+    assert torch.equal(run(every, share=share)[there], alone[there])
+    padded = run(every, share=share, live=live)
+    assert torch.equal(padded[there & (live > 0)], alone[there & (live > 0)]) and float(padded[:, live == 0].abs().sum()) == 0
+    assert torch.equal(run(every)[there], alone[there])
 
 
 def test_moe_experts_of_operands_beyond_the_grouped_products_reach(K):
