@@ -2159,3 +2159,31 @@ def test_bias_attention_of_single_tokens_in_as_many_pieces_as_keys(nq, nkv, dk, 
         assert torch.equal(got, want)
     else:
         assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -9)        # an ulp of bfloat16 where the last bit of the sum differs
+
+
+@pytest.mark.parametrize("nq,nkv,dk,dv,more", [(12, 2, 64, 64, {}), (20, 1, 32, 16, {"window": 30}), (5, 5, 32, 32, {"chunk": 16, "sink": True})])
+@pytest.mark.parametrize("B", [1, 7, 8, 63, 64, 65, 130])
+def test_a_block_of_columns_finds_its_sequence(nq, nkv, dk, dv, more, B):
+    # one by one and 64 at a time: sequences without tokens, of one, of a block and of several; each has the bits it has alone
+    from pico_vllm_amd.ops.attention_bias_fast import FastBiasAttention
+    fast = FastBiasAttention(nq, nkv, dk, dv, dk ** -0.5, **more)
+    g = torch.Generator().manual_seed(B + nq)
+    lens = [int(n) for n in torch.tensor([0, 1, 1, 1, 2, 16, 40])[torch.randint(0, 7, (B,), generator=g)]]
+    lens[-1] = 3
+    ends = [n + int(p) for n, p in zip(lens, torch.randint(0, 200, (B,), generator=g))]
+    per = -(-max(ends) // 16)
+    dev = torch.Generator(device=DEV).manual_seed(B)
+    kc, vc = (torch.randn(B * per, nkv, *s, device=DEV, generator=dev).bfloat16() for s in ((16, dk), (dv, 16)))
+    bt = torch.randperm(B * per, generator=g).int().reshape(B, per).to(DEV)
+    q = torch.randn(sum(lens), nq * dk, device=DEV, generator=dev).bfloat16()
+    at = [sum(lens[:i]) for i in range(B + 1)]
+    cu = torch.tensor(at, dtype=torch.int32, device=DEV)
+    pos = torch.cat([torch.arange(e - n, e) for n, e in zip(lens, ends)]).int().to(DEV)
+    for chunks in (1, 3):
+        got = fast.run(q, kc, vc, bt, cu, pos, B, split=True, chunks=chunks)
+        for b in range(B):
+            if lens[b] and (B < 60 or b % 9 == 0 or b > B - 4):
+                own = slice(at[b], at[b + 1])
+                alone = fast.run(q[own], kc, vc, bt[b:b + 1], torch.tensor([0, lens[b]], dtype=torch.int32, device=DEV), pos[own].contiguous(), 1,
+                                 split=True, chunks=chunks)
+                assert torch.equal(got[own], alone), (b, lens[b])
