@@ -14,7 +14,6 @@ from .kernels import KernelError, _check, _check_cache2, _ptr, _stream
 c_float = ctypes.c_float
 MAX_CHUNKS = 32
 PROMPT_KERNEL_FROM = 64      # tokens of a step from which the prompt kernel serves it (a tile of its workgroups)
-DECODE_TILE_KEYS, DECODE_TILE_PAIRS = 136, 128      # single tokens that it serves too: keys, and (sequence, kv head) pairs, at most
 
 
 def supported(key_dim: int, value_dim: int) -> bool:
@@ -62,9 +61,9 @@ class FastBiasAttention:
     def chunks(self, num_tokens: int, num_seqs: int, max_keys: int = 0) -> int:
         """Into how many pieces every block's keys are cut, each piece a workgroup of its own (their parts are put
         together by a second launch): as many as bring the step to two workgroups a compute unit, at most MAX_CHUNKS.
-        Decided from the step's size alone; a piece is a whole number of 128 keys, found on the device from the block's
-        own range of keys.  max_keys (of steps of single tokens: what the engine's contexts may reach): no more pieces than those have, the
-        others would be empty."""
+        Decided from the step's size, and in steps of single tokens from max_keys, the most keys that the engine's requests or the window allow:
+        no more pieces than those have, the others would be empty (4,096 keys, the engine's default, have MAX_CHUNKS).  A piece is a whole
+        number of 128 keys, found on the device from the block's own range of keys."""
         if not self.split(num_tokens):
             return 1
         R = self.nq // self.nkv
@@ -74,12 +73,12 @@ class FastBiasAttention:
 
     def prompt_shape(self, ctx) -> int:
         """The shape of the prompt kernel's workgroups for this step (0: that kernel does not serve it).  A step of single tokens leaves it 63 of
-        a tile's 64 queries idle; it serves those of few (sequence, kv head) pairs and contexts of a tile or two, where it needs no second
-        launch.  Microseconds a step by the prompt kernel / by blocks of columns, four layers: 64 sequences of 2 kv heads, 560 keys 799 / 720, 250 keys
-        713 / 701, 120 keys 687 / 688, 32 keys 661 / 672; of 4 kv heads 2,156 / 1,955, 32 keys 1,867 / 1,863."""
-        if self.tuned is None or ctx.num_tokens < PROMPT_KERNEL_FROM:
-            return 0
-        if ctx.all_decode and (ctx.max_context > DECODE_TILE_KEYS or ctx.num_seqs * self.nkv > DECODE_TILE_PAIRS):
+        a tile's 64 queries idle and reads every key once a query head: it serves those whose kv heads have one query head each.
+        Microseconds of a launch by the prompt kernel / by blocks of columns, uncut, at 16, 96, 256, 600 keys: 64 sequences of 12 heads over 2
+        8.5 / 7.3, 14.5 / 8.2, 23.8 / 10.7 (in three pieces and merged 10.4, 11.3, 13.1); 256 of them 23.8 / 9.0, 37.0 / 10.7, 66 / 18.4; 64 of 28 over 4
+        14.7 / 7.5, 24.7 / 9.2, 43.0 / 13.7; 64 of 24 over 12 12.9 / 9.5, 21.5 / 12.2, 38.4 / 23.4, 77 / 49; 256 of 16 over 8, of 64 entries, 19.5 / 14.5,
+        29.2 / 17.9, 46 / 32, 97 / 64; of 16 over 16 19.3 / 22.6, 29.8 / 28.7, 55 / 58, 112 / 113; 64 of those 7.3 / 8.3, 10.4 / 10.6, 20.0 / 19.5, 33.4 / 35.0."""
+        if self.tuned is None or ctx.num_tokens < PROMPT_KERNEL_FROM or (ctx.all_decode and self.nq > self.nkv):
             return 0
         key = ("bias_attention_shape", self.nq, self.nkv, self.dk, self.window)
         if key not in ctx.shared:

@@ -101,6 +101,29 @@ def mixed_steps(reqs, page, seed, max_live=3, tail=12):
     return steps, roundup(peak)
 
 
+def decode_together(model_dir, dtype, reqs, tail, page, graph, max_seq_len):
+    """The last ``tail`` tokens of all requests in steps of a token each, recorded or not; {(id, position): logits row}."""
+    from pico_vllm_amd.engine.batch import SeqStep
+    from pico_vllm_amd.engine.step import ModelRunner
+    from pico_vllm_amd.parts.model import load_model
+    longest = max(len(t) for t in reqs.values())
+    run = ModelRunner(load_model(model_dir, dtype), page, len(reqs) * -(-longest // page), len(reqs), 256, max_seq_len, use_graph=graph,
+                      max_graph_batch=len(reqs))
+    rows = {}
+    for rid, toks in reqs.items():
+        assert run.manager.add_request(rid) and run.manager.grow(rid, len(toks))
+        first = [SeqStep(rid, toks[:len(toks) - tail])]
+        run.step(first)
+        run.advance(first)
+    for k in range(tail):
+        seqs = [SeqStep(rid, toks[len(toks) - tail + k:][:1], [0]) for rid, toks in reqs.items()]
+        out = run.step(seqs).double().cpu().numpy()
+        run.advance(seqs)
+        rows.update({(rid, len(toks) - tail + k): out[i] for i, (rid, toks) in enumerate(reqs.items())})
+    assert bool(run._graphs) == graph
+    return rows
+
+
 def step_ctx(new_lens, prefix_lens, slots):
     """The few arrays of a step that kernels with a state read."""
     pos, seq, cu = [], [], [0]

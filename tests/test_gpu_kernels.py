@@ -2187,3 +2187,43 @@ def test_a_block_of_columns_finds_its_sequence(nq, nkv, dk, dv, more, B):
                 alone = fast.run(q[own], kc, vc, bt[b:b + 1], torch.tensor([0, lens[b]], dtype=torch.int32, device=DEV), pos[own].contiguous(), 1,
                                  split=True, chunks=chunks)
                 assert torch.equal(got[own], alone), (b, lens[b])
+
+
+@pytest.mark.parametrize("nq,nkv,d,more", [(12, 2, 64, {"temp_coef": 0.4, "temp_every": 64, "slope_span": 8.0}), (4, 4, 64, {"window": 100}),
+                                           (6, 2, 32, {"sink": True, "gated": True, "gate_heads": True, "out_scale": 0.7})])
+@pytest.mark.parametrize("B,most", [(33, 4096), (64, 4096), (64, 130), (100, 4096), (257, 600)])
+def test_single_tokens_of_many_requests_as_a_step_has_them(nq, nkv, d, more, B, most):
+    # by whatever kernel and in as many pieces as the step's plan says, against the equations in 64 bits
+    from types import SimpleNamespace
+    from pico_vllm_amd.ops.attention_bias_fast import FastBiasAttention
+    fast = FastBiasAttention(nq, nkv, d, d, d ** -0.5, **more)
+    g = torch.Generator().manual_seed(B + nq)
+    contexts = [1 + int(n) for n in torch.randint(0, min(most, 400), (B,), generator=g)]
+    per, R = -(-max(contexts) // 16), nq // nkv
+    bt = torch.randperm(B * per, generator=g).int().reshape(B, per)
+    kc, vc = torch.randn(B * per, nkv, 16, d, generator=g).bfloat16(), torch.randn(B * per, nkv, d, 16, generator=g).bfloat16()
+    q, gate, sinks = torch.randn(B, nq * d, generator=g).bfloat16(), torch.randn(B, nq, generator=g).bfloat16(), torch.randn(nq, generator=g)
+    extra = fast.sink
+    if extra:
+        fast.sinks = sinks.to(DEV)
+    cu, lens = torch.arange(B + 1, dtype=torch.int32), torch.tensor(contexts, dtype=torch.int32)
+    ctx = SimpleNamespace(num_tokens=B, num_seqs=B, all_decode=True, max_context=most, host={"cu_seqlens": cu.numpy(), "context_lens": lens.numpy()}, shared={},
+                          cu_seqlens=cu.to(DEV), positions=lens.to(DEV) - 1, context_lens=lens.to(DEV))
+    got = fast(q.to(DEV), SimpleNamespace(k=kc.to(DEV), v=vc.to(DEV)), bt.to(DEV), ctx, gate=gate.to(DEV) if extra else None).double().cpu().view(B, nq, d)
+    for b, n in enumerate(contexts):
+        pages = bt[b, :-(-n // 16)].long()
+        k = kc[pages].double().permute(1, 0, 2, 3).reshape(nkv, -1, d)[:, :n].repeat_interleave(R, 0)
+        v = vc[pages].double().permute(1, 0, 3, 2).reshape(nkv, -1, d)[:, :n].repeat_interleave(R, 0)
+        s = (k @ q[b].double().view(nq, d, 1))[..., 0] * d ** -0.5
+        if "temp_every" in more:
+            s = s * (1 + 0.4 * math.log(n // 64 + 1))
+            s = s - 2.0 ** (-8.0 * torch.arange(1, nq + 1).double() / nq)[:, None] * (n - 1 - torch.arange(n).double())
+        if fast.window:
+            s[:, :max(0, n - fast.window)] = -math.inf
+        p = torch.exp(s - s.amax(1, keepdim=True))
+        total = p.sum(1, keepdim=True) + (torch.exp(sinks.double()[:, None] - s.amax(1, keepdim=True)) if extra else 0)
+        want = ((p / total)[:, None] @ v)[:, 0]
+        if extra:
+            want = want * torch.sigmoid(gate[b].double())[:, None] * 0.7
+        # probabilities and the output are rounded to bfloat16, and scores are float32 sums of products of bfloat16 numbers
+        assert float((got[b] - want).abs().max()) <= 2.0 ** -7 * float(v.abs().max()), (b, n)

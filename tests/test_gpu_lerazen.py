@@ -506,6 +506,17 @@ def test_batch_equals_each_alone(dtype):
     compare(name, dtype, a, reqs)
 
 
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("name", ["d", "e"])
+def test_many_requests_decode_together(name, graph):
+    """As many single tokens as a tile of the prompt kernel's queries holds, and more; keys and values of one size and not."""
+    from replay_util import decode_together
+    reqs = requests(name, [8 + 41 * i % 150 for i in range(70)], seed=12)
+    rows = decode_together(model_dir(name), "bfloat16", reqs, 3, 16, graph, 300)
+    some = {r: reqs[r] for r in [list(reqs)[i] for i in (0, 1, 3, 7, 18, 31, 38, 69)]}
+    compare(name, "bfloat16", {k: v for k, v in rows.items() if k[0] in some}, some)
+
+
 def draw_config(seed):
     """A configuration drawn at random: sizes, head counts, windows, constants and the order of layers all differ from
     the hand-picked ones, and include the values that make mechanisms vanish (a window of 1, one expert, one head)."""

@@ -11,7 +11,7 @@ import torch
 import plain_tubusun as P
 from begasun_configs import write_model
 from gpu_util import DEV
-from replay_util import DT, F, MixerAlone, alone, close, cut, mixed_steps, replay, requests, rounded, roundup, row_errors, step_ctx
+from replay_util import DT, F, MixerAlone, alone, close, cut, decode_together, mixed_steps, replay, requests, rounded, roundup, row_errors, step_ctx
 from tubusun_configs import CONFIGS, config, dense, left, model_dir, moe, pair, right, tensors_of
 
 pytestmark = pytest.mark.gpu
@@ -701,6 +701,17 @@ def test_long_decoding(dtype):
     reqs = requests(CONFIGS["b"]["vocab"], [330], seed=6)
     rows, _ = replay(model_dir("b"), dtype, alone(reqs, lambda t: cut(t, [30], tail=300)), roundup(330), PAGE["b"])
     compare("b", dtype, rows, reqs)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("many", [40, 70])
+def test_many_requests_decode_together(many, graph):
+    """More single tokens than the search for a block's sequence takes one by one, as many as a tile of the prompt kernel's queries and
+    more (recorded: padded to 64 and 128), contexts of less and more than a piece of keys in a step."""
+    reqs = requests(CONFIGS["b"]["vocab"], [8 + 41 * i % 150 for i in range(many)], seed=12)
+    rows = decode_together(model_dir("b"), "bfloat16", reqs, 3, PAGE["b"], graph, 400)
+    some = {f"r{i}": reqs[f"r{i}"] for i in (0, 1, 3, 7, 18, 31, 38, many - 1)}
+    compare("b", "bfloat16", {k: v for k, v in rows.items() if k[0] in some}, some)
 
 
 def test_sharp_attention_at_a_windows_edge_in_every_pass_of_a_loop():
