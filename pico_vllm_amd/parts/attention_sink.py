@@ -98,6 +98,15 @@ class SinkAttention(OpenMixer):
         kernels.attn_bias_plain(q, cache.k, cache.v, bt, ctx.positions, ctx.token_seq, self.nq, self.nkv, self.dk, self.dv, self.scale,
                                 self.window, gate=gate, gate_heads=True, sinks=self.sinks, out=out, out_scale=self.out_scale)
 
+    def _beside_pieces(self, ctx: StepContext) -> int:
+        """Into how many pieces the keys are cut beside a ``LightningAttention`` (0: not served beside one).  The launch that puts pieces together
+        is shared, so there are two where one would do: contexts that have no more (the second is empty), or so many blocks that the chip is
+        full.  Microseconds a step, four layers, in launches of their own with one piece / so, 1.5B: 64 requests at 32 tokens 816 / 742, 96 at 32
+        and 1,000 947 / 881 and 1,049 / 936, 256 1,210 / 1,133 and 1,405 / 1,314; 7B, 256 2,997 / 2,848 and 3,400 / 3,242; by the prompt kernel / so, a query
+        head a kv head, 64 requests 877 / 788 and 1,142 / 1,036, 256 1,334 / 1,273 and 2,354 / 2,254."""
+        split, pieces, _ = self.fast.plan(ctx)
+        return max(2, pieces) if split and pieces <= kernels.PAIR_MAX_PIECES else 0
+
     def core_beside(self, other: OpenMixer, y: torch.Tensor, col: int, other_col: int, ctx: StepContext, cache, other_cache,
                     out: torch.Tensor, other_out: torch.Tensor) -> bool:
         """This core and a ``LightningAttention``'s in shared launches, for a step of single tokens in bfloat16: norm, rotation
@@ -106,10 +115,9 @@ class SinkAttention(OpenMixer):
         if not (isinstance(other, LightningAttention) and self.fast is not None and cache.k.dtype == torch.bfloat16 and ctx.all_decode
                 and ctx.num_tokens == ctx.num_seqs and other.heads * other.dv <= kernels.PAIR_MAX_ROW):
             return False
-        split, pieces, _ = self.fast.plan(ctx)
-        if not split or pieces > kernels.PAIR_MAX_PIECES:
+        pieces = self._beside_pieces(ctx)
+        if not pieces:
             return False
-        pieces = max(2, pieces)             # (short contexts too: their second piece is empty, the launches saved are worth more)
         table = self.angles.table(ctx) if self.angles is not None else None
         q, o = kernels.pair_open(
             y, (col, col + self.k_col, col + self.v_col, self.nq, self.nkv, self.dk, self.dv), self.norm_eps, table,

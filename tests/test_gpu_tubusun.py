@@ -704,10 +704,11 @@ def test_long_decoding(dtype):
 
 
 @pytest.mark.parametrize("graph", [False, True])
-@pytest.mark.parametrize("many", [40, 70])
+@pytest.mark.parametrize("many", [40, 70, 260])
 def test_many_requests_decode_together(many, graph):
     """More single tokens than the search for a block's sequence takes one by one, as many as a tile of the prompt kernel's queries and
-    more (recorded: padded to 64 and 128), contexts of less and more than a piece of keys in a step."""
+    more (recorded: padded to 64, 128 and 512), and so many that the chip is full without cutting their keys; contexts of less and more than
+    a piece of keys in a step."""
     reqs = requests(CONFIGS["b"]["vocab"], [8 + 41 * i % 150 for i in range(many)], seed=12)
     rows = decode_together(model_dir("b"), "bfloat16", reqs, 3, PAGE["b"], graph, 400)
     some = {f"r{i}": reqs[f"r{i}"] for i in (0, 1, 3, 7, 18, 31, 38, many - 1)}
