@@ -116,12 +116,12 @@ def test_swiglu_of_float32_rows(K, T, I):
 
 @pytest.mark.parametrize("counts,D,F_", [([0, 1, 63, 64, 65], 72, 40), ([129, 0, 48, 2], 64, 264), ([1, 127, 128, 129, 700], 136, 1000),
                                          ([0, 1100], 328, 200), ([0, 0, 5], 1536, 8),
-                                         ([200, 1, 129], 8328, 72), ([128, 300], 5440, 328), ([129] * 16, 1280, 456), ([129] * 16, 1920, 72)])
+                                         ([200, 1, 129], 8328, 72), ([128, 300], 5440, 328), ([129] * 16, 1152, 456), ([129] * 16, 1728, 72)])
 @pytest.mark.parametrize("mode", [0, 1, 2])
 def test_moe_grouped(K, counts, D, F_, mode):
     # experts with rows up to, at and behind the edges of tiles of 64 and 128 rows and of strips of tiles, columns and k that
     # end inside a tile and a stage; a row with a stride; a number that has no matrices; a second product of one round of tiles of 128
-    # columns, of 192, and of more; choices so uneven that what was taken for one round is 320 tiles for 256 workgroups
+    # columns, of 192, and of more; choices so uneven that what was taken for one round is 288 tiles for 256 workgroups
     g = torch.Generator().manual_seed(D + F_)
     E, which = len(counts), [e for e, n in enumerate(counts) for _ in range(n)] + [len(counts)]
     R = len(which)
